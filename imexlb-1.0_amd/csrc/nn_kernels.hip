@@ -3,11 +3,9 @@
 // (C ABI in include/imexlb_nn.h).  Tensors are FP32, NCHW, in device memory
 // the caller owns; every launch goes to the given stream.
 //
-// conv3x3 (padding 1, stride 1): one block computes a 16x16 tile of pixels
-// for 16 output channels; input channels stream through LDS 8 at a time
-// (the tile with its one-pixel halo) together with the matching weights,
-// stored [ci][tap][co] so one 128-bit LDS read feeds four FMAs.  The
-// data gradient is the same kernel on the flipped, transposed weights; the
+// conv3x3 (padding 1, stride 1) in FP32 runs on the matrix cores (k_conv3
+// below); the data gradient is the same kernel on the flipped, transposed
+// weights; the
 // weight gradient gives each thread one (co, ci) pair and its 9 taps over a
 // tile, summed over the batch, then added to dW with atomics.
 //
@@ -36,66 +34,172 @@
 
 namespace imexlb_nn {
 
-constexpr int TS = 16;   // pixel tile edge
-constexpr int COB = 16;  // output channels per block
-constexpr int CIB = 8;   // input channels per LDS chunk
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
-__global__ __launch_bounds__(256) void k_conv3(const float *__restrict__ in, const float *__restrict__ w,
-                                               const float *__restrict__ bias, float *__restrict__ out, int N,
-                                               int CI, int CO, int H, int W, int relu)
+// Order of the blocks of a 1D grid: blocks are dealt to the 8 XCDs in turn,
+// so this gives each XCD one contiguous run of tiles (blocks that share
+// input or weights share an L2).
+__device__ __forceinline__ uint32_t xcd_run(uint32_t b, uint32_t nb)
 {
-    __shared__ float tin[CIB][TS + 2][TS + 2];
-    __shared__ float4 tw[CIB][9][COB / 4];
-    const int tx = threadIdx.x % TS, ty = threadIdx.x / TS;
-    const int x0 = blockIdx.x * TS, y0 = blockIdx.y * TS;
-    const int ncob = (CO + COB - 1) / COB;
-    const int n = blockIdx.z / ncob, co0 = (blockIdx.z % ncob) * COB;
-    float acc[COB];
+    const uint32_t per = nb / 8u;
+    return b < per * 8u ? (b % 8u) * per + b / 8u : b;
+}
+
+// 3x3 convolution, padding 1, as a matrix product over k = 9 ci + tap with
+// v_mfma_f32_32x32x2_f32.  That instruction adds its two products to the
+// accumulator one after the other, each as an FMA (compared bit for bit with
+// a chain of FMAs, subnormals included), so taking k in order gives exactly
+// the sum of a loop over input channels and taps.
+//
+// Bound by the matrix cores (157 TFLOP/s; a plain FMA loop has half).  A
+// block computes 4 MT (32 / TC) rows x TC columns of pixels for 32 NT output
+// channels, a wave MT groups of 32 pixels; rows of the product are output
+// channels and columns pixels, so a half-wave stores 32 consecutive pixels.
+// Eight input channels at a time (the tile with its halo, and the weights
+// [k][co]) go through two LDS buffers in turn, fetched into registers while
+// the previous eight are multiplied; every operand is one 32-bit LDS read
+// without bank conflicts, read one product ahead.  The loads take no branch:
+// one per load made each wait for the one before (80 against 115 TFLOP/s).
+// Against one thread per pixel with 16 accumulators and FMAs: 96 -> 32
+// channels, 8 x 128 x 512: 603 to 248 us (117 TFLOP/s); 64 -> 64, 8 x 64 x
+// 256: 221 to 93 us; 256 -> 256, 8 x 16 x 64: 475 to 99 us; 256 -> 256, 1 x
+// 16 x 64: 429 to 59 us.
+constexpr int CIB = 8;  // input channels per LDS chunk
+
+template <int MT, int NT, int TC>
+__global__ __launch_bounds__(256) void k_conv3(const float *__restrict__ in, const float *__restrict__ w,
+                                               const float *__restrict__ bias, float *__restrict__ out, int CI, int CO,
+                                               int H, int W, int relu, uint32_t ntx, uint32_t nty, uint32_t ncob)
+{
+    constexpr int GR = 32 / TC;  // rows of a 32-pixel group
+    constexpr int TR = 4 * MT * GR, IR = TR + 2, IC = TC + 2, BN = 32 * NT, WS = BN + 1;
+    constexpr int NP = (IR * IC + 63) / 64, NW = (BN + 2) / 3;
+    __shared__ float s_in[2][CIB * IR * IC];
+    __shared__ float s_w[2][CIB * 9 * WS];
+    __shared__ float s_b[BN];
+    const int tid = int(threadIdx.x), lane = tid % 64, wave = tid / 64;
+    const int m = lane % 32, hk = lane / 32;  // operand row / column and which of the two k
+    uint32_t blk = xcd_run(blockIdx.x, gridDim.x);
+    const int co0 = int(blk % ncob) * BN;
+    blk /= ncob;
+    const int x0 = int(blk % ntx) * TC;
+    blk /= ntx;
+    const int y0 = int(blk % nty) * TR;
+    const int64_t n = blk / nty, HW = int64_t(H) * W;
+    const float *const img = in + n * CI * HW;
+
+    // Staging.  A wave brings two channels of the tile with its halo; a
+    // lane's pixels are the same for every channel.  Weights lie k = 9 ci +
+    // tap fastest: a thread brings one k of every third output channel.
+    // Loads have no branches: lanes with nothing to load read a valid
+    // neighbour and drop it.
+    int64_t ioff[NP];
+    bool iok[NP];
 #pragma unroll
-    for (int k = 0; k < COB; ++k) acc[k] = 0.0f;
-    for (int ci0 = 0; ci0 < CI; ci0 += CIB) {
-        for (int i = threadIdx.x; i < CIB * (TS + 2) * (TS + 2); i += 256) {
-            const int c = i / ((TS + 2) * (TS + 2)), r = i % ((TS + 2) * (TS + 2));
-            const int yy = y0 + r / (TS + 2) - 1, xx = x0 + r % (TS + 2) - 1;
-            float v = 0.0f;
-            if (ci0 + c < CI && yy >= 0 && yy < H && xx >= 0 && xx < W)
-                v = in[((int64_t(n) * CI + ci0 + c) * H + yy) * W + xx];
-            tin[c][r / (TS + 2)][r % (TS + 2)] = v;
-        }
-        float *twf = &tw[0][0][0].x;
-        for (int i = threadIdx.x; i < CIB * 9 * COB; i += 256) {
-            const int c = i / (9 * COB), r = i % (9 * COB), k = r / COB, co = r % COB;
-            float v = 0.0f;
-            if (co0 + co < CO && ci0 + c < CI) v = w[(int64_t(co0 + co) * CI + ci0 + c) * 9 + k];
-            twf[i] = v;
-        }
-        __syncthreads();
-#pragma unroll 2
-        for (int c = 0; c < CIB; ++c)
-#pragma unroll
-            for (int k = 0; k < 9; ++k) {
-                const float v = tin[c][ty + k / 3][tx + k % 3];
-#pragma unroll
-                for (int q = 0; q < COB / 4; ++q) {
-                    const float4 wv = tw[c][k][q];
-                    acc[4 * q + 0] = fma_(wv.x, v, acc[4 * q + 0]);
-                    acc[4 * q + 1] = fma_(wv.y, v, acc[4 * q + 1]);
-                    acc[4 * q + 2] = fma_(wv.z, v, acc[4 * q + 2]);
-                    acc[4 * q + 3] = fma_(wv.w, v, acc[4 * q + 3]);
-                }
-            }
-        __syncthreads();
+    for (int i = 0; i < NP; ++i) {
+        const int p = lane + 64 * i, yy = y0 + p / IC - 1, xx = x0 + p % IC - 1;
+        iok[i] = p < IR * IC && yy >= 0 && yy < H && xx >= 0 && xx < W;
+        ioff[i] = iok[i] ? int64_t(yy) * W + xx : int64_t(y0) * W + x0;
     }
-    const int x = x0 + tx, y = y0 + ty;
-    if (x >= W || y >= H) return;
+    const int ch = __builtin_amdgcn_readfirstlane(wave * 2);
+    const int wk = tid % 72, wc = tid / 72;  // threads from 216 on repeat others' loads
+    const int wlast = (min(co0 + BN, CO) - 1 - co0 - min(wc, CO - 1 - co0)) / 3;
+    const float *const wrow = w + int64_t(co0 + min(wc, CO - 1 - co0)) * CI * 9;
+    float xin[2][NP], xw[NW];
+    auto load = [&](int c0) {
 #pragma unroll
-    for (int co = 0; co < COB; ++co) {
-        if (co0 + co >= CO) break;
-        float v = acc[co] + (bias ? bias[co0 + co] : 0.0f);
-        if (relu) v = v > 0.0f ? v : 0.0f;
-        out[((int64_t(n) * CO + co0 + co) * H + y) * W + x] = v;
+        for (int c = 0; c < 2; ++c) {
+            const float *const pl = img + int64_t(min(c0 + ch + c, CI - 1)) * HW;
+#pragma unroll
+            for (int i = 0; i < NP; ++i) xin[c][i] = pl[ioff[i]];
+        }
+        const float *const p = wrow + min(int64_t(c0) * 9 + wk, int64_t(CI) * 9 - 1);
+#pragma unroll
+        for (int i = 0; i < NW; ++i) xw[i] = p[int64_t(min(i, wlast)) * 27 * CI];
+    };
+    auto store = [&](int buf, int c0) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const bool live = c0 + ch + c < CI;
+#pragma unroll
+            for (int i = 0; i < NP; ++i)
+                if (lane + 64 * i < IR * IC)
+                    s_in[buf][(ch + c) * (IR * IC) + lane + 64 * i] = live && iok[i] ? xin[c][i] : 0.0f;
+        }
+        if (tid < 216) {
+            const bool live = wk < (CI - c0) * 9;
+#pragma unroll
+            for (int i = 0; i < NW; ++i)
+                if (wc + 3 * i < BN) s_w[buf][wk * WS + wc + 3 * i] = live ? xw[i] : 0.0f;
+        }
+    };
+    // where the lane's pixel operand of product i of a channel pair lies:
+    // its k is 2 i + hk, i.e. channel k / 9 of the pair and tap k % 9
+    int bo[9];
+    const int px = (wave * MT * GR + m / TC) * IC + m % TC;
+#pragma unroll
+    for (int i = 0; i < 9; ++i) {
+        const int k0 = 2 * i, k1 = 2 * i + 1;
+        const int o0 = k0 / 9 * (IR * IC) + k0 % 9 / 3 * IC + k0 % 3;
+        const int o1 = k1 / 9 * (IR * IC) + k1 % 9 / 3 * IC + k1 % 3;
+        bo[i] = px + (hk ? o1 : o0);
+    }
+    const int ao = hk * WS + m;
+    f32x16 acc[NT][MT] = {};
+    if (tid < BN) s_b[tid] = bias && co0 + tid < CO ? bias[co0 + tid] : 0.0f;
+
+    load(0);
+    store(0, 0);
+    __syncthreads();
+    int buf = 0;
+    for (int c0 = 0; c0 < CI; c0 += CIB) {
+        const bool more = c0 + CIB < CI;
+        if (more) load(c0 + CIB);
+        const float *const si = s_in[buf], *const sw = s_w[buf];
+        // operands of product k2 of the chunk (k = 2 k2 + hk), read one
+        // product ahead of their use
+        float a[2][NT], b[2][MT];
+        auto fetch = [&](int k2, float(&fa)[NT], float(&fb)[MT]) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) fa[t] = sw[ao + 2 * k2 * WS + 32 * t];
+#pragma unroll
+            for (int t = 0; t < MT; ++t) fb[t] = si[bo[k2 % 9] + k2 / 9 * 2 * (IR * IC) + t * GR * IC];
+        };
+        fetch(0, a[0], b[0]);
+#pragma unroll
+        for (int k2 = 0; k2 < CIB * 9 / 2; ++k2) {
+            if (k2 + 1 < CIB * 9 / 2) fetch(k2 + 1, a[(k2 + 1) % 2], b[(k2 + 1) % 2]);
+#pragma unroll
+            for (int s = 0; s < NT; ++s)
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+                    acc[s][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[k2 % 2][s], b[k2 % 2][t], acc[s][t], 0, 0, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, NT + MT, 0);  // the reads of the next product,
+            __builtin_amdgcn_sched_group_barrier(0x008, NT * MT, 0);  // then the products of this one
+        }
+        if (more) store(buf ^ 1, c0 + CIB);  // its last readers passed the barrier before this chunk
+        __syncthreads();
+        buf ^= 1;
+    }
+    // lane holds D[channel 8 (j/4) + 4 hk + j%4][pixel m] of each 32x32 tile
+    const int x = x0 + m % TC;
+    if (x >= W) return;
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        const int y = y0 + (wave * MT + t) * GR + m / TC;
+        if (y >= H) continue;
+        float *const o = out + (n * CO + co0) * HW + int64_t(y) * W + x;
+#pragma unroll
+        for (int s = 0; s < NT; ++s)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const int co = 32 * s + 8 * (j / 4) + 4 * hk + j % 4;
+                float v = acc[s][t][j] + s_b[co];
+                if (relu) v = v > 0.0f ? v : 0.0f;
+                if (co0 + co < CO) o[co * HW] = v;
+            }
     }
 }
 
@@ -108,6 +212,7 @@ __global__ void k_flip(const float *__restrict__ w, float *__restrict__ wt, int 
     wt[(int64_t(ci) * CO + co) * 9 + (8 - k)] = w[i];
 }
 
+constexpr int TS = 16;   // pixel tile edge of the weight gradient
 constexpr int WCO = 16, WCI = 16;
 
 // partial == nullptr: add to dw with atomics; otherwise write the block's
@@ -292,7 +397,6 @@ __global__ void k_adam(float *__restrict__ w, const float *__restrict__ g, float
 
 // ------------------------------------------------------------ BF16 inference
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // FP32 -> bf16, round to nearest even (NaN kept quiet)
 __device__ __forceinline__ uint16_t to_bf16(float f)
@@ -471,8 +575,23 @@ int imexlb_nn_conv3x3(const float *in, const float *w, const float *bias, float 
                       int W, int relu, void *stream)
 {
     if (!in || !w || !out || N <= 0 || CI <= 0 || CO <= 0 || H <= 0 || W <= 0) return -1;
-    const dim3 grid(unsigned((W + TS - 1) / TS), unsigned((H + TS - 1) / TS), unsigned(N * ((CO + COB - 1) / COB)));
-    NN_LAUNCH(k_conv3, grid, dim3(256), 0, (hipStream_t)stream, in, w, bias, out, N, CI, CO, H, W, relu);
+    // The largest tile that still gives every CU two blocks (its operands are
+    // reused most: 8 x 32 pixels for 64 channels 118 TFLOP/s on the deep
+    // layers of a batch of 8, for 32 channels 100); a batch of one gets the
+    // smallest.  Rows of at most 16 pixels take the 16-column tile.
+    const auto run = [&](auto kernel, int rows, int cols, int bn, bool always) {
+        const int64_t tx = (int64_t(W) + cols - 1) / cols, ty = (int64_t(H) + rows - 1) / rows, tc = (CO + bn - 1) / bn;
+        const int64_t nb = tx * ty * tc * N;
+        if (nb < 512 && !always) return 1;  // too few blocks to give every CU two: smaller tiles
+        if (nb > 0x7fffffff) return -2;
+        hipLaunchKernelGGL(kernel, dim3(unsigned(nb)), dim3(256), 0, (hipStream_t)stream, in, w, bias, out, CI, CO, H,
+                           W, relu, uint32_t(tx), uint32_t(ty), uint32_t(tc));
+        return hipGetLastError() == hipSuccess ? 0 : -2;
+    };
+    if (W <= 16) return run(k_conv3<1, 1, 16>, 8, 16, 32, true);
+    int rc = CO > 32 ? run(k_conv3<2, 2, 32>, 8, 32, 64, false) : 1;
+    if (rc > 0) rc = run(k_conv3<2, 1, 32>, 8, 32, 32, false);
+    return rc <= 0 ? rc : run(k_conv3<1, 1, 32>, 4, 32, 32, true);
 }
 
 int imexlb_nn_flip_weights(const float *w, float *wt, int CI, int CO, void *stream)

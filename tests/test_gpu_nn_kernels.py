@@ -1,0 +1,79 @@
+"""The warm-start network's kernels at the edges of their tiles: remainders of
+rows, columns and channels, the smallest and largest tile forms, non-finite
+values.  References are the operations' definitions in 64 bits on the CPU."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _call(name, *args):
+    import torch
+    from imexlb._lib import lib
+    rc = getattr(lib(), "imexlb_nn_" + name)(
+        *[C.c_void_p(a.data_ptr()) if isinstance(a, torch.Tensor) else a for a in args], None)
+    assert rc == 0, (name, rc)
+
+
+def _conv64(x, w, b=None):
+    N, ci, H, W = x.shape
+    xp = np.zeros((N, ci, H + 2, W + 2))
+    xp[:, :, 1:-1, 1:-1] = x
+    y = np.zeros((N, w.shape[0], H, W))
+    for k in range(9):
+        y += np.einsum("oc,nchw->nohw", w[:, :, k // 3, k % 3], xp[:, :, k // 3:k // 3 + H, k % 3:k % 3 + W])
+    return y if b is None else y + b[None, :, None, None]
+
+
+# tile forms: 16-column (W <= 16), 4 x 32 (few blocks), 8 x 32 (512 blocks and more)
+SHAPES = [(1, 1, 1, 1, 1), (2, 3, 5, 9, 7), (1, 15, 31, 8, 16), (1, 16, 32, 4, 17), (2, 17, 33, 5, 33),
+          (1, 33, 65, 3, 32), (3, 8, 3, 2, 70), (1, 100, 4, 1, 40), (20, 5, 31, 61, 97), (9, 17, 65, 121, 64)]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("relu", [0, 1])
+def test_conv3x3_at_tile_edges(shape, relu):
+    import torch
+    N, ci, co, H, W = shape
+    print(f"[nn] conv3x3 {shape} relu {relu}", flush=True)
+    rng = np.random.default_rng(5)
+    x = rng.normal(0, 1, (N, ci, H, W)).astype(np.float32)
+    w = rng.normal(0, 1, (co, ci, 3, 3)).astype(np.float32)
+    b = rng.normal(0, 1, co).astype(np.float32)
+    xd, wd, bd = (torch.tensor(v, device="cuda") for v in (x, w, b))
+    out = torch.full((N, co, H, W), 7.0, device="cuda")
+    _call("conv3x3", xd, wd, bd, out, N, ci, co, H, W, relu)
+    ref = _conv64(x.astype(np.float64), w.astype(np.float64), b.astype(np.float64))
+    size = _conv64(np.abs(x).astype(np.float64), np.abs(w).astype(np.float64), np.abs(b).astype(np.float64))
+    # FP32 summation bound: one rounding of 2^-24 per term, and a few more
+    tol = (9 * ci + 8) * 2.0 ** -24 * size
+    err = np.abs(out.cpu().numpy() - (np.maximum(ref, 0) if relu else ref))
+    assert (err <= tol).all(), (err / tol).max()
+
+
+@pytest.mark.parametrize("shape", [(1, 5, 6, 20, 40), (1, 18, 34, 9, 16), (4, 3, 7, 200, 180)])
+def test_conv3x3_non_finite_values(shape):
+    """Infinities, NaN and overflowing products behave as in FP32."""
+    import torch
+    N, ci, co, H, W = shape
+    print(f"[nn] conv3x3 non-finite {shape}", flush=True)
+    rng = np.random.default_rng(6)
+    x = rng.normal(0, 1, (N, ci, H, W)).astype(np.float32)
+    w = rng.integers(-3, 4, (co, ci, 3, 3)).astype(np.float32)
+    x[0, 0, 3, 3], x[0, 1, H - 1, W - 1], x[0, 2, 5, 9] = np.nan, np.inf, -np.inf
+    x[N - 1, 1, 7, 12] = 3.4e38
+    out = torch.empty((N, co, H, W), device="cuda")
+    _call("conv3x3", torch.tensor(x, device="cuda"), torch.tensor(w, device="cuda"), None, out, N, ci, co, H, W, 0)
+    with np.errstate(all="ignore"):
+        ref = _conv64(x.astype(np.float64), w.astype(np.float64))
+        small = np.where(np.isfinite(x) & (np.abs(x) < 1e30), x, 0).astype(np.float64)
+        ref32 = ref.astype(np.float32)
+    got = out.cpu().numpy()
+    big = np.abs(ref) > 1e30  # products of 3.4e38: overflow depends on the order of the sum
+    assert (np.isnan(got) == np.isnan(ref))[~big].all()
+    assert np.array_equal(got[np.isinf(ref)], ref32[np.isinf(ref)])
+    plain = np.isfinite(ref) & ~big
+    size = _conv64(np.abs(small), np.abs(w).astype(np.float64))
+    assert (np.abs(got[plain] - ref[plain]) <= ((9 * ci + 8) * 2.0 ** -24 * size)[plain]).all()
