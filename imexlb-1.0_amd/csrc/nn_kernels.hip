@@ -5,9 +5,9 @@
 //
 // conv3x3 (padding 1, stride 1) in FP32 runs on the matrix cores (k_conv3
 // below); the data gradient is the same kernel on the flipped, transposed
-// weights; the
-// weight gradient gives each thread one (co, ci) pair and its 9 taps over a
-// tile, summed over the batch, then added to dW with atomics.
+// weights; the weight gradient (k_conv3_dw) sums a 16x16 tile of pixels over
+// the batch on the matrix cores, and the tiles' sums are added in order or
+// with atomics.
 //
 // Inference in BF16: activations NHWC bf16, weights packed
 // [CI/8][tap][CO][8 ci] bf16, products on the matrix cores
@@ -212,69 +212,167 @@ __global__ void k_flip(const float *__restrict__ w, float *__restrict__ wt, int 
     wt[(int64_t(ci) * CO + co) * 9 + (8 - k)] = w[i];
 }
 
-constexpr int TS = 16;   // pixel tile edge of the weight gradient
-constexpr int WCO = 16, WCI = 16;
+constexpr int TS = 16;  // pixel tile edge of the weight gradient
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// Weight gradient of one 16x16 tile of pixels, summed over the batch: for
+// each tap a matrix product over the pixels (image after image, row after
+// row) of the output gradient's channels and the shifted input's, with
+// v_mfma_f32_16x16x4_f32, which adds its four products in order as FMAs --
+// exactly the sum of a loop over the pixels.
 // partial == nullptr: add to dw with atomics; otherwise write the block's
 // sums to partial[blockIdx.x][co][ci][9] for k_dw_reduce (fixed order).
+//
+// Bound by the matrix cores (157 TFLOP/s).  A block takes 16 GCO output x 16
+// GCI input channels, a wave 16 x 16 of them and all 9 taps; with fewer than
+// four such groups the waves share the taps.  Half a tile (8 rows) of an
+// image goes through LDS at a time, fetched into registers while the
+// previous half is multiplied; 32 x 32 channels take 50 KB, three blocks on a
+// CU.  Against one (co, ci) pair per thread and FMAs: 32 -> 32 channels, 8 x
+// 128 x 512: 351 to 121 us; 96 -> 32: 917 to 281 us (103 TFLOP/s); 256 ->
+// 256, 8 x 16 x 64: 274 to 112 us; 4 -> 32, 8 x 128 x 512: 247 to 67 us.
+template <int GCO, int GCI>
 __global__ __launch_bounds__(256) void k_conv3_dw(const float *__restrict__ in, const float *__restrict__ dout,
                                                   float *__restrict__ dw, int N, int CI, int CO, int H, int W,
                                                   float *__restrict__ partial)
 {
-    __shared__ float tin[WCI][TS + 2][TS + 2];
-    __shared__ float tg[WCO][TS * TS];
-    const int co = threadIdx.x / WCI, ci = threadIdx.x % WCI;
+    constexpr int NTAP = GCO * GCI == 4 ? 9 : GCO * GCI == 2 ? 5 : 3;  // taps per wave
+    constexpr int HR = TS / 2, IC = TS + 2, IP = (HR + 2) * IC, GP = HR * TS;
+    // channel strides of 2 (mod 32): the 16 channels x 2 pixels of a
+    // half-wave read fall in 32 banks
+    constexpr int SI = 226, SG = 162;
+    __shared__ float s_in[GCI * 16 * SI];
+    __shared__ float s_g[GCO * 16 * SG];
+    const int tid = int(threadIdx.x), lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int m = lane % 16, kk = lane / 16;  // operand row / column, pixel of four
     const int ntx = (W + TS - 1) / TS;
-    const int x0 = (blockIdx.x % ntx) * TS, y0 = (blockIdx.x / ntx) * TS;
-    const int nci = (CI + WCI - 1) / WCI;
-    const int co0 = (blockIdx.y / nci) * WCO, ci0 = (blockIdx.y % nci) * WCI;
-    float acc[9];
+    const int x0 = int(blockIdx.x) % ntx * TS, y0 = int(blockIdx.x) / ntx * TS;
+    const int nci = (CI + 16 * GCI - 1) / (16 * GCI);
+    const int co0 = int(blockIdx.y) / nci * (16 * GCO), ci0 = int(blockIdx.y) % nci * (16 * GCI);
+    const int wco = wave % GCO, wci = wave / GCO % GCI, tap0 = wave / (GCO * GCI) * NTAP;
+    const int64_t HW = int64_t(H) * W;
+
+    // Staging: half a tile (8 rows) of one image; a wave brings every fourth
+    // channel.  Channels past the end repeat the last one (their sums are
+    // not stored); pixels outside the image are zero.
+    constexpr int NI = (IP + 63) / 64, NG = GP / 64;
+    float xi[GCI * 4][NI], xg[GCO * 4][NG];
+    bool iok[NI], gok[NG];
+    auto load = [&](int n, int h) {
+        int64_t io[NI], go[NG];
 #pragma unroll
-    for (int k = 0; k < 9; ++k) acc[k] = 0.0f;
-    for (int n = 0; n < N; ++n) {
-        for (int i = threadIdx.x; i < WCI * (TS + 2) * (TS + 2); i += 256) {
-            const int c = i / ((TS + 2) * (TS + 2)), r = i % ((TS + 2) * (TS + 2));
-            const int yy = y0 + r / (TS + 2) - 1, xx = x0 + r % (TS + 2) - 1;
-            float v = 0.0f;
-            if (ci0 + c < CI && yy >= 0 && yy < H && xx >= 0 && xx < W)
-                v = in[((int64_t(n) * CI + ci0 + c) * H + yy) * W + xx];
-            tin[c][r / (TS + 2)][r % (TS + 2)] = v;
+        for (int i = 0; i < NI; ++i) {
+            const int p = lane + 64 * i, yy = y0 + h * HR + p / IC - 1, xx = x0 + p % IC - 1;
+            iok[i] = p < IP && yy >= 0 && yy < H && xx >= 0 && xx < W;
+            io[i] = iok[i] ? int64_t(yy) * W + xx : 0;
         }
-        for (int i = threadIdx.x; i < WCO * TS * TS; i += 256) {
-            const int c = i / (TS * TS), p = i % (TS * TS);
-            const int yy = y0 + p / TS, xx = x0 + p % TS;
-            float v = 0.0f;
-            if (co0 + c < CO && yy < H && xx < W) v = dout[((int64_t(n) * CO + co0 + c) * H + yy) * W + xx];
-            tg[c][p] = v;
-        }
-        __syncthreads();
-        for (int p = 0; p < TS * TS; ++p) {
-            const float g = tg[co][p];
-            const int py = p / TS, px = p % TS;
 #pragma unroll
-            for (int k = 0; k < 9; ++k) acc[k] = fma_(g, tin[ci][py + k / 3][px + k % 3], acc[k]);
+        for (int i = 0; i < NG; ++i) {
+            const int p = lane + 64 * i, yy = y0 + h * HR + p / TS, xx = x0 + p % TS;
+            gok[i] = yy < H && xx < W;
+            go[i] = gok[i] ? int64_t(yy) * W + xx : 0;
         }
-        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < GCI * 4; ++c) {
+            const float *const pl = in + (int64_t(n) * CI + min(ci0 + wave + 4 * c, CI - 1)) * HW;
+#pragma unroll
+            for (int i = 0; i < NI; ++i) xi[c][i] = pl[io[i]];
+        }
+#pragma unroll
+        for (int c = 0; c < GCO * 4; ++c) {
+            const float *const pl = dout + (int64_t(n) * CO + min(co0 + wave + 4 * c, CO - 1)) * HW;
+#pragma unroll
+            for (int i = 0; i < NG; ++i) xg[c][i] = pl[go[i]];
+        }
+    };
+    f32x4 acc[NTAP] = {};
+    int bo[NTAP];  // the tap's offset in the lane's input channel
+#pragma unroll
+    for (int t = 0; t < NTAP; ++t) {
+        const int tap = min(tap0 + t, 8);  // (a wave with fewer taps repeats the last, not stored)
+        bo[t] = (wci * 16 + m) * SI + tap / 3 * IC + tap % 3 + kk;
     }
-    if (co0 + co >= CO || ci0 + ci >= CI) return;
-    const int64_t o = (int64_t(co0 + co) * CI + ci0 + ci) * 9;
-    if (partial) {
-        float *pb = partial + int64_t(blockIdx.x) * CO * CI * 9 + o;
+    const int ao = (wco * 16 + m) * SG + kk;
+    const int halves = y0 + HR < H ? 2 : 1;
+
+    load(0, 0);
+    for (int n = 0, h = 0; n < N;) {
+        __syncthreads();  // the previous part has been multiplied
 #pragma unroll
-        for (int k = 0; k < 9; ++k) pb[k] = acc[k];
-        return;
+        for (int c = 0; c < GCI * 4; ++c)
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+                if (lane + 64 * i < IP) s_in[(wave + 4 * c) * SI + lane + 64 * i] = iok[i] ? xi[c][i] : 0.0f;
+#pragma unroll
+        for (int c = 0; c < GCO * 4; ++c)
+#pragma unroll
+            for (int i = 0; i < NG; ++i) s_g[(wave + 4 * c) * SG + lane + 64 * i] = gok[i] ? xg[c][i] : 0.0f;
+        __syncthreads();
+        const int rows = min(HR, H - y0 - h * HR);
+        if (++h == halves) {
+            h = 0;
+            ++n;
+        }
+        if (n < N) load(n, h);
+        // 4 pixels per product, in pixel order; operands read one product
+        // ahead (past the last row: read, not used)
+        float a[2], b[2][NTAP];
+        a[0] = s_g[ao];
+#pragma unroll
+        for (int t = 0; t < NTAP; ++t) b[0][t] = s_in[bo[t]];
+        for (int r = 0; r < rows; ++r) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int nx = (g + 1) % 2, ro = g == 3 ? r + 1 : r, go = (g + 1) % 4 * 4;
+                a[nx] = s_g[ao + ro * TS + go];
+#pragma unroll
+                for (int t = 0; t < NTAP; ++t) b[nx][t] = s_in[bo[t] + ro * IC + go];
+#pragma unroll
+                for (int t = 0; t < NTAP; ++t)
+                    acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[g % 2], b[g % 2][t], acc[t], 0, 0, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, NTAP + 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, NTAP, 0);
+            }
+        }
     }
+    // lane holds D[co 4 kk + j][ci m]
+    const int ci = ci0 + wci * 16 + m;
+    if (ci >= CI) return;
 #pragma unroll
-    for (int k = 0; k < 9; ++k) atomicAdd(&dw[o + k], acc[k]);
+    for (int j = 0; j < 4; ++j) {
+        const int co = co0 + wco * 16 + 4 * kk + j;
+        if (co >= CO) continue;
+        const int64_t o = (int64_t(co) * CI + ci) * 9;
+        float *const pb = partial ? partial + int64_t(blockIdx.x) * CO * CI * 9 + o : dw + o;
+#pragma unroll
+        for (int t = 0; t < NTAP; ++t) {
+            if (tap0 + t >= 9) continue;
+            if (partial)
+                pb[tap0 + t] = acc[t][j];
+            else
+                atomicAdd(&pb[tap0 + t], acc[t][j]);
+        }
+    }
 }
 
-// dw[i] += sum over tiles b = 0..nb-1 of partial[b][i], in that order
-__global__ void k_dw_reduce(const float *__restrict__ partial, float *__restrict__ dw, int64_t nb, int64_t n)
+// dw[i] += sum over tiles b = 0..nb-1 of partial[b][i], in that order, kRed
+// loads in flight per thread
+constexpr int kRed = 32;
+__global__ __launch_bounds__(64) void k_dw_reduce(const float *__restrict__ partial, float *__restrict__ dw, int64_t nb,
+                                                  int64_t n)
 {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t i = int64_t(blockIdx.x) * 64 + threadIdx.x;
     if (i >= n) return;
     float s = 0.0f;
-    for (int64_t b = 0; b < nb; ++b) s += partial[b * n + i];
+    int64_t b = 0;
+    for (; b + kRed <= nb; b += kRed) {
+        float v[kRed];
+#pragma unroll
+        for (int k = 0; k < kRed; ++k) v[k] = partial[(b + k) * n + i];
+#pragma unroll
+        for (int k = 0; k < kRed; ++k) s += v[k];
+    }
+    for (; b < nb; ++b) s += partial[b * n + i];
     dw[i] += s;
 }
 
@@ -559,6 +657,36 @@ __global__ void k_up2_bf16(const uint4 *__restrict__ in, uint4 *__restrict__ out
 
 inline unsigned blocks(int64_t n) { return unsigned((n + 255) / 256); }
 
+// weight gradient: the tiles' sums to `work` and from there to dw in tile
+// order, or (work == nullptr) to dw with atomics.
+int launch_dw(const float *in, const float *dout, float *dw, float *work, int N, int CI, int CO, int H, int W,
+              hipStream_t s)
+{
+    const int64_t tiles = int64_t((W + TS - 1) / TS) * ((H + TS - 1) / TS), n = int64_t(CO) * CI * 9;
+    // blocks of 32 x 32 channels share their staged pixels most; where they
+    // leave CUs without a block, smaller ones, whose waves share the taps
+    // (64 -> 128, 8 x 32 x 128: 108 us with 128 blocks, 69 us with 256),
+    // and 16 x 16 as the last resort
+    const auto pairs = [&](int gco, int gci) {
+        return int64_t((CO + 16 * gco - 1) / (16 * gco)) * ((CI + 16 * gci - 1) / (16 * gci));
+    };
+    int gco = 1, gci = 1;
+    if (CO > 16 && CI > 16 && tiles * pairs(2, 2) >= 256)
+        gco = gci = 2;
+    else if (CO > 16 && tiles * pairs(2, 1) >= 256)
+        gco = 2;
+    else if (CI > 16 && tiles * pairs(1, 2) >= 256)
+        gci = 2;
+    const dim3 grid(unsigned(tiles), unsigned(pairs(gco, gci)));
+    const auto kernel = gco == 2 ? (gci == 2 ? k_conv3_dw<2, 2> : k_conv3_dw<2, 1>)
+                                 : (gci == 2 ? k_conv3_dw<1, 2> : k_conv3_dw<1, 1>);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, in, dout, dw, N, CI, CO, H, W, work);
+    if (hipGetLastError() != hipSuccess) return -2;
+    if (!work) return 0;
+    hipLaunchKernelGGL(k_dw_reduce, dim3(unsigned((n + 63) / 64)), dim3(64), 0, s, work, dw, tiles, n);
+    return hipGetLastError() == hipSuccess ? 0 : -2;
+}
+
 }  // namespace imexlb_nn
 
 using namespace imexlb_nn;
@@ -604,9 +732,7 @@ int imexlb_nn_conv3x3_dw(const float *in, const float *dout, float *dw, int N, i
                          void *stream)
 {
     if (!in || !dout || !dw || N <= 0 || CI <= 0 || CO <= 0 || H <= 0 || W <= 0) return -1;
-    const dim3 grid(unsigned(((W + TS - 1) / TS) * ((H + TS - 1) / TS)),
-                    unsigned(((CO + WCO - 1) / WCO) * ((CI + WCI - 1) / WCI)));
-    NN_LAUNCH(k_conv3_dw, grid, dim3(256), 0, (hipStream_t)stream, in, dout, dw, N, CI, CO, H, W, nullptr);
+    return launch_dw(in, dout, dw, nullptr, N, CI, CO, H, W, (hipStream_t)stream);
 }
 
 int64_t imexlb_nn_conv3x3_dw_work(int CI, int CO, int H, int W)
@@ -622,10 +748,7 @@ int imexlb_nn_conv3x3_dw_ordered(const float *in, const float *dout, float *dw, 
     const int64_t tiles = int64_t((W + TS - 1) / TS) * ((H + TS - 1) / TS);
     const int64_t n = int64_t(CO) * CI * 9;
     if (work_floats < tiles * n) return -1;
-    const dim3 grid(unsigned(tiles), unsigned(((CO + WCO - 1) / WCO) * ((CI + WCI - 1) / WCI)));
-    hipLaunchKernelGGL(k_conv3_dw, grid, dim3(256), 0, (hipStream_t)stream, in, dout, dw, N, CI, CO, H, W, work);
-    if (hipGetLastError() != hipSuccess) return -2;
-    NN_LAUNCH(k_dw_reduce, dim3(blocks(n)), dim3(256), 0, (hipStream_t)stream, work, dw, tiles, n);
+    return launch_dw(in, dout, dw, work, N, CI, CO, H, W, (hipStream_t)stream);
 }
 
 }  // extern "C"
@@ -688,10 +811,7 @@ int imexlb_nn_conv3x3_dw_ordered_noalloc(const float *in, const float *dout, flo
     }
     float *work = scratch_here();
     if (!work) return -2;
-    const dim3 grid(unsigned(tiles), unsigned(((CO + WCO - 1) / WCO) * ((CI + WCI - 1) / WCI)));
-    hipLaunchKernelGGL(k_conv3_dw, grid, dim3(256), 0, (hipStream_t)stream, in, dout, dw, N, CI, CO, H, W, work);
-    if (hipGetLastError() != hipSuccess) return -2;
-    NN_LAUNCH(k_dw_reduce, dim3(blocks(n)), dim3(256), 0, (hipStream_t)stream, work, dw, tiles, n);
+    return launch_dw(in, dout, dw, work, N, CI, CO, H, W, (hipStream_t)stream);
 }
 
 int imexlb_nn_bias_grad(const float *dout, float *db, int N, int C, int H, int W, void *stream)

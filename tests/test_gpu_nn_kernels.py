@@ -77,3 +77,47 @@ def test_conv3x3_non_finite_values(shape):
     plain = np.isfinite(ref) & ~big
     size = _conv64(np.abs(small), np.abs(w).astype(np.float64))
     assert (np.abs(got[plain] - ref[plain]) <= ((9 * ci + 8) * 2.0 ** -24 * size)[plain]).all()
+
+
+# channel groups of 16 and 32 on either side and past them, ragged tiles, one
+# and two tile halves, tile counts around the reduction's 32 loads in flight
+DW_SHAPES = [(1, 1, 1, 1, 1), (3, 15, 16, 8, 16), (2, 16, 17, 9, 17), (2, 17, 15, 16, 33), (1, 33, 34, 31, 5),
+             (2, 20, 40, 260, 190), (1, 3, 65, 65, 500), (2, 40, 9, 100, 300)]
+
+
+@pytest.mark.parametrize("shape", DW_SHAPES)
+def test_weight_gradient_at_tile_edges(shape):
+    import torch
+    from imexlb._lib import lib
+    N, ci, co, H, W = shape
+    print(f"[nn] conv3x3_dw {shape}", flush=True)
+    rng = np.random.default_rng(7)
+    x = rng.normal(0, 1, (N, ci, H, W)).astype(np.float32)
+    g = rng.normal(0, 1, (N, co, H, W)).astype(np.float32)
+    start = rng.normal(0, 1, (co, ci, 3, 3)).astype(np.float32)
+
+    def dw64(x, g):
+        xp = np.zeros((N, ci, H + 2, W + 2))
+        xp[:, :, 1:-1, 1:-1] = x
+        r = np.zeros((co, ci, 3, 3))
+        for k in range(9):
+            s = xp[:, :, k // 3:k // 3 + H, k % 3:k % 3 + W].transpose(1, 0, 2, 3).reshape(ci, -1)
+            r[:, :, k // 3, k % 3] = g.astype(np.float64).transpose(1, 0, 2, 3).reshape(co, -1) @ s.T
+        return r
+
+    xd, gd = torch.tensor(x, device="cuda"), torch.tensor(g, device="cuda")
+    n = lib().imexlb_nn_conv3x3_dw_work(ci, co, H, W)
+    work = torch.empty(n, device="cuda")
+    dw = torch.tensor(start, device="cuda")
+    _call("conv3x3_dw_ordered", xd, gd, dw, work, n, N, ci, co, H, W)
+    again = torch.tensor(start, device="cuda")
+    _call("conv3x3_dw_ordered_noalloc", xd, gd, again, N, ci, co, H, W)
+    assert torch.equal(dw, again)
+    loose = torch.tensor(start, device="cuda")
+    _call("conv3x3_dw", xd, gd, loose, N, ci, co, H, W)
+    # one rounding of 2^-24 per product and per tile
+    tiles = -(-H // 16) * -(-W // 16)
+    tol = (N * H * W + tiles + 4) * 2.0 ** -24 * (dw64(np.abs(x), np.abs(g)) + np.abs(start))
+    for got in (dw, loose):
+        err = np.abs(got.cpu().numpy() - (dw64(x, g) + start))
+        assert (err <= tol).all(), (err / tol).max()
