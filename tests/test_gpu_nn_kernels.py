@@ -121,3 +121,43 @@ def test_weight_gradient_at_tile_edges(shape):
     for got in (dw, loose):
         err = np.abs(got.cpu().numpy() - (dw64(x, g) + start))
         assert (err <= tol).all(), (err / tol).max()
+
+
+# rows of 256 pixels: one ragged, exactly one, more than a batch of loads in
+# flight, images shorter than a batch
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (2, 3, 15, 17), (3, 5, 16, 16), (2, 7, 131, 129), (5, 4, 16, 112),
+                                   (1, 33, 16, 1040)])
+def test_bias_gradient(shape):
+    import torch
+    N, C_, H, W = shape
+    rng = np.random.default_rng(8)
+    g = rng.normal(0, 1, shape).astype(np.float32)
+    db = torch.empty(C_, device="cuda")
+    _call("bias_grad", torch.tensor(g, device="cuda"), db, N, C_, H, W)
+    # the order of the sum: thread t adds pixels t, t + 256, ..., then a tree
+    rows = -(-H * W // 256)
+    v = np.zeros((N, C_, rows * 256), np.float32)
+    v[:, :, :H * W] = g.reshape(N, C_, -1)
+    v = v.reshape(N, C_, rows, 256).transpose(1, 0, 2, 3).reshape(C_, N * rows, 256)
+    s = np.zeros((C_, 256), np.float32)
+    for k in range(N * rows):
+        s += v[:, k]
+    o = 128
+    while o:
+        s[:, :o] += s[:, o:2 * o]
+        o //= 2
+    assert np.array_equal(db.cpu().numpy(), s[:, 0])
+
+
+@pytest.mark.parametrize("n", [1, 255, 1024, 1025, 131072, 131073, 400003])
+def test_mse(n):
+    import torch
+    rng = np.random.default_rng(9)
+    p, t = (rng.normal(0, 1, n).astype(np.float32) for _ in range(2))
+    g, loss = torch.empty(n, device="cuda"), torch.full((1,), 0.5, device="cuda")
+    _call("mse", torch.tensor(p, device="cuda"), torch.tensor(t, device="cuda"), g, n, loss)
+    d = p - t
+    assert np.array_equal(g.cpu().numpy(), np.float32(2) * d / np.float32(n))
+    ref = 0.5 + np.mean(d.astype(np.float64) ** 2)
+    # each term rounded twice, at most 128 additions to the loss
+    assert abs(loss.item() - ref) <= 130 * 2.0 ** -24 * ref
