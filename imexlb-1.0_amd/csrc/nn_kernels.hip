@@ -27,6 +27,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <initializer_list>
 #include <mutex>
 #include <string>
 #include <type_traits>
@@ -70,10 +71,17 @@ __device__ __forceinline__ uint32_t xcd_run(uint32_t b, uint32_t nb)
 // 16 x 64: 429 to 59 us.
 constexpr int CIB = 8;  // input channels per LDS chunk
 
-template <int MT, int NT, int TC>
+//
+// The output goes to channels of a buffer with ototal of them per image
+// (out points at the first).  DGRAD: w is [CI][CO][3][3], read flipped and
+// transposed -- the data gradient of a layer from CO to CI channels -- and,
+// with a gate (gtotal channels per image), the value is kept only where the
+// gate is positive: the ReLU of the layer before.
+template <int MT, int NT, int TC, bool DGRAD>
 __global__ __launch_bounds__(256) void k_conv3(const float *__restrict__ in, const float *__restrict__ w,
-                                               const float *__restrict__ bias, float *__restrict__ out, int CI, int CO,
-                                               int H, int W, int relu, uint32_t ntx, uint32_t nty, uint32_t ncob)
+                                               const float *__restrict__ bias, float *__restrict__ out, int ototal,
+                                               const float *__restrict__ gate, int gtotal, int CI, int CO, int H, int W,
+                                               int relu, uint32_t ntx, uint32_t nty, uint32_t ncob)
 {
     constexpr int GR = 32 / TC;  // rows of a 32-pixel group
     constexpr int TR = 4 * MT * GR, IR = TR + 2, IC = TC + 2, BN = 32 * NT, WS = BN + 1;
@@ -108,7 +116,8 @@ __global__ __launch_bounds__(256) void k_conv3(const float *__restrict__ in, con
     const int ch = __builtin_amdgcn_readfirstlane(wave * 2);
     const int wk = tid % 72, wc = tid / 72;  // threads from 216 on repeat others' loads
     const int wlast = (min(co0 + BN, CO) - 1 - co0 - min(wc, CO - 1 - co0)) / 3;
-    const float *const wrow = w + int64_t(co0 + min(wc, CO - 1 - co0)) * CI * 9;
+    const int wco = co0 + min(wc, CO - 1 - co0);
+    const float *const wrow = DGRAD ? w + int64_t(wco) * 9 + 8 - wk % 9 : w + int64_t(wco) * CI * 9;
     float xin[2][NP], xw[NW];
     auto load = [&](int c0) {
 #pragma unroll
@@ -117,9 +126,10 @@ __global__ __launch_bounds__(256) void k_conv3(const float *__restrict__ in, con
 #pragma unroll
             for (int i = 0; i < NP; ++i) xin[c][i] = pl[ioff[i]];
         }
-        const float *const p = wrow + min(int64_t(c0) * 9 + wk, int64_t(CI) * 9 - 1);
+        const float *const p = wrow + (DGRAD ? min(c0 + wk / 9, CI - 1) * int64_t(CO) * 9
+                                             : min(int64_t(c0) * 9 + wk, int64_t(CI) * 9 - 1));
 #pragma unroll
-        for (int i = 0; i < NW; ++i) xw[i] = p[int64_t(min(i, wlast)) * 27 * CI];
+        for (int i = 0; i < NW; ++i) xw[i] = p[min(i, wlast) * (DGRAD ? 27 : int64_t(27) * CI)];
     };
     auto store = [&](int buf, int c0) {
 #pragma unroll
@@ -192,16 +202,25 @@ __global__ __launch_bounds__(256) void k_conv3(const float *__restrict__ in, con
     for (int t = 0; t < MT; ++t) {
         const int y = y0 + (wave * MT + t) * GR + m / TC;
         if (y >= H) continue;
-        float *const o = out + (n * CO + co0) * HW + int64_t(y) * W + x;
+        float *const o = out + (n * ototal + co0) * HW + int64_t(y) * W + x;
+        const float *const g = DGRAD && gate ? gate + (n * gtotal + co0) * HW + int64_t(y) * W + x : nullptr;
 #pragma unroll
-        for (int s = 0; s < NT; ++s)
+        for (int s = 0; s < NT; ++s) {
+            float gv[16];  // all gate values in flight before the first is used
+            if (DGRAD && g) {
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+                    gv[j] = g[min(32 * s + 8 * (j / 4) + 4 * hk + j % 4, CO - 1 - co0) * HW];
+            }
 #pragma unroll
             for (int j = 0; j < 16; ++j) {
                 const int co = 32 * s + 8 * (j / 4) + 4 * hk + j % 4;
                 float v = acc[s][t][j] + s_b[co];
                 if (relu) v = v > 0.0f ? v : 0.0f;
+                if (DGRAD && g) v = gv[j] > 0.0f ? v : 0.0f;
                 if (co0 + co < CO) o[co * HW] = v;
             }
+        }
     }
 }
 
@@ -212,6 +231,59 @@ __global__ void k_flip(const float *__restrict__ w, float *__restrict__ wt, int 
     if (i >= int64_t(CO) * CI * 9) return;
     const int k = int(i % 9), ci = int((i / 9) % CI), co = int(i / (9 * int64_t(CI)));
     wt[(int64_t(ci) * CO + co) * 9 + (8 - k)] = w[i];
+}
+
+// db[c] = sum of dout over batch and pixels (one block per channel): thread
+// t adds pixels t, t + 256, ... of image after image, then a tree over the
+// threads.  Bound by the latency of its loads (one channel's values pass
+// through one CU): kBias of them are in flight per thread, the additions
+// keep their order.  32 channels, 8 x 128 x 512: 505 us with one load in
+// flight, 76 us now.
+constexpr int kBias = 64;
+__device__ __forceinline__ void bias_sum(const float *__restrict__ dout, float *__restrict__ db, int N, int C,
+                                         int64_t HW, int c, float *red)
+{
+    const int64_t rows = (HW + 255) / 256;  // of 256 pixels per image, the last one ragged
+    const float *p = dout + c * HW + threadIdx.x;
+    const int64_t next = C * HW - rows * 256;  // from past the last row to the next image's first
+    int64_t left = N * rows, i = 0;
+    const bool tail = (rows - 1) * 256 + threadIdx.x < HW;  // this thread's pixel of the last row exists
+    float s = 0.0f;
+    const auto sum = [&](auto count) {
+        constexpr int K = decltype(count)::value;
+        for (; left >= K; left -= K) {
+            float v[K];
+            bool ok[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const bool last = i + 1 == rows;
+                ok[k] = !last || tail;
+                v[k] = p[ok[k] ? 0 : -int64_t(threadIdx.x)];  // (no branch: a missing pixel reads its row's first)
+                p += last ? next + 256 : 256;
+                i = last ? 0 : i + 1;
+            }
+#pragma unroll
+            for (int k = 0; k < K; ++k) s += ok[k] ? v[k] : 0.0f;
+        }
+    };
+    sum(std::integral_constant<int, kBias>{});
+    sum(std::integral_constant<int, 8>{});
+    sum(std::integral_constant<int, 1>{});
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if (int(threadIdx.x) < o) red[threadIdx.x] += red[threadIdx.x + o];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) db[c] = red[0];
+    __syncthreads();  // (red is used again)
+}
+
+__global__ __launch_bounds__(256) void k_bias_grad(const float *__restrict__ dout, float *__restrict__ db, int N,
+                                                   int C, int64_t HW)
+{
+    __shared__ float red[256];
+    bias_sum(dout, db, N, C, HW, int(blockIdx.x), red);
 }
 
 constexpr int TS = 16;  // pixel tile edge of the weight gradient
@@ -236,7 +308,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 template <int GCO, int GCI>
 __global__ __launch_bounds__(256) void k_conv3_dw(const float *__restrict__ in, const float *__restrict__ dout,
                                                   float *__restrict__ dw, int N, int CI, int CO, int H, int W,
-                                                  float *__restrict__ partial)
+                                                  float *__restrict__ partial, float *__restrict__ db)
 {
     constexpr int NTAP = GCO * GCI == 4 ? 9 : GCO * GCI == 2 ? 5 : 3;  // taps per wave
     constexpr int HR = TS / 2, IC = TS + 2, IP = (HR + 2) * IC, GP = HR * TS;
@@ -247,10 +319,17 @@ __global__ __launch_bounds__(256) void k_conv3_dw(const float *__restrict__ in, 
     __shared__ float s_g[GCO * 16 * SG];
     const int tid = int(threadIdx.x), lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const int m = lane % 16, kk = lane / 16;  // operand row / column, pixel of four
+    // with db, the first row of blocks sums the bias gradient (the waits of
+    // those few chains of additions pass while the others multiply)
+    if (db && blockIdx.y == 0) {
+        for (int c = int(blockIdx.x); c < CO; c += int(gridDim.x)) bias_sum(dout, db, N, CO, int64_t(H) * W, c, s_in);
+        return;
+    }
+    const int by = int(blockIdx.y) - (db ? 1 : 0);
     const int ntx = (W + TS - 1) / TS;
     const int x0 = int(blockIdx.x) % ntx * TS, y0 = int(blockIdx.x) / ntx * TS;
     const int nci = (CI + 16 * GCI - 1) / (16 * GCI);
-    const int co0 = int(blockIdx.y) / nci * (16 * GCO), ci0 = int(blockIdx.y) % nci * (16 * GCI);
+    const int co0 = by / nci * (16 * GCO), ci0 = by % nci * (16 * GCI);
     const int wco = wave % GCO, wci = wave / GCO % GCI, tap0 = wave / (GCO * GCI) * NTAP;
     const int64_t HW = int64_t(H) * W;
 
@@ -332,8 +411,12 @@ __global__ __launch_bounds__(256) void k_conv3_dw(const float *__restrict__ in, 
 #pragma unroll
                 for (int t = 0; t < NTAP; ++t)
                     acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[g % 2], b[g % 2][t], acc[t], 0, 0, 0);
-                __builtin_amdgcn_sched_group_barrier(0x100, NTAP + 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, NTAP, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+#pragma unroll
+                for (int t = 0; t < NTAP; ++t) {  // one read between two products
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                }
             }
         }
     }
@@ -378,53 +461,6 @@ __global__ __launch_bounds__(64) void k_dw_reduce(const float *__restrict__ part
     dw[i] += s;
 }
 
-// db[c] = sum of dout over batch and pixels (one block per channel): thread
-// t adds pixels t, t + 256, ... of image after image, then a tree over the
-// threads.  Bound by the latency of its loads (one channel's values pass
-// through one CU): kBias of them are in flight per thread, the additions
-// keep their order.  32 channels, 8 x 128 x 512: 505 us with one load in
-// flight, 76 us now.
-constexpr int kBias = 64;
-__global__ __launch_bounds__(256) void k_bias_grad(const float *__restrict__ dout, float *__restrict__ db, int N,
-                                                   int C, int64_t HW)
-{
-    __shared__ float red[256];
-    const int c = blockIdx.x;
-    const int64_t rows = (HW + 255) / 256;  // of 256 pixels per image, the last one ragged
-    const float *p = dout + c * HW + threadIdx.x;
-    const int64_t next = C * HW - rows * 256;  // from past the last row to the next image's first
-    int64_t left = N * rows, i = 0;
-    const bool tail = (rows - 1) * 256 + threadIdx.x < HW;  // this thread's pixel of the last row exists
-    float s = 0.0f;
-    const auto sum = [&](auto count) {
-        constexpr int K = decltype(count)::value;
-        for (; left >= K; left -= K) {
-            float v[K];
-            bool ok[K];
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                const bool last = i + 1 == rows;
-                ok[k] = !last || tail;
-                v[k] = p[ok[k] ? 0 : -int64_t(threadIdx.x)];  // (no branch: a missing pixel reads its row's first)
-                p += last ? next + 256 : 256;
-                i = last ? 0 : i + 1;
-            }
-#pragma unroll
-            for (int k = 0; k < K; ++k) s += ok[k] ? v[k] : 0.0f;
-        }
-    };
-    sum(std::integral_constant<int, kBias>{});
-    sum(std::integral_constant<int, 8>{});
-    sum(std::integral_constant<int, 1>{});
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (int(threadIdx.x) < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) db[c] = red[0];
-}
-
 __global__ void k_relu_bwd(const float *__restrict__ out, const float *__restrict__ dout, float *__restrict__ dz,
                            int64_t n)
 {
@@ -432,49 +468,141 @@ __global__ void k_relu_bwd(const float *__restrict__ out, const float *__restric
     if (i < n) dz[i] = out[i] > 0.0f ? dout[i] : 0.0f;
 }
 
-// 2x2 average pool: in [N][C][2h][2w] -> out [N][C][h][w]
-__global__ void k_pool2(const float *__restrict__ in, float *__restrict__ out, int64_t NC, int h, int w)
+// K consecutive values, as one access where the buffers allow it (A)
+template <int K>
+struct Px {
+    float v[K];
+};
+template <bool A, int K>
+__device__ __forceinline__ Px<K> ld_px(const float *p)
 {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= NC * h * w) return;
-    const int x = int(i % w), y = int((i / w) % h);
-    const int64_t nc = i / (int64_t(h) * w);
-    const float *p = in + (nc * 2 * h + 2 * y) * (2 * w) + 2 * x;
-    out[i] = 0.25f * ((p[0] + p[1]) + (p[2 * w] + p[2 * w + 1]));
+    if constexpr (A && K == 4)
+        return __builtin_bit_cast(Px<K>, *reinterpret_cast<const float4 *>(p));
+    else if constexpr (A && K == 2)
+        return __builtin_bit_cast(Px<K>, *reinterpret_cast<const float2 *>(p));
+    Px<K> r;
+#pragma unroll
+    for (int k = 0; k < K; ++k) r.v[k] = p[k];
+    return r;
+}
+template <bool A, int K>
+__device__ __forceinline__ void st_px(float *p, const Px<K> &v)
+{
+    if constexpr (A && K == 4)
+        *reinterpret_cast<float4 *>(p) = __builtin_bit_cast(float4, v);
+    else if constexpr (A && K == 2)
+        *reinterpret_cast<float2 *>(p) = __builtin_bit_cast(float2, v);
+    else {
+#pragma unroll
+        for (int k = 0; k < K; ++k) p[k] = v.v[k];
+    }
 }
 
-__global__ void k_pool2_bwd(const float *__restrict__ dout, float *__restrict__ din, int64_t NC, int h, int w)
+// Pooling and upsampling: a wave takes a low-resolution row of one channel
+// of one image, its place found once with scalar divisions (a 64-bit
+// division per value cost more than the memory access), two pixels per
+// thread with 8- and 16-byte accesses (A) where w is even and the buffers
+// are aligned, else one.  Bound by HBM: the three upsamplings of a training
+// step of 8 cases on 128 x 512 took 64 us each, now 18; the gradients with the
+// ReLU and the skip connection joined 19 and 22 us instead of 46 and 104 in
+// two and four launches.
+template <bool A, class F>
+__device__ __forceinline__ void for_rows(int N, int C, int h, int w, F f)
 {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;  // over din
-    if (i >= NC * 4 * h * w) return;
-    const int X = int(i % (2 * w)), Y = int((i / (2 * w)) % (2 * h));
-    const int64_t nc = i / (int64_t(4) * h * w);
-    din[i] = 0.25f * dout[(nc * h + Y / 2) * w + X / 2];
+    constexpr int V = A ? 2 : 1;
+    const int64_t rows = int64_t(N) * C * h;
+    for (int64_t r = int64_t(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / 64); r < rows;
+         r += int64_t(gridDim.x) * 4) {
+        const int64_t nc = r / h, n = nc / C;
+        const int y = int(r - nc * h), c = int(nc - n * C);
+        for (int x = int(threadIdx.x % 64) * V; x < w; x += 64 * V) f(n, c, y, x);
+    }
 }
 
-// nearest 2x upsample: in [N][C][h][w] -> channels [coff, coff+C) of out [N][Ctot][2h][2w]
-__global__ void k_up2(const float *__restrict__ in, float *__restrict__ out, int N, int C, int h, int w, int Ctot,
-                      int coff)
+// 2x2 average pool of channels [coff, coff + C) of in [N][Ctot][2h][2w]
+// (in points at channel coff) into out [N][C][h][w]
+template <bool A>
+__global__ __launch_bounds__(256) void k_pool2(const float *__restrict__ in, int Ctot, float *__restrict__ out, int N,
+                                               int C, int h, int w)
 {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;  // over the C output channels
-    const int64_t per = int64_t(C) * 4 * h * w;
-    if (i >= N * per) return;
-    const int n = int(i / per);
-    const int64_t r = i % per;
-    const int c = int(r / (int64_t(4) * h * w));
-    const int X = int(r % (2 * w)), Y = int((r / (2 * w)) % (2 * h));
-    out[((int64_t(n) * Ctot + coff + c) * 2 * h + Y) * 2 * w + X] = in[((int64_t(n) * C + c) * h + Y / 2) * w + X / 2];
+    constexpr int V = A ? 2 : 1;
+    for_rows<A>(N, C, h, w, [&](int64_t n, int c, int y, int x) {
+        const float *p = in + ((n * Ctot + c) * 2 * h + 2 * y) * (2 * int64_t(w)) + 2 * x;
+        const Px<2 * V> a = ld_px<A, 2 * V>(p), b = ld_px<A, 2 * V>(p + 2 * int64_t(w));
+        Px<V> o;
+#pragma unroll
+        for (int k = 0; k < V; ++k) o.v[k] = 0.25f * ((a.v[2 * k] + a.v[2 * k + 1]) + (b.v[2 * k] + b.v[2 * k + 1]));
+        st_px<A, V>(out + ((n * C + c) * h + y) * int64_t(w) + x, o);
+    });
 }
 
-__global__ void k_up2_bwd(const float *__restrict__ dout, float *__restrict__ din, int N, int C, int h, int w,
-                          int Ctot, int coff)
+// Gradient of the pool, din [N][C][2h][2w]: 0.25 dout of the pixel's cell,
+// plus skip (stot channels per image) if given, where gate (gtot channels
+// per image) is positive if given.
+template <bool A>
+__global__ __launch_bounds__(256) void k_pool2_bwd(const float *__restrict__ dout, const float *__restrict__ skip,
+                                                   int stot, const float *__restrict__ gate, int gtot,
+                                                   float *__restrict__ din, int N, int C, int h, int w)
 {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;  // over din
-    if (i >= int64_t(N) * C * h * w) return;
-    const int x = int(i % w), y = int((i / w) % h);
-    const int c = int((i / (int64_t(h) * w)) % C), n = int(i / (int64_t(C) * h * w));
-    const float *p = dout + ((int64_t(n) * Ctot + coff + c) * 2 * h + 2 * y) * 2 * w + 2 * x;
-    din[i] = (p[0] + p[1]) + (p[2 * w] + p[2 * w + 1]);
+    constexpr int V = A ? 2 : 1;
+    const int64_t W = 2 * int64_t(w);
+    for_rows<A>(N, C, h, w, [&](int64_t n, int c, int y, int x) {
+        const Px<V> g = ld_px<A, V>(dout + ((n * C + c) * h + y) * int64_t(w) + x);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int64_t row = 2 * y + k;
+            Px<2 * V> o, s, a;
+            if (skip) s = ld_px<A, 2 * V>(skip + ((n * stot + c) * 2 * h + row) * W + 2 * x);
+            if (gate) a = ld_px<A, 2 * V>(gate + ((n * gtot + c) * 2 * h + row) * W + 2 * x);
+#pragma unroll
+            for (int j = 0; j < 2 * V; ++j) {
+                o.v[j] = 0.25f * g.v[j / 2];
+                if (skip) o.v[j] = o.v[j] + s.v[j];
+                if (gate && !(a.v[j] > 0.0f)) o.v[j] = 0.0f;
+            }
+            st_px<A, 2 * V>(din + ((n * C + c) * 2 * h + row) * W + 2 * x, o);
+        }
+    });
+}
+
+// nearest 2x upsample: in [N][C][h][w] -> C channels of out [N][Ctot][2h][2w]
+// (out points at the first)
+template <bool A>
+__global__ __launch_bounds__(256) void k_up2(const float *__restrict__ in, float *__restrict__ out, int N, int C, int h,
+                                             int w, int Ctot)
+{
+    constexpr int V = A ? 2 : 1;
+    const int64_t W = 2 * int64_t(w);
+    for_rows<A>(N, C, h, w, [&](int64_t n, int c, int y, int x) {
+        const Px<V> v = ld_px<A, V>(in + ((n * C + c) * h + y) * int64_t(w) + x);
+        Px<2 * V> o;
+#pragma unroll
+        for (int j = 0; j < 2 * V; ++j) o.v[j] = v.v[j / 2];
+        float *const p = out + ((n * Ctot + c) * 2 * h + 2 * y) * W + 2 * x;
+        st_px<A, 2 * V>(p, o);
+        st_px<A, 2 * V>(p + W, o);
+    });
+}
+
+// its gradient, where gate (gtot channels per image) is positive if given
+template <bool A>
+__global__ __launch_bounds__(256) void k_up2_bwd(const float *__restrict__ dout, int Ctot,
+                                                 const float *__restrict__ gate, int gtot, float *__restrict__ din,
+                                                 int N, int C, int h, int w)
+{
+    constexpr int V = A ? 2 : 1;
+    for_rows<A>(N, C, h, w, [&](int64_t n, int c, int y, int x) {
+        const float *p = dout + ((n * Ctot + c) * 2 * h + 2 * y) * (2 * int64_t(w)) + 2 * x;
+        const Px<2 * V> a = ld_px<A, 2 * V>(p), b = ld_px<A, 2 * V>(p + 2 * int64_t(w));
+        Px<V> o, t;
+        if (gate) t = ld_px<A, V>(gate + ((n * gtot + c) * h + y) * int64_t(w) + x);
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+            o.v[k] = (a.v[2 * k] + a.v[2 * k + 1]) + (b.v[2 * k] + b.v[2 * k + 1]);
+            if (gate && !(t.v[k] > 0.0f)) o.v[k] = 0.0f;
+        }
+        st_px<A, V>(din + ((n * C + c) * h + y) * int64_t(w) + x, o);
+    });
 }
 
 // dst[:, dcoff+c] (=|+=) src[:, scoff+c] for c < C
@@ -693,10 +821,47 @@ __global__ void k_up2_bf16(const uint4 *__restrict__ in, uint4 *__restrict__ out
 
 inline unsigned blocks(int64_t n) { return unsigned((n + 255) / 256); }
 
+// blocks of a kernel that walks rows (four per block, at most 2^20 blocks)
+inline dim3 row_blocks(int N, int C, int h)
+{
+    return dim3(unsigned(std::min<int64_t>((int64_t(N) * C * h + 3) / 4, int64_t(1) << 20)));
+}
+// the buffers of a pooling or upsampling call take 8- and 16-byte accesses
+inline bool vec_ok(int w, std::initializer_list<const void *> ptrs)
+{
+    uintptr_t bits = 0;
+    for (const void *p : ptrs) bits |= reinterpret_cast<uintptr_t>(p);
+    return w % 2 == 0 && bits % 16 == 0;
+}
+
+// the convolution's tile for these sizes and its launch
+template <bool DGRAD>
+int launch_conv(const float *in, const float *w, const float *bias, float *out, int ototal, const float *gate,
+                int gtotal, int N, int CI, int CO, int H, int W, int relu, hipStream_t stream)
+{
+    // The largest tile that still gives every CU two blocks (its operands are
+    // reused most: 8 x 32 pixels for 64 channels 118 TFLOP/s on the deep
+    // layers of a batch of 8, for 32 channels 100); a batch of one gets the
+    // smallest.  Rows of at most 16 pixels take the 16-column tile.
+    const auto run = [&](auto kernel, int rows, int cols, int bn, bool always) {
+        const int64_t tx = (int64_t(W) + cols - 1) / cols, ty = (int64_t(H) + rows - 1) / rows, tc = (CO + bn - 1) / bn;
+        const int64_t nb = tx * ty * tc * N;
+        if (nb < 512 && !always) return 1;  // too few blocks to give every CU two: smaller tiles
+        if (nb > 0x7fffffff) return -2;
+        hipLaunchKernelGGL(kernel, dim3(unsigned(nb)), dim3(256), 0, stream, in, w, bias, out, ototal, gate,
+                           gtotal, CI, CO, H, W, relu, uint32_t(tx), uint32_t(ty), uint32_t(tc));
+        return hipGetLastError() == hipSuccess ? 0 : -2;
+    };
+    if (W <= 16) return run(k_conv3<1, 1, 16, DGRAD>, 8, 16, 32, true);
+    int rc = CO > 32 ? run(k_conv3<2, 2, 32, DGRAD>, 8, 32, 64, false) : 1;
+    if (rc > 0) rc = run(k_conv3<2, 1, 32, DGRAD>, 8, 32, 32, false);
+    return rc <= 0 ? rc : run(k_conv3<1, 1, 32, DGRAD>, 4, 32, 32, true);
+}
+
 // weight gradient: the tiles' sums to `work` and from there to dw in tile
-// order, or (work == nullptr) to dw with atomics.
-int launch_dw(const float *in, const float *dout, float *dw, float *work, int N, int CI, int CO, int H, int W,
-              hipStream_t s)
+// order, or (work == nullptr) to dw with atomics; db: the bias gradient too.
+int launch_dw(const float *in, const float *dout, float *dw, float *db, float *work, int N, int CI, int CO, int H,
+              int W, hipStream_t s)
 {
     const int64_t tiles = int64_t((W + TS - 1) / TS) * ((H + TS - 1) / TS), n = int64_t(CO) * CI * 9;
     // blocks of 32 x 32 channels share their staged pixels most; where they
@@ -713,10 +878,10 @@ int launch_dw(const float *in, const float *dout, float *dw, float *work, int N,
         gco = 2;
     else if (CI > 16 && tiles * pairs(1, 2) >= 256)
         gci = 2;
-    const dim3 grid(unsigned(tiles), unsigned(pairs(gco, gci)));
+    const dim3 grid(unsigned(tiles), unsigned(pairs(gco, gci) + (db ? 1 : 0)));
     const auto kernel = gco == 2 ? (gci == 2 ? k_conv3_dw<2, 2> : k_conv3_dw<2, 1>)
                                  : (gci == 2 ? k_conv3_dw<1, 2> : k_conv3_dw<1, 1>);
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, in, dout, dw, N, CI, CO, H, W, work);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, in, dout, dw, N, CI, CO, H, W, work, db);
     if (hipGetLastError() != hipSuccess) return -2;
     if (!work) return 0;
     hipLaunchKernelGGL(k_dw_reduce, dim3(unsigned((n + 63) / 64)), dim3(64), 0, s, work, dw, tiles, n);
@@ -739,23 +904,26 @@ int imexlb_nn_conv3x3(const float *in, const float *w, const float *bias, float 
                       int W, int relu, void *stream)
 {
     if (!in || !w || !out || N <= 0 || CI <= 0 || CO <= 0 || H <= 0 || W <= 0) return -1;
-    // The largest tile that still gives every CU two blocks (its operands are
-    // reused most: 8 x 32 pixels for 64 channels 118 TFLOP/s on the deep
-    // layers of a batch of 8, for 32 channels 100); a batch of one gets the
-    // smallest.  Rows of at most 16 pixels take the 16-column tile.
-    const auto run = [&](auto kernel, int rows, int cols, int bn, bool always) {
-        const int64_t tx = (int64_t(W) + cols - 1) / cols, ty = (int64_t(H) + rows - 1) / rows, tc = (CO + bn - 1) / bn;
-        const int64_t nb = tx * ty * tc * N;
-        if (nb < 512 && !always) return 1;  // too few blocks to give every CU two: smaller tiles
-        if (nb > 0x7fffffff) return -2;
-        hipLaunchKernelGGL(kernel, dim3(unsigned(nb)), dim3(256), 0, (hipStream_t)stream, in, w, bias, out, CI, CO, H,
-                           W, relu, uint32_t(tx), uint32_t(ty), uint32_t(tc));
-        return hipGetLastError() == hipSuccess ? 0 : -2;
-    };
-    if (W <= 16) return run(k_conv3<1, 1, 16>, 8, 16, 32, true);
-    int rc = CO > 32 ? run(k_conv3<2, 2, 32>, 8, 32, 64, false) : 1;
-    if (rc > 0) rc = run(k_conv3<2, 1, 32>, 8, 32, 32, false);
-    return rc <= 0 ? rc : run(k_conv3<1, 1, 32>, 4, 32, 32, true);
+    return launch_conv<false>(in, w, bias, out, CO, nullptr, 0, N, CI, CO, H, W, relu, (hipStream_t)stream);
+}
+
+int imexlb_nn_conv3x3_into(const float *in, const float *w, const float *bias, float *out, int ototal, int ooff, int N,
+                           int CI, int CO, int H, int W, int relu, void *stream)
+{
+    if (!in || !w || !out || N <= 0 || CI <= 0 || CO <= 0 || H <= 0 || W <= 0 || ooff < 0 || ooff + CO > ototal)
+        return -1;
+    return launch_conv<false>(in, w, bias, out + int64_t(ooff) * H * W, ototal, nullptr, 0, N, CI, CO, H, W, relu,
+                              (hipStream_t)stream);
+}
+
+int imexlb_nn_conv3x3_dgrad(const float *dz, const float *w, const float *gate, int gtotal, int goff, float *dx, int N,
+                            int CI, int CO, int H, int W, void *stream)
+{
+    if (!dz || !w || !dx || N <= 0 || CI <= 0 || CO <= 0 || H <= 0 || W <= 0 ||
+        (gate && (goff < 0 || goff + CI > gtotal)))
+        return -1;
+    return launch_conv<true>(dz, w, nullptr, dx, CI, gate ? gate + int64_t(goff) * H * W : nullptr, gtotal, N, CO, CI, H,
+                             W, 0, (hipStream_t)stream);
 }
 
 int imexlb_nn_flip_weights(const float *w, float *wt, int CI, int CO, void *stream)
@@ -768,7 +936,7 @@ int imexlb_nn_conv3x3_dw(const float *in, const float *dout, float *dw, int N, i
                          void *stream)
 {
     if (!in || !dout || !dw || N <= 0 || CI <= 0 || CO <= 0 || H <= 0 || W <= 0) return -1;
-    return launch_dw(in, dout, dw, nullptr, N, CI, CO, H, W, (hipStream_t)stream);
+    return launch_dw(in, dout, dw, nullptr, nullptr, N, CI, CO, H, W, (hipStream_t)stream);
 }
 
 int64_t imexlb_nn_conv3x3_dw_work(int CI, int CO, int H, int W)
@@ -784,7 +952,7 @@ int imexlb_nn_conv3x3_dw_ordered(const float *in, const float *dout, float *dw, 
     const int64_t tiles = int64_t((W + TS - 1) / TS) * ((H + TS - 1) / TS);
     const int64_t n = int64_t(CO) * CI * 9;
     if (work_floats < tiles * n) return -1;
-    return launch_dw(in, dout, dw, work, N, CI, CO, H, W, (hipStream_t)stream);
+    return launch_dw(in, dout, dw, nullptr, work, N, CI, CO, H, W, (hipStream_t)stream);
 }
 
 }  // extern "C"
@@ -847,7 +1015,15 @@ int imexlb_nn_conv3x3_dw_ordered_noalloc(const float *in, const float *dout, flo
     }
     float *work = scratch_here();
     if (!work) return -2;
-    return launch_dw(in, dout, dw, work, N, CI, CO, H, W, (hipStream_t)stream);
+    return launch_dw(in, dout, dw, nullptr, work, N, CI, CO, H, W, (hipStream_t)stream);
+}
+
+int imexlb_nn_conv3x3_grads(const float *in, const float *dout, float *dw, float *db, float *work, int64_t work_floats,
+                            int N, int CI, int CO, int H, int W, void *stream)
+{
+    if (!in || !dout || !dw || !db || !work || N <= 0 || CI <= 0 || CO <= 0 || H <= 0 || W <= 0) return -1;
+    if (work_floats < imexlb_nn_conv3x3_dw_work(CI, CO, H, W)) return -1;
+    return launch_dw(in, dout, dw, db, work, N, CI, CO, H, W, (hipStream_t)stream);
 }
 
 int imexlb_nn_bias_grad(const float *dout, float *db, int N, int C, int H, int W, void *stream)
@@ -862,32 +1038,60 @@ int imexlb_nn_relu_bwd(const float *out, const float *dout, float *dz, int64_t n
     NN_LAUNCH(k_relu_bwd, dim3(blocks(n)), dim3(256), 0, (hipStream_t)stream, out, dout, dz, n);
 }
 
+int imexlb_nn_pool2_from(const float *in, int Ctot, int coff, float *out, int N, int C, int h, int w, void *stream)
+{
+    if (!in || !out || N <= 0 || C <= 0 || h <= 0 || w <= 0 || coff < 0 || coff + C > Ctot) return -1;
+    in += int64_t(coff) * 4 * h * w;
+    NN_LAUNCH(vec_ok(w, {in, out}) ? k_pool2<true> : k_pool2<false>, row_blocks(N, C, h), dim3(256), 0,
+              (hipStream_t)stream, in, Ctot, out, N, C, h, w);
+}
+
 int imexlb_nn_pool2(const float *in, float *out, int N, int C, int h, int w, void *stream)
 {
-    if (!in || !out || N <= 0 || C <= 0 || h <= 0 || w <= 0) return -1;
-    const int64_t NC = int64_t(N) * C;
-    NN_LAUNCH(k_pool2, dim3(blocks(NC * h * w)), dim3(256), 0, (hipStream_t)stream, in, out, NC, h, w);
+    return imexlb_nn_pool2_from(in, C, 0, out, N, C, h, w, stream);
+}
+
+int imexlb_nn_pool2_bwd_join(const float *dout, const float *skip, int stotal, int soff, const float *gate, int gtotal,
+                             int goff, float *din, int N, int C, int h, int w, void *stream)
+{
+    if (!dout || !din || N <= 0 || C <= 0 || h <= 0 || w <= 0 || (skip && (soff < 0 || soff + C > stotal)) ||
+        (gate && (goff < 0 || goff + C > gtotal)))
+        return -1;
+    const int64_t hw = int64_t(4) * h * w;
+    if (skip) skip += soff * hw;
+    if (gate) gate += goff * hw;
+    NN_LAUNCH(vec_ok(w, {dout, skip, gate, din}) ? k_pool2_bwd<true> : k_pool2_bwd<false>, row_blocks(N, C, h),
+              dim3(256), 0, (hipStream_t)stream, dout, skip, stotal, gate, gtotal, din, N, C, h, w);
 }
 
 int imexlb_nn_pool2_bwd(const float *dout, float *din, int N, int C, int h, int w, void *stream)
 {
-    if (!dout || !din || N <= 0 || C <= 0 || h <= 0 || w <= 0) return -1;
-    const int64_t NC = int64_t(N) * C;
-    NN_LAUNCH(k_pool2_bwd, dim3(blocks(NC * 4 * h * w)), dim3(256), 0, (hipStream_t)stream, dout, din, NC, h, w);
+    return imexlb_nn_pool2_bwd_join(dout, nullptr, 0, 0, nullptr, 0, 0, din, N, C, h, w, stream);
 }
 
 int imexlb_nn_up2(const float *in, float *out, int N, int C, int h, int w, int Ctot, int coff, void *stream)
 {
     if (!in || !out || N <= 0 || C <= 0 || h <= 0 || w <= 0 || coff < 0 || coff + C > Ctot) return -1;
-    NN_LAUNCH(k_up2, dim3(blocks(int64_t(N) * C * 4 * h * w)), dim3(256), 0, (hipStream_t)stream, in, out, N, C, h,
-              w, Ctot, coff);
+    out += int64_t(coff) * 4 * h * w;
+    NN_LAUNCH(vec_ok(w, {in, out}) ? k_up2<true> : k_up2<false>, row_blocks(N, C, h), dim3(256), 0,
+              (hipStream_t)stream, in, out, N, C, h, w, Ctot);
+}
+
+int imexlb_nn_up2_bwd_gate(const float *dout, int Ctot, int coff, const float *gate, int gtotal, int goff, float *din,
+                           int N, int C, int h, int w, void *stream)
+{
+    if (!dout || !din || N <= 0 || C <= 0 || h <= 0 || w <= 0 || coff < 0 || coff + C > Ctot ||
+        (gate && (goff < 0 || goff + C > gtotal)))
+        return -1;
+    dout += int64_t(coff) * 4 * h * w;
+    if (gate) gate += int64_t(goff) * h * w;
+    NN_LAUNCH(vec_ok(w, {dout, gate, din}) ? k_up2_bwd<true> : k_up2_bwd<false>, row_blocks(N, C, h), dim3(256), 0,
+              (hipStream_t)stream, dout, Ctot, gate, gtotal, din, N, C, h, w);
 }
 
 int imexlb_nn_up2_bwd(const float *dout, float *din, int N, int C, int h, int w, int Ctot, int coff, void *stream)
 {
-    if (!dout || !din || N <= 0 || C <= 0 || h <= 0 || w <= 0 || coff < 0 || coff + C > Ctot) return -1;
-    NN_LAUNCH(k_up2_bwd, dim3(blocks(int64_t(N) * C * h * w)), dim3(256), 0, (hipStream_t)stream, dout, din, N, C,
-              h, w, Ctot, coff);
+    return imexlb_nn_up2_bwd_gate(dout, Ctot, coff, nullptr, 0, 0, din, N, C, h, w, stream);
 }
 
 int imexlb_nn_copy_channels(const float *src, int sctot, int scoff, float *dst, int dctot, int dcoff, int N, int C,

@@ -74,6 +74,8 @@ SIGNATURES = {
     "imexlb_batch_info": (C.c_int, [_P, _I64P]),
     # warm-start network kernels (include/imexlb_nn.h); float pointers are device addresses
     "imexlb_nn_conv3x3": (C.c_int, [_P, _P, _P, _P, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _P]),
+    "imexlb_nn_conv3x3_into": (C.c_int, [_P, _P, _P, _P] + [C.c_int] * 8 + [_P]),
+    "imexlb_nn_conv3x3_dgrad": (C.c_int, [_P, _P, _P, C.c_int, C.c_int, _P] + [C.c_int] * 5 + [_P]),
     "imexlb_nn_flip_weights": (C.c_int, [_P, _P, C.c_int, C.c_int, _P]),
     "imexlb_nn_conv3x3_dw": (C.c_int, [_P, _P, _P, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _P]),
     "imexlb_nn_conv3x3_dw_work": (C.c_int64, [C.c_int, C.c_int, C.c_int, C.c_int]),
@@ -81,10 +83,14 @@ SIGNATURES = {
                                                _P]),
     "imexlb_nn_conv3x3_dw_ordered_noalloc": (C.c_int, [_P, _P, _P, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int,
                                                        _P]),
-    "imexlb_nn_bias_grad":(C.c_int, [_P, _P, C.c_int, C.c_int, C.c_int, C.c_int, _P]),
+    "imexlb_nn_conv3x3_grads": (C.c_int, [_P] * 5 + [C.c_int64] + [C.c_int] * 5 + [_P]),
+    "imexlb_nn_bias_grad": (C.c_int, [_P, _P, C.c_int, C.c_int, C.c_int, C.c_int, _P]),
     "imexlb_nn_relu_bwd": (C.c_int, [_P, _P, _P, C.c_int64, _P]),
     "imexlb_nn_pool2": (C.c_int, [_P, _P, C.c_int, C.c_int, C.c_int, C.c_int, _P]),
     "imexlb_nn_pool2_bwd": (C.c_int, [_P, _P, C.c_int, C.c_int, C.c_int, C.c_int, _P]),
+    "imexlb_nn_pool2_from": (C.c_int, [_P, C.c_int, C.c_int, _P] + [C.c_int] * 4 + [_P]),
+    "imexlb_nn_pool2_bwd_join": (C.c_int, [_P, _P, C.c_int, C.c_int, _P, C.c_int, C.c_int, _P] + [C.c_int] * 4 + [_P]),
+    "imexlb_nn_up2_bwd_gate": (C.c_int, [_P, C.c_int, C.c_int, _P, C.c_int, C.c_int, _P] + [C.c_int] * 4 + [_P]),
     "imexlb_nn_up2": (C.c_int, [_P, _P, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _P]),
     "imexlb_nn_up2_bwd": (C.c_int, [_P, _P, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _P]),
     "imexlb_nn_copy_channels": (C.c_int, [_P, C.c_int, C.c_int, _P, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int,

@@ -65,6 +65,22 @@ def layer_shapes(cin, cout, chans):
     return shapes
 
 
+class _InputGradients:
+    """dx[k]: the loss gradient of convolution k's input as the last
+    backward pass left it, formed when asked for (the pass itself forms it
+    together with the ReLU, pooling or upsampling before it)."""
+
+    def __init__(self, net):
+        self.net = net
+
+    def __getitem__(self, k):
+        n = self.net
+        dz = n.dz[k] if k < len(n.dz) else n.gout
+        dx = n.t.empty_like(n.inp[k])
+        n._dgrad(k, dz, dx)
+        return dx
+
+
 class UNet:
     """Encoder-decoder on device buffers; batch N of H x W fields."""
 
@@ -79,23 +95,24 @@ class UNet:
         rng = np.random.default_rng(seed)
         dev = "cuda"
         f32 = torch.float32
-        self.w, self.b = [], []
+        # weights then biases, their gradients and both moments in one buffer
+        # each (one Adam launch for all); the lists are views into them
+        sizes = [co * ci * 9 for co, ci in self.shapes] + [co for co, ci in self.shapes]
+        self.nw = sum(sizes[:len(self.shapes)])
+        host = []
         for k, (co, ci) in enumerate(self.shapes):
-            if params is not None:
-                w0, b0 = params[k]
-            else:
-                w0 = rng.normal(0.0, np.sqrt(2.0 / (9 * ci)), (co, ci, 3, 3))
-                b0 = np.zeros(co)
-            self.w.append(torch.tensor(np.asarray(w0, np.float32), device=dev))
-            self.b.append(torch.tensor(np.asarray(b0, np.float32), device=dev))
-        z = lambda like: torch.zeros_like(like)
-        self.dw = [z(w) for w in self.w]
-        self.db = [z(b) for b in self.b]
-        self.mw = [z(w) for w in self.w]
-        self.vw = [z(w) for w in self.w]
-        self.mb = [z(b) for b in self.b]
-        self.vb = [z(b) for b in self.b]
-        self.wt = [torch.empty((ci, co, 3, 3), dtype=f32, device=dev) for co, ci in self.shapes]
+            host.append(params[k][0] if params is not None
+                        else rng.normal(0.0, np.sqrt(2.0 / (9 * ci)), (co, ci, 3, 3)))
+        host += [np.zeros(co) if params is None else params[k][1] for k, (co, ci) in enumerate(self.shapes)]
+        self.flat = torch.from_numpy(np.concatenate([np.asarray(v, np.float32).ravel() for v in host])).to(dev)
+        self.grads, self.mom1, self.mom2 = torch.zeros((3, self.flat.numel()), dtype=f32, device=dev)
+
+        def views(buf):
+            parts = buf.split(sizes)
+            n = len(self.shapes)
+            return [p.view(co, ci, 3, 3) for p, (co, ci) in zip(parts, self.shapes)], list(parts[n:])
+
+        (self.w, self.b), (self.dw, self.db) = views(self.flat), views(self.grads)
         self.step_count = 0
         # per-level sizes and buffers
         self.hw = [(H >> l, W >> l) for l in range(L)]
@@ -106,107 +123,107 @@ class UNet:
         for l in range(L - 2, -1, -1):
             self.level_of += [l, l]
         self.level_of.append(0)
-        self.out = [e(co, self.level_of[k]) for k, (co, ci) in enumerate(self.shapes)]
-        self.dz = [e(co, self.level_of[k]) for k, (co, ci) in enumerate(self.shapes)]
-        self.dx = [e(ci, self.level_of[k]) for k, (co, ci) in enumerate(self.shapes)]
-        self.pooled = [None] + [e(self.chans[l - 1], l) for l in range(1, L)]
+        # the second convolution of encoder level l < L-1 writes into its
+        # channels of the decoder's concatenated input
+        self.skip_of = {2 * l + 1: l for l in range(L - 1)}
         self.cat = [e(self.chans[l + 1] + self.chans[l], l) for l in range(L - 1)]
-        self.denc = [e(self.chans[l], l) for l in range(L - 1)]
-        self.dpool = [None] + [e(self.chans[l - 1], l - 1) for l in range(1, L)]
-        self.dup = [e(self.chans[l + 1], l + 1) for l in range(L - 1)]
+        self.out = [self.cat[self.skip_of[k]][:, self.chans[self.skip_of[k] + 1]:] if k in self.skip_of
+                    else e(co, self.level_of[k]) for k, (co, ci) in enumerate(self.shapes)]
+        self.pooled = [None] + [e(self.chans[l - 1], l) for l in range(1, L)]
+        # gradients: of every convolution's sum (before its ReLU), of the
+        # concatenated inputs and of the pooled inputs
+        self.dz = [e(co, self.level_of[k]) for k, (co, ci) in enumerate(self.shapes[:-1])]
+        self.dcat = [e(self.chans[l + 1] + self.chans[l], l) for l in range(L - 1)]
+        self.dpool = [None] + [e(self.chans[l - 1], l) for l in range(1, L)]
+        self.dx = _InputGradients(self)
         self.inp = [None] * len(self.shapes)
         self.loss_buf = torch.zeros(1, dtype=f32, device=dev)
         # per-tile weight-gradient sums, added in a fixed order (training repeats bit for bit)
         work = max(lib().imexlb_nn_conv3x3_dw_work(ci, co, *self.hw[self.level_of[k]])
                    for k, (co, ci) in enumerate(self.shapes))
         self.dw_work = torch.empty(int(work), dtype=f32, device=dev)
-        self.grad_out = e(cout, 0)
+        self.grad_out = self.gout = e(cout, 0)
 
     # ---------------------------------------------------------------- layers
+    def _act(self, k):
+        """(buffer, its channels, first channel) of convolution k's output"""
+        if k in self.skip_of:
+            l = self.skip_of[k]
+            return self.cat[l], self.chans[l + 1] + self.chans[l], self.chans[l + 1]
+        return self.out[k], self.shapes[k][0], 0
+
+    def _dgrad(self, k, dz, dx, gate=None):
+        co, ci = self.shapes[k]
+        act, total, off = self._act(gate) if gate is not None else (None, 0, 0)
+        _ok(lib().imexlb_nn_conv3x3_dgrad(_ptr(dz), _ptr(self.w[k]), None if act is None else _ptr(act), total, off,
+                                          _ptr(dx), self.N, ci, co, *self.hw[self.level_of[k]], None),
+            "conv3x3 (data gradient)")
+
     def _conv(self, k, x, relu=True):
         co, ci = self.shapes[k]
         h, w = self.hw[self.level_of[k]]
         self.inp[k] = x
-        _ok(lib().imexlb_nn_conv3x3(_ptr(x), _ptr(self.w[k]), _ptr(self.b[k]), _ptr(self.out[k]), self.N, ci, co, h,
-                                    w, 1 if relu else 0, None), "conv3x3")
-        return self.out[k]
+        out, total, off = self._act(k)
+        _ok(lib().imexlb_nn_conv3x3_into(_ptr(x), _ptr(self.w[k]), _ptr(self.b[k]), _ptr(out), total, off, self.N, ci,
+                                         co, h, w, 1 if relu else 0, None), "conv3x3")
+        return out
 
-    def _conv_back(self, k, g, relu=True, need_dx=True):
+    def _conv_back(self, k, dz, dx, gate=None):
+        """Gradients of convolution k from that of its sum; dx (None: not
+        needed) takes its input's, 0 where the convolution `gate` that made
+        the input gave 0."""
         co, ci = self.shapes[k]
         h, w = self.hw[self.level_of[k]]
-        n = self.N * co * h * w
-        if relu:
-            _ok(lib().imexlb_nn_relu_bwd(_ptr(self.out[k]), _ptr(g), _ptr(self.dz[k]), n, None), "relu_bwd")
-            dz = self.dz[k]
-        else:
-            dz = g
-        _ok(lib().imexlb_nn_conv3x3_dw_ordered(_ptr(self.inp[k]), _ptr(dz), _ptr(self.dw[k]), _ptr(self.dw_work),
-                                               self.dw_work.numel(), self.N, ci, co, h, w, None), "conv3x3_dw")
-        _ok(lib().imexlb_nn_bias_grad(_ptr(dz), _ptr(self.db[k]), self.N, co, h, w, None), "bias_grad")
-        if not need_dx:
-            return None
-        _ok(lib().imexlb_nn_flip_weights(_ptr(self.w[k]), _ptr(self.wt[k]), ci, co, None), "flip")
-        _ok(lib().imexlb_nn_conv3x3(_ptr(dz), _ptr(self.wt[k]), None, _ptr(self.dx[k]), self.N, co, ci, h, w, 0,
-                                    None), "conv3x3 (data gradient)")
-        return self.dx[k]
+        _ok(lib().imexlb_nn_conv3x3_grads(_ptr(self.inp[k]), _ptr(dz), _ptr(self.dw[k]), _ptr(self.db[k]),
+                                          _ptr(self.dw_work), self.dw_work.numel(), self.N, ci, co, h, w, None),
+            "conv3x3 (weight gradient)")
+        if dx is not None:
+            self._dgrad(k, dz, dx, gate)
 
     # ------------------------------------------------------------------ passes
     def forward(self, x):
         """x: (N, cin, H, W) float32 device tensor; returns the output buffer."""
         L, ch, N = len(self.chans), self.chans, self.N
-        k, h, enc = 0, x, []
+        k, h = 0, x
         for l in range(L):
             if l > 0:
-                hh, ww = self.hw[l]
-                _ok(lib().imexlb_nn_pool2(_ptr(enc[l - 1]), _ptr(self.pooled[l]), N, ch[l - 1], hh, ww, None), "pool2")
+                _ok(lib().imexlb_nn_pool2_from(_ptr(h), ch[l] + ch[l - 1], ch[l], _ptr(self.pooled[l]), N, ch[l - 1],
+                                               *self.hw[l], None), "pool2")
                 h = self.pooled[l]
             h = self._conv(k, h)
             h = self._conv(k + 1, h)
             k += 2
-            enc.append(h)
-        d = enc[-1]
         for l in range(L - 2, -1, -1):
-            hh, ww = self.hw[l + 1]
-            ctot = ch[l + 1] + ch[l]
-            _ok(lib().imexlb_nn_up2(_ptr(d), _ptr(self.cat[l]), N, ch[l + 1], hh, ww, ctot, 0, None), "up2")
-            H0, W0 = self.hw[l]
-            _ok(lib().imexlb_nn_copy_channels(_ptr(enc[l]), ch[l], 0, _ptr(self.cat[l]), ctot, ch[l + 1], N, ch[l], H0,
-                                              W0, 0, None), "concat")
-            d = self._conv(k, self.cat[l])
-            d = self._conv(k + 1, d)
+            _ok(lib().imexlb_nn_up2(_ptr(h), _ptr(self.cat[l]), N, ch[l + 1], *self.hw[l + 1], ch[l + 1] + ch[l], 0,
+                                    None), "up2")
+            h = self._conv(k, self.cat[l])
+            h = self._conv(k + 1, h)
             k += 2
-        return self._conv(k, d, relu=False)
+        return self._conv(k, h, relu=False)
 
     def backward(self, g):
         """g: gradient of the loss w.r.t. the output; fills dw, db."""
         L, ch, N = len(self.chans), self.chans, self.N
-        for t in self.dw:
-            t.zero_()
+        self.gout = g
+        self.grads[:self.nw].zero_()
         k = len(self.shapes) - 1
-        g = self._conv_back(k, g, relu=False)
-        k -= 1
-        for l in range(0, L - 1):
-            g = self._conv_back(k, g)
-            g = self._conv_back(k - 1, g)
+        self._conv_back(k, g, self.dz[k - 1], gate=k - 1)
+        for l in range(0, L - 1):  # decoder, from the output down
             k -= 2
-            ctot, cu = ch[l + 1] + ch[l], ch[l + 1]
-            H0, W0 = self.hw[l]
-            _ok(lib().imexlb_nn_copy_channels(_ptr(g), ctot, cu, _ptr(self.denc[l]), ch[l], 0, N, ch[l], H0, W0, 0,
-                                              None), "split")
-            hh, ww = self.hw[l + 1]
-            _ok(lib().imexlb_nn_up2_bwd(_ptr(g), _ptr(self.dup[l]), N, cu, hh, ww, ctot, 0, None), "up2_bwd")
-            g = self.dup[l]
-        for l in range(L - 1, -1, -1):
-            g = self._conv_back(k, g)
-            g = self._conv_back(k - 1, g, need_dx=(k - 1) > 0)
+            self._conv_back(k + 1, self.dz[k + 1], self.dz[k], gate=k)
+            self._conv_back(k, self.dz[k], self.dcat[l])
+            act, total, off = self._act(k - 1)
+            _ok(lib().imexlb_nn_up2_bwd_gate(_ptr(self.dcat[l]), ch[l + 1] + ch[l], 0, _ptr(act), total, off,
+                                             _ptr(self.dz[k - 1]), N, ch[l + 1], *self.hw[l + 1], None), "up2_bwd")
+        for l in range(L - 1, -1, -1):  # encoder, from the bottom up
             k -= 2
+            self._conv_back(k + 1, self.dz[k + 1], self.dz[k], gate=k)
+            self._conv_back(k, self.dz[k], self.dpool[l] if l > 0 else None)
             if l > 0:
-                hh, ww = self.hw[l]
-                _ok(lib().imexlb_nn_pool2_bwd(_ptr(g), _ptr(self.dpool[l]), N, ch[l - 1], hh, ww, None), "pool2_bwd")
-                H0, W0 = self.hw[l - 1]
-                _ok(lib().imexlb_nn_copy_channels(_ptr(self.denc[l - 1]), ch[l - 1], 0, _ptr(self.dpool[l]), ch[l - 1],
-                                                  0, N, ch[l - 1], H0, W0, 1, None), "skip gradient")
-                g = self.dpool[l]
+                act, total, off = self._act(k - 1)
+                _ok(lib().imexlb_nn_pool2_bwd_join(_ptr(self.dpool[l]), _ptr(self.dcat[l - 1]), ch[l] + ch[l - 1],
+                                                   ch[l], _ptr(act), total, off, _ptr(self.dz[k - 1]), N, ch[l - 1],
+                                                   *self.hw[l], None), "pool2_bwd")
 
     def loss(self, pred, target, with_grad=True):
         self.loss_buf.zero_()
@@ -216,10 +233,8 @@ class UNet:
 
     def adam(self, lr, b1=0.9, b2=0.999, eps=1e-8):
         self.step_count += 1
-        for group in ((self.w, self.dw, self.mw, self.vw), (self.b, self.db, self.mb, self.vb)):
-            for p, g, m, v in zip(*group):
-                _ok(lib().imexlb_nn_adam(_ptr(p), _ptr(g), _ptr(m), _ptr(v), p.numel(), lr, b1, b2, eps,
-                                         self.step_count, None), "adam")
+        _ok(lib().imexlb_nn_adam(_ptr(self.flat), _ptr(self.grads), _ptr(self.mom1), _ptr(self.mom2),
+                                 self.flat.numel(), lr, b1, b2, eps, self.step_count, None), "adam")
 
     def params_numpy(self):
         return [(w.cpu().numpy().astype(np.float64), b.cpu().numpy().astype(np.float64)) for w, b in zip(self.w, self.b)]

@@ -17,6 +17,17 @@ extern "C" {
  * w is [CO][CI][3][3]; bias may be NULL; relu: 1 applies max(0, .). */
 int imexlb_nn_conv3x3(const float *in, const float *w, const float *bias, float *out, int N, int CI, int CO, int H,
                       int W, int relu, void *stream);
+/* The same into channels [ooff, ooff+CO) of out [N][ototal][H][W] (a skip
+ * connection written straight into the decoder's concatenated input). */
+int imexlb_nn_conv3x3_into(const float *in, const float *w, const float *bias, float *out, int ototal, int ooff, int N,
+                           int CI, int CO, int H, int W, int relu, void *stream);
+/* Data gradient of a layer from CI to CO channels, weights w [CO][CI][3][3]:
+ * dx[n,ci] = sum_co flipped w[co,ci] (*) dz[n,co], equal bit for bit to
+ * imexlb_nn_conv3x3 with imexlb_nn_flip_weights.  With a gate
+ * [N][gtotal][H][W], the layer's input activations at channels [goff,
+ * goff+CI), dx is 0 where they are not positive (the ReLU that made them). */
+int imexlb_nn_conv3x3_dgrad(const float *dz, const float *w, const float *gate, int gtotal, int goff, float *dx, int N,
+                            int CI, int CO, int H, int W, void *stream);
 /* wt[ci][co][2-ky][2-kx] = w[co][ci][ky][kx]: with it, imexlb_nn_conv3x3 of
  * the output gradient gives the input gradient. */
 int imexlb_nn_flip_weights(const float *w, float *wt, int CI, int CO, void *stream);
@@ -43,6 +54,10 @@ int imexlb_nn_conv3x3_dw_ordered(const float *in, const float *dout, float *dw, 
  * (several streams or threads) share the array and race: serialise them. */
 int imexlb_nn_conv3x3_dw_ordered_noalloc(const float *in, const float *dout, float *dw, int N, int CI, int CO,
                                          int H, int W, void *stream);
+/* imexlb_nn_conv3x3_dw_ordered and imexlb_nn_bias_grad in one launch (the
+ * same bits) */
+int imexlb_nn_conv3x3_grads(const float *in, const float *dout, float *dw, float *db, float *work, int64_t work_floats,
+                            int N, int CI, int CO, int H, int W, void *stream);
 /* db[c] = sum of dout[:, c] */
 int imexlb_nn_bias_grad(const float *dout, float *db, int N, int C, int H, int W, void *stream);
 /* dz = dout where out > 0, else 0 (out: the ReLU output) */
@@ -50,10 +65,21 @@ int imexlb_nn_relu_bwd(const float *out, const float *dout, float *dz, int64_t n
 /* 2x2 average pool, in [N][C][2h][2w] -> out [N][C][h][w], and its gradient */
 int imexlb_nn_pool2(const float *in, float *out, int N, int C, int h, int w, void *stream);
 int imexlb_nn_pool2_bwd(const float *dout, float *din, int N, int C, int h, int w, void *stream);
+/* The pool of channels [coff, coff+C) of in [N][Ctot][2h][2w]; the pool's
+ * gradient plus a skip connection's (channels [soff, soff+C) of skip
+ * [N][stotal][2h][2w]; may be NULL), 0 where the gate (channels [goff,
+ * goff+C) of [N][gtotal][2h][2w]; may be NULL) is not positive */
+int imexlb_nn_pool2_from(const float *in, int Ctot, int coff, float *out, int N, int C, int h, int w, void *stream);
+int imexlb_nn_pool2_bwd_join(const float *dout, const float *skip, int stotal, int soff, const float *gate, int gtotal,
+                             int goff, float *din, int N, int C, int h, int w, void *stream);
 /* nearest 2x upsample of in [N][C][h][w] into channels [coff, coff+C) of
- * out [N][Ctot][2h][2w], and its gradient (din overwritten) */
+ * out [N][Ctot][2h][2w], and its gradient (din overwritten; the second form:
+ * 0 where the gate, channels [goff, goff+C) of [N][gtotal][h][w], is not
+ * positive) */
 int imexlb_nn_up2(const float *in, float *out, int N, int C, int h, int w, int Ctot, int coff, void *stream);
 int imexlb_nn_up2_bwd(const float *dout, float *din, int N, int C, int h, int w, int Ctot, int coff, void *stream);
+int imexlb_nn_up2_bwd_gate(const float *dout, int Ctot, int coff, const float *gate, int gtotal, int goff, float *din,
+                           int N, int C, int h, int w, void *stream);
 /* dst[:, dcoff+c] = src[:, scoff+c] (accumulate: +=), c < C; src has sctot
  * channels, dst dctot */
 int imexlb_nn_copy_channels(const float *src, int sctot, int scoff, float *dst, int dctot, int dcoff, int N, int C,

@@ -161,3 +161,85 @@ def test_mse(n):
     ref = 0.5 + np.mean(d.astype(np.float64) ** 2)
     # each term rounded twice, at most 128 additions to the loss
     assert abs(loss.item() - ref) <= 130 * 2.0 ** -24 * ref
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1, 1), (2, 5, 33, 9, 33), (1, 40, 7, 6, 16), (1, 17, 64, 70, 31),
+                                   (9, 32, 65, 121, 64)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_data_gradient_equals_flipped_convolution(shape, gated):
+    import torch
+    N, ci, co, H, W = shape
+    g = torch.Generator("cuda").manual_seed(10)
+    r = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    dz, w, gate = r(N, co, H, W), r(co, ci, 3, 3), r(N, ci + 5, H, W)
+    wt, ref, dx = torch.empty(ci, co, 3, 3, device="cuda"), r(N, ci, H, W), r(N, ci, H, W)
+    _call("flip_weights", w, wt, ci, co)
+    _call("conv3x3", dz, wt, None, ref, N, co, ci, H, W, 0)
+    _call("conv3x3_dgrad", dz, w, gate if gated else None, ci + 5, 3, dx, N, ci, co, H, W)
+    if gated:
+        ref = torch.where(gate[:, 3:3 + ci] > 0, ref, torch.zeros_like(ref))
+    assert torch.equal(dx, ref)
+
+
+@pytest.mark.parametrize("shape", [(2, 5, 33, 9, 33), (1, 40, 70, 6, 16), (3, 17, 18, 70, 31)])
+def test_joined_entries_equal_their_parts(shape):
+    """Output into a channel slice; weight and bias gradient in one launch."""
+    import torch
+    from imexlb._lib import lib
+    N, ci, co, H, W = shape
+    g = torch.Generator("cuda").manual_seed(11)
+    r = lambda *s: torch.randn(s, generator=g, device="cuda")  # noqa: E731
+    x, w, b, dz = r(N, ci, H, W), r(co, ci, 3, 3), r(co), r(N, co, H, W)
+    ref, wide = torch.empty(N, co, H, W, device="cuda"), r(N, co + 9, H, W)
+    keep = wide.clone()
+    _call("conv3x3", x, w, b, ref, N, ci, co, H, W, 1)
+    _call("conv3x3_into", x, w, b, wide, co + 9, 4, N, ci, co, H, W, 1)
+    assert torch.equal(wide[:, 4:4 + co], ref)
+    assert torch.equal(wide[:, :4], keep[:, :4]) and torch.equal(wide[:, 4 + co:], keep[:, 4 + co:])
+    n = lib().imexlb_nn_conv3x3_dw_work(ci, co, H, W)
+    work = torch.empty(n, device="cuda")
+    dw, dw2 = torch.zeros_like(w), torch.zeros_like(w)
+    db, db2 = torch.empty_like(b), torch.empty_like(b)
+    _call("conv3x3_dw_ordered", x, dz, dw, work, n, N, ci, co, H, W)
+    _call("bias_grad", dz, db, N, co, H, W)
+    _call("conv3x3_grads", x, dz, dw2, db2, work, n, N, ci, co, H, W)
+    assert torch.equal(dw, dw2) and torch.equal(db, db2)
+
+
+# odd and even widths, one pixel, rows longer than a wave's 128 pixels, more
+# rows than blocks of a small launch; buffers that start off 16 bytes
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (2, 3, 5, 7), (1, 4, 3, 64), (2, 5, 2, 131), (1, 3, 9, 258)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_pooling_and_upsampling(shape, shift):
+    import torch
+    N, C_, h, w = shape
+    g = torch.Generator("cuda").manual_seed(12)
+
+    def r(*s):
+        n = int(np.prod(s))
+        return torch.randn(n + shift, generator=g, device="cuda")[shift:].view(s)
+
+    f = np.float32
+    big, low = r(N, C_ + 6, 2 * h, 2 * w), r(N, C_, h, w)
+    B, Lo = big.cpu().numpy(), low.cpu().numpy()
+    sl = B[:, 4:4 + C_]
+    quad = ((sl[..., 0::2, 0::2] + sl[..., 0::2, 1::2]) + (sl[..., 1::2, 0::2] + sl[..., 1::2, 1::2]))
+    out = r(N, C_, h, w)
+    _call("pool2_from", big, C_ + 6, 4, out, N, C_, h, w)
+    assert np.array_equal(out.cpu().numpy(), f(0.25) * quad)
+    gate = r(N, C_ + 2, h, w)
+    _call("up2_bwd_gate", big, C_ + 6, 4, gate, C_ + 2, 1, out, N, C_, h, w)
+    assert np.array_equal(out.cpu().numpy(), np.where(gate.cpu().numpy()[:, 1:1 + C_] > 0, quad, f(0)))
+    _call("up2_bwd", big, out, N, C_, h, w, C_ + 6, 4)
+    assert np.array_equal(out.cpu().numpy(), quad)
+    din, gate2 = r(N, C_, 2 * h, 2 * w), r(N, C_ + 1, 2 * h, 2 * w)
+    spread = f(0.25) * Lo.repeat(2, 2).repeat(2, 3)
+    _call("pool2_bwd", low, din, N, C_, h, w)
+    assert np.array_equal(din.cpu().numpy(), spread)
+    _call("pool2_bwd_join", low, big, C_ + 6, 4, gate2, C_ + 1, 1, din, N, C_, h, w)
+    assert np.array_equal(din.cpu().numpy(), np.where(gate2.cpu().numpy()[:, 1:] > 0, spread + sl, f(0)))
+    wide = r(N, C_ + 3, 2 * h, 2 * w)
+    keep = wide.cpu().numpy()
+    _call("up2", low, wide, N, C_, h, w, C_ + 3, 2)
+    keep[:, 2:2 + C_] = Lo.repeat(2, 2).repeat(2, 3)
+    assert np.array_equal(wide.cpu().numpy(), keep)
