@@ -9,20 +9,12 @@
 // the batch on the matrix cores, and the tiles' sums are added in order or
 // with atomics.
 //
-// Inference in BF16: activations NHWC bf16, weights packed
+// Inference in BF16 (k_conv3_bf16): activations NHWC bf16, weights packed
 // [CI/8][tap][CO][8 ci] bf16, products on the matrix cores
 // (v_mfma_f32_32x32x16_bf16, FP32 accumulation), bias, ReLU and the
-// rounding to bf16 (round to nearest even) fused into the store.  One block
-// computes 8x16 pixels for 32 output channels, one 32-pixel row pair per
-// wave; the input tile with its halo and the block's weights go through LDS
-// 16 channels at a time (15 KB), stored in 16-byte groups of 8 channels so
-// that every lane's operand is one 128-bit LDS read and the 32 lanes of a
-// half-wave read consecutive groups.  The small blocks keep up to 8 of them
-// on a CU, which hides the staging better than larger blocks with more
-// products per chunk (measured: 32- or 64-channel chunks and 64-channel
-// blocks run 15-20 % slower).  Skip connections cost no copy: an
-// encoder convolution writes into its channel slice of the decoder's
-// concatenated input (output channel stride and offset).
+// rounding to bf16 (round to nearest even) fused into the store, with the
+// pooled copy; a decoder layer reads the upsampled and the skip channels from
+// their own buffers.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -669,97 +661,362 @@ __device__ __forceinline__ uint16_t to_bf16(float f)
     return uint16_t(u >> 16);
 }
 
+// two values to bf16 in one instruction, the same rounding (NaN quiet)
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack2(float a, float b)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, bf16x2));
+}
+
 __device__ __forceinline__ float from_bf16(uint32_t h) { return __uint_as_float(h << 16); }
 
-constexpr int PR = 8, PC = 16;  // pixel tile of the BF16 convolution: 8 rows x 16 columns
-
-// KC input channels per LDS chunk (16 or 32), BN output channels per block
-// (32 or 64).  in: [N][H][W][CIP] bf16 as 16-byte groups; wp: [CIP/8][9][COP]
-// groups of 8 input channels.  Output channel co < CO of pixel (n, y, x):
-// bf16 at out[((n H + y) W + x) ostride + ooff + co], or with f32_nchw FP32
-// at out[((n CO + co) H + y) W + x].
-template <int KC, int BN>
-__global__ __launch_bounds__(256) void k_conv3_bf16(const uint4 *__restrict__ in, const uint4 *__restrict__ wp,
-                                                    const float *__restrict__ bias, void *__restrict__ out, int H,
-                                                    int W, int CIP, int CO, int COP, int ostride, int ooff, int relu,
-                                                    int f32_nchw)
+// average of four pixels' 8 channels, in FP32, rounded to bf16
+__device__ __forceinline__ uint4 average4(uint4 a, uint4 b, uint4 c, uint4 d)
 {
-    constexpr int G = KC / 8;  // channel groups per chunk
-    constexpr int NT = BN / 32;
-    __shared__ uint4 s_in[G][PR + 2][PC + 2];
-    __shared__ uint4 s_w[9][G][BN];
-    const int lane = int(threadIdx.x) % 64, wave = int(threadIdx.x) / 64;
-    const int ntx = (W + PC - 1) / PC;
-    const int x0 = int(blockIdx.x) % ntx * PC, y0 = int(blockIdx.x) / ntx * PR;
-    const int co0 = int(blockIdx.y) * BN, n = int(blockIdx.z);
-    const int cg = CIP / 8;
-    const int m = lane % 32, hk = lane / 32;        // operand row (pixel / channel) and K half
-    const int pr = wave * 2 + m / 16, pc = m % 16;  // this lane's pixel in the tile
-    f32x16 acc[NT];
+    const uint4 v[4] = {a, b, c, d};
+    uint32_t o[4];
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int k = 0; k < 4; ++k) {
+        float avg[2];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) acc[t][j] = 0.0f;
-    const int64_t img = int64_t(n) * H;
-    for (int c0 = 0; c0 < CIP; c0 += KC) {
-        for (int e = int(threadIdx.x); e < (PR + 2) * (PC + 2) * G; e += 256) {
-            const int g = e % G, p = e / G;
-            const int r = p / (PC + 2), c = p % (PC + 2);
-            const int yy = y0 + r - 1, xx = x0 + c - 1;
-            uint4 v = make_uint4(0u, 0u, 0u, 0u);
-            if (yy >= 0 && yy < H && xx >= 0 && xx < W) v = in[((img + yy) * W + xx) * cg + c0 / 8 + g];
-            s_in[g][r][c] = v;
-        }
-        for (int e = int(threadIdx.x); e < 9 * G * BN; e += 256) {
-            const int co = e % BN, t = (e / BN) % 9, g = e / (9 * BN);
-            s_w[t][g][co] = wp[(int64_t(c0 / 8 + g) * 9 + t) * COP + co0 + co];
-        }
-        __syncthreads();
+        for (int half = 0; half < 2; ++half) {
+            float s[4];
 #pragma unroll
-        for (int t = 0; t < 9; ++t)
-#pragma unroll
-            for (int s = 0; s < KC / 16; ++s) {
-                const bf16x8 a = __builtin_bit_cast(bf16x8, s_in[2 * s + hk][pr + t / 3][pc + t % 3]);
-#pragma unroll
-                for (int q = 0; q < NT; ++q) {
-                    const bf16x8 b = __builtin_bit_cast(bf16x8, s_w[t][2 * s + hk][q * 32 + m]);
-                    acc[q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[q], 0, 0, 0);
-                }
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t word = k == 0 ? v[q].x : k == 1 ? v[q].y : k == 2 ? v[q].z : v[q].w;
+                s[q] = from_bf16(half ? word >> 16 : word & 0xffffu);
             }
-        __syncthreads();
-    }
-    // lane holds D[pixel 8 (j/4) + 4 hk + j%4][channel m] of each 32x32 tile
-#pragma unroll
-    for (int q = 0; q < NT; ++q) {
-        const int co = co0 + q * 32 + m;
-        if (co >= CO) continue;
-        const float bv = bias ? bias[co] : 0.0f;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int px = 8 * (j / 4) + 4 * hk + j % 4;
-            const int y = y0 + wave * 2 + px / 16, x = x0 + px % 16;
-            if (y >= H || x >= W) continue;
-            float v = acc[q][j] + bv;
-            if (relu) v = v > 0.0f ? v : 0.0f;
-            if (f32_nchw)
-                static_cast<float *>(out)[((int64_t(n) * CO + co) * H + y) * W + x] = v;
-            else
-                static_cast<uint16_t *>(out)[((img + y) * W + x) * ostride + ooff + co] = to_bf16(v);
+            avg[half] = 0.25f * ((s[0] + s[1]) + (s[2] + s[3]));
         }
+        o[k] = pack2(avg[0], avg[1]);
+    }
+    return make_uint4(o[0], o[1], o[2], o[3]);
+}
+
+// slot of 8-channel group g of the pixel in column c, in the pixel's run of G
+// slots in LDS: turned by the column so that 8 neighbours' slots of one group
+// fall in different banks
+template <int G>
+__device__ __forceinline__ int turn(int g, int c)
+{
+    return G == 4 ? g ^ ((c >> 1) & 3) : g ^ ((c >> 2) & 1);
+}
+
+// The store of a tile of MT groups of 32 pixels and 32 channels per wave, WY
+// waves down and 4 / WY across the channels: bias, ReLU, and for bf16 output
+// through LDS (every wave's reads of it are over) so that the stores are 16
+// bytes wide, with the pooled copy if asked for.
+template <int MT, int WY, int TC>
+__device__ __forceinline__ void conv_store(const f32x16 (&acc)[MT], uint4 *sh, const float *__restrict__ bias,
+                                           void *__restrict__ out, uint16_t *__restrict__ pool, int H, int W, int CO,
+                                           int ostride, int ooff, int relu, int f32_nchw, int vec, int n, int y0,
+                                           int x0, int cob)
+{
+    constexpr int GR = 32 / TC, WC = 4 / WY, TR = WY * MT * GR, kOut = TR * TC * 4 * WC;
+    const int tid = int(threadIdx.x), lane = tid % 64, wave = tid / 64, m = lane % 32, hk = lane / 32;
+    const int wy = wave % WY, wc = wave / WY, co0 = cob + 32 * wc;
+    // lane holds D[channel 8 (j/4) + 4 hk + j%4][pixel m] of each 32x32 tile
+    float bv[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const int co = co0 + 8 * (j / 4) + 4 * hk + j % 4;
+        bv[j] = bias && co < CO ? bias[co] : 0.0f;
+    }
+    const auto value = [&](int t, int j) {
+        const float v = acc[t][j] + bv[j];
+        return relu ? __builtin_fmaxf(v, 0.0f) : v;
+    };
+    if (f32_nchw) {
+        const int x = x0 + m % TC;
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            const int y = y0 + (wy * MT + t) * GR + m / TC;
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const int co = co0 + 8 * (j / 4) + 4 * hk + j % 4;
+                if (co < CO && y < H && x < W)
+                    static_cast<float *>(out)[((int64_t(n) * CO + co) * H + y) * W + x] = value(t, j);
+            }
+        }
+        return;
+    }
+    // slot 4 p + group of each of the WC channel blocks
+    __syncthreads();
+    uint2 *const so = reinterpret_cast<uint2 *>(sh + wc * (TR * TC * 4));
+#pragma unroll
+    for (int t = 0; t < MT; ++t) {
+        const int p = (wy * MT + t) * 32 + m;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            so[(4 * p + turn<4>(q, p)) * 2 + hk] = make_uint2(pack2(value(t, 4 * q), value(t, 4 * q + 1)),
+                                                              pack2(value(t, 4 * q + 2), value(t, 4 * q + 3)));
+        }
+    }
+    __syncthreads();
+    uint16_t *const o = static_cast<uint16_t *>(out);
+    for (int e = tid; e < kOut; e += 256) {
+        const int b = e / (TR * TC * 4), p = e / 4 % (TR * TC), g = e % 4;
+        const int y = y0 + p / TC, x = x0 + p % TC, co = cob + 32 * b + 8 * g;
+        if (y >= H || x >= W || co >= CO) continue;
+        const uint4 v = sh[b * (TR * TC * 4) + 4 * p + turn<4>(g, p)];
+        uint16_t *const d = o + ((int64_t(n) * H + y) * W + x) * ostride + ooff + co;
+        if (vec) {
+            *reinterpret_cast<uint4 *>(d) = v;
+        } else {
+            const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (co + k < CO) d[k] = uint16_t(w4[k / 2] >> (16 * (k % 2)));
+        }
+    }
+    if (!pool) return;
+    for (int e = tid; e < kOut / 4; e += 256) {
+        const int b = e / (TR * TC), q = e / 4 % (TR * TC / 4), g = e % 4;
+        const int py = q / (TC / 2), px = q % (TC / 2), p = 2 * py * TC + 2 * px;
+        const int y = y0 / 2 + py, x = x0 / 2 + px, co = cob + 32 * b + 8 * g;
+        if (y >= H / 2 || x >= W / 2 || co >= CO) continue;
+        const uint4 *const t = sh + b * (TR * TC * 4);
+        *reinterpret_cast<uint4 *>(pool + ((int64_t(n) * (H / 2) + y) * (W / 2) + x) * CO + co) =
+            average4(t[4 * p + turn<4>(g, p)], t[4 * (p + 1) + turn<4>(g, p + 1)],
+                     t[4 * (p + TC) + turn<4>(g, p + TC)], t[4 * (p + TC + 1) + turn<4>(g, p + TC + 1)]);
     }
 }
 
-// x [N][C][H][W] FP32 -> y [N][H][W][CP] bf16, channels C..CP-1 zero
-__global__ void k_pack_in(const float *__restrict__ x, uint16_t *__restrict__ y, int C, int CP, int H, int W,
-                          int64_t total)
+// Every sum takes its products in one order, 16 input channels after
+// another and tap after tap, whatever the tile.  A plain tile (one 32-pixel
+// operand read per product, weights and pixels through LDS) was bound by
+// LDS reads: 2 KB per product and wave, twice what LDS gives in the 32 cycles
+// of a product.  Here a wave takes MT groups of rows and holds the 9 taps'
+// weights of 16 channels in registers, so that a row read once serves as the
+// upper, middle and lower row of three groups: 0.5 KB per product.  The
+// input goes from memory straight to LDS; two or three blocks on a CU hide
+// one another's waits.  40 cases on 128 x 512: 384 -> 128 channels 210 to
+// 127 us (1,140 TFLOP/s), 256 -> 256 81 to 52 us, 32 -> 32 (bound by memory,
+// 336 MB) 153 to 97 us; the whole network 2.20 to 1.13 ms.
+//
+// 3x3 convolution, padding 1, NHWC bf16.  Input channels [0, C0) come from
+// in0 at half the resolution (nearest upsampling), the following C1 from in1;
+// wp: [CIP/8][9][COP] groups of 8 input channels.  Output channel co < CO of
+// pixel (n, y, x): bf16 at out[((n H + y) W + x) ostride + ooff + co], or with
+// f32_nchw FP32 at out[((n CO + co) H + y) W + x]; with pool also the 2x2
+// average of the bf16 values at pool[((n H/2 + y/2) W/2 + x/2) CO + co].
+template <int MT, int WY, int TC, int KC>
+__global__ __launch_bounds__(256, MT == 4 ? 3 : 4) void k_conv3_bf16(const uint4 *__restrict__ in0, int C0,
+                                                    const uint4 *__restrict__ in1, int C1,
+                                                    const uint4 *__restrict__ wp, const float *__restrict__ bias,
+                                                    void *__restrict__ out, uint16_t *__restrict__ pool, int H, int W,
+                                                    int CO, int COP, int ostride, int ooff, int relu, int f32_nchw,
+                                                    int vec, uint32_t ntx, uint32_t nty, uint32_t ncob)
 {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    constexpr int G = KC / 8, GR = 32 / TC, WC = 4 / WY;
+    constexpr int TR = WY * MT * GR, IR = TR + 2, IC = TC + 2, NPX = IR * IC;
+    constexpr int NI = (NPX * G + 255) / 256;
+    constexpr int kIn = NPX * G, kOut = TR * TC * 4 * WC;
+    __shared__ uint4 sh[kIn > kOut ? kIn : kOut];
+    const int tid = int(threadIdx.x), lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int m = lane % 32, hk = lane / 32;  // operand row / column and K half
+    const int wy = wave % WY, wc = wave / WY;
+    uint32_t blk = xcd_run(blockIdx.x, gridDim.x);
+    const int cob = int(blk % ncob) * (32 * WC);
+    blk /= ncob;
+    const int x0 = int(blk % ntx) * TC;
+    blk /= ntx;
+    const int y0 = int(blk % nty) * TR, n = int(blk / nty);
+    const int co0 = cob + 32 * wc;
+
+    // staging, straight to LDS in 16-byte slots (slot e of the block is lane
+    // e % 64's of its wave's load e / 256); slots outside the image stay
+    // zero.  A slot's pixel is kept as row and column of the tile, -1 where
+    // there is nothing to load.
+    int at[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int e = tid + 256 * i, p = e / G, r = p / IC, c = p % IC;
+        const int yy = y0 + r - 1, xx = x0 + c - 1;
+        const bool ok = e < kIn && yy >= 0 && yy < H && xx >= 0 && xx < W;
+        at[i] = ok ? r << 8 | c : -1;
+        if (e < kIn && !ok) sh[e] = make_uint4(0u, 0u, 0u, 0u);
+    }
+    const uint4 *const t1 = in1 + ((int64_t(n) * H + y0) * W + x0) * (C1 / 8);
+    const uint4 *const t0 = C0 ? in0 + ((int64_t(n) * (H / 2) + y0 / 2) * (W / 2) + x0 / 2) * (C0 / 8) : nullptr;
+    int pa[3];  // the lane's pixel operand of tap column kx, row 0, first group
+#pragma unroll
+    for (int kx = 0; kx < 3; ++kx)
+        pa[kx] = ((wy * MT * GR + m / TC) * IC + m % TC + kx) * G + turn<G>(hk, m % TC + kx);
+    f32x16 acc[MT] = {};
+    const int CIP = C0 + C1;
+    for (int c0 = 0; c0 < CIP; c0 += KC) {
+        __syncthreads();  // the previous channels have been multiplied
+        const auto stage = [&](const uint4 *base, int stride, int half, int w) {
+#pragma unroll
+            for (int i = 0; i < NI; ++i)
+                if (at[i] >= 0) {
+                    const int r = (at[i] >> 8) - 1 >> half, c = (at[i] & 255) - 1 >> half;
+                    const int g = turn<G>(tid % G, at[i] & 255);
+                    __builtin_amdgcn_global_load_lds(
+                        (const __attribute__((address_space(1))) void *)(base + int64_t(r * w + c) * stride + g),
+                        (__attribute__((address_space(3))) void *)(sh + 256 * i + 64 * wave), 16, 0, 0);
+                }
+        };
+        if (c0 < C0)
+            stage(t0 + c0 / 8, C0 / 8, 1, W / 2);
+        else
+            stage(t1 + (c0 - C0) / 8, C1 / 8, 0, W);
+        // the weights of 16 channels: every lane its output channel's 8 of K
+        bf16x8 wf[9];
+        auto weights = [&](int c) {
+            const uint4 *const p = wp + (int64_t(c / 8 + hk) * 9) * COP + co0 + m;
+#pragma unroll
+            for (int t = 0; t < 9; ++t) wf[t] = __builtin_bit_cast(bf16x8, p[int64_t(t) * COP]);
+        };
+        weights(c0);
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's slots are in LDS
+        __syncthreads();
+#pragma unroll
+        for (int cc = 0; cc < KC / 16; ++cc) {
+            if (cc > 0) weights(c0 + 16 * cc);
+            // input rows in order; each serves the (up to three) groups of
+            // output rows that it is the upper, middle or lower row of, so
+            // every sum takes its taps in order
+#pragma unroll
+            for (int s = 0; s < (MT - 1) * GR + 3; ++s)
+#pragma unroll
+                for (int kx = 0; kx < 3; ++kx) {
+                    const bf16x8 a = __builtin_bit_cast(bf16x8, sh[(pa[kx] ^ 2 * cc) + s * IC * G]);
+#pragma unroll
+                    for (int ky = 0; ky < 3; ++ky)
+                        if ((s - ky) % GR == 0 && s - ky >= 0 && (s - ky) / GR < MT)
+                            acc[(s - ky) / GR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[3 * ky + kx], a,
+                                                                                         acc[(s - ky) / GR], 0, 0, 0);
+                }
+        }
+    }
+    conv_store<MT, WY, TC>(acc, sh, bias, out, pool, H, W, CO, ostride, ooff, relu, f32_nchw, vec, n, y0, x0, cob);
+}
+
+// The same for few tiles (a block or less per CU), where the time is that of
+// one block's chain of chunks: input and weights of the next three chunks
+// are on their way to LDS while one is multiplied.  Every wave issues the
+// same number of loads per chunk (a slot with nothing to load takes zeros),
+// so it can wait for the oldest chunk alone.
+__device__ const uint4 zero_slot = {0u, 0u, 0u, 0u};
+template <int TC, int KC>
+__global__ __launch_bounds__(256) void k_conv3_bf16_deep(const uint4 *__restrict__ in0, int C0,
+                                                         const uint4 *__restrict__ in1, int C1,
+                                                         const uint4 *__restrict__ wp, const float *__restrict__ bias,
+                                                         void *__restrict__ out, uint16_t *__restrict__ pool, int H,
+                                                         int W, int CO, int COP, int ostride, int ooff, int relu,
+                                                         int f32_nchw, int vec, uint32_t ntx, uint32_t nty,
+                                                         uint32_t ncob)
+{
+    constexpr int G = KC / 8, GR = 32 / TC, TR = 4 * GR, IR = TR + 2, IC = TC + 2;
+    constexpr int kIn = IR * IC * G, NI = (kIn + 255) / 256, kW = 9 * G * 32, NW = (kW + 255) / 256;
+    constexpr int kBuf = (NI + NW) * 256, ND = 4;
+    __shared__ uint4 sh[ND * kBuf];
+    const int tid = int(threadIdx.x), lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int m = lane % 32, hk = lane / 32;
+    uint32_t blk = xcd_run(blockIdx.x, gridDim.x);
+    const int co0 = int(blk % ncob) * 32;
+    blk /= ncob;
+    const int x0 = int(blk % ntx) * TC;
+    blk /= ntx;
+    const int y0 = int(blk % nty) * TR, n = int(blk / nty);
+    const uint4 *const t1 = in1 + ((int64_t(n) * H + y0) * W + x0) * (C1 / 8);
+    const uint4 *const t0 = C0 ? in0 + ((int64_t(n) * (H / 2) + y0 / 2) * (W / 2) + x0 / 2) * (C0 / 8) : nullptr;
+    const auto put = [&](const uint4 *a, uint4 *d) {
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)a,
+                                         (__attribute__((address_space(3))) void *)d, 16, 0, 0);
+    };
+    const auto stage = [&](int c0, int buf) {
+        uint4 *const d = sh + buf * kBuf + 64 * wave;
+        const bool low = c0 < C0;
+        const uint4 *const base = low ? t0 + c0 / 8 : t1 + (c0 - C0) / 8;
+        const int stride = (low ? C0 : C1) / 8, w = low ? W / 2 : W, half = low ? 1 : 0;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int e = tid + 256 * i, p = e / G, r = p / IC - 1, c = p % IC - 1;
+            const bool ok = e < kIn && unsigned(y0 + r) < unsigned(H) && unsigned(x0 + c) < unsigned(W);
+            const int64_t o = int64_t((r >> half) * w + (c >> half)) * stride + turn<G>(tid % G, c + 1);
+            put(ok ? base + o : &zero_slot, d + 256 * i);
+        }
+        const uint4 *const wb = wp + int64_t(c0 / 8) * 9 * COP + co0;
+#pragma unroll
+        for (int i = 0; i < NW; ++i) {
+            const int e = tid + 256 * i;
+            put(e < kW ? wb + int64_t(e / 32) * COP + e % 32 : &zero_slot, d + 256 * (NI + i));
+        }
+    };
+    int pa[3];
+#pragma unroll
+    for (int kx = 0; kx < 3; ++kx)
+        pa[kx] = ((wave * GR + m / TC) * IC + m % TC + kx) * G + turn<G>(hk, m % TC + kx);
+    f32x16 acc[1] = {};
+    const int nst = (C0 + C1) / KC;
+#pragma unroll
+    for (int k = 0; k < ND - 1; ++k)
+        if (k < nst) stage(k * KC, k);
+    for (int st = 0; st < nst; ++st) {
+        // this chunk has arrived once only the later ones' loads are out
+        const int later = min(ND - 2, nst - 1 - st);
+        static_assert(ND == 4 && 2 * (NI + NW) < 64, "the counts below");
+        constexpr int v2 = 2 * (NI + NW), v1 = NI + NW;
+        if (later == 2)
+            __builtin_amdgcn_s_waitcnt(0x0f70 | (v2 & 15) | (v2 >> 4) << 14);
+        else if (later == 1)
+            __builtin_amdgcn_s_waitcnt(0x0f70 | (v1 & 15) | (v1 >> 4) << 14);
+        else
+            __builtin_amdgcn_s_waitcnt(0x0f70);
+        // for every wave; and the previous chunk has been multiplied.  (Not
+        // __syncthreads(), whose fence waits for the later chunks too.)
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (st + ND - 1 < nst) stage((st + ND - 1) * KC, (st + ND - 1) % ND);
+        const uint4 *const si = sh + st % ND * kBuf, *const sw = si + 256 * NI;
+        // operands read three products ahead
+        constexpr int NP = KC / 16 * 9, AH = 3;
+        bf16x8 a[AH + 1], b[AH + 1];
+        const auto fetch = [&](int q) {
+            const int cc = q / 9, t = q % 9;
+            a[q % (AH + 1)] = __builtin_bit_cast(bf16x8, sw[((2 * cc + hk) * 9 + t) * 32 + m]);
+            b[q % (AH + 1)] = __builtin_bit_cast(bf16x8, si[(pa[t % 3] ^ 2 * cc) + t / 3 * IC * G]);
+        };
+#pragma unroll
+        for (int q = 0; q < AH; ++q) fetch(q);
+        __builtin_amdgcn_sched_group_barrier(0x100, 2 * AH, 0);
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            if (q + AH < NP) fetch(q + AH);
+            acc[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[q % (AH + 1)], b[q % (AH + 1)], acc[0], 0, 0, 0);
+            if (q + AH < NP) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
+    }
+    __syncthreads();
+    conv_store<1, 4, TC>(acc, sh, bias, out, pool, H, W, CO, ostride, ooff, relu, f32_nchw, vec, n, y0, x0, co0);
+}
+
+// x [N][C][H][W] FP32 -> y [N][H][W][CP] bf16, channels C..CP-1 zero; K
+// channels per thread (8 where CP is a multiple of 8: one 16-byte store)
+template <int K>
+__global__ __launch_bounds__(256) void k_pack_in(const float *__restrict__ x, uint16_t *__restrict__ y, int C, int CP,
+                                                 int64_t hw, int64_t total)
+{
+    const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
     if (i >= total) return;
-    const int c = int(i % CP);
-    const int64_t p = i / CP;
-    const int64_t hw = int64_t(H) * W;
-    const int64_t n = p / hw, r = p % hw;
-    y[i] = c < C ? to_bf16(x[(n * C + c) * hw + r]) : uint16_t(0);
+    const int cg = CP / K;
+    const int64_t n = i / (hw * cg), j = i - n * hw * cg;
+    const int c = int(j / hw) * K;  // a wave reads consecutive pixels of a channel
+    const int64_t r = j - (c / K) * hw;
+    uint16_t v[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) v[k] = c + k < C ? to_bf16(x[(n * C + c + k) * hw + r]) : uint16_t(0);
+    uint16_t *const o = y + (n * hw + r) * CP + c;
+    if constexpr (K == 8)
+        *reinterpret_cast<uint4 *>(o) =
+            make_uint4(v[0] | uint32_t(v[1]) << 16, v[2] | uint32_t(v[3]) << 16, v[4] | uint32_t(v[5]) << 16,
+                       v[6] | uint32_t(v[7]) << 16);
+    else
+        *o = v[0];
 }
 
 // w [CO][CI][3][3] FP32 -> wp [CIP/8][9][COP][8] bf16, zero outside CO x CI
@@ -785,24 +1042,7 @@ __global__ void k_pool2_bf16(const uint4 *__restrict__ in, uint4 *__restrict__ o
     const int x = int(p % w), y = int((p / w) % h);
     const int64_t n = p / (int64_t(w) * h);
     const int64_t b = ((n * 2 * h + 2 * y) * 2 * w + 2 * x) * cs8 + coff8 + g;
-    const uint4 v[4] = {in[b], in[b + cs8], in[b + 2 * int64_t(w) * cs8], in[b + (2 * int64_t(w) + 1) * cs8]};
-    uint32_t o[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        uint32_t r = 0;
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            float s[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const uint32_t word = k == 0 ? v[q].x : k == 1 ? v[q].y : k == 2 ? v[q].z : v[q].w;
-                s[q] = from_bf16(half ? word >> 16 : word & 0xffffu);
-            }
-            r |= uint32_t(to_bf16(0.25f * ((s[0] + s[1]) + (s[2] + s[3])))) << (16 * half);
-        }
-        o[k] = r;
-    }
-    out[i] = make_uint4(o[0], o[1], o[2], o[3]);
+    out[i] = average4(in[b], in[b + cs8], in[b + 2 * int64_t(w) * cs8], in[b + (2 * int64_t(w) + 1) * cs8]);
 }
 
 // nearest 2x upsample of in [N][h][w][8 C8] into channels [coff, coff + 8 C8)
@@ -1128,8 +1368,11 @@ int imexlb_nn_adam(float *w, const float *g, float *m, float *v, int64_t n, floa
 int imexlb_nn_pack_input_bf16(const float *x, uint16_t *y, int N, int C, int CP, int H, int W, void *stream)
 {
     if (!x || !y || N <= 0 || C <= 0 || CP < C || H <= 0 || W <= 0) return -1;
-    const int64_t total = int64_t(N) * H * W * CP;
-    NN_LAUNCH(k_pack_in, dim3(blocks(total)), dim3(256), 0, (hipStream_t)stream, x, y, C, CP, H, W, total);
+    const int64_t hw = int64_t(H) * W;
+    const bool wide = CP % 8 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0;
+    const int64_t total = N * hw * (wide ? CP / 8 : CP);
+    NN_LAUNCH(wide ? k_pack_in<8> : k_pack_in<1>, dim3(blocks(total)), dim3(256), 0, (hipStream_t)stream, x, y, C, CP,
+              hw, total);
 }
 
 int imexlb_nn_pack_weights_bf16(const float *w, uint16_t *wp, int CI, int CO, int CIP, int COP, void *stream)
@@ -1142,18 +1385,54 @@ int imexlb_nn_pack_weights_bf16(const float *w, uint16_t *wp, int CI, int CO, in
 int imexlb_nn_conv3x3_bf16(const uint16_t *in, const uint16_t *wp, const float *bias, void *out, int N, int CIP,
                            int CO, int COP, int H, int W, int ostride, int ooff, int relu, int f32_nchw, void *stream)
 {
-    if (!in || !wp || !out || N <= 0 || N > 65535 || H <= 0 || W <= 0 || CIP <= 0 || CIP % 16 || CO <= 0 ||
-        COP < CO || COP % 32)
+    return imexlb_nn_conv3x3_bf16_join(nullptr, 0, in, CIP, wp, bias, out, nullptr, N, CO, COP, H, W, ostride, ooff,
+                                       relu, f32_nchw, stream);
+}
+
+int imexlb_nn_conv3x3_bf16_join(const uint16_t *low, int CL, const uint16_t *in, int CI, const uint16_t *wp,
+                                const float *bias, void *out, uint16_t *pool, int N, int CO, int COP, int H, int W,
+                                int ostride, int ooff, int relu, int f32_nchw, void *stream)
+{
+    if (!in || !wp || !out || N <= 0 || N > 65535 || H <= 0 || W <= 0 || CI <= 0 || CI % 16 || CO <= 0 || COP < CO ||
+        COP % 32)
         return -1;
+    if (low ? CL <= 0 || CL % 16 || H % 2 || W % 2 : CL != 0) return -1;
+    if (pool && (f32_nchw || H % 2 || W % 2 || CO % 8)) return -1;
     if (!f32_nchw && (ooff < 0 || ooff + CO > ostride)) return -1;
-    if ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(wp)) & 15) return -1;
-    const int64_t tiles = int64_t((W + PC - 1) / PC) * ((H + PR - 1) / PR);
-    if (tiles > 0x7fffffff) return -1;
-    const dim3 grid(unsigned(tiles), unsigned(COP / 32), unsigned(N));
-    hipLaunchKernelGGL((k_conv3_bf16<16, 32>), grid, dim3(256), 0, (hipStream_t)stream,
-                       reinterpret_cast<const uint4 *>(in), reinterpret_cast<const uint4 *>(wp), bias, out, H, W, CIP,
-                       CO, COP, ostride, ooff, relu, f32_nchw);
-    return hipGetLastError() == hipSuccess ? 0 : -2;
+    if ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(wp) | reinterpret_cast<uintptr_t>(low) |
+         reinterpret_cast<uintptr_t>(pool)) & 15)
+        return -1;
+    const int vec = CO % 8 == 0 && ostride % 8 == 0 && ooff % 8 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0;
+    const auto count = [&](int rows, int cols, int bn) {
+        return ((int64_t(W) + cols - 1) / cols) * ((int64_t(H) + rows - 1) / rows) * ((COP + bn - 1) / bn) * N;
+    };
+    const auto run = [&](auto kernel, int rows, int cols, int bn) {
+        if (count(rows, cols, bn) > 0x7fffffff) return -1;
+        hipLaunchKernelGGL(kernel, dim3(unsigned(count(rows, cols, bn))), dim3(256), 0, (hipStream_t)stream,
+                           reinterpret_cast<const uint4 *>(low), CL, reinterpret_cast<const uint4 *>(in), CI,
+                           reinterpret_cast<const uint4 *>(wp), bias, out, pool, H, W, CO, COP, ostride, ooff, relu,
+                           f32_nchw, vec, uint32_t((W + cols - 1) / cols), uint32_t((H + rows - 1) / rows),
+                           uint32_t((COP + bn - 1) / bn));
+        return hipGetLastError() == hipSuccess ? 0 : -2;
+    };
+    // 32 channels a chunk where the inputs allow it.  The widest tile that
+    // gives every CU two blocks; for 32 output channels of few input channels
+    // (bound by memory) 16 rows of 16-channel chunks, else 8 rows (40 x 128 x
+    // 512, 32 -> 32 channels 93 against 100 us, 96 -> 32 245 against 229 us).
+    // Below that the chain of chunks is the time: three chunks ahead (a batch
+    // of one on 128 x 512: 118 us for the whole network, 137 with the plain
+    // 4-row tile for the layers of one and two chunks, 223 for all).
+    const bool wide = CI % 32 == 0 && CL % 32 == 0;
+#define CONV_BF16(MT, WY, TC) (wide ? k_conv3_bf16<MT, WY, TC, 32> : k_conv3_bf16<MT, WY, TC, 16>)
+#define CONV_BF16_DEEP(TC) (wide ? k_conv3_bf16_deep<TC, 32> : k_conv3_bf16_deep<TC, 16>)
+    if (W <= 16)
+        return count(8, 16, 32) < 1024 ? run(CONV_BF16_DEEP(16), 8, 16, 32) : run(CONV_BF16(1, 4, 16), 8, 16, 32);
+    if (COP % 64 == 0 && count(8, 32, 64) >= 512) return run(CONV_BF16(4, 2, 32), 8, 32, 64);
+    if (CL + CI <= 32 && count(16, 32, 32) >= 512) return run(k_conv3_bf16<4, 4, 32, 16>, 16, 32, 32);
+    if (count(8, 32, 32) >= 512) return run(CONV_BF16(2, 4, 32), 8, 32, 32);
+    return run(CONV_BF16_DEEP(32), 4, 32, 32);
+#undef CONV_BF16_DEEP
+#undef CONV_BF16
 }
 
 int imexlb_nn_pool2_bf16(const uint16_t *in, uint16_t *out, int N, int C, int h, int w, int cstride, int coff,

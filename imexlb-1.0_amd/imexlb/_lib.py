@@ -102,6 +102,7 @@ SIGNATURES = {
     "imexlb_nn_pack_weights_bf16": (C.c_int, [_P, _P, C.c_int, C.c_int, C.c_int, C.c_int, _P]),
     "imexlb_nn_conv3x3_bf16": (C.c_int, [_P, _P, _P, _P, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int,
                                          C.c_int, C.c_int, C.c_int, C.c_int, _P]),
+    "imexlb_nn_conv3x3_bf16_join": (C.c_int, [_P, C.c_int, _P, C.c_int] + [_P] * 4 + [C.c_int] * 9 + [_P]),
     "imexlb_nn_pool2_bf16": (C.c_int, [_P, _P, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _P]),
     "imexlb_nn_up2_bf16": (C.c_int, [_P, _P, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _P]),
 }

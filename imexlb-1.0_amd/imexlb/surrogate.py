@@ -245,8 +245,10 @@ class UNet:
 
 class UNetBF16:
     """Inference with the weights of a UNet in BF16 on the matrix cores
-    (imexlb_nn_conv3x3_bf16): activations NHWC bf16, every encoder output
-    written straight into its slice of the decoder's concatenated input.
+    (imexlb_nn_conv3x3_bf16_join): activations NHWC bf16; the encoder's
+    second convolutions write their pooled output too, and the decoder's
+    first ones read the upsampled and the skip channels from their own
+    buffers, so nothing is pooled, upsampled or concatenated separately.
     Channel counts must be multiples of 16; the input is padded to 16
     channels.  forward() returns (N, cout, H, W) FP32."""
 
@@ -269,8 +271,7 @@ class UNetBF16:
         e = lambda c, l: torch.empty((N, *hw[l], c), dtype=bf, device=dev)
         self.x = e(self.cinp, 0)
         self.t1 = [e(ch[l], l) for l in range(L)]
-        self.cat = [e(ch[l + 1] + ch[l], l) for l in range(L - 1)]
-        self.bottom = e(ch[L - 1], L - 1)
+        self.enc = [e(ch[l], l) for l in range(L)]
         self.pooled = [None] + [e(ch[l - 1], l) for l in range(1, L)]
         self.dec = [e(ch[l], l) for l in range(L - 1)]
         self.out = torch.empty((N, self.cout, self.H, self.W), dtype=torch.float32, device=dev)
@@ -281,45 +282,36 @@ class UNetBF16:
             _ok(lib().imexlb_nn_pack_weights_bf16(_ptr(self.net.w[k]), _ptr(self.wp[k]), ci, co, self.cip[k],
                                                   self.cop[k], None), "pack weights")
 
-    def _conv(self, k, x, out, level, ostride, ooff, relu=True, f32=False):
+    def _conv(self, k, x, out, level, low=None, pool=None, relu=True, f32=False):
         co, ci = self.net.shapes[k]
-        h, w = self.hw[level]
-        _ok(lib().imexlb_nn_conv3x3_bf16(_ptr(x), _ptr(self.wp[k]), _ptr(self.net.b[k]), _ptr(out), self.N,
-                                         self.cip[k], co, self.cop[k], h, w, ostride, ooff, 1 if relu else 0,
-                                         1 if f32 else 0, None), "conv3x3_bf16")
+        cl = 0 if low is None else low.shape[3]
+        _ok(lib().imexlb_nn_conv3x3_bf16_join(None if low is None else _ptr(low), cl, _ptr(x), self.cip[k] - cl,
+                                              _ptr(self.wp[k]), _ptr(self.net.b[k]), _ptr(out),
+                                              None if pool is None else _ptr(pool), self.N, co, self.cop[k],
+                                              *self.hw[level], co, 0, 1 if relu else 0, 1 if f32 else 0, None),
+            "conv3x3_bf16")
 
     def forward(self, x):
         """x: (N, cin, H, W) contiguous FP32 device tensor."""
         if tuple(x.shape) != (self.N, self.net.cin, self.H, self.W) or x.dtype != self.t.float32 \
                 or not x.is_contiguous():
             raise ValueError(f"input must be a contiguous float32 ({self.N}, {self.net.cin}, {self.H}, {self.W})")
-        L, ch, N = len(self.chans), self.chans, self.N
+        L, N = len(self.chans), self.N
         _ok(lib().imexlb_nn_pack_input_bf16(_ptr(x), _ptr(self.x), N, self.net.cin, self.cinp, self.H, self.W, None),
             "pack input")
-        k = 0
+        k, src = 0, self.x
         for l in range(L):
-            src = self.x
-            if l > 0:
-                hh, ww = self.hw[l]
-                _ok(lib().imexlb_nn_pool2_bf16(_ptr(self.cat[l - 1]), _ptr(self.pooled[l]), N, ch[l - 1], hh, ww,
-                                               ch[l] + ch[l - 1], ch[l], None), "pool2_bf16")
-                src = self.pooled[l]
-            self._conv(k, src, self.t1[l], l, ch[l], 0)
-            if l < L - 1:
-                self._conv(k + 1, self.t1[l], self.cat[l], l, ch[l + 1] + ch[l], ch[l + 1])
-            else:
-                self._conv(k + 1, self.t1[l], self.bottom, l, ch[l], 0)
+            self._conv(k, src, self.t1[l], l)
+            src = self.pooled[l + 1] if l < L - 1 else None
+            self._conv(k + 1, self.t1[l], self.enc[l], l, pool=src)
             k += 2
-        d = self.bottom
+        d = self.enc[-1]
         for l in range(L - 2, -1, -1):
-            hh, ww = self.hw[l + 1]
-            _ok(lib().imexlb_nn_up2_bf16(_ptr(d), _ptr(self.cat[l]), N, ch[l + 1], hh, ww, ch[l + 1] + ch[l], 0,
-                                         None), "up2_bf16")
-            self._conv(k, self.cat[l], self.t1[l], l, ch[l], 0)
-            self._conv(k + 1, self.t1[l], self.dec[l], l, ch[l], 0)
+            self._conv(k, self.enc[l], self.t1[l], l, low=d)
+            self._conv(k + 1, self.t1[l], self.dec[l], l)
             d = self.dec[l]
             k += 2
-        self._conv(k, d, self.out, 0, 0, 0, relu=False, f32=True)
+        self._conv(k, d, self.out, 0, relu=False, f32=True)
         return self.out
 
 

@@ -108,6 +108,16 @@ int imexlb_nn_pack_weights_bf16(const float *w, uint16_t *wp, int CI, int CO, in
  * be NULL; relu: 1 applies max(0, .); N <= 65535. */
 int imexlb_nn_conv3x3_bf16(const uint16_t *in, const uint16_t *wp, const float *bias, void *out, int N, int CIP,
                            int CO, int COP, int H, int W, int ostride, int ooff, int relu, int f32_nchw, void *stream);
+/* The same with the first CL input channels (a multiple of 16; 0 with low
+ * NULL) read from low [N][H/2][W/2][CL], upsampled to nearest, before the CI
+ * channels of in: the weights are those of CL + CI channels, and the result
+ * is that of imexlb_nn_up2_bf16 into a concatenated input.  With pool (CO a
+ * multiple of 8) the 2x2 average of the bf16 output goes to
+ * pool[N][H/2][W/2][CO], as imexlb_nn_pool2_bf16 forms it.  H and W even for
+ * either. */
+int imexlb_nn_conv3x3_bf16_join(const uint16_t *low, int CL, const uint16_t *in, int CI, const uint16_t *wp,
+                                const float *bias, void *out, uint16_t *pool, int N, int CO, int COP, int H, int W,
+                                int ostride, int ooff, int relu, int f32_nchw, void *stream);
 /* 2x2 average pool of channels [coff, coff+C) of in [N][2h][2w][cstride]
  * into out [N][h][w][C] (C, cstride, coff multiples of 8) */
 int imexlb_nn_pool2_bf16(const uint16_t *in, uint16_t *out, int N, int C, int h, int w, int cstride, int coff,

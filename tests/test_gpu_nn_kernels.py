@@ -243,3 +243,73 @@ def test_pooling_and_upsampling(shape, shift):
     _call("up2", low, wide, N, C_, h, w, C_ + 3, 2)
     keep[:, 2:2 + C_] = Lo.repeat(2, 2).repeat(2, 3)
     assert np.array_equal(wide.cpu().numpy(), keep)
+
+
+# the tiles: 16 columns (narrow images, few and many blocks), 32 columns four
+# rows with chunks ahead, 8 rows, 16 rows, 64 channels a block; chunks of 16
+# and 32 channels, one to nine of them; ragged sizes and channel counts
+BF16_SHAPES = [(1, 16, 3, 1, 1), (1, 48, 40, 9, 16), (80, 32, 8, 41, 13), (2, 96, 32, 5, 33), (1, 288, 33, 7, 40),
+               (3, 16, 31, 130, 190), (9, 32, 64, 130, 62), (12, 80, 30, 130, 200), (16, 32, 32, 134, 260)]
+
+
+def _bf16_ref(x, w, b):
+    """Exact products in FP64 of bf16 values (torch's float64 on the CPU)."""
+    return _conv64(x.astype(np.float64), w.astype(np.float64), b.astype(np.float64))
+
+
+@pytest.mark.parametrize("shape", BF16_SHAPES)
+def test_bf16_convolution_at_tile_edges(shape):
+    import torch
+    N, ci, co, H, W = shape
+    print(f"[nn] conv3x3_bf16 {shape}", flush=True)
+    g = torch.Generator().manual_seed(13)
+    x = torch.randn(N, H, W, ci, generator=g).to(torch.bfloat16)
+    w = (torch.randn(co, ci, 3, 3, generator=g) / np.sqrt(9 * ci)).to(torch.bfloat16).float()
+    b = torch.randn(co, generator=g)
+    cop = 32 * -(-co // 32)
+    wp = torch.empty(ci * 9 * cop, dtype=torch.bfloat16, device="cuda")
+    wd, bd, xd = w.cuda(), b.cuda(), x.cuda()
+    _call("pack_weights_bf16", wd, wp, ci, co, ci, cop)
+    few = max(1, min(N, 2))  # (the reference of a few images; the rest by repetition)
+    xd[few:] = xd[:1]
+    ref = _bf16_ref(xd[:few].cpu().float().permute(0, 3, 1, 2).numpy(), w.numpy(), b.numpy())
+    size = _bf16_ref(xd[:few].cpu().float().abs().permute(0, 3, 1, 2).numpy(), w.abs().numpy(), b.abs().numpy())
+    wide = torch.full((N, H, W, co + 3), 7.0, dtype=torch.bfloat16, device="cuda")
+    f32 = torch.empty(N, co, H, W, device="cuda")
+    _call("conv3x3_bf16", xd, wp, bd, wide, N, ci, co, cop, H, W, co + 3, 2, 0, 0)
+    _call("conv3x3_bf16", xd, wp, bd, f32, N, ci, co, cop, H, W, 0, 0, 1, 1)
+    # FP32 sums of exact products, then one rounding to bf16
+    tol = (9 * ci + 8) * 2.0 ** -24 * size
+    got = f32[:few].cpu().numpy()
+    assert (np.abs(got - np.maximum(ref, 0)) <= tol).all()
+    full = wide.float().cpu().numpy().transpose(0, 3, 1, 2)
+    assert (full[:, :2] == 7).all() and (full[:, 2 + co:] == 7).all()
+    assert (np.abs(full[:few, 2:2 + co] - ref) <= 2.0 ** -8 * np.abs(ref) + 2 * tol).all()
+    for k in range(few, N):
+        assert torch.equal(f32[k], f32[0]) and torch.equal(wide[k], wide[0])
+
+
+@pytest.mark.parametrize("shape", [(1, 32, 16, 16, 4, 6), (1, 16, 32, 40, 34, 18), (2, 64, 32, 32, 66, 70),
+                                   (9, 64, 64, 64, 130, 66), (5, 32, 32, 96, 260, 130)])
+def test_bf16_joined_layer_equals_its_parts(shape):
+    """Upsampled and skip channels from their own buffers, and the pooled
+    output, against the separate calls: the same bits."""
+    import torch
+    N, cl, cs, co, H, W = shape
+    print(f"[nn] conv3x3_bf16_join {shape}", flush=True)
+    g = torch.Generator("cuda").manual_seed(14)
+    bf = lambda *s: torch.randn(s, generator=g, device="cuda").to(torch.bfloat16)  # noqa: E731
+    low, skip, b = bf(N, H // 2, W // 2, cl), bf(N, H, W, cs), torch.randn(co, generator=g, device="cuda")
+    ci, cop = cl + cs, 32 * -(-co // 32)
+    wp = torch.empty(ci * 9 * cop, dtype=torch.bfloat16, device="cuda")
+    _call("pack_weights_bf16", torch.randn(co, ci, 3, 3, generator=g, device="cuda") / np.sqrt(9 * ci), wp, ci, co, ci,
+          cop)
+    cat = torch.empty(N, H, W, ci, dtype=torch.bfloat16, device="cuda")
+    _call("up2_bf16", low, cat, N, cl, H // 2, W // 2, ci, 0)
+    cat[..., cl:] = skip
+    ref, out = bf(N, H, W, co), bf(N, H, W, co)
+    pref, pool = bf(N, H // 2, W // 2, co), bf(N, H // 2, W // 2, co)
+    _call("conv3x3_bf16", cat, wp, b, ref, N, ci, co, cop, H, W, co, 0, 1, 0)
+    _call("pool2_bf16", ref, pref, N, co, H // 2, W // 2, co, 0)
+    _call("conv3x3_bf16_join", low, cl, skip, cs, wp, b, out, pool, N, co, cop, H, W, co, 0, 1, 0)
+    assert torch.equal(out, ref) and torch.equal(pool, pref)
