@@ -273,6 +273,18 @@ int imexlb_create(imexlb_ctx **out, int dim, int nx, int ny, int nz, int device,
     // multiple of `align` cells (IMEXLB_ROW_ALIGN) so that the y- and
     // z-shifted pulls of a tile start on a tile boundary
     int64_t align = 1;
+    // The small-lattice step form pays while the two population buffers stay
+    // in the 256 MB Infinity Cache from step to step: up to 240 MiB of them
+    // and 5 Mi cells (measured on MI355X from 400x100 to 8192x2048 in every
+    // storage form; against two steps per pass FP64 2048x512 23.4 and 26.3 us
+    // a step, 2560x640 35.0 and 33.4, FP16 4096x1024 25.3 and 29.0, 5001x1251
+    // 40.0 and 38.0 us); IMEXLB_SMALL_CELLS overrides the cell limit.
+    c->small_cells = std::min<int64_t>(int64_t(5) << 20, (int64_t(240) << 20) / (2 * 9 * int64_t(c->ssz)));
+    if (const char *sv = std::getenv("IMEXLB_SMALL_CELLS")) c->small_cells = std::atoll(sv);
+    const char *dv = std::getenv("IMEXLB_DOUBLE");
+    c->dbl_enabled = !(dv && dv[0] == '0');
+    // rows of whole tiles where two steps are made per pass (k_double2)
+    if (device >= 0 && c->dbl_enabled && dim == 2 && int64_t(nx + 3) * (ny + 3) > c->small_cells) align = 64;
     if (const char *av = std::getenv("IMEXLB_ROW_ALIGN")) align = std::max<int64_t>(1, std::atoll(av));
     if (align > 4096) return fail(IMEXLB_E_ARG, "IMEXLB_ROW_ALIGN above 4096 cells");
     c->Px = ((int64_t(nx) + 3 + align - 1) / align) * align;
@@ -306,6 +318,7 @@ int imexlb_create(imexlb_ctx **out, int dim, int nx, int ny, int nz, int device,
     k.plane = c->plane;
     k.ncell = uint32_t(c->Px * c->Py * c->Pz);
     k.Py = c->Py;
+    k.row_pad = uint32_t(c->Px - (int64_t(nx) + 3));
     k.div_px.init(uint32_t(c->Px));
     k.div_py.init(uint32_t(c->Py));
     for (uint32_t n : {0u, uint32_t(c->Px), k.ncell - 1u, 0xfffffffeu})
@@ -314,12 +327,6 @@ int imexlb_create(imexlb_ctx **out, int dim, int nx, int ny, int nz, int device,
     k.back_tiles = uint32_t((1 + k.Px + k.PxPy + 63) / 64);
     k.rdy = c->g.dy;
     k.rdz = c->g.dz;
-    // The small-lattice step form pays while the two population buffers stay
-    // in the 256 MB Infinity Cache from step to step: up to 240 MiB of them
-    // and 5 Mi cells (measured on MI355X from 400x100 to 8192x2048 in every
-    // storage form); IMEXLB_SMALL_CELLS overrides the cell limit.
-    c->small_cells = std::min<int64_t>(int64_t(5) << 20, (int64_t(240) << 20) / (2 * 9 * int64_t(c->ssz)));
-    if (const char *sv = std::getenv("IMEXLB_SMALL_CELLS")) c->small_cells = std::atoll(sv);
     // XCD-contiguous block order (each XCD steps the same eighth of the
     // lattice every step, so a step reads the previous one's output from its
     // own L2) pays for D3Q27 FP64 and for the small 2D lattices that stay in
@@ -400,6 +407,61 @@ int imexlb_set_params(imexlb_ctx *c, double ome, double rho0, double uu)
         HIP_TRY(hipStreamSynchronize(c->stream));
         c->drop_graphs();
     }
+    return IMEXLB_OK;
+}
+
+static bool double_suits(const imexlb_ctx *c)
+{
+    return c->dim == 2 && IMEXLB_TILE == 64 && c->Px % 64 == 0 && c->kp.nx >= 16 && c->kp.ny >= 16 &&
+           size_t(c->Q) * size_t(c->plane) * c->ssz < (size_t(1) << 32) - (size_t(1) << 16) &&
+           int64_t(c->kp.ncell) > c->small_cells;
+}
+
+// The two-steps-per-pass plan of the new geometry: the frame's lists, the
+// bulk's marks in the node types, the scratch buffer.  A lattice it does not
+// suit, or without memory for the scratch buffer, keeps single steps.
+static int build_double(imexlb_ctx *c)
+{
+    c->drop_double();
+    if (!c->dbl_enabled || !c->push_on || !double_suits(c)) return IMEXLB_OK;
+    DoublePlan &d = c->dbl;
+    struct Tmp {  // freed on every return
+        void *p = nullptr;
+        ~Tmp()
+        {
+            if (p) (void)hipFree(p);
+        }
+    } zones, counts;
+    const size_t pop = size_t(c->Q) * size_t(c->plane) * c->ssz, n = size_t(c->plane);
+    if (hipMalloc(&d.scratch, pop) != hipSuccess) {
+        (void)hipGetLastError();
+        d.scratch = nullptr;
+        return IMEXLB_OK;
+    }
+    HIP_TRY(hipMemset(d.scratch, 0, pop));
+    HIP_TRY(hipMalloc(&zones.p, 3 * n));
+    HIP_TRY(hipMalloc(&counts.p, 4 * sizeof(uint32_t)));
+    HIP_TRY(hipMemset(zones.p, 0, 3 * n));
+    HIP_TRY(hipMemset(counts.p, 0, 4 * sizeof(uint32_t)));
+    uint8_t *const z = static_cast<uint8_t *>(zones.p);
+    uint32_t *const cnt = static_cast<uint32_t *>(counts.p);
+    const StepArgs a = c->args();
+    // special nodes, the second step's frame (one node around them), the
+    // first step's (one more)
+    HIP_TRY(launch_zone(c->dim, 0, a, c->geo, nullptr, z, nullptr, nullptr, 0, nullptr));
+    HIP_TRY(launch_zone(c->dim, 1, a, c->geo, z, z + n, nullptr, nullptr, 0, nullptr));
+    HIP_TRY(launch_zone(c->dim, 1, a, c->geo, z + n, z + 2 * n, nullptr, nullptr, 0, nullptr));
+    for (int k = 0; k < 2; ++k)
+        HIP_TRY(launch_zone(c->dim, 2, a, c->geo, z + (2 - k) * n, nullptr, cnt + k, nullptr, k, nullptr));
+    HIP_TRY(hipMemcpy(d.count, cnt, sizeof(d.count), hipMemcpyDeviceToHost));
+    for (int k = 0; k < 2; ++k) {
+        HIP_TRY(hipMalloc((void **)&d.list[k], std::max<size_t>(d.count[k], 1) * sizeof(uint32_t)));
+        HIP_TRY(launch_zone(c->dim, 2, a, c->geo, z + (2 - k) * n, nullptr, cnt + 2 + k, d.list[k], 0, nullptr));
+    }
+    HIP_TRY(hipDeviceSynchronize());
+    d.idx64 = !c->fill32;
+    plan_double(c->dim, int(c->ssz), c->kp, d);
+    c->dbl_on = true;
     return IMEXLB_OK;
 }
 
@@ -491,6 +553,7 @@ int imexlb_set_geometry_shape(imexlb_ctx *c, double pos, double radius, double a
         HIP_TRY(hipMemcpy(c->link_back, t.link_back.data(), t.link_back.size() * 8, hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(c->link_q, t.link_q.data(), t.link_q.size(), hipMemcpyHostToDevice));
     }
+    if ((rc = build_double(c))) return rc;
     commit.done = c->geom_set = true;
     return IMEXLB_OK;
 }
@@ -799,11 +862,85 @@ static int step_graph(imexlb_ctx *c, int size, int X, hipGraphExec_t *out)
     return IMEXLB_OK;
 }
 
-// n fused steps, the first reading fb[A]: one alone if n is odd, then pairs
-// as replays of the largest graphs that fit (the state they leave is the
-// one n launches one by one would)
+// kQuads[size] times two double steps (four steps, back in the same buffer),
+// the first reading fb[A], as one graph
+static int quad_graph(imexlb_ctx *c, int size, int A, hipGraphExec_t *out)
+{
+    hipGraphExec_t &slot = c->quad_graph[size][A];
+    if (slot) {
+        *out = slot;
+        return IMEXLB_OK;
+    }
+    StepArgs a = c->args();
+    HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+    hipError_t e = hipSuccess;
+    for (int k = 0; k < 2 * imexlb_ctx::kQuads[size] && e == hipSuccess; ++k) {
+        a.src = c->fb[A ^ (k & 1)];
+        a.dst = c->fb[A ^ 1 ^ (k & 1)];
+        e = launch_double(c->dim, c->prec, a, c->dbl, c->stream);
+    }
+    hipGraph_t g = nullptr;
+    hipError_t e2 = hipStreamEndCapture(c->stream, &g);
+    if (e != hipSuccess || e2 != hipSuccess) {
+        if (g) (void)hipGraphDestroy(g);
+        return fail(IMEXLB_E_HIP, std::string("graph capture: ") + hipGetErrorString(e != hipSuccess ? e : e2));
+    }
+    hipGraphExec_t x = nullptr;
+    e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(g);
+    if (e != hipSuccess) return fail(IMEXLB_E_HIP, std::string("graph instantiate: ") + hipGetErrorString(e));
+    slot = x;
+    *out = x;
+    return IMEXLB_OK;
+}
+
+// The part of n fused steps from fb[A] that runs two steps per pass: fours,
+// which end in the buffer they began in, leaving at least one single step
+// (the last step's source buffer has to hold the step before).  Returns the
+// steps taken in *done.
+static int run_double_steps(imexlb_ctx *c, int A, int64_t n, int64_t *done)
+{
+    int64_t quads = c->dbl_on ? (n - 1) / 4 : 0;
+    *done = 4 * quads;
+    if (!c->graphs || c->prof) {
+        for (int64_t k = 0; k < 2 * quads; ++k) {
+            StepArgs a = c->args();
+            a.src = c->fb[A ^ int(k & 1)];
+            a.dst = c->fb[A ^ 1 ^ int(k & 1)];
+            int rc = c->launch(0, [&] { return launch_double(c->dim, c->prec, a, c->dbl, c->stream); }, 2);
+            if (rc) return rc;
+        }
+        return IMEXLB_OK;
+    }
+    for (int j = 0; j < imexlb_ctx::kGraphSizes && quads > 0; ++j) {
+        const int64_t reps = quads / imexlb_ctx::kQuads[j];
+        if (reps <= 0) continue;
+        hipGraphExec_t g;
+        int rc = quad_graph(c, j, A, &g);
+        if (rc) return rc;
+        for (int64_t k = 0; k < reps; ++k) HIP_TRY(hipGraphLaunch(g, c->stream));
+        quads -= reps * imexlb_ctx::kQuads[j];
+    }
+    return IMEXLB_OK;
+}
+
+// n fused steps, the first reading fb[A]: two steps per pass where the
+// lattice has the plan for it, then one alone if an odd number is left, then
+// pairs as replays of the largest graphs that fit (the state they leave is
+// the one n launches one by one would)
 static int run_fused_steps(imexlb_ctx *c, int A, int64_t n)
 {
+    int64_t done = 0;
+    int rd = run_double_steps(c, A, n, &done);
+    if (rd) return rd;
+    n -= done;
+    if (!c->graphs || c->prof) {
+        for (; n > 0; --n, A = 1 - A) {
+            int rc = c->run_step(c->collide_mode(), c->fb[A], c->fb[1 - A], nullptr);
+            if (rc) return rc;
+        }
+        return IMEXLB_OK;
+    }
     if (n & 1) {
         int rc = c->run_step(c->collide_mode(), c->fb[A], c->fb[1 - A], nullptr);
         if (rc) return rc;
@@ -838,7 +975,7 @@ int imexlb_advance(imexlb_ctx *c, int64_t nsteps)
     if (nsteps < 0) return fail(IMEXLB_E_ARG, "negative step count");
     int64_t i = 0;
     // timed (profiled) runs launch kernel by kernel so each one is bracketed
-    if (c->can_defer()) {
+    if (c->can_defer() || (c->fused && c->dbl_on)) {
         for (; i < nsteps && c->stage != S_FUSED; ++i) {
             int rc = one_step(c);
             if (rc) return rc;

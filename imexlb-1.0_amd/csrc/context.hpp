@@ -38,7 +38,7 @@ inline int fail(int code, const std::string &msg)
 enum Stage { S_NONE, S_PRE, S_COLLIDED, S_FILLED, S_PENDING, S_STREAMED, S_FUSED };
 
 struct TimedLaunch {
-    int cls;
+    int cls, steps;  // steps: lattice steps the launch makes (counted as so many launches)
     hipEvent_t a, b;
 };
 
@@ -96,7 +96,7 @@ struct imexlb_ctx {
     {
         geom_set = false;
         nfill = nlink = 0;
-        push_on = prefilled = false;
+        push_on = prefilled = dbl_on = false;
         stage = S_NONE;
         have_pu = have_f = have_fb = false;
         lazy_src = -1;
@@ -120,12 +120,13 @@ struct imexlb_ctx {
     hipGraphExec_t graph[kGraphSizes][2] = {};
     void drop_graphs()
     {
-        for (auto &set : graph)
-            for (int k = 0; k < 2; ++k)
-                if (set[k]) {
-                    (void)hipGraphExecDestroy(set[k]);
-                    set[k] = nullptr;
-                }
+        for (auto *all : {&graph, &quad_graph})
+            for (auto &set : *all)
+                for (int k = 0; k < 2; ++k)
+                    if (set[k]) {
+                        (void)hipGraphExecDestroy(set[k]);
+                        set[k] = nullptr;
+                    }
     }
 
     // Fused steps asked for through the phase calls (PostProcessing of a
@@ -138,6 +139,20 @@ struct imexlb_ctx {
     int defer_src = 0;
     static constexpr int64_t kDeferChunk = 16;
     bool can_defer() const { return fused && graphs && !prof && push_on; }
+
+    // Two steps in one pass over memory, for lattices that do not stay in the
+    // caches (built with the geometry; IMEXLB_DOUBLE=0 keeps single steps)
+    DoublePlan dbl;
+    bool dbl_enabled = true, dbl_on = false;
+    hipGraphExec_t quad_graph[kGraphSizes][2] = {};  // kQuads[j] pairs of double steps, by starting buffer
+    static constexpr int kQuads[kGraphSizes] = {16, 4, 1};
+    void drop_double()
+    {
+        for (void *q : {(void *)dbl.list[0], (void *)dbl.list[1], dbl.scratch})
+            if (q) (void)hipFree(q);
+        dbl = DoublePlan{};
+        dbl_on = false;
+    }
 
     // profiling
     bool prof = false;
@@ -172,13 +187,13 @@ struct imexlb_ctx {
         HIP_TRY(hipEventRecord(b, stream));
         return IMEXLB_OK;
     }
-    int end(int cls, hipEvent_t b)
+    int end(int cls, hipEvent_t b, int steps)
     {
         if (!prof) return IMEXLB_OK;
         hipEvent_t e;
         HIP_TRY(hipEventCreate(&e));
         HIP_TRY(hipEventRecord(e, stream));
-        timed.push_back(TimedLaunch{cls, b, e});
+        timed.push_back(TimedLaunch{cls, steps, b, e});
         // bound the live event pairs of a long timed run: fold the oldest
         // half into the totals (waiting for them) once kMaxTimed are held
         if (timed.size() >= kMaxTimed) return harvest(kMaxTimed / 2);
@@ -195,7 +210,7 @@ struct imexlb_ctx {
             HIP_TRY(hipEventSynchronize(t.b));
             float v = 0.0f;
             HIP_TRY(hipEventElapsedTime(&v, t.a, t.b));
-            prof_n[t.cls] += 1;
+            prof_n[t.cls] += t.steps;
             prof_ms[t.cls] += double(v);
             (void)hipEventDestroy(t.a);
             (void)hipEventDestroy(t.b);
@@ -205,14 +220,14 @@ struct imexlb_ctx {
     }
 
     template <class F>
-    int launch(int cls, F &&fn)
+    int launch(int cls, F &&fn, int steps = 1)
     {
         hipEvent_t b = nullptr;
         int rc = begin(cls, b);
         if (rc) return rc;
         hipError_t e = fn();
         if (e != hipSuccess) return fail(IMEXLB_E_HIP, std::string("kernel launch: ") + hipGetErrorString(e));
-        return end(cls, b);
+        return end(cls, b, steps);
     }
 
     // BoundaryCondition on buffer `buf`; the other buffer holds the previous
@@ -275,6 +290,7 @@ struct imexlb_ctx {
                         force_out, push_beg, push_q,   push_dst, push_lds, mass_partial};
         for (void *q : ptrs)
             if (q) (void)hipFree(q);
+        drop_double();
         fb[0] = fb[1] = f = nullptr;
         push_beg = nullptr;
         push_q = nullptr;

@@ -59,6 +59,7 @@ struct KParams {
     double inv_rho0;     // 1/rho0 (FP32-compute forms multiply by it)
     uint32_t xcd_remap;  // block order over the XCDs: 0 hardware, 1 an eighth each, R >= 2 runs of R
     float ome_f, rho0_f, uu_f, inv_rho0_f;  // the same scalars rounded to FP32 once
+    uint32_t row_pad = 0; // padding cells of a row past its ghost cells
     uint32_t back_tiles; // ceil((1 + Px + PxPy) / 64): the farthest tile a pull reads behind its own
 };
 
@@ -98,8 +99,9 @@ inline int64_t pop_slot(int64_t q, int64_t c, int64_t plane, int Q)
 enum : int { K_COLLIDE = 1, K_WRITE_F = 2, K_WRITE_PU = 4, K_NOSHIFT = 8, K_PUSH = 16, K_IDX64 = 32, K_SMALL = 64 };
 constexpr unsigned kSmallBlock = 64;
 
-// node-type byte on the device: fluid node; node with boundary copies to push
-enum : uint8_t { G_FLUID = 1, G_PUSH = 2 };
+// node-type byte on the device: fluid node; node with boundary copies to push;
+// node that two steps in one pass may write
+enum : uint8_t { G_FLUID = 1, G_PUSH = 2, G_BULK = 4 };
 
 // The resolved boundary table grouped by source node: entries beg[c] ..
 // beg[c+1]-1 of padded cell c copy its direction q[e] to slot dst[e] of the
@@ -133,6 +135,25 @@ struct StepArgs {
     const uint8_t *geo = nullptr;
     PushTable push;
 };
+
+// Two steps in one pass (launch_double): the frame's cells of the first and
+// second step, the scratch buffer of its first step, and the bulk's split
+// into strips of columns and segments of rows.
+struct DoublePlan {
+    uint32_t *list[2] = {nullptr, nullptr};
+    uint32_t count[2] = {0, 0};
+    void *scratch = nullptr;
+    bool idx64 = false;  // the push table's slots are int64
+    uint32_t strips = 0, segments = 0;
+    int rows = 0;
+};
+void plan_double(int dim, int bytes, const KParams &kp, DoublePlan &d);
+hipError_t launch_double(int dim, int prec, const StepArgs &a, const DoublePlan &d, hipStream_t s);
+// passes that find the frame: 0 special nodes to out; 1 in grown by a node to
+// out; 2 the nodes marked in `in` appended to list (nullptr: counted), the
+// others marked G_BULK in geo with bulk
+hipError_t launch_zone(int dim, int pass, const StepArgs &a, uint8_t *geo, const uint8_t *in, uint8_t *out,
+                       uint32_t *count, uint32_t *list, int bulk, hipStream_t s);
 
 // prec: 0 FP64, 1 FP32, 2 FP16 storage + FP32 arithmetic, 3 BF16 storage + FP32 arithmetic
 hipError_t launch_step(int dim, int prec, int mode, const StepArgs &a, hipStream_t s);

@@ -177,6 +177,17 @@ __device__ __forceinline__ uint32_t sr_word(C p, uint32_t c)
         return 0u;
 }
 
+// The cell's index for sr_word: its padded index without the row padding that
+// some lattices have, so that the dither does not depend on it.
+template <class S>
+__device__ __forceinline__ uint32_t sr_cell(const KParams &kp, uint32_t c, int y, int z)
+{
+    if constexpr (std::is_same<S, bf16sr_t>::value)
+        return c - kp.row_pad * uint32_t(y + 1 + (z + 1) * (kp.PxPy ? int(kp.Py) : 0));
+    else
+        return c;
+}
+
 // streaming (non-temporal) store of one population value
 template <class S>
 __device__ __forceinline__ void nt_store(S *p, S v)
@@ -686,7 +697,7 @@ __device__ __forceinline__ void finish_node(const C (&f)[Lat<D>::Q], uint8_t g, 
         // base plus the lane
         S *const wdst = (MODE & K_WAVE) ? dst + uint64_t(wave_tile(c)) * (L::Q * 64u) : dst;
         S out[kRegPush ? L::Q : 1];  // the stored values, for the copies
-        const uint32_t srw = sr_word<S>(p, c);
+        const uint32_t srw = sr_word<S>(p, sr_cell<S>(kp, c, y, z));
         collide<D, C>(f, p, ux, uy, uz, kp, [&](int q, C v) {
             S *o = (MODE & K_WAVE) ? wdst + (uint32_t(store_q(q, L::Q)) * 64u + (c & 63u)) : dst + cslot<L::Q>(kp, q, c);
             const S sv = Store<S>::template st<C>(v, srw + uint32_t(q) * kGolden);
@@ -770,7 +781,7 @@ __device__ __forceinline__ void step_small(const S *__restrict__ src, S *__restr
         if (g & G_FLUID) {
             C p, ux, uy, uz;
             moments<D, C>(f, kp, x, y, z, p, ux, uy, uz);
-            const uint32_t srw = sr_word<S>(p, c);
+            const uint32_t srw = sr_word<S>(p, sr_cell<S>(kp, c, y, z));
             collide<D, C>(f, p, ux, uy, uz, kp, [&](int q, C v) {
                 const S sv = Store<S>::template st<C>(v, srw + uint32_t(q) * kGolden);
                 tdst[uint32_t(store_q(q, L::Q)) * 64u + lane] = sv;
@@ -834,7 +845,7 @@ __device__ __forceinline__ void step_wave_copies(const S *__restrict__ src, S *_
         if (g & G_FLUID) {
             C p, ux, uy, uz;
             moments<D, C>(f, kp, x, y, z, p, ux, uy, uz);
-            const uint32_t srw = sr_word<S>(p, c);
+            const uint32_t srw = sr_word<S>(p, sr_cell<S>(kp, c, y, z));
             collide<D, C>(f, p, ux, uy, uz, kp, [&](int q, C v) {
                 S sv;
                 if constexpr (std::is_same<S, bf16_t>::value)
@@ -956,6 +967,208 @@ __global__ IMEXLB_STEP_BOUNDS void k_step(const S *__restrict__ src, S *__restri
 }
 
 // ---------------------------------------------------------------------------
+// Two steps in one pass over memory.  The cells two steps away from
+// everything that is not a plain pull (k_zone_*: G_BULK) are stepped by
+// k_double2: the populations of the first step stay on the chip, so two steps
+// read and write each population once instead of twice.  The frame that is
+// left -- cells near the walls, the body, the inlet and outlet -- is stepped
+// twice one step at a time from lists of its cells (k_step_list), its first
+// step going to a scratch buffer.  Results are those of two steps, bit for
+// bit: the same arithmetic on the same stored (rounded) values.
+constexpr int kStripX = 256;          // columns a block of k_double2 writes
+constexpr int kDouble2 = kStripX + 64;  // its threads: one more wave for the columns beside the strip
+
+// One step of the cells of a list.
+template <int D, class S, class C, int MODE>
+__global__ __launch_bounds__(256) void k_step_list(const S *__restrict__ src, S *__restrict__ dst,
+                                                   const uint8_t *__restrict__ geo, KParams kp, PushTable pt,
+                                                   const uint32_t *__restrict__ list, uint32_t n)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    int x, y, z;
+    uint32_t c;
+    if (!decode_cell<D>(kp, list[i], x, y, z, c)) return;
+    step_node<D, S, C, MODE>(src, dst, nullptr, nullptr, nullptr, nullptr, nullptr, geo, kp, x, y, z, c, pt);
+}
+
+// Two steps of the bulk of a D2Q9 lattice.  A block takes a strip of columns
+// and walks up `rows` rows: each thread makes the first step of its column's
+// next row, leaves the populations that move sideways in LDS (six of nine;
+// the rest stay in its registers), and makes the second step of the row
+// below, whose pulls come from the last three rows of the ring.
+//
+// Bound by HBM: a pass moves 144 B per FP64 node for two steps (plus two rows
+// a segment and two columns a strip).  Whole-line stores matter most: strips
+// of 254 columns on unpadded rows, whose waves straddle lines, took 0.279 ms
+// a step at 8192 x 2048 FP64 (4.5 TB/s), tile-aligned ones 0.243 (5.1 TB/s);
+// the single step 0.412.  FP32 0.207 to 0.127, FP16 0.103 to 0.082 (bound by
+// instructions), BF16 with stochastic rounding 0.105 to 0.090.  Gathering two
+// rows ahead measured slower in every form but FP32.
+template <class S, class C>
+__global__ __launch_bounds__(kDouble2) void k_double2(const S *__restrict__ src, S *__restrict__ dst,
+                                                      const uint8_t *__restrict__ geo, KParams kp, int rows,
+                                                      uint32_t nstrips)
+{
+    using L = Lat<2>;
+    using U = BitsOf<S>;
+    // e_x = -1, +1 populations of direction e_y = -1, 0, +1: needed this row,
+    // one and two rows later; one more slot each lets a row be written while
+    // slower waves still read.  Column x0 - 1 + i of the strip is entry i.
+    constexpr int W = kStripX + 2;
+    __shared__ U down[2][2][W], level[3][2][W], up[4][2][W];
+    // All waves but the last take the strip's columns, a tile each (rows are
+    // whole tiles), so that their stores are whole lines; two lanes of the
+    // last the columns beside it.
+    const int th = int(threadIdx.x);
+    const int t = th < kStripX ? th + 1 : th == kStripX ? 0 : W - 1;
+    const int x0 = int(blockIdx.x % nstrips) * kStripX - 1;
+    const int y0 = 2 + int(blockIdx.x / nstrips) * rows, y1 = min(y0 + rows - 1, kp.ny - 2);
+    const int x = min(max(x0 - 1 + t, 0), kp.nx);
+    const bool writes = th < kStripX && x0 - 1 + t >= 2 && x0 - 1 + t <= kp.nx - 2, leaves = th < W;
+    const uint32_t Px = uint32_t(kp.Px);
+    uint32_t c = uint32_t(kp.o0 + x) + Px * uint32_t(y0 - 1);  // the first step's cell
+    // Byte offsets (32 bits: plan_double) of direction 0 of the cells x + 1,
+    // x, x - 1 in the rows above, at and below the next gather; a row's
+    // offsets are formed once and serve three gathers and a store.
+    constexpr uint32_t QT = L::Q * 64u * sizeof(S), QS = 64u * sizeof(S);
+    const auto slot0 = [&](uint32_t cell) { return (cell >> 6) * QT + (cell & 63u) * uint32_t(sizeof(S)); };
+    uint32_t off[3][3];  // [row: above, at, below][x + 1, x, x - 1]
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) off[r][k] = slot0(c + Px - uint32_t(r) * Px + 1u - uint32_t(k));
+    const char *const sb = reinterpret_cast<const char *>(src);
+    char *const db = reinterpret_cast<char *>(dst);
+    const auto pull = [&](C(&f)[L::Q]) {
+#pragma unroll
+        for (int q = 0; q < L::Q; ++q)  // from x - e_x, row - e_y
+            f[q] = Store<S>::ld(*reinterpret_cast<const S *>(sb + off[L::ey(q) + 1][L::ex(q) + 1] +
+                                                             uint32_t(store_q(q, L::Q)) * QS));
+    };
+    const auto next_row = [&](uint32_t cell) {  // the gather moves on to the row of `cell`
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            off[2][k] = off[1][k];
+            off[1][k] = off[0][k];
+            off[0][k] = slot0(cell + Px + 1u - uint32_t(k));
+        }
+    };
+    C f[L::Q];
+    pull(f);
+    uint32_t out1 = 0, out0 = slot0(c);  // the second step's store, this row and next
+    uint8_t g = 0, gn = 0;               // node types of the rows the second step takes now and next
+    C same = C(0), rise1 = C(0), rise2 = C(0);  // own column: e = (0, 0) of a row ago, (0, 1) of one and two
+    int l3 = 0;
+    for (int j = y0 - 1; j <= y1 + 1; ++j) {
+        C p, ux, uy, uz;
+        U sv[L::Q];
+        moments<2, C>(f, kp, -1, 0, 0, p, ux, uy, uz);  // (no inlet or outlet in the bulk)
+        const uint32_t srw = sr_word<S>(p, sr_cell<S>(kp, c, j, 0));
+        collide<2, C>(f, p, ux, uy, uz, kp, [&](int q, C v) {
+            sv[q] = __builtin_bit_cast(U, Store<S>::template st<C>(v, srw + uint32_t(q) * kGolden));
+        });
+        const auto back = [&](U u) { return C(Store<S>::ld(__builtin_bit_cast(S, u))); };
+        out1 = out0;
+        out0 = slot0(c);
+        const uint32_t cell2 = c - Px;  // the second step's cell
+        c += Px;
+        if (j <= y1) {  // the next row's loads pass while this row's second step is made
+            next_row(c);
+            pull(f);
+        }
+        g = gn;
+        gn = geo[c - Px];
+        if (leaves) {
+            down[j & 1][0][t] = sv[0];
+            down[j & 1][1][t] = sv[6];
+            level[l3][0][t] = sv[1];
+            level[l3][1][t] = sv[7];
+            up[j & 3][0][t] = sv[2];
+            up[j & 3][1][t] = sv[8];
+        }
+        __syncthreads();
+        const int l1 = l3 == 0 ? 2 : l3 - 1;  // the level slot of a row ago
+        if (j > y0 && writes) {
+            C h[L::Q];
+            h[0] = back(down[j & 1][0][t + 1]);
+            h[6] = back(down[j & 1][1][t - 1]);
+            h[3] = back(sv[3]);
+            h[1] = back(level[l1][0][t + 1]);
+            h[7] = back(level[l1][1][t - 1]);
+            h[4] = same;
+            h[2] = back(up[(j - 2) & 3][0][t + 1]);
+            h[8] = back(up[(j - 2) & 3][1][t - 1]);
+            h[5] = rise2;
+            moments<2, C>(h, kp, -1, 0, 0, p, ux, uy, uz);
+            const uint32_t srw2 = sr_word<S>(p, sr_cell<S>(kp, cell2, j - 1, 0));
+            if (g & G_BULK)
+                collide<2, C>(h, p, ux, uy, uz, kp, [&](int q, C v) {
+                    nt_store(reinterpret_cast<S *>(db + out1 + uint32_t(store_q(q, L::Q)) * QS),
+                             Store<S>::template st<C>(v, srw2 + uint32_t(q) * kGolden));
+                });
+        }
+        rise2 = rise1;
+        rise1 = back(sv[5]);
+        same = back(sv[4]);
+        l3 = l3 == 2 ? 0 : l3 + 1;
+    }
+}
+
+// Zones of a lattice, one byte per padded cell.  k_zone_special: interior
+// nodes whose step is more than a pull from fluid neighbours -- solid, next
+// to a solid or ghost cell, or the source of boundary copies.
+template <int D>
+__global__ __launch_bounds__(256) void k_zone_special(const uint8_t *__restrict__ geo, uint8_t *__restrict__ out,
+                                                      KParams kp)
+{
+    int x, y, z;
+    uint32_t c;
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (!decode_cell<D>(kp, i, x, y, z, c)) return;
+    bool plain = !(geo[c] & G_PUSH);
+#pragma unroll
+    for (int q = 0; q < Lat<D>::Q; ++q) plain &= (geo[c - shift32<D>(kp, q)] & G_FLUID) != 0;
+    out[c] = plain ? 0 : 1;
+}
+
+// out: interior nodes with a marked neighbour (or marked themselves)
+template <int D>
+__global__ __launch_bounds__(256) void k_zone_grow(const uint8_t *__restrict__ in, uint8_t *__restrict__ out,
+                                                   KParams kp)
+{
+    int x, y, z;
+    uint32_t c;
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (!decode_cell<D>(kp, i, x, y, z, c)) return;
+    uint8_t any = 0;
+#pragma unroll
+    for (int q = 0; q < Lat<D>::Q; ++q) any |= in[c - shift32<D>(kp, q)];
+    out[c] = any;
+}
+
+// The marked cells with work (fluid, or body cells that copy) as a list: a
+// wave appends its 64 cells' in order (list == nullptr: counts only).  With
+// bulk the unmarked interior cells get G_BULK.
+template <int D>
+__global__ __launch_bounds__(256) void k_zone_list(const uint8_t *__restrict__ mark, uint8_t *__restrict__ geo,
+                                                   KParams kp, int bulk, uint32_t *__restrict__ count,
+                                                   uint32_t *__restrict__ list)
+{
+    int x, y, z;
+    uint32_t c;
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    const bool in = decode_cell<D>(kp, i, x, y, z, c);
+    const bool take = in && mark[c] && (geo[c] & (G_FLUID | G_PUSH));
+    const uint64_t m = __ballot(take);
+    uint32_t base = 0;
+    if (m && (threadIdx.x & 63u) == 0) base = atomicAdd(count, uint32_t(__popcll(m)));
+    base = __builtin_amdgcn_readfirstlane(base);
+    if (take && list) list[base + uint32_t(__popcll(m & ((uint64_t(1) << (threadIdx.x & 63u)) - 1)))] = c;
+    if (in && bulk && !mark[c]) geo[c] |= G_BULK;
+}
+
+// ---------------------------------------------------------------------------
 // Batched ensemble: many independent lattices advanced by one launch.  The
 // interior nodes of every case are cut into tiles of BLOCK*CPT nodes; a
 // block takes a tile (by its index, or from a queue when PERSIST), reads the
@@ -1029,7 +1242,7 @@ __global__ __launch_bounds__(256) void k_collide(const S *__restrict__ fin, S *_
 #pragma unroll
     for (int q = 0; q < L::Q; ++q) f[q] = Store<S>::ld(fin[cslot<L::Q>(kp, q, c)]);
     collide<D, C>(f, C(p[c]), C(ux[c]), C(uy[c]), D == 3 ? C(uz[c]) : C(0), kp,
-                  [&, srw = sr_word<S>(C(p[c]), c)](int q, C v) {
+                  [&, srw = sr_word<S>(C(p[c]), sr_cell<S>(kp, c, y, z))](int q, C v) {
                       dst[cslot<L::Q>(kp, q, c)] = Store<S>::template st<C>(v, srw + uint32_t(q) * kGolden);
                   });
 }
@@ -1068,7 +1281,7 @@ __global__ __launch_bounds__(256) void k_init_pdf(S *__restrict__ fout, const do
         term(L::ey(q), u1);
         if (D == 3) term(L::ez(q), u2);
         const C feq = C(L::w(q)) * (pp * C(3) + rho0 * ((C(3) * edu + C(4.5) * (edu * edu)) - C(1.5) * udu));
-        fout[cslot<L::Q>(kp, q, c)] = Store<S>::template st<C>(feq, sr_word<S>(pp, c) + uint32_t(q) * kGolden);
+        fout[cslot<L::Q>(kp, q, c)] = Store<S>::template st<C>(feq, sr_word<S>(pp, sr_cell<S>(kp, c, y, z)) + uint32_t(q) * kGolden);
     }
 }
 
@@ -1351,6 +1564,79 @@ static hipError_t step_d(int prec, int mode, const StepArgs &a, hipStream_t s)
 hipError_t launch_step(int dim, int prec, int mode, const StepArgs &a, hipStream_t s)
 {
     return dim == 2 ? step_d<2>(prec, mode, a, s) : step_d<3>(prec, mode, a, s);
+}
+
+template <int D, int MODE>
+static hipError_t list_dm(int prec, const StepArgs &a, const uint32_t *list, uint32_t n, hipStream_t s)
+{
+    return dispatch_prec(prec, [&](auto *sp, auto *cp) {
+        using S = std::remove_pointer_t<decltype(sp)>;
+        using C = std::remove_pointer_t<decltype(cp)>;
+        hipLaunchKernelGGL((k_step_list<D, S, C, MODE>), dim3(nblocks(n)), dim3(256), 0, s, (const S *)a.src,
+                           (S *)a.dst, a.geo, a.kp, a.push, list, n);
+        return hipGetLastError();
+    });
+}
+
+static hipError_t launch_step_list(int dim, int prec, bool idx64, const StepArgs &a, const uint32_t *list, uint32_t n,
+                                   hipStream_t s)
+{
+    constexpr int M = K_COLLIDE | K_PUSH, M64 = M | K_IDX64;
+    if (n == 0) return hipSuccess;
+    if (dim == 2) return idx64 ? list_dm<2, M64>(prec, a, list, n, s) : list_dm<2, M>(prec, a, list, n, s);
+    return idx64 ? list_dm<3, M64>(prec, a, list, n, s) : list_dm<3, M>(prec, a, list, n, s);
+}
+
+hipError_t launch_double(int dim, int prec, const StepArgs &a, const DoublePlan &d, hipStream_t s)
+{
+    StepArgs first = a, second = a;
+    first.dst = d.scratch;
+    second.src = d.scratch;
+    hipError_t e = launch_step_list(dim, prec, d.idx64, first, d.list[0], d.count[0], s);
+    if (e != hipSuccess) return e;
+    if (dim != 2) return hipErrorInvalidValue;
+    e = dispatch_prec(prec, [&](auto *sp, auto *cp) {
+        using S = std::remove_pointer_t<decltype(sp)>;
+        using C = std::remove_pointer_t<decltype(cp)>;
+        hipLaunchKernelGGL((k_double2<S, C>), dim3(d.strips * d.segments), dim3(kDouble2), 0, s, (const S *)a.src,
+                           (S *)a.dst, a.geo, a.kp, d.rows, d.strips);
+        return hipGetLastError();
+    });
+    if (e != hipSuccess) return e;
+    return launch_step_list(dim, prec, d.idx64, second, d.list[1], d.count[1], s);
+}
+
+hipError_t launch_zone(int dim, int pass, const StepArgs &a, uint8_t *geo, const uint8_t *in, uint8_t *out,
+                       uint32_t *count, uint32_t *list, int bulk, hipStream_t s)
+{
+    const dim3 grid(nblocks(a.kp.ncell)), block(256);
+    const auto go = [&](auto dtag) {
+        constexpr int D = decltype(dtag)::value;
+        if (pass == 0)
+            hipLaunchKernelGGL((k_zone_special<D>), grid, block, 0, s, geo, out, a.kp);
+        else if (pass == 1)
+            hipLaunchKernelGGL((k_zone_grow<D>), grid, block, 0, s, in, out, a.kp);
+        else
+            hipLaunchKernelGGL((k_zone_list<D>), grid, block, 0, s, in, geo, a.kp, bulk, count, list);
+        return hipGetLastError();
+    };
+    return dim == 2 ? go(std::integral_constant<int, 2>{}) : go(std::integral_constant<int, 3>{});
+}
+
+// The bulk of k_double2 in strips of columns and segments of rows: as many
+// blocks as fit on 256 CUs at a time -- three on each, five in 16-bit storage
+// -- since a block that starts when others end leaves them idle (8192 x 2048
+// per step: FP64 0.243 ms with 768 blocks, 0.245 with 1024, 0.266 with 1536;
+// FP16 0.098 with 1024, 0.082 with 1280, 0.100 with 1536).  A segment costs
+// two more rows, so it has at least 8.
+void plan_double(int dim, int bytes, const KParams &kp, DoublePlan &d)
+{
+    (void)dim;
+    const uint32_t fit = bytes == 2 ? 1280 : 768, rows = uint32_t(kp.ny - 3);  // rows 2 .. ny-2
+    d.strips = uint32_t((kp.nx + kStripX - 1) / kStripX);                       // columns -1 .. nx-2
+    const uint32_t seg = std::max(1u, fit / d.strips);
+    d.rows = std::max<int>(8, int((rows + seg - 1) / seg));
+    d.segments = (rows + uint32_t(d.rows) - 1) / uint32_t(d.rows);
 }
 
 hipError_t launch_collide(int dim, int prec, const StepArgs &a, hipStream_t s)

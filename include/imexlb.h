@@ -208,7 +208,8 @@ int imexlb_synchronize(imexlb_ctx *ctx);
 /* Kernel timing with HIP events on the context stream.  While enabled,
  * every launch is bracketed by events; imexlb_profile_read returns, for
  * kernel class k (0 fused step, 1 boundary fill, 2 other), the launch count
- * and the summed milliseconds since the last reset. */
+ * and the summed milliseconds since the last reset.  A pass that makes two
+ * steps counts as two launches. */
 int imexlb_profile(imexlb_ctx *ctx, int enable);
 int imexlb_profile_read(imexlb_ctx *ctx, int64_t launches[3], double ms[3]);
 
