@@ -20,6 +20,7 @@
 #include <memory>
 #include <new>
 #include <string>
+#include <unordered_map>
 #include <vector>
 
 #include "context.hpp"
@@ -278,11 +279,26 @@ int imexlb_create(imexlb_ctx **out, int dim, int nx, int ny, int nz, int device,
     // and 5 Mi cells (measured on MI355X from 400x100 to 8192x2048 in every
     // storage form; against two steps per pass FP64 2048x512 23.4 and 26.3 us
     // a step, 2560x640 35.0 and 33.4, FP16 4096x1024 25.3 and 29.0, 5001x1251
-    // 40.0 and 38.0 us); IMEXLB_SMALL_CELLS overrides the cell limit.
+    // 40.0 and 38.0 us); IMEXLB_SMALL_CELLS overrides the cell limit (and
+    // that of several steps per launch).
     c->small_cells = std::min<int64_t>(int64_t(5) << 20, (int64_t(240) << 20) / (2 * 9 * int64_t(c->ssz)));
     if (const char *sv = std::getenv("IMEXLB_SMALL_CELLS")) c->small_cells = std::atoll(sv);
+    // Several steps per launch pay in FP32 at every size, in 16-bit storage up
+    // to 8 Mi cells and in FP64 up to 2.5 Mi; above, the cells that neighbouring
+    // windows both compute cost more than a second pass (against two steps per
+    // pass, us a step: FP32 8192x2048 107 and 129, FP16 5001x1251 35.2 and
+    // 38.1, 8192x2048 95 and 83, FP64 3000x750 39.8 and 41.5, 8192x2048 285 and
+    // 244); with stochastic rounding, more arithmetic per cell, up to 4 Mi
+    // (5001x1251 42.9 and 40.9).
+    c->multi_cells = c->ssz == 4                     ? INT64_MAX
+                     : precision == IMEXLB_BF16SR_F32 ? int64_t(4) << 20
+                     : c->ssz == 2                    ? int64_t(8) << 20
+                                                      : int64_t(5) << 19;
+    if (std::getenv("IMEXLB_SMALL_CELLS")) c->multi_cells = c->small_cells;
     const char *dv = std::getenv("IMEXLB_DOUBLE");
     c->dbl_enabled = !(dv && dv[0] == '0');
+    const char *mv = std::getenv("IMEXLB_MULTI");
+    c->multi_enabled = !(mv && mv[0] == '0');
     // rows of whole tiles where two steps are made per pass (k_double2)
     if (device >= 0 && c->dbl_enabled && dim == 2 && int64_t(nx + 3) * (ny + 3) > c->small_cells) align = 64;
     if (const char *av = std::getenv("IMEXLB_ROW_ALIGN")) align = std::max<int64_t>(1, std::atoll(av));
@@ -423,7 +439,7 @@ static bool double_suits(const imexlb_ctx *c)
 static int build_double(imexlb_ctx *c)
 {
     c->drop_double();
-    if (!c->dbl_enabled || !c->push_on || !double_suits(c)) return IMEXLB_OK;
+    if (!c->dbl_enabled || !c->push_on || c->multi_on || !double_suits(c)) return IMEXLB_OK;
     DoublePlan &d = c->dbl;
     struct Tmp {  // freed on every return
         void *p = nullptr;
@@ -462,6 +478,82 @@ static int build_double(imexlb_ctx *c)
     d.idx64 = !c->fill32;
     plan_double(c->dim, int(c->ssz), c->kp, d);
     c->dbl_on = true;
+    return IMEXLB_OK;
+}
+
+// Whether every boundary copy of a previous step's body value is always 0: such
+// values mostly go round among body cells (a mirror's mirror is the cell
+// itself) and stay the 0 they start with.
+static bool body_copies_zero(const DeviceTables &t)
+{
+    std::unordered_map<int64_t, int64_t> src;
+    for (size_t k = 0; k < t.fill_dst.size(); ++k) src.emplace(t.fill_dst[k], t.fill_src[k]);
+    for (size_t k = 0; k < t.fill_dst.size(); ++k) {
+        int64_t s = t.fill_src[k];
+        for (size_t hops = 0; s <= -2 && hops <= t.fill_dst.size(); ++hops) {
+            const int64_t at = decode_prev(s);
+            if (at == t.fill_dst[k]) break;  // a ring
+            const auto it = src.find(at);
+            s = it == src.end() ? -1 : it->second;
+        }
+        if (t.fill_src[k] <= -2 && s >= 0) return false;
+    }
+    return true;
+}
+
+// The several-steps-per-launch plan of the new geometry.  A lattice it does
+// not suit, or without memory for its tables, keeps single steps.
+static int build_multi(imexlb_ctx *c, const DeviceTables &t)
+{
+    c->drop_multi();
+    if (!c->multi_enabled || !c->push_on || !c->fill32 || c->dim != 2 || IMEXLB_TILE != 64 ||
+        int64_t(c->kp.ncell) > c->multi_cells || !body_copies_zero(t))
+        return IMEXLB_OK;
+    plan_multi(int(c->ssz), c->kp, c->multi);
+    struct Tmp {  // freed on every return
+        void *p = nullptr;
+        ~Tmp()
+        {
+            if (p) (void)hipFree(p);
+        }
+    } dfrom, dbad;
+    const MultiPlan &m = c->multi;
+    const size_t nw = size_t(m.nx) * size_t(m.ny), nslots = size_t(c->Q) * size_t(c->plane);
+    const auto no_memory = [&] {
+        (void)hipGetLastError();
+        c->drop_multi();
+        return IMEXLB_OK;
+    };
+    if (hipMalloc((void **)&c->multi_table, nw * sizeof(int32_t)) != hipSuccess ||
+        hipMalloc(&dfrom.p, nslots * sizeof(int32_t)) != hipSuccess || hipMalloc(&dbad.p, 4) != hipSuccess)
+        return no_memory();
+    uint32_t bad = 0;
+    std::vector<int32_t> mark(nw);
+    HIP_TRY(hipMemset(dbad.p, 0, 4));
+    HIP_TRY(launch_multi_from(c->args(), static_cast<int32_t *>(dfrom.p), int64_t(nslots),
+                              static_cast<const int32_t *>(c->fill_dst), static_cast<const int32_t *>(c->fill_src),
+                              c->nfill, nullptr));
+    const auto plan = [&](uint16_t *place) {
+        return launch_multi_plan(c->args(), static_cast<int32_t *>(dfrom.p), m, c->multi_table, place,
+                                 static_cast<uint32_t *>(dbad.p), nullptr);
+    };
+    HIP_TRY(plan(nullptr));
+    HIP_TRY(hipMemcpy(&bad, dbad.p, 4, hipMemcpyDeviceToHost));
+    HIP_TRY(hipMemcpy(mark.data(), c->multi_table, nw * sizeof(int32_t), hipMemcpyDeviceToHost));
+    if (bad) {
+        c->drop_multi();
+        return IMEXLB_OK;
+    }
+    int32_t tables = 0;
+    for (int32_t &v : mark) v = v ? tables++ : -1;
+    if (hipMalloc((void **)&c->multi_place, std::max<size_t>(1, size_t(tables) * 9 * size_t(m.wx * m.wy) * 2)) != hipSuccess)
+        return no_memory();
+    HIP_TRY(hipMemcpy(c->multi_table, mark.data(), nw * sizeof(int32_t), hipMemcpyHostToDevice));
+    HIP_TRY(plan(c->multi_place));
+    HIP_TRY(hipDeviceSynchronize());
+    c->multi.table = c->multi_table;
+    c->multi.place = c->multi_place;
+    c->multi_on = true;
     return IMEXLB_OK;
 }
 
@@ -553,7 +645,7 @@ int imexlb_set_geometry_shape(imexlb_ctx *c, double pos, double radius, double a
         HIP_TRY(hipMemcpy(c->link_back, t.link_back.data(), t.link_back.size() * 8, hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(c->link_q, t.link_q.data(), t.link_q.size(), hipMemcpyHostToDevice));
     }
-    if ((rc = build_double(c))) return rc;
+    if ((rc = build_multi(c, t)) || (rc = build_double(c))) return rc;
     commit.done = c->geom_set = true;
     return IMEXLB_OK;
 }
@@ -787,7 +879,7 @@ int imexlb_post_processing(imexlb_ctx *c)
         c->lazy_src = c->cur;
         c->have_f = c->have_pu = false;
         c->stage = S_FUSED;
-        if (c->deferred >= imexlb_ctx::kDeferChunk) FLUSH(c);
+        if (c->deferred >= c->defer_chunk()) FLUSH(c);
         return IMEXLB_OK;
     }
     if (c->stage != S_STREAMED) return fail(IMEXLB_E_STATE, "PostProcessing must follow Propagation");
@@ -862,22 +954,19 @@ static int step_graph(imexlb_ctx *c, int size, int X, hipGraphExec_t *out)
     return IMEXLB_OK;
 }
 
-// kQuads[size] times two double steps (four steps, back in the same buffer),
-// the first reading fb[A], as one graph
-static int quad_graph(imexlb_ctx *c, int size, int A, hipGraphExec_t *out)
+// n launches of `one` from fb[A], one after the other between the two buffers,
+// as a graph
+extern "C++" template <class F>
+static int capture_passes(imexlb_ctx *c, int n, int A, hipGraphExec_t &slot, F &&one)
 {
-    hipGraphExec_t &slot = c->quad_graph[size][A];
-    if (slot) {
-        *out = slot;
-        return IMEXLB_OK;
-    }
+    if (slot) return IMEXLB_OK;
     StepArgs a = c->args();
     HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     hipError_t e = hipSuccess;
-    for (int k = 0; k < 2 * imexlb_ctx::kQuads[size] && e == hipSuccess; ++k) {
+    for (int k = 0; k < n && e == hipSuccess; ++k) {
         a.src = c->fb[A ^ (k & 1)];
         a.dst = c->fb[A ^ 1 ^ (k & 1)];
-        e = launch_double(c->dim, c->prec, a, c->dbl, c->stream);
+        e = one(a);
     }
     hipGraph_t g = nullptr;
     hipError_t e2 = hipStreamEndCapture(c->stream, &g);
@@ -885,12 +974,12 @@ static int quad_graph(imexlb_ctx *c, int size, int A, hipGraphExec_t *out)
         if (g) (void)hipGraphDestroy(g);
         return fail(IMEXLB_E_HIP, std::string("graph capture: ") + hipGetErrorString(e != hipSuccess ? e : e2));
     }
-    hipGraphExec_t x = nullptr;
-    e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
+    e = hipGraphInstantiate(&slot, g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
-    if (e != hipSuccess) return fail(IMEXLB_E_HIP, std::string("graph instantiate: ") + hipGetErrorString(e));
-    slot = x;
-    *out = x;
+    if (e != hipSuccess) {
+        slot = nullptr;
+        return fail(IMEXLB_E_HIP, std::string("graph instantiate: ") + hipGetErrorString(e));
+    }
     return IMEXLB_OK;
 }
 
@@ -915,11 +1004,49 @@ static int run_double_steps(imexlb_ctx *c, int A, int64_t n, int64_t *done)
     for (int j = 0; j < imexlb_ctx::kGraphSizes && quads > 0; ++j) {
         const int64_t reps = quads / imexlb_ctx::kQuads[j];
         if (reps <= 0) continue;
-        hipGraphExec_t g;
-        int rc = quad_graph(c, j, A, &g);
+        hipGraphExec_t &g = c->quad_graph[j][A];
+        int rc = capture_passes(c, 2 * imexlb_ctx::kQuads[j], A, g,
+                                [&](const StepArgs &a) { return launch_double(c->dim, c->prec, a, c->dbl, c->stream); });
         if (rc) return rc;
         for (int64_t k = 0; k < reps; ++k) HIP_TRY(hipGraphLaunch(g, c->stream));
         quads -= reps * imexlb_ctx::kQuads[j];
+    }
+    return IMEXLB_OK;
+}
+
+// The part of n fused steps from fb[A] that runs several steps per launch,
+// leaving at least one single step.  Every launch makes an odd number of
+// steps, so that the buffers end up as after as many single steps; only the
+// last leaves the boundary copies that single steps read.
+static int run_multi_steps(imexlb_ctx *c, int A, int64_t n, int64_t *done)
+{
+    *done = 0;
+    if (!c->multi_on || n < 4) return IMEXLB_OK;
+    const int K = c->multi.halo;
+    int64_t full = (n - 1) / K;
+    int rest = int((n - 1) % K);
+    if (!(rest & 1)) --rest;
+    if (rest < 3) rest = 0;
+    *done = K * full + rest;
+    if (rest == 0) --full;  // the last launch, with copies
+    if (c->graphs && !c->prof) {
+        for (int j = 0; j < imexlb_ctx::kGraphSizes; ++j)
+            for (; full >= imexlb_ctx::kMulti[j]; full -= imexlb_ctx::kMulti[j]) {
+                hipGraphExec_t &g = c->multi_graph[j][A];
+                int rc = capture_passes(c, imexlb_ctx::kMulti[j], A, g, [&](const StepArgs &a) {
+                    return launch_multi(c->prec, a, c->multi, K, false, c->stream);
+                });
+                if (rc) return rc;
+                HIP_TRY(hipGraphLaunch(g, c->stream));
+            }
+    }
+    for (; full >= 0; --full, A = 1 - A) {
+        const int steps = full > 0 || rest == 0 ? K : rest;
+        StepArgs a = c->args();
+        a.src = c->fb[A];
+        a.dst = c->fb[1 - A];
+        int rc = c->launch(0, [&] { return launch_multi(c->prec, a, c->multi, steps, full == 0, c->stream); }, steps);
+        if (rc) return rc;
     }
     return IMEXLB_OK;
 }
@@ -931,9 +1058,10 @@ static int run_double_steps(imexlb_ctx *c, int A, int64_t n, int64_t *done)
 static int run_fused_steps(imexlb_ctx *c, int A, int64_t n)
 {
     int64_t done = 0;
-    int rd = run_double_steps(c, A, n, &done);
+    int rd = c->dbl_on ? run_double_steps(c, A, n, &done) : run_multi_steps(c, A, n, &done);
     if (rd) return rd;
     n -= done;
+    A ^= int(done & 1);
     if (!c->graphs || c->prof) {
         for (; n > 0; --n, A = 1 - A) {
             int rc = c->run_step(c->collide_mode(), c->fb[A], c->fb[1 - A], nullptr);
@@ -975,7 +1103,7 @@ int imexlb_advance(imexlb_ctx *c, int64_t nsteps)
     if (nsteps < 0) return fail(IMEXLB_E_ARG, "negative step count");
     int64_t i = 0;
     // timed (profiled) runs launch kernel by kernel so each one is bracketed
-    if (c->can_defer() || (c->fused && c->dbl_on)) {
+    if (c->can_defer() || (c->fused && (c->dbl_on || c->multi_on))) {
         for (; i < nsteps && c->stage != S_FUSED; ++i) {
             int rc = one_step(c);
             if (rc) return rc;

@@ -96,7 +96,7 @@ struct imexlb_ctx {
     {
         geom_set = false;
         nfill = nlink = 0;
-        push_on = prefilled = dbl_on = false;
+        push_on = prefilled = dbl_on = multi_on = false;
         stage = S_NONE;
         have_pu = have_f = have_fb = false;
         lazy_src = -1;
@@ -120,7 +120,7 @@ struct imexlb_ctx {
     hipGraphExec_t graph[kGraphSizes][2] = {};
     void drop_graphs()
     {
-        for (auto *all : {&graph, &quad_graph})
+        for (auto *all : {&graph, &quad_graph, &multi_graph})
             for (auto &set : *all)
                 for (int k = 0; k < 2; ++k)
                     if (set[k]) {
@@ -138,6 +138,7 @@ struct imexlb_ctx {
     int64_t deferred = 0;
     int defer_src = 0;
     static constexpr int64_t kDeferChunk = 16;
+    int64_t defer_chunk() const { return multi_on ? 2 * multi.halo + 1 : kDeferChunk; }
     bool can_defer() const { return fused && graphs && !prof && push_on; }
 
     // Two steps in one pass over memory, for lattices that do not stay in the
@@ -146,6 +147,23 @@ struct imexlb_ctx {
     bool dbl_enabled = true, dbl_on = false;
     hipGraphExec_t quad_graph[kGraphSizes][2] = {};  // kQuads[j] pairs of double steps, by starting buffer
     static constexpr int kQuads[kGraphSizes] = {16, 4, 1};
+    // Several steps in one launch (built with the geometry; IMEXLB_MULTI=0
+    // keeps the other forms)
+    MultiPlan multi;
+    int32_t *multi_table = nullptr;
+    uint16_t *multi_place = nullptr;
+    bool multi_enabled = true, multi_on = false;
+    hipGraphExec_t multi_graph[kGraphSizes][2] = {};  // kMulti[j] launches of multi.halo steps
+    static constexpr int kMulti[kGraphSizes] = {16, 4, 2};  // even: they end in the buffer they began in
+    void drop_multi()
+    {
+        for (void *q : {(void *)multi_table, (void *)multi_place})
+            if (q) (void)hipFree(q);
+        multi_table = nullptr;
+        multi_place = nullptr;
+        multi = MultiPlan{};
+        multi_on = false;
+    }
     void drop_double()
     {
         for (void *q : {(void *)dbl.list[0], (void *)dbl.list[1], dbl.scratch})
@@ -249,6 +267,7 @@ struct imexlb_ctx {
         return K_COLLIDE | K_PUSH | (dim == 2 && int64_t(kp.ncell) <= small_cells ? K_SMALL : 0);
     }
     int64_t small_cells = 0;  // set at creation (IMEXLB_SMALL_CELLS)
+    int64_t multi_cells = 0;  // up to it several steps per launch
 
     int run_step(int mode, const void *src, void *dst, void *fout)
     {
@@ -291,6 +310,7 @@ struct imexlb_ctx {
         for (void *q : ptrs)
             if (q) (void)hipFree(q);
         drop_double();
+        drop_multi();
         fb[0] = fb[1] = f = nullptr;
         push_beg = nullptr;
         push_q = nullptr;

@@ -147,6 +147,21 @@ struct DoublePlan {
     uint32_t strips = 0, segments = 0;
     int rows = 0;
 };
+// Several steps of a small 2D lattice per launch (launch_multi): windows of
+// wx x wy cells, nx and ny of them along the axes, the steps a launch can make
+// at most (odd), and where each cell of a window pulls from.
+struct MultiPlan {
+    int nx = 0, ny = 0, wx = 0, wy = 0, halo = 0;
+    const int32_t *table = nullptr;   // a window's table of places, -1: plain
+    const uint16_t *place = nullptr;  // the tables
+};
+void plan_multi(int bytes, const KParams &kp, MultiPlan &m);
+hipError_t launch_multi_from(const StepArgs &a, int32_t *from, int64_t nslots, const int32_t *dslot,
+                             const int32_t *sslot, int64_t nfill, hipStream_t s);
+hipError_t launch_multi_plan(const StepArgs &a, const int32_t *from, const MultiPlan &m, int32_t *mark, uint16_t *place,
+                             uint32_t *bad, hipStream_t s);
+// copies: also the boundary copies of the last step
+hipError_t launch_multi(int prec, const StepArgs &a, const MultiPlan &m, int steps, bool copies, hipStream_t s);
 void plan_double(int dim, int bytes, const KParams &kp, DoublePlan &d);
 hipError_t launch_double(int dim, int prec, const StepArgs &a, const DoublePlan &d, hipStream_t s);
 // passes that find the frame: 0 special nodes to out; 1 in grown by a node to

@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <type_traits>
 
@@ -407,6 +408,23 @@ __device__ __forceinline__ void collide_f32(const float (&f)[Lat<D>::Q], float p
 }
 
 // ---------------------------------------------------------------------------
+// v / 3, correctly rounded as the division is, in three operations instead of
+// a dozen: with y the rounded reciprocal and q = v y within one unit in the
+// last place, q + (v - 3 q) y rounds to the quotient where v - 3 q is exact
+// (P. Markstein, IBM J. Res. Dev. 34, 1990).  Zero, infinite, NaN and values
+// so small that the remainder could be subnormal take the division.  (With the
+// divisions by rho0 = 1 gone as well, FP64 401 x 101 2.43 to 2.28 us a step.)
+__device__ __forceinline__ float third(float v) { return v / 3.0f; }
+__device__ __forceinline__ double third(double v)
+{
+    constexpr double y = 1.0 / 3.0;
+    const double q = v * y;
+    double t = __builtin_fma(__builtin_fma(-3.0, q, v), y, q);
+    const double a = __builtin_fabs(v);
+    if (!(a > 0x1p-960 && a < 0x1p1000)) t = v / 3.0;
+    return t;
+}
+
 // PostProcessing arithmetic on one node (lbm.f90:163-199): moments summed in
 // q order, divided by 3 and by rho0, then the inlet Dirichlet velocity at
 // x = 0 and the outlet p = 0 at x = nx.
@@ -431,10 +449,15 @@ __device__ __forceinline__ void moments(const C (&f)[Lat<D>::Q], const KParams &
         if (D == 3 && L::ez(q) < 0) sz = sz - f[q];
     }
     const C rho0 = C(kp.rho0);
-    p = ps / C(3);
-    ux = sx / rho0;
-    uy = sy / rho0;
-    uz = D == 3 ? sz / rho0 : C(0);
+    p = third(ps);
+    ux = sx;
+    uy = sy;
+    uz = D == 3 ? sz : C(0);
+    if (rho0 != C(1)) {  // the same for every node: no division where it changes nothing
+        ux = sx / rho0;
+        uy = sy / rho0;
+        if (D == 3) uz = sz / rho0;
+    }
     if (x == 0) {  // inlet, lbm.f90:186-191 (3D: profile in z, u_z kept, lbm_3d.f90:188-193)
         const int h = D == 2 ? y : z;
         const int nh = D == 2 ? kp.ny : kp.nz;
@@ -1169,6 +1192,211 @@ __global__ __launch_bounds__(256) void k_zone_list(const uint8_t *__restrict__ m
 }
 
 // ---------------------------------------------------------------------------
+// Several steps of a D2Q9 lattice in one launch.  A small lattice's step
+// launched alone takes the time of a launch and of one wave's chain of loads,
+// arithmetic and stores, 3 to 5 us whatever the size; a large one's that of
+// moving every population.  Here a block loads a window of WX x WY cells, makes up to `halo` steps of it in LDS
+// and writes the cells that are still right: those `halo` cells from a side of
+// the window that is not a side of the lattice.  One thread per cell, which
+// keeps the LDS places of the nine populations it pulls in registers (from a
+// table, k_multi_plan): a pull that would read a boundary copy reads the copy's
+// source, so a step is nine LDS reads, the arithmetic and nine LDS writes, and
+// no copies are made but after the last step of a run.  Windows of fluid nodes
+// only need no table: their places are constants.
+//
+// Bound by the arithmetic, a third to half of it on cells that a neighbouring
+// window writes, and for small lattices by the 3 us of a launch per 5 to 9
+// steps.  us a step, single steps and now: FP64 49 x 25 3.36 and 1.26, 401 x
+// 101 3.67 and 2.36, 2001 x 501 22.5 and 17.1; FP32 401 x 101 3.06 and 1.45,
+// 2801 x 701 22.2 and 12.4; FP16 401 x 101 3.08 and 1.29, 5002 x 1252 (two
+// steps per pass) 38.1 and 35.2.  Tables for all windows cost FP32 2801 x 701
+// 14.3.
+
+// Windows along an axis of n nodes: one where they all fit (m == 1), else m
+// that write W - 2 halo nodes each.  In x they go round the lattice like a
+// ring, since the corner cells' copies come from the other end of the channel
+// (the periodic image); in y the first and last begin and end at the walls.
+struct WinAxis {
+    int first, lo, hi;  // first node (x: may be < 0), the nodes it writes: lo <= node < hi
+};
+template <int W>
+__device__ __forceinline__ WinAxis win_axis(int i, int m, int n, int halo, bool ring)
+{
+    const int out = W - 2 * halo;
+    if (m == 1) return {0, 0, n};
+    if (ring) return {i * out - halo, i * out, min(n, (i + 1) * out)};
+    const bool left = i == 0, right = i == m - 1;
+    return {left ? 0 : right ? n - W : i * out, left ? 0 : i * out + halo, right ? n : (i + 1) * out + halo};
+}
+
+// cell of a thread of a window; false outside the lattice
+template <int WX, int WY>
+__device__ __forceinline__ bool win_cell(const KParams &kp, const MultiPlan &m, WinAxis &ax, WinAxis &ay, int &x, int &y)
+{
+    const int i = int(blockIdx.x) % m.nx, j = int(blockIdx.x) / m.nx, n = kp.nx + 1;
+    ax = win_axis<WX>(i, m.nx, n, m.halo, true);
+    ay = win_axis<WY>(j, m.ny, kp.ny + 1, m.halo, false);
+    x = ax.first + int(threadIdx.x) % WX;
+    y = ay.first + int(threadIdx.x) / WX;
+    if (m.nx > 1) x = x < 0 ? x + n : x >= n ? x - n : x;
+    return x <= kp.nx && y <= kp.ny;
+}
+__device__ __forceinline__ bool win_writes(int l, const WinAxis &a) { return a.first + l >= a.lo && a.first + l < a.hi; }
+
+// Slot that each slot of the populations takes its value from within a step:
+// itself for a fluid node, the source for a boundary copy (k_multi_copies), -1
+// where the value is always 0.
+__global__ __launch_bounds__(256) void k_multi_from(const uint8_t *__restrict__ geo, int32_t *__restrict__ from,
+                                                    int64_t n)
+{
+    const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t s = uint32_t(i);
+    from[i] = (geo[s / (9u * 64u) * 64u + s % 64u] & G_FLUID) ? int32_t(s) : -1;
+}
+__global__ __launch_bounds__(256) void k_multi_copies(int32_t *__restrict__ from, const int32_t *__restrict__ dslot,
+                                                      const int32_t *__restrict__ sslot, int64_t n)
+{
+    const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    if (i < n) from[dslot[i]] = max(sslot[i], -1);  // (a previous step's body value: 0)
+}
+
+// The tables of places, [table][direction][cell], of the windows that are not
+// plain; a plain one holds fluid nodes only that all pull from their
+// neighbours.  from: the slot that each slot of a boundary copy takes its value
+// from (its own slot: no copy; -1: it is 0).  First pass (place == nullptr):
+// marks the windows that need a table, and sets *bad where a cell that is
+// written would not be right for `halo` steps; second pass: writes them.
+template <int WX, int WY>
+__global__ __launch_bounds__(WX *WY) void k_multi_plan(const int32_t *__restrict__ from,
+                                                       const uint8_t *__restrict__ geo, KParams kp, MultiPlan m,
+                                                       int32_t *__restrict__ mark, uint16_t *__restrict__ place,
+                                                       uint32_t *__restrict__ bad)
+{
+    using L = Lat<2>;
+    constexpr uint32_t N = WX * WY;
+    __shared__ int right[2][N];  // steps for which a cell is right
+    const uint32_t th = threadIdx.x;
+    WinAxis ax, ay;
+    int x, y;
+    const bool in = win_cell<WX, WY>(kp, m, ax, ay, x, y);
+    const uint32_t c = in ? uint32_t(kp.o0 + x + kp.Px * y) : 0u;
+    const bool fluid = in && (geo[c] & G_FLUID);
+    bool special = !fluid || (geo[c] & G_PUSH) || x == 0 || x == kp.nx;
+    int source[L::Q];  // cell of the window a pull reads; -1 outside; -2 none
+    for (int q = 0; q < L::Q; ++q) {
+        uint32_t at = uint32_t(q) * N + th;
+        source[q] = -2;
+        if (fluid) {
+            const uint32_t pulled = cslot<L::Q>(kp, uint32_t(q), c - shift32<2>(kp, q));
+            const int32_t s = from[pulled];
+            special |= s != int32_t(pulled);
+            if (s < 0) {
+                at = 9u * N;  // the place that holds 0
+            } else {          // slot -> cell and direction -> place in the window
+                const uint32_t sc = uint32_t(s) / (9u * 64u) * 64u + uint32_t(s) % 64u, sq = uint32_t(s) / 64u % 9u;
+                int sx = int(sc % uint32_t(kp.Px)) - 1 - ax.first;
+                const int sy = int(sc / uint32_t(kp.Px)) - 1 - ay.first;
+                if (m.nx > 1) sx = sx < 0 ? sx + kp.nx + 1 : sx > kp.nx ? sx - kp.nx - 1 : sx;
+                source[q] = -1;
+                if (sx >= 0 && sx < WX && sy >= 0 && sy < WY) {
+                    source[q] = sy * WX + sx;
+                    at = sq * N + uint32_t(source[q]);
+                }
+            }
+        }
+        if (place && mark[blockIdx.x] >= 0) place[(uint32_t(mark[blockIdx.x]) * 9u + uint32_t(q)) * N + th] = uint16_t(at);
+    }
+    if (place) return;
+    int mine = fluid ? m.halo : 0;
+    right[0][th] = mine;
+    for (int k = 0; k < m.halo; ++k) {
+        __syncthreads();
+        for (int q = 0; q < L::Q; ++q)
+            if (source[q] != -2) mine = min(mine, source[q] < 0 ? 0 : right[k & 1][source[q]] + 1);
+        right[(k & 1) ^ 1][th] = mine;
+    }
+    if (fluid && mine < m.halo && win_writes(int(th) % WX, ax) && win_writes(int(th) / WX, ay)) atomicOr(bad, 1u);
+    const int any = __syncthreads_or(special);
+    if (th == 0) mark[blockIdx.x] = any;
+}
+
+template <class S, class C, int WX, int WY>
+__global__ __launch_bounds__(WX *WY) void k_multi2(const S *__restrict__ src, S *__restrict__ dst,
+                                                   const uint8_t *__restrict__ geo, KParams kp, PushTable pt,
+                                                   MultiPlan m, int steps, int copies)
+{
+    using L = Lat<2>;
+    using U = BitsOf<S>;
+    constexpr uint32_t N = WX * WY;
+    __shared__ U cells[2][9 * N + 8];
+    const uint32_t th = threadIdx.x;
+    const int32_t table = m.table[blockIdx.x];
+    WinAxis ax, ay;
+    int x, y;
+    const bool in = win_cell<WX, WY>(kp, m, ax, ay, x, y);
+    const uint32_t c = uint32_t(kp.o0 + min(x, kp.nx) + kp.Px * min(y, kp.ny));
+#pragma unroll
+    for (int q = 0; q < L::Q; ++q)
+        cells[0][uint32_t(q) * N + th] = __builtin_bit_cast(U, src[cslot<L::Q>(kp, uint32_t(q), c)]);
+    uint8_t g = G_FLUID;
+    U out[L::Q] = {};
+    const auto node = [&](const C(&f)[L::Q], int xn) {
+        C p, ux, uy, uz;
+        moments<2, C>(f, kp, xn, y, 0, p, ux, uy, uz);
+        const uint32_t srw = sr_word<S>(p, sr_cell<S>(kp, c, y, 0));
+        collide<2, C>(f, p, ux, uy, uz, kp, [&](int q, C v) {
+            out[q] = __builtin_bit_cast(U, Store<S>::template st<C>(v, srw + uint32_t(q) * kGolden));
+        });
+    };
+    const auto keep = [&](int k) {
+        if (k + 1 < steps) {
+            U *const b = cells[(k & 1) ^ 1] + th;
+#pragma unroll
+            for (int q = 0; q < L::Q; ++q) b[uint32_t(q) * N] = out[q];
+        }
+    };
+    if (table < 0) {  // the same for the block
+        // (at the window's edges these reads fall on other cells of the array:
+        // direction 0 reads ahead, 8 back)
+        for (int k = 0; k < steps; ++k) {
+            __syncthreads();
+            C f[L::Q];
+#pragma unroll
+            for (int q = 0; q < L::Q; ++q)
+                f[q] = Store<S>::ld(
+                    __builtin_bit_cast(S, cells[k & 1][uint32_t(q) * N + th - uint32_t(L::ey(q) * WX + L::ex(q))]));
+            node(f, -1);
+            keep(k);
+        }
+    } else {
+        uint32_t at[L::Q];
+#pragma unroll
+        for (int q = 0; q < L::Q; ++q) at[q] = m.place[(uint32_t(table) * 9u + uint32_t(q)) * N + th];
+        g = in ? geo[c] : uint8_t(0);
+        if (th < 2) cells[th][9 * N] = U(0);
+        for (int k = 0; k < steps; ++k) {
+            __syncthreads();
+            if (g & G_FLUID) {
+                C f[L::Q];
+#pragma unroll
+                for (int q = 0; q < L::Q; ++q) f[q] = Store<S>::ld(__builtin_bit_cast(S, cells[k & 1][at[q]]));
+                node(f, x);
+                keep(k);
+            }
+        }
+    }
+    if (!(g & G_FLUID) || !win_writes(int(th) % WX, ax) || !win_writes(int(th) / WX, ay)) return;
+#pragma unroll
+    for (int q = 0; q < L::Q; ++q) dst[cslot<L::Q>(kp, uint32_t(q), c)] = __builtin_bit_cast(S, out[q]);
+    if (copies && (g & G_PUSH)) {
+        const int32_t *const to = static_cast<const int32_t *>(pt.dst);
+        for (int32_t e = pt.beg[c], ee = pt.beg[c + 1]; e < ee; ++e)
+            dst[uint32_t(to[e])] = __builtin_bit_cast(S, pick(out, pt.q[e]));
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Batched ensemble: many independent lattices advanced by one launch.  The
 // interior nodes of every case are cut into tiles of BLOCK*CPT nodes; a
 // block takes a tile (by its index, or from a queue when PERSIST), reads the
@@ -1604,6 +1832,86 @@ hipError_t launch_double(int dim, int prec, const StepArgs &a, const DoublePlan 
     });
     if (e != hipSuccess) return e;
     return launch_step_list(dim, prec, d.idx64, second, d.list[1], d.count[1], s);
+}
+
+template <class F>
+static hipError_t dispatch_window(const MultiPlan &m, F &&f)
+{
+    if (m.wx == 16) return f(std::integral_constant<int, 16>{}, std::integral_constant<int, 16>{});
+    if (m.wy == 16) return f(std::integral_constant<int, 32>{}, std::integral_constant<int, 16>{});
+    return f(std::integral_constant<int, 32>{}, std::integral_constant<int, 32>{});
+}
+
+// Window and steps per launch by an estimate of the time per step (us): a
+// launch costs 3.1 and its loads and stores 1 per 5 MB; a step 0.3 and, for
+// each wave that a SIMD of the fullest CU has to run, 0.27 in FP64 or 0.1.
+// Small lattices leave CUs idle, so small windows serve them best; larger ones
+// pay for the cells computed twice; with several rounds of blocks on a CU the
+// memory time and the arithmetic overlap unless a block fills the CU's LDS.
+// Within 15 % of the times measured from 49 x 25 to 2001 x 501 in FP64, FP32
+// and FP16, and the best or next best of the seven windows in each.
+void plan_multi(int bytes, const KParams &kp, MultiPlan &m)
+{
+    struct Window {
+        int wx, wy, halo;
+    };
+    constexpr Window windows[] = {{32, 32, 5}, {32, 32, 7}, {32, 32, 9}, {32, 16, 3}, {32, 16, 5}, {16, 16, 5}};
+    const int nx = kp.nx + 1, ny = kp.ny + 1;
+    double best = 1e300;
+    for (const Window &w : windows) {
+        const int ox = w.wx - 2 * w.halo, oy = w.wy - 2 * w.halo, cells = w.wx * w.wy;
+        const int mx = nx <= w.wx ? 1 : (nx + ox - 1) / ox;
+        const int my = ny <= w.wy ? 1 : 2 + std::max(0, (ny - 2 * (w.wy - w.halo) + oy - 1) / oy);
+        const double blocks = double(mx) * my, slots = 9.0 * bytes;
+        const int fit = std::min(2048 / cells, int(160 * 1024 / (18.0 * cells * bytes)));  // blocks of a CU
+        const double waves = std::ceil(blocks / 256.0) * cells / 256.0;
+        const double arith = 0.3 + (bytes == 8 ? 0.27 : 0.1) * waves;
+        const double memory = (3.1 + (blocks * cells + double(nx) * ny) * slots / 5e6) / w.halo;
+        const bool overlap = fit > 1 && blocks > 512.0 * fit;
+        const double t = overlap ? std::max(arith, memory) + 0.3 * std::min(arith, memory) : arith + memory;
+        if (t < best) {
+            best = t;
+            m.wx = w.wx;
+            m.wy = w.wy;
+            m.halo = w.halo;
+            m.nx = mx;
+            m.ny = my;
+        }
+    }
+}
+
+hipError_t launch_multi_from(const StepArgs &a, int32_t *from, int64_t nslots, const int32_t *dslot,
+                             const int32_t *sslot, int64_t nfill, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_multi_from, dim3(nblocks(uint64_t(nslots))), dim3(256), 0, s, a.geo, from, nslots);
+    if (nfill > 0)
+        hipLaunchKernelGGL(k_multi_copies, dim3(nblocks(uint64_t(nfill))), dim3(256), 0, s, from, dslot, sslot, nfill);
+    return hipGetLastError();
+}
+
+hipError_t launch_multi_plan(const StepArgs &a, const int32_t *from, const MultiPlan &m, int32_t *mark, uint16_t *place,
+                             uint32_t *bad, hipStream_t s)
+{
+    return dispatch_window(m, [&](auto wx, auto wy) {
+        constexpr int WX = decltype(wx)::value, WY = decltype(wy)::value;
+        hipLaunchKernelGGL((k_multi_plan<WX, WY>), dim3(unsigned(m.nx * m.ny)), dim3(WX * WY), 0, s, from, a.geo, a.kp,
+                           m, mark, place, bad);
+        return hipGetLastError();
+    });
+}
+
+hipError_t launch_multi(int prec, const StepArgs &a, const MultiPlan &m, int steps, bool copies, hipStream_t s)
+{
+    return dispatch_prec(prec, [&](auto *sp, auto *cp) {
+        using S = std::remove_pointer_t<decltype(sp)>;
+        using C = std::remove_pointer_t<decltype(cp)>;
+        return dispatch_window(m, [&](auto wx, auto wy) {
+            constexpr int WX = decltype(wx)::value, WY = decltype(wy)::value;
+            hipLaunchKernelGGL((k_multi2<S, C, WX, WY>), dim3(unsigned(m.nx * m.ny)), dim3(WX * WY), 0, s,
+                               (const S *)a.src, (S *)a.dst, a.geo, a.kp, a.push, m, steps, int(copies));
+            return hipGetLastError();
+        });
+    });
 }
 
 hipError_t launch_zone(int dim, int pass, const StepArgs &a, uint8_t *geo, const uint8_t *in, uint8_t *out,
