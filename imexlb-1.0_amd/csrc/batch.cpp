@@ -7,7 +7,8 @@
 // cases whose table does not qualify need the fill.  The step kernel takes the cases'
 // nodes in tiles of block*cells_per_thread nodes, by block index or from a
 // queue (persistent blocks); imexlb_batch_tune times the configurations and
-// keeps the fastest.  Pairs of steps replay as a HIP graph.
+// keeps the fastest.  Pairs of steps replay as a HIP graph.  Where every case
+// suits it, all but the last steps of an advance run several per launch.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -63,6 +64,16 @@ struct imexlb_batch {
     hipGraphExec_t graph[kGraphSizes][2] = {};
     bool graphs = true;  // replay captured pairs of steps (IMEXLB_GRAPHS=0: launch every step)
 
+    // several steps per launch (every case qualifies): a window's case, the
+    // cases' tables; IMEXLB_MULTI=0 keeps single steps
+    uint32_t *window_case = nullptr;
+    int32_t *multi_table = nullptr;
+    uint16_t *multi_place = nullptr;
+    uint32_t nwindows = 0;
+    bool multi_on = false;
+    static constexpr int kMulti = 8;  // launches per graph: even, it ends in the buffer it began in
+    hipGraphExec_t multi_graph[2] = {};
+
     int cur = 1, lazy = -1;
     bool initialized = false, have_pu = false;
 
@@ -74,6 +85,11 @@ struct imexlb_batch {
                     (void)hipGraphExecDestroy(g);
                     g = nullptr;
                 }
+        for (auto &g : multi_graph)
+            if (g) {
+                (void)hipGraphExecDestroy(g);
+                g = nullptr;
+            }
     }
 
     void release()
@@ -86,7 +102,7 @@ struct imexlb_batch {
         void *ptrs[] = {fb[0],     fb[1],      f,        p,         ux,        uy,            rv,
                         geo,       fill_dst,   fill_src, link_out,  link_back, link_q,        force_partial,
                         force_out, mon,        d_cases,  queue,     tile_case, tile_first,
-                        push_beg,  push_dst,   push_q};
+                        push_beg,  push_dst,   push_q,   window_case, multi_table, multi_place};
         for (void *q : ptrs)
             if (q) (void)hipFree(q);
         if (stream) (void)hipStreamDestroy(stream);
@@ -158,6 +174,56 @@ struct imexlb_batch {
         return IMEXLB_OK;
     }
 
+    hipError_t enqueue_multi(int b, int steps, bool copies)
+    {
+        return launch_batch_multi(prec, cases[0].multi, fb[b], fb[1 - b], geo, d_cases, window_case, nwindows, steps,
+                                  copies, stream);
+    }
+
+    // The part of n steps that runs several per launch, leaving at least one
+    // single step; every launch makes an odd number of steps, so that the
+    // buffers end up as after as many single steps, and the last leaves the
+    // boundary copies that single steps read.
+    int multi_steps(int64_t n, int64_t *done)
+    {
+        *done = 0;
+        if (!multi_on || n < 4) return IMEXLB_OK;
+        const int K = cases[0].multi.halo;
+        int64_t full = (n - 1) / K;
+        int rest = int((n - 1) % K);
+        if (!(rest & 1)) --rest;
+        if (rest < 3) rest = 0;
+        *done = K * full + rest;
+        if (rest == 0) --full;  // the last launch, with copies
+        if (graphs && full >= kMulti) {
+            hipGraphExec_t &g = multi_graph[cur];
+            if (!g) {
+                HIP_TRY(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+                hipError_t e = hipSuccess;
+                for (int k = 0; k < kMulti && e == hipSuccess; ++k) e = enqueue_multi(cur ^ (k & 1), K, false);
+                hipGraph_t gr = nullptr;
+                const hipError_t e2 = hipStreamEndCapture(stream, &gr);
+                if (e == hipSuccess) e = e2;
+                if (e == hipSuccess) e = hipGraphInstantiate(&g, gr, nullptr, nullptr, 0);
+                if (gr) (void)hipGraphDestroy(gr);
+                if (e != hipSuccess) {
+                    g = nullptr;
+                    return fail(IMEXLB_E_HIP, std::string("batch graph: ") + hipGetErrorString(e));
+                }
+            }
+            for (; full >= kMulti; full -= kMulti) HIP_TRY(hipGraphLaunch(g, stream));
+        }
+        for (; full >= 0; --full) {
+            const hipError_t e = enqueue_multi(cur, full > 0 || rest == 0 ? K : rest, full == 0);
+            if (e != hipSuccess) return fail(IMEXLB_E_HIP, std::string("batch steps: ") + hipGetErrorString(e));
+            cur = 1 - cur;
+        }
+        have_pu = false;
+        return IMEXLB_OK;
+    }
+
+    int build_multi(const std::vector<int32_t> &fd, const std::vector<int32_t> &fs, const std::vector<int64_t> &first);
+
     int pair_graph(int size, hipGraphExec_t *out)
     {
         hipGraphExec_t &slot = graph[size][cur];
@@ -215,6 +281,14 @@ int balloc(imexlb_batch *b, void **ptr, size_t bytes)
     return IMEXLB_OK;
 }
 
+struct DeviceTemp {  // freed on every return
+    void *p = nullptr;
+    ~DeviceTemp()
+    {
+        if (p) (void)hipFree(p);
+    }
+};
+
 #define CHECK_BATCH(b)                                                    \
     do {                                                                  \
         if (!(b)) return fail(IMEXLB_E_ARG, "null batch");               \
@@ -222,6 +296,82 @@ int balloc(imexlb_batch *b, void **ptr, size_t bytes)
     } while (0)
 
 }  // namespace
+
+// The windows of every case and their tables; fd, fs: the cases' boundary
+// fills in slots within the case, those of case i from first[i] on.  Batches
+// that have no memory for them or a case they do not suit keep single steps.
+int imexlb_batch::build_multi(const std::vector<int32_t> &fd, const std::vector<int32_t> &fs,
+                              const std::vector<int64_t> &first)
+{
+    std::vector<const KParams *> lattices;
+    int64_t slots = 0;
+    for (const BatchCase &bc : cases) lattices.push_back(&bc.kp);
+    for (const imexlb_ctx *c : host) slots = std::max(slots, int64_t(c->Q) * c->plane);
+    std::vector<MultiPlan> plans;
+    plan_multi(int(ssz), lattices, plans);
+    std::vector<uint32_t> wc;
+    for (int i = 0; i < ncase; ++i) {
+        cases[size_t(i)].first_window = int(wc.size());
+        wc.insert(wc.end(), size_t(plans[size_t(i)].nx) * size_t(plans[size_t(i)].ny), uint32_t(i));
+    }
+    DeviceTemp from, dbad, dfd, dfs;
+    const auto drop = [&] {
+        (void)hipGetLastError();
+        for (void *q : {(void *)window_case, (void *)multi_table, (void *)multi_place})
+            if (q) (void)hipFree(q);
+        window_case = nullptr;
+        multi_table = nullptr;
+        multi_place = nullptr;
+        return IMEXLB_OK;
+    };
+    const size_t nw = wc.size(), nf = std::max<size_t>(fd.size(), 1);
+    if (hipMalloc((void **)&window_case, nw * 4) != hipSuccess || hipMalloc((void **)&multi_table, nw * 4) != hipSuccess ||
+        hipMalloc(&from.p, size_t(slots) * 4) != hipSuccess || hipMalloc(&dbad.p, 4) != hipSuccess ||
+        hipMalloc(&dfd.p, nf * 4) != hipSuccess || hipMalloc(&dfs.p, nf * 4) != hipSuccess)
+        return drop();
+    HIP_TRY(hipMemcpy(window_case, wc.data(), nw * 4, hipMemcpyHostToDevice));
+    if (!fd.empty()) {
+        HIP_TRY(hipMemcpy(dfd.p, fd.data(), fd.size() * 4, hipMemcpyHostToDevice));
+        HIP_TRY(hipMemcpy(dfs.p, fs.data(), fs.size() * 4, hipMemcpyHostToDevice));
+    }
+    HIP_TRY(hipMemsetAsync(dbad.p, 0, 4, stream));
+    int32_t *const fr = static_cast<int32_t *>(from.p);
+    const auto plan = [&](uint16_t *place) {
+        for (int i = 0; i < ncase; ++i) {
+            const StepArgs a = case_args(i);
+            const int64_t f0 = first[size_t(i)], f1 = size_t(i) + 1 < first.size() ? first[size_t(i) + 1] : int64_t(fd.size());
+            hipError_t e = launch_multi_from(a, fr, int64_t(host[size_t(i)]->Q) * host[size_t(i)]->plane,
+                                             static_cast<int32_t *>(dfd.p) + f0, static_cast<int32_t *>(dfs.p) + f0,
+                                             f1 - f0, stream);
+            if (e == hipSuccess)
+                e = launch_multi_plan(a, fr, plans[size_t(i)], multi_table + cases[size_t(i)].first_window, place,
+                                      static_cast<uint32_t *>(dbad.p), stream);
+            if (e != hipSuccess) return e;
+        }
+        return hipStreamSynchronize(stream);
+    };
+    HIP_TRY(plan(nullptr));
+    uint32_t bad = 0;
+    std::vector<int32_t> mark(nw);
+    HIP_TRY(hipMemcpy(&bad, dbad.p, 4, hipMemcpyDeviceToHost));
+    HIP_TRY(hipMemcpy(mark.data(), multi_table, nw * 4, hipMemcpyDeviceToHost));
+    if (bad) return drop();
+    int32_t tables = 0;
+    for (int32_t &v : mark) v = v ? tables++ : -1;
+    const size_t cells = size_t(plans[0].wx * plans[0].wy);
+    if (hipMalloc((void **)&multi_place, std::max<size_t>(1, size_t(tables) * 9 * cells * 2)) != hipSuccess) return drop();
+    HIP_TRY(hipMemcpy(multi_table, mark.data(), nw * 4, hipMemcpyHostToDevice));
+    HIP_TRY(plan(multi_place));
+    for (int i = 0; i < ncase; ++i) {
+        BatchCase &bc = cases[size_t(i)];
+        bc.multi = plans[size_t(i)];
+        bc.multi.table = multi_table + bc.first_window;
+        bc.multi.place = multi_place;
+    }
+    nwindows = uint32_t(nw);
+    multi_on = true;
+    return IMEXLB_OK;
+}
 
 extern "C" {
 
@@ -260,6 +410,10 @@ int imexlb_batch_create_shapes(imexlb_batch **out, int ncase, const int32_t *nxn
     std::vector<int64_t> beg_off, ent_off;  // per case (-1: the case is filled every step)
     std::vector<int8_t> lq;
     std::vector<uint8_t> geo;
+    const char *mv = std::getenv("IMEXLB_MULTI");
+    bool multi = !(mv && mv[0] == '0') && IMEXLB_TILE == 64;
+    std::vector<int32_t> mfd, mfs;  // every case's fill in slots within the case
+    std::vector<int64_t> mfirst;
     const char *pv = std::getenv("IMEXLB_PUSH");
     const bool push_enabled = !(pv && pv[0] == '0');
     for (int i = 0; i < ncase; ++i) {
@@ -288,6 +442,12 @@ int imexlb_batch_create_shapes(imexlb_batch **out, int ncase, const int32_t *nxn
             const int64_t s = t.fill_src[k];
             fdc.push_back(t.fill_dst[k] + pb);
             fsc.push_back(s >= 0 ? s + pb : s == -1 ? -1 : encode_prev(decode_prev(s) + pb));
+        }
+        multi = multi && push && body_copies_zero(t);
+        mfirst.push_back(int64_t(mfd.size()));
+        for (size_t k = 0; multi && k < t.fill_dst.size(); ++k) {
+            mfd.push_back(int32_t(t.fill_dst[k]));
+            mfs.push_back(int32_t(t.fill_src[k]));
         }
         if (push) {  // slots within the case: the step offsets dst by pop_base
             beg_off.push_back(int64_t(pbeg.size()));
@@ -366,6 +526,7 @@ int imexlb_batch_create_shapes(imexlb_batch **out, int ncase, const int32_t *nxn
         HIP_TRY(hipMemcpy(B->link_back, lbk.data(), lbk.size() * 8, hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(B->link_q, lq.data(), lq.size(), hipMemcpyHostToDevice));
     }
+    if (multi && (rc = B->build_multi(mfd, mfs, mfirst))) return rc;
     HIP_TRY(hipMemcpy(B->d_cases, B->cases.data(), size_t(ncase) * sizeof(BatchCase), hipMemcpyHostToDevice));
     if ((rc = B->build_tiles())) return rc;
     *out = b.release();
@@ -494,6 +655,9 @@ int imexlb_batch_advance(imexlb_batch *b, int64_t nsteps)
         if (rc) return rc;
         --nsteps;
     }
+    int64_t done = 0;
+    if (int rc = b->multi_steps(nsteps, &done)) return rc;
+    nsteps -= done;
     if (!b->graphs) {
         for (int64_t k = 0; k < nsteps; ++k) {
             int rc = b->one_step();

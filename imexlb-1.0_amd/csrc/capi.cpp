@@ -20,7 +20,6 @@
 #include <memory>
 #include <new>
 #include <string>
-#include <unordered_map>
 #include <vector>
 
 #include "context.hpp"
@@ -212,6 +211,24 @@ int build_device_tables(const imexlb_ctx *c, DeviceTables &t)
                 }
             }
     return IMEXLB_OK;
+}
+
+bool body_copies_zero(const DeviceTables &t)
+{
+    const size_t n = t.fill_dst.size();
+    std::vector<uint8_t> seen(n, 0);  // entries found to be 0, or on the way there (a ring)
+    for (size_t k = 0; k < n; ++k) {
+        size_t at = k;
+        while (!seen[at] && t.fill_src[at] <= -2) {
+            seen[at] = 1;
+            const int64_t s = decode_prev(t.fill_src[at]);
+            const auto it = std::lower_bound(t.fill_dst.begin(), t.fill_dst.end(), s);  // in order
+            if (it == t.fill_dst.end() || *it != s) break;  // never written
+            at = size_t(it - t.fill_dst.begin());
+            if (t.fill_src[at] >= 0) return false;
+        }
+    }
+    return true;
 }
 
 }  // namespace imexlb
@@ -481,26 +498,6 @@ static int build_double(imexlb_ctx *c)
     return IMEXLB_OK;
 }
 
-// Whether every boundary copy of a previous step's body value is always 0: such
-// values mostly go round among body cells (a mirror's mirror is the cell
-// itself) and stay the 0 they start with.
-static bool body_copies_zero(const DeviceTables &t)
-{
-    std::unordered_map<int64_t, int64_t> src;
-    for (size_t k = 0; k < t.fill_dst.size(); ++k) src.emplace(t.fill_dst[k], t.fill_src[k]);
-    for (size_t k = 0; k < t.fill_dst.size(); ++k) {
-        int64_t s = t.fill_src[k];
-        for (size_t hops = 0; s <= -2 && hops <= t.fill_dst.size(); ++hops) {
-            const int64_t at = decode_prev(s);
-            if (at == t.fill_dst[k]) break;  // a ring
-            const auto it = src.find(at);
-            s = it == src.end() ? -1 : it->second;
-        }
-        if (t.fill_src[k] <= -2 && s >= 0) return false;
-    }
-    return true;
-}
-
 // The several-steps-per-launch plan of the new geometry.  A lattice it does
 // not suit, or without memory for its tables, keeps single steps.
 static int build_multi(imexlb_ctx *c, const DeviceTables &t)
@@ -509,7 +506,9 @@ static int build_multi(imexlb_ctx *c, const DeviceTables &t)
     if (!c->multi_enabled || !c->push_on || !c->fill32 || c->dim != 2 || IMEXLB_TILE != 64 ||
         int64_t(c->kp.ncell) > c->multi_cells || !body_copies_zero(t))
         return IMEXLB_OK;
-    plan_multi(int(c->ssz), c->kp, c->multi);
+    std::vector<MultiPlan> plans;
+    plan_multi(int(c->ssz), {&c->kp}, plans);
+    c->multi = plans[0];
     struct Tmp {  // freed on every return
         void *p = nullptr;
         ~Tmp()

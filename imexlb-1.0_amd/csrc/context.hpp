@@ -366,6 +366,11 @@ struct DeviceTables {
 };
 int build_device_tables(const imexlb_ctx *c, DeviceTables &t);
 
+// Whether every boundary copy of a previous step's body value is always 0: such
+// values mostly go round among body cells (a mirror's mirror is the cell
+// itself) and stay the 0 they start with.
+bool body_copies_zero(const DeviceTables &t);
+
 // The boundary fill's slot tables fit int32 entries when every slot and its
 // previous-step encoding (-slot-2) do.
 inline bool fill_fits_32(int64_t nslots) { return nslots < (int64_t(1) << 31) - 2; }

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <vector>
 
 namespace imexlb {
 
@@ -117,6 +118,15 @@ struct PushTable {
     const uint16_t *lds = nullptr;
 };
 
+// Several steps of a 2D lattice per launch (launch_multi): windows of
+// wx x wy cells, nx and ny of them along the axes, the steps a launch can make
+// at most (odd), and where each cell of a window pulls from.
+struct MultiPlan {
+    int nx = 0, ny = 0, wx = 0, wy = 0, halo = 0;
+    const int32_t *table = nullptr;   // a window's table of places, -1: plain
+    const uint16_t *place = nullptr;  // the tables
+};
+
 // One case of a batched ensemble: its parameters and where its populations
 // and node types start in the shared arrays.
 struct BatchCase {
@@ -124,6 +134,8 @@ struct BatchCase {
     int64_t pop_base;  // first population slot of the case
     int64_t geo_base;  // first cell of the case (node types, p, u)
     PushTable pt;      // the case's boundary copies (int32 slots within the case), pushed by the step
+    MultiPlan multi;   // its windows of several steps per launch, the first being first_window
+    int first_window = 0;
 };
 
 struct StepArgs {
@@ -147,19 +159,15 @@ struct DoublePlan {
     uint32_t strips = 0, segments = 0;
     int rows = 0;
 };
-// Several steps of a small 2D lattice per launch (launch_multi): windows of
-// wx x wy cells, nx and ny of them along the axes, the steps a launch can make
-// at most (odd), and where each cell of a window pulls from.
-struct MultiPlan {
-    int nx = 0, ny = 0, wx = 0, wy = 0, halo = 0;
-    const int32_t *table = nullptr;   // a window's table of places, -1: plain
-    const uint16_t *place = nullptr;  // the tables
-};
-void plan_multi(int bytes, const KParams &kp, MultiPlan &m);
+// one window and step count for all the lattices, their plans without tables
+void plan_multi(int bytes, const std::vector<const KParams *> &lattices, std::vector<MultiPlan> &plans);
 hipError_t launch_multi_from(const StepArgs &a, int32_t *from, int64_t nslots, const int32_t *dslot,
                              const int32_t *sslot, int64_t nfill, hipStream_t s);
 hipError_t launch_multi_plan(const StepArgs &a, const int32_t *from, const MultiPlan &m, int32_t *mark, uint16_t *place,
                              uint32_t *bad, hipStream_t s);
+hipError_t launch_batch_multi(int prec, const MultiPlan &m, const void *src, void *dst, const uint8_t *geo,
+                              const BatchCase *cases, const uint32_t *window_case, uint32_t nwindows, int steps,
+                              bool copies, hipStream_t s);
 // copies: also the boundary copies of the last step
 hipError_t launch_multi(int prec, const StepArgs &a, const MultiPlan &m, int steps, bool copies, hipStream_t s);
 void plan_double(int dim, int bytes, const KParams &kp, DoublePlan &d);

@@ -1229,11 +1229,12 @@ __device__ __forceinline__ WinAxis win_axis(int i, int m, int n, int halo, bool 
     return {left ? 0 : right ? n - W : i * out, left ? 0 : i * out + halo, right ? n : (i + 1) * out + halo};
 }
 
-// cell of a thread of a window; false outside the lattice
+// cell of a thread of window w; false outside the lattice
 template <int WX, int WY>
-__device__ __forceinline__ bool win_cell(const KParams &kp, const MultiPlan &m, WinAxis &ax, WinAxis &ay, int &x, int &y)
+__device__ __forceinline__ bool win_cell(const KParams &kp, const MultiPlan &m, int w, WinAxis &ax, WinAxis &ay, int &x,
+                                         int &y)
 {
-    const int i = int(blockIdx.x) % m.nx, j = int(blockIdx.x) / m.nx, n = kp.nx + 1;
+    const int i = w % m.nx, j = w / m.nx, n = kp.nx + 1;
     ax = win_axis<WX>(i, m.nx, n, m.halo, true);
     ay = win_axis<WY>(j, m.ny, kp.ny + 1, m.halo, false);
     x = ax.first + int(threadIdx.x) % WX;
@@ -1279,7 +1280,7 @@ __global__ __launch_bounds__(WX *WY) void k_multi_plan(const int32_t *__restrict
     const uint32_t th = threadIdx.x;
     WinAxis ax, ay;
     int x, y;
-    const bool in = win_cell<WX, WY>(kp, m, ax, ay, x, y);
+    const bool in = win_cell<WX, WY>(kp, m, int(blockIdx.x), ax, ay, x, y);
     const uint32_t c = in ? uint32_t(kp.o0 + x + kp.Px * y) : 0u;
     const bool fluid = in && (geo[c] & G_FLUID);
     bool special = !fluid || (geo[c] & G_PUSH) || x == 0 || x == kp.nx;
@@ -1321,20 +1322,21 @@ __global__ __launch_bounds__(WX *WY) void k_multi_plan(const int32_t *__restrict
     if (th == 0) mark[blockIdx.x] = any;
 }
 
+// `steps` steps of window w of a lattice
 template <class S, class C, int WX, int WY>
-__global__ __launch_bounds__(WX *WY) void k_multi2(const S *__restrict__ src, S *__restrict__ dst,
-                                                   const uint8_t *__restrict__ geo, KParams kp, PushTable pt,
-                                                   MultiPlan m, int steps, int copies)
+__device__ __forceinline__ void multi_window(const S *__restrict__ src, S *__restrict__ dst,
+                                             const uint8_t *__restrict__ geo, const KParams &kp, const PushTable &pt,
+                                             const MultiPlan &m, int w, int steps, int copies)
 {
     using L = Lat<2>;
     using U = BitsOf<S>;
     constexpr uint32_t N = WX * WY;
     __shared__ U cells[2][9 * N + 8];
     const uint32_t th = threadIdx.x;
-    const int32_t table = m.table[blockIdx.x];
+    const int32_t table = m.table[w];
     WinAxis ax, ay;
     int x, y;
-    const bool in = win_cell<WX, WY>(kp, m, ax, ay, x, y);
+    const bool in = win_cell<WX, WY>(kp, m, w, ax, ay, x, y);
     const uint32_t c = uint32_t(kp.o0 + min(x, kp.nx) + kp.Px * min(y, kp.ny));
 #pragma unroll
     for (int q = 0; q < L::Q; ++q)
@@ -1394,6 +1396,32 @@ __global__ __launch_bounds__(WX *WY) void k_multi2(const S *__restrict__ src, S 
         for (int32_t e = pt.beg[c], ee = pt.beg[c + 1]; e < ee; ++e)
             dst[uint32_t(to[e])] = __builtin_bit_cast(S, pick(out, pt.q[e]));
     }
+}
+
+template <class S, class C, int WX, int WY>
+__global__ __launch_bounds__(WX *WY) void k_multi2(const S *__restrict__ src, S *__restrict__ dst,
+                                                   const uint8_t *__restrict__ geo, KParams kp, PushTable pt,
+                                                   MultiPlan m, int steps, int copies)
+{
+    multi_window<S, C, WX, WY>(src, dst, geo, kp, pt, m, int(blockIdx.x), steps, copies);
+}
+
+// The same for every lattice of an ensemble: window_case gives a block its
+// case.  96 uneven cylinders (11.3 M nodes), us a step, single steps and now:
+// FP64 293 and 205, FP32 143 and 87, FP16 92 and 79; 3 of them 19.7 and 13.2,
+// 11.7 and 5.8, 8.1 and 5.4.
+template <class S, class C, int WX, int WY>
+__global__ __launch_bounds__(WX *WY) void k_batch_multi(const S *__restrict__ src, S *__restrict__ dst,
+                                                        const uint8_t *__restrict__ geo,
+                                                        const BatchCase *__restrict__ cases,
+                                                        const uint32_t *__restrict__ window_case, int steps, int copies)
+{
+    const BatchCase &bc = cases[window_case[blockIdx.x]];
+    const KParams kp = bc.kp;  // copies: kept in scalar registers across the stores
+    const PushTable pt = bc.pt;
+    const MultiPlan m = bc.multi;
+    multi_window<S, C, WX, WY>(src + bc.pop_base, dst + bc.pop_base, geo + bc.geo_base, kp, pt, m,
+                               int(blockIdx.x) - bc.first_window, steps, copies);
 }
 
 // ---------------------------------------------------------------------------
@@ -1850,32 +1878,38 @@ static hipError_t dispatch_window(const MultiPlan &m, F &&f)
 // memory time and the arithmetic overlap unless a block fills the CU's LDS.
 // Within 15 % of the times measured from 49 x 25 to 2001 x 501 in FP64, FP32
 // and FP16, and the best or next best of the seven windows in each.
-void plan_multi(int bytes, const KParams &kp, MultiPlan &m)
+void plan_multi(int bytes, const std::vector<const KParams *> &lattices, std::vector<MultiPlan> &plans)
 {
     struct Window {
         int wx, wy, halo;
     };
     constexpr Window windows[] = {{32, 32, 5}, {32, 32, 7}, {32, 32, 9}, {32, 16, 3}, {32, 16, 5}, {16, 16, 5}};
-    const int nx = kp.nx + 1, ny = kp.ny + 1;
     double best = 1e300;
     for (const Window &w : windows) {
         const int ox = w.wx - 2 * w.halo, oy = w.wy - 2 * w.halo, cells = w.wx * w.wy;
-        const int mx = nx <= w.wx ? 1 : (nx + ox - 1) / ox;
-        const int my = ny <= w.wy ? 1 : 2 + std::max(0, (ny - 2 * (w.wy - w.halo) + oy - 1) / oy);
-        const double blocks = double(mx) * my, slots = 9.0 * bytes;
+        std::vector<MultiPlan> plan;
+        double blocks = 0.0, nodes = 0.0;
+        for (const KParams *kp : lattices) {
+            const int nx = kp->nx + 1, ny = kp->ny + 1;
+            MultiPlan m;
+            m.wx = w.wx;
+            m.wy = w.wy;
+            m.halo = w.halo;
+            m.nx = nx <= w.wx ? 1 : (nx + ox - 1) / ox;
+            m.ny = ny <= w.wy ? 1 : 2 + std::max(0, (ny - 2 * (w.wy - w.halo) + oy - 1) / oy);
+            plan.push_back(m);
+            blocks += double(m.nx) * m.ny;
+            nodes += double(nx) * ny;
+        }
         const int fit = std::min(2048 / cells, int(160 * 1024 / (18.0 * cells * bytes)));  // blocks of a CU
         const double waves = std::ceil(blocks / 256.0) * cells / 256.0;
         const double arith = 0.3 + (bytes == 8 ? 0.27 : 0.1) * waves;
-        const double memory = (3.1 + (blocks * cells + double(nx) * ny) * slots / 5e6) / w.halo;
+        const double memory = (3.1 + (blocks * cells + nodes) * 9.0 * bytes / 5e6) / w.halo;
         const bool overlap = fit > 1 && blocks > 512.0 * fit;
         const double t = overlap ? std::max(arith, memory) + 0.3 * std::min(arith, memory) : arith + memory;
         if (t < best) {
             best = t;
-            m.wx = w.wx;
-            m.wy = w.wy;
-            m.halo = w.halo;
-            m.nx = mx;
-            m.ny = my;
+            plans = plan;
         }
     }
 }
@@ -1911,6 +1945,25 @@ hipError_t launch_multi(int prec, const StepArgs &a, const MultiPlan &m, int ste
                                (const S *)a.src, (S *)a.dst, a.geo, a.kp, a.push, m, steps, int(copies));
             return hipGetLastError();
         });
+    });
+}
+
+hipError_t launch_batch_multi(int prec, const MultiPlan &m, const void *src, void *dst, const uint8_t *geo,
+                              const BatchCase *cases, const uint32_t *window_case, uint32_t nwindows, int steps,
+                              bool copies, hipStream_t s)
+{
+    return dispatch_prec(prec, [&](auto *sp, auto *cp) {
+        using S = std::remove_pointer_t<decltype(sp)>;
+        using C = std::remove_pointer_t<decltype(cp)>;
+        if constexpr (std::is_same<S, bf16_t>::value || std::is_same<S, bf16sr_t>::value)
+            return hipErrorInvalidValue;  // (no ensembles in these forms)
+        else
+            return dispatch_window(m, [&](auto wx, auto wy) {
+                constexpr int WX = decltype(wx)::value, WY = decltype(wy)::value;
+                hipLaunchKernelGGL((k_batch_multi<S, C, WX, WY>), dim3(nwindows), dim3(WX * WY), 0, s, (const S *)src,
+                                   (S *)dst, geo, cases, window_case, steps, int(copies));
+                return hipGetLastError();
+            });
     });
 }
 

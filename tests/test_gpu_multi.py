@@ -106,3 +106,27 @@ def test_multi_steps_match_oracle(name):
     assert_state_equal(lat, o)
     lat.close()
     o.close()
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32", "f16"])
+def test_ensemble_multi_steps_equal_single_steps(monkeypatch, prec):
+    """Uneven cases, one within a window and one with a turned ellipse."""
+    from imexlb.ensemble import Batch, cylinder_cases
+    out = []
+    for multi in ("1", "0"):
+        monkeypatch.setenv("IMEXLB_MULTI", multi)
+        b = Batch([_deck(n) for n in ((28, 24), (61, 20), (150, 60), (90, 33))] + cylinder_cases(3, seed=2),
+                  precision=PRECS[prec])
+        b.init(np.linspace(0.0, 1.0, 100))
+        res = []
+        for n in (1, 4, 5, 12, 131):
+            b.advance(n)
+            res.append([b.forces(), b.monitor()[0]] + [v for i in range(b.ncase) for v in b.download_fields(i)])
+        b.init(np.linspace(1.0, 0.0, 100))
+        b.advance(60)
+        res.append([v for i in range(b.ncase) for v in b.download_fields(i)])
+        out.append(res)
+        del b
+    for r, s in zip(*out):
+        for x, y in zip(r, s):
+            assert np.array_equal(x, y)
