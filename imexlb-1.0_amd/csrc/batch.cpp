@@ -74,6 +74,8 @@ struct imexlb_batch {
     static constexpr int kMulti = 8;  // launches per graph: even, it ends in the buffer it began in
     hipGraphExec_t multi_graph[2] = {};
 
+    Staging staging;
+
     int cur = 1, lazy = -1;
     bool initialized = false, have_pu = false;
 
@@ -99,6 +101,7 @@ struct imexlb_batch {
             (void)hipStreamSynchronize(stream);
         }
         drop_graphs();
+        staging.release();
         void *ptrs[] = {fb[0],     fb[1],      f,        p,         ux,        uy,            rv,
                         geo,       fill_dst,   fill_src, link_out,  link_back, link_q,        force_partial,
                         force_out, mon,        d_cases,  queue,     tile_case, tile_first,
@@ -799,9 +802,15 @@ int imexlb_batch_download_fields(imexlb_batch *b, int i, double *p, double *u)
     if (rc) return rc;
     const imexlb_ctx *c = b->host[size_t(i)];
     const size_t n = size_t(c->plane);
-    std::vector<double> h(n);
     const int64_t N = c->kp.N;
     double *srcs[3] = {b->p, b->ux, b->uy};
+    const int64_t cb = b->cases[size_t(i)].geo_base;
+    hipError_t e;
+    if (download_interior(b->staging, b->device, b->stream, 2, c->kp,
+                          {{b->p + cb, p}, {b->ux + cb, u}, {b->uy + cb, u + N}}, e))
+        return e == hipSuccess ? IMEXLB_OK
+                               : fail(IMEXLB_E_HIP, std::string("batch download: ") + hipGetErrorString(e));
+    std::vector<double> h(n);
     for (int k = 0; k < 3; ++k) {
         HIP_TRY(hipMemcpyAsync(h.data(), srcs[k] + b->cases[size_t(i)].geo_base, n * sizeof(double),
                                hipMemcpyDeviceToHost, b->stream));

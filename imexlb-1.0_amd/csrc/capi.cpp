@@ -1219,9 +1219,19 @@ int imexlb_download_fields(imexlb_ctx *c, double *p, double *u, int layout)
     if (rc) return rc;
     const int dim = c->dim;
     const size_t bytes = size_t(c->plane) * sizeof(double);
-    std::vector<double> h(size_t(c->plane));
     const int64_t N = c->kp.N;
     double *srcs[4] = {c->p, c->ux, c->uy, c->uz};
+    if (layout == IMEXLB_LAYOUT_INTERIOR) {
+        std::vector<FieldCopy> fields;
+        for (int k = 0; k <= dim; ++k)
+            if (k == 0 ? p != nullptr : u != nullptr) fields.push_back({srcs[k], k == 0 ? p : u + int64_t(k - 1) * N});
+        hipError_t e;
+        if (fields.empty()) return IMEXLB_OK;
+        if (download_interior(c->staging, c->device, c->stream, dim, c->kp, fields, e))
+            return e == hipSuccess ? IMEXLB_OK
+                                   : fail(IMEXLB_E_HIP, std::string("field download: ") + hipGetErrorString(e));
+    }
+    std::vector<double> h(size_t(c->plane));
     for (int k = 0; k <= dim; ++k) {
         double *out = k == 0 ? p : u;
         if (!out) continue;

@@ -43,6 +43,26 @@ struct TimedLaunch {
 };
 
 
+// Pinned buffers of the downloads, one per thread, kept by the object that
+// downloads (its calls are not concurrent) and freed with it: at most 16 MiB.
+struct Staging {
+    static constexpr int kWorkers = 8;
+    double *host[kWorkers] = {};
+    hipEvent_t done[kWorkers] = {};
+    int64_t values = 0;  // of each buffer
+    void release();
+};
+
+struct FieldCopy {
+    const double *from;  // padded device array
+    double *to;          // the caller's dense interior array
+};
+
+// The interior of padded device arrays to dense host arrays, after the work on
+// the stream; false if there is no memory for the buffers (nothing was copied).
+bool download_interior(Staging &s, int device, hipStream_t stream, int dim, const KParams &kp,
+                       const std::vector<FieldCopy> &fields, hipError_t &err);
+
 }  // namespace imexlb
 
 using namespace imexlb;
@@ -83,6 +103,7 @@ struct imexlb_ctx {
     int8_t *link_q = nullptr;
     int64_t nlink = 0;
     double *force_partial = nullptr, *force_out = nullptr;
+    Staging staging;
     double *mass_partial = nullptr;  // MASS_BLOCKS partial sums, then the total
     size_t dev_bytes = 0;
     // test hook: IMEXLB_FAIL_ALLOC=N (read at creation) makes this
@@ -311,6 +332,7 @@ struct imexlb_ctx {
             if (q) (void)hipFree(q);
         drop_double();
         drop_multi();
+        staging.release();
         fb[0] = fb[1] = f = nullptr;
         push_beg = nullptr;
         push_q = nullptr;

@@ -196,6 +196,9 @@ hipError_t launch_body_mask(const StepArgs &a, float *out, int H, int W, hipStre
 // Boundary fill; the slot tables hold int32 (idx32) or int64 entries.
 hipError_t launch_fill(int prec, void *buf, const void *prev, const void *dslot, const void *sslot, bool idx32,
                        int64_t n, hipStream_t s);
+// out[i] = field value of interior node first + i, i < count
+hipError_t launch_pack(int dim, const KParams &kp, const double *field, int64_t first, int64_t count, double *out,
+                       hipStream_t s);
 hipError_t launch_monitor(int dim, const StepArgs &a, uint32_t skip, unsigned long long *out, hipStream_t s);
 // Batched ensemble (D2Q9; prec 0, 1 or 2).  block in {64,128,256,512},
 // cpt in {1,2,4}; persist launches `grid` blocks that take tiles from

@@ -1601,6 +1601,18 @@ __global__ __launch_bounds__(256) void k_body_mask(float *__restrict__ out, cons
     if (x < W && y < H) out[int64_t(y) * W + x] = (geo[c] & G_FLUID) ? 0.0f : 1.0f;
 }
 
+// Values of `count` interior nodes from node `first` on (scan order), dense:
+// `out` may be pinned host memory, written over the bus in whole lines.
+template <int D>
+__global__ __launch_bounds__(256) void k_pack(const double *__restrict__ field, KParams kp, uint32_t first,
+                                              uint32_t count, double *__restrict__ out)
+{
+    int x, y, z;
+    uint32_t c;
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i < count && decode<D>(kp, first + i, x, y, z, c)) out[i] = field[c];
+}
+
 // Boundary fill of this step's buffer: dst slot <- this step's fluid slot
 // (s >= 0), 0 (s == -1), or a body-cell slot of the previous step's buffer
 // (s <= -2, slot -s-2).  Sources are never destinations, so the order of
@@ -2103,6 +2115,18 @@ hipError_t launch_forces(int dim, int prec, const void *buf, const int64_t *out_
     });
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_forces_final, dim3(1), dim3(64), 0, s, partial, int64_t(nb), out);
+    return hipGetLastError();
+}
+
+hipError_t launch_pack(int dim, const KParams &kp, const double *field, int64_t first, int64_t count, double *out,
+                       hipStream_t s)
+{
+    if (dim == 2)
+        hipLaunchKernelGGL((k_pack<2>), dim3(nblocks(uint64_t(count))), dim3(256), 0, s, field, kp, uint32_t(first),
+                           uint32_t(count), out);
+    else
+        hipLaunchKernelGGL((k_pack<3>), dim3(nblocks(uint64_t(count))), dim3(256), 0, s, field, kp, uint32_t(first),
+                           uint32_t(count), out);
     return hipGetLastError();
 }
 
