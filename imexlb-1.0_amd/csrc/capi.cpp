@@ -303,12 +303,12 @@ int imexlb_create(imexlb_ctx **out, int dim, int nx, int ny, int nz, int device,
     // Several steps per launch pay in FP32 at every size, in 16-bit storage up
     // to 8 Mi cells and in FP64 up to 2.5 Mi; above, the cells that neighbouring
     // windows both compute cost more than a second pass (against two steps per
-    // pass, us a step: FP32 8192x2048 107 and 129, FP16 5001x1251 35.2 and
-    // 38.1, 8192x2048 95 and 83, FP64 3000x750 39.8 and 41.5, 8192x2048 285 and
-    // 244); with stochastic rounding, more arithmetic per cell, up to 4 Mi
-    // (5001x1251 42.9 and 40.9).
+    // pass, us a step: FP32 8192x2048 97 and 129, FP16 5001x1251 32.1 and 38.1,
+    // 8192x2048 83.6 and 82.8, FP64 3000x750 39.8 and 41.5, 8192x2048 285 and
+    // 244); with stochastic rounding, more arithmetic per cell, up to 0.75 Mi
+    // (1000x250 3.60 and, single steps, 4.45; 2000x500 9.73 and 9.24).
     c->multi_cells = c->ssz == 4                     ? INT64_MAX
-                     : precision == IMEXLB_BF16SR_F32 ? int64_t(4) << 20
+                     : precision == IMEXLB_BF16SR_F32 ? int64_t(3) << 18
                      : c->ssz == 2                    ? int64_t(8) << 20
                                                       : int64_t(5) << 19;
     if (std::getenv("IMEXLB_SMALL_CELLS")) c->multi_cells = c->small_cells;

@@ -1206,11 +1206,11 @@ __global__ __launch_bounds__(256) void k_zone_list(const uint8_t *__restrict__ m
 //
 // Bound by the arithmetic, a third to half of it on cells that a neighbouring
 // window writes, and for small lattices by the 3 us of a launch per 5 to 9
-// steps.  us a step, single steps and now: FP64 49 x 25 3.36 and 1.26, 401 x
-// 101 3.67 and 2.36, 2001 x 501 22.5 and 17.1; FP32 401 x 101 3.06 and 1.45,
-// 2801 x 701 22.2 and 12.4; FP16 401 x 101 3.08 and 1.29, 5002 x 1252 (two
-// steps per pass) 38.1 and 35.2.  Tables for all windows cost FP32 2801 x 701
-// 14.3.
+// steps.  us a step, before (single steps; 5002 x 1252 and 8193 x 2049 two per
+// pass) and now: FP64 49 x 25 3.36 and 1.19, 401 x 101 3.67 and 2.35, 2001 x
+// 501 22.5 and 16.6; FP32 401 x 101 3.06 and 1.29, 2801 x 701 22.2 and 12.8,
+// 8193 x 2049 129 and 97; FP16 401 x 101 3.08 and 1.25, 5002 x 1252 38.1 and
+// 32.1.
 
 // Windows along an axis of n nodes: one where they all fit (m == 1), else m
 // that write W - 2 halo nodes each.  In x they go round the lattice like a
@@ -1229,16 +1229,27 @@ __device__ __forceinline__ WinAxis win_axis(int i, int m, int n, int halo, bool 
     return {left ? 0 : right ? n - W : i * out, left ? 0 : i * out + halo, right ? n : (i + 1) * out + halo};
 }
 
-// cell of a thread of window w; false outside the lattice
+// threads of a window's block, one cell each, or several cells N threads apart
 template <int WX, int WY>
-__device__ __forceinline__ bool win_cell(const KParams &kp, const MultiPlan &m, int w, WinAxis &ax, WinAxis &ay, int &x,
-                                         int &y)
+constexpr int win_threads()
 {
-    const int i = w % m.nx, j = w / m.nx, n = kp.nx + 1;
-    ax = win_axis<WX>(i, m.nx, n, m.halo, true);
-    ay = win_axis<WY>(j, m.ny, kp.ny + 1, m.halo, false);
-    x = ax.first + int(threadIdx.x) % WX;
-    y = ay.first + int(threadIdx.x) / WX;
+    return WX * WY < 1024 ? WX * WY : 1024;
+}
+
+template <int WX, int WY>
+__device__ __forceinline__ void win_place(const KParams &kp, const MultiPlan &m, int w, WinAxis &ax, WinAxis &ay)
+{
+    ax = win_axis<WX>(w % m.nx, m.nx, kp.nx + 1, m.halo, true);
+    ay = win_axis<WY>(w / m.nx, m.ny, kp.ny + 1, m.halo, false);
+}
+// node of a window's cell l; false outside the lattice
+template <int WX>
+__device__ __forceinline__ bool win_cell(const KParams &kp, const MultiPlan &m, const WinAxis &ax, const WinAxis &ay,
+                                         uint32_t l, int &x, int &y)
+{
+    const int n = kp.nx + 1;
+    x = ax.first + int(l) % WX;
+    y = ay.first + int(l) / WX;
     if (m.nx > 1) x = x < 0 ? x + n : x >= n ? x - n : x;
     return x <= kp.nx && y <= kp.ny;
 }
@@ -1269,57 +1280,71 @@ __global__ __launch_bounds__(256) void k_multi_copies(int32_t *__restrict__ from
 // marks the windows that need a table, and sets *bad where a cell that is
 // written would not be right for `halo` steps; second pass: writes them.
 template <int WX, int WY>
-__global__ __launch_bounds__(WX *WY) void k_multi_plan(const int32_t *__restrict__ from,
-                                                       const uint8_t *__restrict__ geo, KParams kp, MultiPlan m,
-                                                       int32_t *__restrict__ mark, uint16_t *__restrict__ place,
-                                                       uint32_t *__restrict__ bad)
+__global__ __launch_bounds__((win_threads<WX, WY>())) void k_multi_plan(const int32_t *__restrict__ from,
+                                                                        const uint8_t *__restrict__ geo, KParams kp,
+                                                                        MultiPlan m, int32_t *__restrict__ mark,
+                                                                        uint16_t *__restrict__ place,
+                                                                        uint32_t *__restrict__ bad)
 {
     using L = Lat<2>;
-    constexpr uint32_t N = WX * WY;
+    constexpr uint32_t N = WX * WY, T = win_threads<WX, WY>(), P = N / T;
     __shared__ int right[2][N];  // steps for which a cell is right
-    const uint32_t th = threadIdx.x;
     WinAxis ax, ay;
-    int x, y;
-    const bool in = win_cell<WX, WY>(kp, m, int(blockIdx.x), ax, ay, x, y);
-    const uint32_t c = in ? uint32_t(kp.o0 + x + kp.Px * y) : 0u;
-    const bool fluid = in && (geo[c] & G_FLUID);
-    bool special = !fluid || (geo[c] & G_PUSH) || x == 0 || x == kp.nx;
-    int source[L::Q];  // cell of the window a pull reads; -1 outside; -2 none
-    for (int q = 0; q < L::Q; ++q) {
-        uint32_t at = uint32_t(q) * N + th;
-        source[q] = -2;
-        if (fluid) {
-            const uint32_t pulled = cslot<L::Q>(kp, uint32_t(q), c - shift32<2>(kp, q));
-            const int32_t s = from[pulled];
-            special |= s != int32_t(pulled);
-            if (s < 0) {
-                at = 9u * N;  // the place that holds 0
-            } else {          // slot -> cell and direction -> place in the window
-                const uint32_t sc = uint32_t(s) / (9u * 64u) * 64u + uint32_t(s) % 64u, sq = uint32_t(s) / 64u % 9u;
-                int sx = int(sc % uint32_t(kp.Px)) - 1 - ax.first;
-                const int sy = int(sc / uint32_t(kp.Px)) - 1 - ay.first;
-                if (m.nx > 1) sx = sx < 0 ? sx + kp.nx + 1 : sx > kp.nx ? sx - kp.nx - 1 : sx;
-                source[q] = -1;
-                if (sx >= 0 && sx < WX && sy >= 0 && sy < WY) {
-                    source[q] = sy * WX + sx;
-                    at = sq * N + uint32_t(source[q]);
+    win_place<WX, WY>(kp, m, int(blockIdx.x), ax, ay);
+    int source[P][L::Q];  // cell of the window a pull reads; -1 outside; -2 none
+    bool special = false;
+    for (uint32_t p = 0; p < P; ++p) {
+        const uint32_t l = threadIdx.x + p * T;
+        int x, y;
+        const bool in = win_cell<WX>(kp, m, ax, ay, l, x, y);
+        const uint32_t c = in ? uint32_t(kp.o0 + x + kp.Px * y) : 0u;
+        const bool fluid = in && (geo[c] & G_FLUID);
+        special |= !fluid || (geo[c] & G_PUSH) || x == 0 || x == kp.nx;
+        for (int q = 0; q < L::Q; ++q) {
+            uint32_t at = uint32_t(q) * N + l;
+            source[p][q] = -2;
+            if (fluid) {
+                const uint32_t pulled = cslot<L::Q>(kp, uint32_t(q), c - shift32<2>(kp, q));
+                const int32_t s = from[pulled];
+                special |= s != int32_t(pulled);
+                if (s < 0) {
+                    at = 9u * N;  // the place that holds 0
+                } else {          // slot -> cell and direction -> place in the window
+                    const uint32_t sc = uint32_t(s) / (9u * 64u) * 64u + uint32_t(s) % 64u, sq = uint32_t(s) / 64u % 9u;
+                    int sx = int(sc % uint32_t(kp.Px)) - 1 - ax.first;
+                    const int sy = int(sc / uint32_t(kp.Px)) - 1 - ay.first;
+                    if (m.nx > 1) sx = sx < 0 ? sx + kp.nx + 1 : sx > kp.nx ? sx - kp.nx - 1 : sx;
+                    source[p][q] = -1;
+                    if (sx >= 0 && sx < WX && sy >= 0 && sy < WY) {
+                        source[p][q] = sy * WX + sx;
+                        at = sq * N + uint32_t(source[p][q]);
+                    }
                 }
             }
+            if (place && mark[blockIdx.x] >= 0) place[(uint32_t(mark[blockIdx.x]) * 9u + uint32_t(q)) * N + l] = uint16_t(at);
         }
-        if (place && mark[blockIdx.x] >= 0) place[(uint32_t(mark[blockIdx.x]) * 9u + uint32_t(q)) * N + th] = uint16_t(at);
+        right[0][l] = fluid ? m.halo : 0;
     }
     if (place) return;
-    int mine = fluid ? m.halo : 0;
-    right[0][th] = mine;
     for (int k = 0; k < m.halo; ++k) {
         __syncthreads();
-        for (int q = 0; q < L::Q; ++q)
-            if (source[q] != -2) mine = min(mine, source[q] < 0 ? 0 : right[k & 1][source[q]] + 1);
-        right[(k & 1) ^ 1][th] = mine;
+        for (uint32_t p = 0; p < P; ++p) {
+            const uint32_t l = threadIdx.x + p * T;
+            int mine = right[k & 1][l];
+            for (int q = 0; q < L::Q; ++q)
+                if (source[p][q] != -2) mine = min(mine, source[p][q] < 0 ? 0 : right[k & 1][source[p][q]] + 1);
+            right[(k & 1) ^ 1][l] = mine;
+        }
     }
-    if (fluid && mine < m.halo && win_writes(int(th) % WX, ax) && win_writes(int(th) / WX, ay)) atomicOr(bad, 1u);
+    for (uint32_t p = 0; p < P; ++p) {
+        const uint32_t l = threadIdx.x + p * T;
+        int x, y;
+        if (win_cell<WX>(kp, m, ax, ay, l, x, y) && (geo[uint32_t(kp.o0 + x + kp.Px * y)] & G_FLUID) &&
+            right[m.halo & 1][l] < m.halo && win_writes(int(l) % WX, ax) && win_writes(int(l) / WX, ay))
+            atomicOr(bad, 1u);
+    }
     const int any = __syncthreads_or(special);
-    if (th == 0) mark[blockIdx.x] = any;
+    if (threadIdx.x == 0) mark[blockIdx.x] = any;
 }
 
 // `steps` steps of window w of a lattice
@@ -1330,32 +1355,45 @@ __device__ __forceinline__ void multi_window(const S *__restrict__ src, S *__res
 {
     using L = Lat<2>;
     using U = BitsOf<S>;
-    constexpr uint32_t N = WX * WY;
+    constexpr uint32_t N = WX * WY, T = win_threads<WX, WY>(), P = N / T;
     __shared__ U cells[2][9 * N + 8];
     const uint32_t th = threadIdx.x;
     const int32_t table = m.table[w];
     WinAxis ax, ay;
-    int x, y;
-    const bool in = win_cell<WX, WY>(kp, m, w, ax, ay, x, y);
-    const uint32_t c = uint32_t(kp.o0 + min(x, kp.nx) + kp.Px * min(y, kp.ny));
+    win_place<WX, WY>(kp, m, w, ax, ay);
+    int x[P], y[P];
+    uint32_t c[P], g[P];
 #pragma unroll
-    for (int q = 0; q < L::Q; ++q)
-        cells[0][uint32_t(q) * N + th] = __builtin_bit_cast(U, src[cslot<L::Q>(kp, uint32_t(q), c)]);
-    uint8_t g = G_FLUID;
-    U out[L::Q] = {};
-    const auto node = [&](const C(&f)[L::Q], int xn) {
-        C p, ux, uy, uz;
-        moments<2, C>(f, kp, xn, y, 0, p, ux, uy, uz);
-        const uint32_t srw = sr_word<S>(p, sr_cell<S>(kp, c, y, 0));
-        collide<2, C>(f, p, ux, uy, uz, kp, [&](int q, C v) {
+    for (uint32_t p = 0; p < P; ++p) {
+        const bool in = win_cell<WX>(kp, m, ax, ay, th + p * T, x[p], y[p]);
+        c[p] = uint32_t(kp.o0 + min(x[p], kp.nx) + kp.Px * min(y[p], kp.ny));
+        g[p] = in ? G_FLUID : 0;
+#pragma unroll
+        for (int q = 0; q < L::Q; ++q)
+            cells[0][uint32_t(q) * N + th + p * T] = __builtin_bit_cast(U, src[cslot<L::Q>(kp, uint32_t(q), c[p])]);
+    }
+    // one step of a cell: to LDS, or after the last step to memory
+    const auto node = [&](const C(&f)[L::Q], int k, uint32_t p, int xn) {
+        C pr, ux, uy, uz;
+        moments<2, C>(f, kp, xn, y[p], 0, pr, ux, uy, uz);
+        const uint32_t srw = sr_word<S>(pr, sr_cell<S>(kp, c[p], y[p], 0));
+        U out[L::Q];
+        collide<2, C>(f, pr, ux, uy, uz, kp, [&](int q, C v) {
             out[q] = __builtin_bit_cast(U, Store<S>::template st<C>(v, srw + uint32_t(q) * kGolden));
         });
-    };
-    const auto keep = [&](int k) {
+        const uint32_t l = th + p * T;
         if (k + 1 < steps) {
-            U *const b = cells[(k & 1) ^ 1] + th;
 #pragma unroll
-            for (int q = 0; q < L::Q; ++q) b[uint32_t(q) * N] = out[q];
+            for (int q = 0; q < L::Q; ++q) cells[(k & 1) ^ 1][uint32_t(q) * N + l] = out[q];
+            return;
+        }
+        if (!win_writes(int(l) % WX, ax) || !win_writes(int(l) / WX, ay)) return;
+#pragma unroll
+        for (int q = 0; q < L::Q; ++q) dst[cslot<L::Q>(kp, uint32_t(q), c[p])] = __builtin_bit_cast(S, out[q]);
+        if (copies && (g[p] & G_PUSH)) {
+            const int32_t *const to = static_cast<const int32_t *>(pt.dst);
+            for (int32_t e = pt.beg[c[p]], ee = pt.beg[c[p] + 1]; e < ee; ++e)
+                dst[uint32_t(to[e])] = __builtin_bit_cast(S, pick(out, pt.q[e]));
         }
     };
     if (table < 0) {  // the same for the block
@@ -1363,43 +1401,41 @@ __device__ __forceinline__ void multi_window(const S *__restrict__ src, S *__res
         // direction 0 reads ahead, 8 back)
         for (int k = 0; k < steps; ++k) {
             __syncthreads();
-            C f[L::Q];
 #pragma unroll
-            for (int q = 0; q < L::Q; ++q)
-                f[q] = Store<S>::ld(
-                    __builtin_bit_cast(S, cells[k & 1][uint32_t(q) * N + th - uint32_t(L::ey(q) * WX + L::ex(q))]));
-            node(f, -1);
-            keep(k);
+            for (uint32_t p = 0; p < P; ++p) {
+                C f[L::Q];
+#pragma unroll
+                for (int q = 0; q < L::Q; ++q)
+                    f[q] = Store<S>::ld(__builtin_bit_cast(
+                        S, cells[k & 1][uint32_t(q) * N + th + p * T - uint32_t(L::ey(q) * WX + L::ex(q))]));
+                node(f, k, p, -1);
+            }
         }
     } else {
-        uint32_t at[L::Q];
+        uint32_t at[P][L::Q];
 #pragma unroll
-        for (int q = 0; q < L::Q; ++q) at[q] = m.place[(uint32_t(table) * 9u + uint32_t(q)) * N + th];
-        g = in ? geo[c] : uint8_t(0);
+        for (uint32_t p = 0; p < P; ++p) {
+#pragma unroll
+            for (int q = 0; q < L::Q; ++q) at[p][q] = m.place[(uint32_t(table) * 9u + uint32_t(q)) * N + th + p * T];
+            g[p] = g[p] ? geo[c[p]] : 0u;
+        }
         if (th < 2) cells[th][9 * N] = U(0);
         for (int k = 0; k < steps; ++k) {
             __syncthreads();
-            if (g & G_FLUID) {
+#pragma unroll
+            for (uint32_t p = 0; p < P; ++p) {
+                if (!(g[p] & G_FLUID)) continue;
                 C f[L::Q];
 #pragma unroll
-                for (int q = 0; q < L::Q; ++q) f[q] = Store<S>::ld(__builtin_bit_cast(S, cells[k & 1][at[q]]));
-                node(f, x);
-                keep(k);
+                for (int q = 0; q < L::Q; ++q) f[q] = Store<S>::ld(__builtin_bit_cast(S, cells[k & 1][at[p][q]]));
+                node(f, k, p, x[p]);
             }
         }
-    }
-    if (!(g & G_FLUID) || !win_writes(int(th) % WX, ax) || !win_writes(int(th) / WX, ay)) return;
-#pragma unroll
-    for (int q = 0; q < L::Q; ++q) dst[cslot<L::Q>(kp, uint32_t(q), c)] = __builtin_bit_cast(S, out[q]);
-    if (copies && (g & G_PUSH)) {
-        const int32_t *const to = static_cast<const int32_t *>(pt.dst);
-        for (int32_t e = pt.beg[c], ee = pt.beg[c + 1]; e < ee; ++e)
-            dst[uint32_t(to[e])] = __builtin_bit_cast(S, pick(out, pt.q[e]));
     }
 }
 
 template <class S, class C, int WX, int WY>
-__global__ __launch_bounds__(WX *WY) void k_multi2(const S *__restrict__ src, S *__restrict__ dst,
+__global__ __launch_bounds__((win_threads<WX, WY>())) void k_multi2(const S *__restrict__ src, S *__restrict__ dst,
                                                    const uint8_t *__restrict__ geo, KParams kp, PushTable pt,
                                                    MultiPlan m, int steps, int copies)
 {
@@ -1408,10 +1444,10 @@ __global__ __launch_bounds__(WX *WY) void k_multi2(const S *__restrict__ src, S 
 
 // The same for every lattice of an ensemble: window_case gives a block its
 // case.  96 uneven cylinders (11.3 M nodes), us a step, single steps and now:
-// FP64 293 and 205, FP32 143 and 87, FP16 92 and 79; 3 of them 19.7 and 13.2,
-// 11.7 and 5.8, 8.1 and 5.4.
+// FP64 293 and 199, FP32 143 and 80, FP16 92 and 75; 3 of them 19.7 and 12.9,
+// 11.7 and 5.4, 8.1 and 5.4.
 template <class S, class C, int WX, int WY>
-__global__ __launch_bounds__(WX *WY) void k_batch_multi(const S *__restrict__ src, S *__restrict__ dst,
+__global__ __launch_bounds__((win_threads<WX, WY>())) void k_batch_multi(const S *__restrict__ src, S *__restrict__ dst,
                                                         const uint8_t *__restrict__ geo,
                                                         const BatchCase *__restrict__ cases,
                                                         const uint32_t *__restrict__ window_case, int steps, int copies)
@@ -1874,9 +1910,13 @@ hipError_t launch_double(int dim, int prec, const StepArgs &a, const DoublePlan 
     return launch_step_list(dim, prec, d.idx64, second, d.list[1], d.count[1], s);
 }
 
-template <class F>
+template <int BYTES, class F>
 static hipError_t dispatch_window(const MultiPlan &m, F &&f)
 {
+    if constexpr (BYTES == 2)
+        if (m.wy == 64) return f(std::integral_constant<int, 64>{}, std::integral_constant<int, 64>{});
+    if constexpr (BYTES <= 4)
+        if (m.wx == 64) return f(std::integral_constant<int, 64>{}, std::integral_constant<int, 32>{});
     if (m.wx == 16) return f(std::integral_constant<int, 16>{}, std::integral_constant<int, 16>{});
     if (m.wy == 16) return f(std::integral_constant<int, 32>{}, std::integral_constant<int, 16>{});
     return f(std::integral_constant<int, 32>{}, std::integral_constant<int, 32>{});
@@ -1884,20 +1924,26 @@ static hipError_t dispatch_window(const MultiPlan &m, F &&f)
 
 // Window and steps per launch by an estimate of the time per step (us): a
 // launch costs 3.1 and its loads and stores 1 per 5 MB; a step 0.3 and, for
-// each wave that a SIMD of the fullest CU has to run, 0.27 in FP64 or 0.1.
-// Small lattices leave CUs idle, so small windows serve them best; larger ones
-// pay for the cells computed twice; with several rounds of blocks on a CU the
-// memory time and the arithmetic overlap unless a block fills the CU's LDS.
-// Within 15 % of the times measured from 49 x 25 to 2001 x 501 in FP64, FP32
-// and FP16, and the best or next best of the seven windows in each.
+// each wave of cells that a SIMD of the fullest CU has to run, 0.27 in FP64,
+// 0.12 in FP32, 0.14 in 16-bit storage.  Small lattices leave CUs idle, so
+// small windows serve them best; larger ones pay for the cells computed twice
+// (53 % of a 32 x 32 window of five steps, 29 % of a 64 x 64 one, which only
+// fits LDS in 16-bit storage).  With several rounds of blocks on a CU the memory
+// time and the arithmetic overlap, less where a block fills the CU.  Mostly
+// within 20 % of the times measured from 49 x 25 to 8193 x 2049, and the chosen
+// window within 6 % of the best; us a step by window (32 x 32 / 64 x 32 / 64 x
+// 64): FP16 5002 x 1252 34.6 / 33.1 / 31.7, 401 x 101 1.28 / 2.00 / 3.34; FP32
+// 8193 x 2049 108 / 97, 901 x 226 2.69 / 2.43.
 void plan_multi(int bytes, const std::vector<const KParams *> &lattices, std::vector<MultiPlan> &plans)
 {
     struct Window {
         int wx, wy, halo;
     };
-    constexpr Window windows[] = {{32, 32, 5}, {32, 32, 7}, {32, 32, 9}, {32, 16, 3}, {32, 16, 5}, {16, 16, 5}};
+    constexpr Window windows[] = {{32, 32, 5}, {32, 32, 7}, {32, 32, 9}, {32, 16, 3}, {32, 16, 5},
+                                  {16, 16, 5}, {64, 32, 5}, {64, 32, 7}, {64, 64, 5}, {64, 64, 7}};
     double best = 1e300;
     for (const Window &w : windows) {
+        if (18 * w.wx * w.wy * bytes > 160 * 1024 - 1024) continue;  // LDS
         const int ox = w.wx - 2 * w.halo, oy = w.wy - 2 * w.halo, cells = w.wx * w.wy;
         std::vector<MultiPlan> plan;
         double blocks = 0.0, nodes = 0.0;
@@ -1913,12 +1959,12 @@ void plan_multi(int bytes, const std::vector<const KParams *> &lattices, std::ve
             blocks += double(m.nx) * m.ny;
             nodes += double(nx) * ny;
         }
-        const int fit = std::min(2048 / cells, int(160 * 1024 / (18.0 * cells * bytes)));  // blocks of a CU
+        const int fit = cells > 1024 ? 1 : std::min(2048 / cells, int(160 * 1024 / (18.0 * cells * bytes)));  // blocks of a CU
         const double waves = std::ceil(blocks / 256.0) * cells / 256.0;
-        const double arith = 0.3 + (bytes == 8 ? 0.27 : 0.1) * waves;
+        const double arith = 0.3 + (bytes == 8 ? 0.27 : bytes == 4 ? 0.12 : 0.14) * waves;
         const double memory = (3.1 + (blocks * cells + nodes) * 9.0 * bytes / 5e6) / w.halo;
-        const bool overlap = fit > 1 && blocks > 512.0 * fit;
-        const double t = overlap ? std::max(arith, memory) + 0.3 * std::min(arith, memory) : arith + memory;
+        const double apart = blocks <= 512.0 * fit ? 1.0 : fit > 1 ? 0.3 : bytes == 8 ? 1.0 : 0.5;
+        const double t = std::max(arith, memory) + apart * std::min(arith, memory);
         if (t < best) {
             best = t;
             plans = plan;
@@ -1938,9 +1984,9 @@ hipError_t launch_multi_from(const StepArgs &a, int32_t *from, int64_t nslots, c
 hipError_t launch_multi_plan(const StepArgs &a, const int32_t *from, const MultiPlan &m, int32_t *mark, uint16_t *place,
                              uint32_t *bad, hipStream_t s)
 {
-    return dispatch_window(m, [&](auto wx, auto wy) {
+    return dispatch_window<2>(m, [&](auto wx, auto wy) {
         constexpr int WX = decltype(wx)::value, WY = decltype(wy)::value;
-        hipLaunchKernelGGL((k_multi_plan<WX, WY>), dim3(unsigned(m.nx * m.ny)), dim3(WX * WY), 0, s, from, a.geo, a.kp,
+        hipLaunchKernelGGL((k_multi_plan<WX, WY>), dim3(unsigned(m.nx * m.ny)), dim3(win_threads<WX, WY>()), 0, s, from, a.geo, a.kp,
                            m, mark, place, bad);
         return hipGetLastError();
     });
@@ -1951,9 +1997,9 @@ hipError_t launch_multi(int prec, const StepArgs &a, const MultiPlan &m, int ste
     return dispatch_prec(prec, [&](auto *sp, auto *cp) {
         using S = std::remove_pointer_t<decltype(sp)>;
         using C = std::remove_pointer_t<decltype(cp)>;
-        return dispatch_window(m, [&](auto wx, auto wy) {
+        return dispatch_window<int(sizeof(S))>(m, [&](auto wx, auto wy) {
             constexpr int WX = decltype(wx)::value, WY = decltype(wy)::value;
-            hipLaunchKernelGGL((k_multi2<S, C, WX, WY>), dim3(unsigned(m.nx * m.ny)), dim3(WX * WY), 0, s,
+            hipLaunchKernelGGL((k_multi2<S, C, WX, WY>), dim3(unsigned(m.nx * m.ny)), dim3(win_threads<WX, WY>()), 0, s,
                                (const S *)a.src, (S *)a.dst, a.geo, a.kp, a.push, m, steps, int(copies));
             return hipGetLastError();
         });
@@ -1970,9 +2016,9 @@ hipError_t launch_batch_multi(int prec, const MultiPlan &m, const void *src, voi
         if constexpr (std::is_same<S, bf16_t>::value || std::is_same<S, bf16sr_t>::value)
             return hipErrorInvalidValue;  // (no ensembles in these forms)
         else
-            return dispatch_window(m, [&](auto wx, auto wy) {
+            return dispatch_window<int(sizeof(S))>(m, [&](auto wx, auto wy) {
                 constexpr int WX = decltype(wx)::value, WY = decltype(wy)::value;
-                hipLaunchKernelGGL((k_batch_multi<S, C, WX, WY>), dim3(nwindows), dim3(WX * WY), 0, s, (const S *)src,
+                hipLaunchKernelGGL((k_batch_multi<S, C, WX, WY>), dim3(nwindows), dim3(win_threads<WX, WY>()), 0, s, (const S *)src,
                                    (S *)dst, geo, cases, window_case, steps, int(copies));
                 return hipGetLastError();
             });

@@ -95,6 +95,19 @@ def test_multi_steps_in_every_storage_form(monkeypatch, prec):
     b.close()
 
 
+# lattices that take windows of two and four cells per thread
+@pytest.mark.parametrize("n,prec", [((900, 225), "f32"), ((900, 225), "f16"), ((2999, 301), "f32"),
+                                    ((3601, 1003), "f16"), ((3601, 1003), "bf16")])
+def test_large_windows_equal_other_forms(monkeypatch, n, prec):
+    print(f"[multi] {n} {prec}", flush=True)
+    a, b = _pair(monkeypatch, _deck(n), PRECS[prec])
+    for lat in (a, b):
+        lat.advance(22)
+    _same(a, b)
+    a.close()
+    b.close()
+
+
 @pytest.mark.parametrize("name", ["tiny2d", "inletbody2d", "ragged2d", "channel3", "input.in"])
 def test_multi_steps_match_oracle(name):
     rv = np.random.default_rng(4).random(100)
