@@ -299,6 +299,11 @@ int imexlb_create(imexlb_ctx **out, int dim, int nx, int ny, int nz, int device,
     // 40.0 and 38.0 us); IMEXLB_SMALL_CELLS overrides the cell limit (and
     // that of several steps per launch).
     c->small_cells = std::min<int64_t>(int64_t(5) << 20, (int64_t(240) << 20) / (2 * 9 * int64_t(c->ssz)));
+    // 3D lattices of the same size store their outputs through the caches
+    // (us a step: 129x49x49 FP64 41 and 31, 161x65x65 FP32 37 and 27, 201x81x81
+    // FP16 37 and 28; above, where they leave the cache before they are read
+    // again, 201x81x81 FP32 62 and 65, FP64 121 and 138).
+    if (dim == 3) c->small_cells = (int64_t(240) << 20) / (2 * 27 * int64_t(c->ssz));
     if (const char *sv = std::getenv("IMEXLB_SMALL_CELLS")) c->small_cells = std::atoll(sv);
     // Several steps per launch pay in FP32 at every size, in 16-bit storage up
     // to 8 Mi cells and in FP64 up to 2.5 Mi; above, the cells that neighbouring
@@ -362,12 +367,14 @@ int imexlb_create(imexlb_ctx **out, int dim, int nx, int ny, int nz, int device,
     k.rdz = c->g.dz;
     // XCD-contiguous block order (each XCD steps the same eighth of the
     // lattice every step, so a step reads the previous one's output from its
-    // own L2) pays for D3Q27 FP64 and for the small 2D lattices that stay in
-    // the caches between steps (measured on MI355X); IMEXLB_XCD_REMAP=0/1/R
-    // overrides
+    // own L2) pays for the lattices that stay in the caches between steps;
+    // larger ones take the hardware's order (D3Q27 FP64 us a step, contiguous
+    // and hardware order: 513x129x129 707 and 693, 258x132x130 389 and 376,
+    // 513x257x257 2744 and 2734; FP16 208 and 187, 113 and 103, 794 and 717);
+    // IMEXLB_XCD_REMAP=0/1/R overrides
     const char *xv = std::getenv("IMEXLB_XCD_REMAP");
     k.xcd_remap = xv ? uint32_t(std::max(0, std::atoi(xv)))
-                     : uint32_t(dim == 3 ? precision == IMEXLB_F64 : int64_t(k.ncell) <= c->small_cells);
+                     : uint32_t(int64_t(k.ncell) <= c->small_cells);
 
     if (const char *fv = std::getenv("IMEXLB_FAIL_ALLOC")) c->fail_alloc_at = std::atoll(fv);
     if (device >= 0) {

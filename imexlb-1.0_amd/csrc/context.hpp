@@ -279,13 +279,14 @@ struct imexlb_ctx {
         });
     }
 
-    // mode bits of the fused collide step for this lattice (K_SMALL for 2D
-    // lattices of at most small_cells padded cells)
+    // mode bits of the fused collide step for this lattice (K_SMALL in 2D and
+    // K_CACHED in 3D for lattices of at most small_cells padded cells)
     int collide_mode() const
     {
         if (!push_on) return K_COLLIDE;
         if (!fill32) return K_COLLIDE | K_PUSH | K_IDX64;
-        return K_COLLIDE | K_PUSH | (dim == 2 && int64_t(kp.ncell) <= small_cells ? K_SMALL : 0);
+        if (int64_t(kp.ncell) > small_cells) return K_COLLIDE | K_PUSH;
+        return K_COLLIDE | K_PUSH | (dim == 2 ? K_SMALL : K_CACHED);
     }
     int64_t small_cells = 0;  // set at creation (IMEXLB_SMALL_CELLS)
     int64_t multi_cells = 0;  // up to it several steps per launch

@@ -96,8 +96,9 @@ inline int64_t pop_slot(int64_t q, int64_t c, int64_t plane, int Q)
 // latency-bound 2D lattice -- blocks of one wave, each a 64-cell tile whose
 // boundary copies are spread over its lanes through LDS, the output written
 // with ordinary (cached) stores (with the XCD-contiguous block order each
-// XCD keeps stepping the same eighth of the lattice, in its own L2).
-enum : int { K_COLLIDE = 1, K_WRITE_F = 2, K_WRITE_PU = 4, K_NOSHIFT = 8, K_PUSH = 16, K_IDX64 = 32, K_SMALL = 64 };
+// XCD keeps stepping the same eighth of the lattice, in its own L2); K_CACHED:
+// ordinary output stores in 3D too.
+enum : int { K_COLLIDE = 1, K_WRITE_F = 2, K_WRITE_PU = 4, K_NOSHIFT = 8, K_PUSH = 16, K_IDX64 = 32, K_SMALL = 64, K_CACHED = 256 };
 constexpr unsigned kSmallBlock = 64;
 
 // node-type byte on the device: fluid node; node with boundary copies to push;

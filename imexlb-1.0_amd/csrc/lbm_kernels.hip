@@ -555,7 +555,7 @@ __device__ __forceinline__ void gather(const S *__restrict__ src, const KParams 
 // Internal mode bit of the step kernel: the wave covers exactly one 64-cell
 // tile (cell-mapped threads, 64-cell tiles, one cell per thread), so slots
 // are formed from a wave-uniform tile base plus a 32-bit lane offset.
-constexpr int K_WAVE = 64;
+constexpr int K_WAVE = 512;
 #ifndef IMEXLB_ADDR32
 #define IMEXLB_ADDR32 0
 #endif
@@ -725,7 +725,7 @@ __device__ __forceinline__ void finish_node(const C (&f)[Lat<D>::Q], uint8_t g, 
             S *o = (MODE & K_WAVE) ? wdst + (uint32_t(store_q(q, L::Q)) * 64u + (c & 63u)) : dst + cslot<L::Q>(kp, q, c);
             const S sv = Store<S>::template st<C>(v, srw + uint32_t(q) * kGolden);
             if constexpr (kRegPush) out[q] = sv;
-            if (IMEXLB_STEP_NT)
+            if (IMEXLB_STEP_NT && !(MODE & K_CACHED))
                 nt_store(o, sv);
             else
                 *o = sv;
@@ -876,7 +876,7 @@ __device__ __forceinline__ void step_wave_copies(const S *__restrict__ src, S *_
                 else
                     sv = Store<S>::template st<C>(v, srw + uint32_t(q) * kGolden);
                 S *const o = tdst + (uint32_t(store_q(q, L::Q)) * 64u + lane);
-                if (IMEXLB_STEP_NT)
+                if (IMEXLB_STEP_NT && !(MODE & K_CACHED))
                     nt_store(o, sv);
                 else
                     *o = sv;
@@ -940,7 +940,7 @@ __global__ IMEXLB_STEP_BOUNDS void k_step(const S *__restrict__ src, S *__restri
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x, kp.xcd_remap);
     if constexpr ((MODE & K_SMALL) != 0) {
         step_small<D, S, C, MODE>(src, dst, geo, kp, pt, blk);
-    } else if constexpr (D == 3 && sizeof(S) <= 4 && MODE == (K_COLLIDE | K_PUSH) && CPT == 1 && IMEXLB_CELLMAP &&
+    } else if constexpr (D == 3 && sizeof(S) <= 4 && (MODE & ~K_CACHED) == (K_COLLIDE | K_PUSH) && CPT == 1 && IMEXLB_CELLMAP &&
                          IMEXLB_TILE == 64) {
         __shared__ BitsOf<S> sh[step_block<D, S, MODE>() / 64][Lat<D>::Q * 64];
         step_wave_copies<D, S, C, MODE>(src, dst, geo, kp, pt, blk * step_block<D, S, MODE>() + (threadIdx.x & ~63u),
@@ -955,7 +955,8 @@ __global__ IMEXLB_STEP_BOUNDS void k_step(const S *__restrict__ src, S *__restri
             C f[Lat<D>::Q];
             gather_wave<D, S, C>(src, kp, c, f);
             finish_node<D, S, C, MODE | K_WAVE>(f, g, src, dst, fout, pout, uxo, uyo, uzo, kp, x, y, z, c, pt);
-        } else if constexpr (IMEXLB_CELLMAP && IMEXLB_TILE == 64 && MODE == (MODE & (K_COLLIDE | K_PUSH | K_IDX64))) {
+        } else if constexpr (IMEXLB_CELLMAP && IMEXLB_TILE == 64 &&
+                             MODE == (MODE & (K_COLLIDE | K_PUSH | K_IDX64 | K_CACHED))) {
             // the wave is one tile: output slots from its wave-uniform base
             const uint8_t g = geo[c];
             C f[Lat<D>::Q];
@@ -1857,6 +1858,9 @@ static hipError_t step_d(int prec, int mode, const StepArgs &a, hipStream_t s)
     case K_COLLIDE | K_PUSH | K_IDX64: return step_dm<D, K_COLLIDE | K_PUSH | K_IDX64>(prec, a, s);
     case K_COLLIDE | K_PUSH | K_SMALL:  // the small-lattice form is 2D only
         if constexpr (D == 2) return step_dm<D, K_COLLIDE | K_PUSH | K_SMALL>(prec, a, s);
+        return hipErrorInvalidValue;
+    case K_COLLIDE | K_PUSH | K_CACHED:
+        if constexpr (D == 3) return step_dm<D, K_COLLIDE | K_PUSH | K_CACHED>(prec, a, s);
         return hipErrorInvalidValue;
     case K_WRITE_F: return step_dm<D, K_WRITE_F>(prec, a, s);
     case K_WRITE_F | K_WRITE_PU: return step_dm<D, K_WRITE_F | K_WRITE_PU>(prec, a, s);
