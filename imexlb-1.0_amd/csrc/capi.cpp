@@ -300,7 +300,7 @@ int imexlb_create(imexlb_ctx **out, int dim, int nx, int ny, int nz, int device,
     // that of several steps per launch).
     c->small_cells = std::min<int64_t>(int64_t(5) << 20, (int64_t(240) << 20) / (2 * 9 * int64_t(c->ssz)));
     // 3D lattices of the same size store their outputs through the caches
-    // (us a step: 129x49x49 FP64 41 and 31, 161x65x65 FP32 37 and 27, 201x81x81
+    // (us a step: 129x49x49 FP64 41 and 31 (25 with LDS copies), 161x65x65 FP32 37 and 27, 201x81x81
     // FP16 37 and 28; above, where they leave the cache before they are read
     // again, 201x81x81 FP32 62 and 65, FP64 121 and 138).
     if (dim == 3) c->small_cells = (int64_t(240) << 20) / (2 * 27 * int64_t(c->ssz));

@@ -825,13 +825,15 @@ __device__ __forceinline__ void step_small(const S *__restrict__ src, S *__restr
     }
 }
 
-// The fused step of a D3Q27 lattice in 16- or 32-bit storage, one wave per
-// 64-cell tile [c0, c0 + 64): as step_small, each wave with boundary copies
-// leaves its cells' values in LDS (27 x 64 values) and spreads the tile's
-// run of the push table over its lanes, one LDS read and one store per copy,
-// instead of each cell reading back its own output per copy.  Output stores
-// non-temporal.  (FP64 keeps the read-back: 13.8 KB of LDS per wave would
-// cost the kernel a wave per SIMD.)
+// The fused step of a D3Q27 lattice in 16- or 32-bit storage, and in FP64 where
+// it stays in the caches, one wave per 64-cell tile [c0, c0 + 64): as
+// step_small, each wave with boundary copies leaves its cells' values in LDS
+// (27 x 64 values) and spreads the tile's run of the push table over its lanes,
+// one LDS read and one store per copy, instead of each cell reading back its
+// own output per copy.  Output stores non-temporal but with K_CACHED.  A small
+// lattice's step is one wave's chain of accesses: FP64 49 x 17 x 17 10.5 to 7.0
+// us, 129 x 49 x 49 31 to 24.6.  (Larger FP64 lattices keep the read-back: 13.8
+// KB of LDS per wave would cost the kernel a wave per SIMD.)
 template <int D, class S, class C, int MODE>
 __device__ __forceinline__ void step_wave_copies(const S *__restrict__ src, S *__restrict__ dst,
                                                  const uint8_t *__restrict__ geo, const KParams &kp,
@@ -901,15 +903,16 @@ __device__ __forceinline__ void step_wave_copies(const S *__restrict__ src, S *_
     }
 }
 
-// Threads per block of the fused step: one wave for the small-lattice form
-// and for D3Q27 in FP32 storage (2.8 % faster on the sphere than 256), 128
+// Threads per block of the fused step: one wave for the small-lattice form,
+// for D3Q27 in FP32 storage (2.8 % faster on the sphere than 256) and in FP64
+// with LDS copies, 128
 // for D2Q9 in FP64 storage (2.5 % faster on the 8192x2048 cylinder), and
 // IMEXLB_STEP_BLOCK otherwise (the 16-bit forms lose 2-4 % at 128 and
 // 11-18 % at 64, FP64 D3Q27 0.4-0.6 % at 64 and 128).
 template <int D, class S, int MODE>
 __host__ __device__ constexpr unsigned step_block()
 {
-    return (MODE & K_SMALL) || (D == 3 && sizeof(S) == 4) ? unsigned(kSmallBlock)
+    return (MODE & K_SMALL) || (D == 3 && (sizeof(S) == 4 || (sizeof(S) == 8 && (MODE & K_CACHED)))) ? unsigned(kSmallBlock)
            : (D == 2 && sizeof(S) == 8 && IMEXLB_STEP_BLOCK >= 128) ? 128u
                                                                    : unsigned(IMEXLB_STEP_BLOCK);
 }
@@ -940,7 +943,7 @@ __global__ IMEXLB_STEP_BOUNDS void k_step(const S *__restrict__ src, S *__restri
     const uint32_t blk = xcd_block(blockIdx.x, gridDim.x, kp.xcd_remap);
     if constexpr ((MODE & K_SMALL) != 0) {
         step_small<D, S, C, MODE>(src, dst, geo, kp, pt, blk);
-    } else if constexpr (D == 3 && sizeof(S) <= 4 && (MODE & ~K_CACHED) == (K_COLLIDE | K_PUSH) && CPT == 1 && IMEXLB_CELLMAP &&
+    } else if constexpr (D == 3 && (sizeof(S) <= 4 || (MODE & K_CACHED)) && (MODE & ~K_CACHED) == (K_COLLIDE | K_PUSH) && CPT == 1 && IMEXLB_CELLMAP &&
                          IMEXLB_TILE == 64) {
         __shared__ BitsOf<S> sh[step_block<D, S, MODE>() / 64][Lat<D>::Q * 64];
         step_wave_copies<D, S, C, MODE>(src, dst, geo, kp, pt, blk * step_block<D, S, MODE>() + (threadIdx.x & ~63u),
