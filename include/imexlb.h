@@ -149,8 +149,8 @@ int imexlb_init_pdf(imexlb_ctx *ctx);
 
 /* The four phases of one time step, main.f90:57-61.  In fused mode, on a
  * lattice whose step writes its own boundary copies, the step's kernel is
- * queued rather than launched by PostProcessing: queued steps run as graph
- * replays once 16 are pending and before any other call that launches work
+ * queued rather than launched by PostProcessing: queued steps run together
+ * once 7 to 19 are pending (by size) and before any other call that launches work
  * or reads device state (so results are the same; an error of such a launch
  * is returned by the call that runs it).  set_params after a fused step
  * relaxes the next Collision with the new parameters, as the reference. */
