@@ -1031,12 +1031,26 @@ __global__ __launch_bounds__(256) void k_step_list(const S *__restrict__ src, S 
 // a step at 8192 x 2048 FP64 (4.5 TB/s), tile-aligned ones 0.243 (5.1 TB/s);
 // the single step 0.412.  FP32 0.207 to 0.127, FP16 0.103 to 0.082 (bound by
 // instructions), BF16 with stochastic rounding 0.105 to 0.090.  Gathering two
-// rows ahead measured slower in every form but FP32.
+// rows ahead measured slower in every form but FP32.  The blocks from nbulk on
+// make the second step of the frame's cells (from the first step in `first`)
+// beside the bulk, which leaves a CU room for one: FP64 4001 x 1201 83.2 to
+// 82.0 us a step, BF16 with stochastic rounding 7002 x 1502 61.0 to 56.7.
 template <class S, class C>
 __global__ __launch_bounds__(kDouble2) void k_double2(const S *__restrict__ src, S *__restrict__ dst,
                                                       const uint8_t *__restrict__ geo, KParams kp, int rows,
-                                                      uint32_t nstrips)
+                                                      uint32_t nstrips, uint32_t nbulk, PushTable pt,
+                                                      const S *__restrict__ first, const uint32_t *__restrict__ list,
+                                                      uint32_t n)
 {
+    if (blockIdx.x >= nbulk) {
+        const uint32_t i = (blockIdx.x - nbulk) * uint32_t(kDouble2) + threadIdx.x;
+        int fx, fy, fz;
+        uint32_t fc;
+        if (i < n && decode_cell<2>(kp, list[i], fx, fy, fz, fc))
+            step_node<2, S, C, K_COLLIDE | K_PUSH>(first, dst, nullptr, nullptr, nullptr, nullptr, nullptr, geo, kp, fx,
+                                                   fy, fz, fc, pt);
+        return;
+    }
     using L = Lat<2>;
     using U = BitsOf<S>;
     // e_x = -1, +1 populations of direction e_y = -1, 0, +1: needed this row,
@@ -1909,11 +1923,13 @@ hipError_t launch_double(int dim, int prec, const StepArgs &a, const DoublePlan 
     e = dispatch_prec(prec, [&](auto *sp, auto *cp) {
         using S = std::remove_pointer_t<decltype(sp)>;
         using C = std::remove_pointer_t<decltype(cp)>;
-        hipLaunchKernelGGL((k_double2<S, C>), dim3(d.strips * d.segments), dim3(kDouble2), 0, s, (const S *)a.src,
-                           (S *)a.dst, a.geo, a.kp, d.rows, d.strips);
+        const uint32_t nbulk = d.strips * d.segments, n = d.idx64 ? 0u : d.count[1];
+        hipLaunchKernelGGL((k_double2<S, C>), dim3(nbulk + (n + kDouble2 - 1) / kDouble2), dim3(kDouble2), 0, s,
+                           (const S *)a.src, (S *)a.dst, a.geo, a.kp, d.rows, d.strips, nbulk, a.push,
+                           (const S *)d.scratch, d.list[1], n);
         return hipGetLastError();
     });
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess || !d.idx64) return e;
     return launch_step_list(dim, prec, d.idx64, second, d.list[1], d.count[1], s);
 }
 
