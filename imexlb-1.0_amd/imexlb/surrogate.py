@@ -96,7 +96,8 @@ class UNet:
         dev = "cuda"
         f32 = torch.float32
         # weights then biases, their gradients and both moments in one buffer
-        # each (one Adam launch for all); the lists are views into them
+        # each (one Adam launch for all); the lists are views into them.  A
+        # list entry may be replaced by another tensor (_whole)
         sizes = [co * ci * 9 for co, ci in self.shapes] + [co for co, ci in self.shapes]
         self.nw = sum(sizes[:len(self.shapes)])
         host = []
@@ -113,6 +114,8 @@ class UNet:
             return [p.view(co, ci, 3, 3) for p, (co, ci) in zip(parts, self.shapes)], list(parts[n:])
 
         (self.w, self.b), (self.dw, self.db) = views(self.flat), views(self.grads)
+        (self.mw, self.mb), (self.vw, self.vb) = views(self.mom1), views(self.mom2)
+        self.places = [v.data_ptr() for v in self._all()]
         self.step_count = 0
         # per-level sizes and buffers
         self.hw = [(H >> l, W >> l) for l in range(L)]
@@ -145,6 +148,13 @@ class UNet:
         self.grad_out = self.gout = e(cout, 0)
 
     # ---------------------------------------------------------------- layers
+    def _all(self):
+        return [v for vs in (self.w, self.b, self.dw, self.db, self.mw, self.mb, self.vw, self.vb) for v in vs]
+
+    def _whole(self):
+        """whether every list still holds the parts of the common buffers"""
+        return [v.data_ptr() for v in self._all()] == self.places
+
     def _act(self, k):
         """(buffer, its channels, first channel) of convolution k's output"""
         if k in self.skip_of:
@@ -205,7 +215,11 @@ class UNet:
         """g: gradient of the loss w.r.t. the output; fills dw, db."""
         L, ch, N = len(self.chans), self.chans, self.N
         self.gout = g
-        self.grads[:self.nw].zero_()
+        if self._whole():
+            self.grads[:self.nw].zero_()
+        else:
+            for t in self.dw:
+                t.zero_()
         k = len(self.shapes) - 1
         self._conv_back(k, g, self.dz[k - 1], gate=k - 1)
         for l in range(0, L - 1):  # decoder, from the output down
@@ -233,8 +247,13 @@ class UNet:
 
     def adam(self, lr, b1=0.9, b2=0.999, eps=1e-8):
         self.step_count += 1
-        _ok(lib().imexlb_nn_adam(_ptr(self.flat), _ptr(self.grads), _ptr(self.mom1), _ptr(self.mom2),
-                                 self.flat.numel(), lr, b1, b2, eps, self.step_count, None), "adam")
+        if self._whole():
+            groups = [(self.flat, self.grads, self.mom1, self.mom2)]
+        else:
+            groups = [*zip(self.w, self.dw, self.mw, self.vw), *zip(self.b, self.db, self.mb, self.vb)]
+        for p, g, m, v in groups:
+            _ok(lib().imexlb_nn_adam(_ptr(p), _ptr(g), _ptr(m), _ptr(v), p.numel(), lr, b1, b2, eps, self.step_count,
+                                     None), "adam")
 
     def params_numpy(self):
         return [(w.cpu().numpy().astype(np.float64), b.cpu().numpy().astype(np.float64)) for w, b in zip(self.w, self.b)]
