@@ -361,8 +361,8 @@ int imexlb_batch::build_multi(const std::vector<int32_t> &fd, const std::vector<
     if (bad) return drop();
     int32_t tables = 0;
     for (int32_t &v : mark) v = v ? tables++ : -1;
-    const size_t cells = size_t(plans[0].wx * plans[0].wy);
-    if (hipMalloc((void **)&multi_place, std::max<size_t>(1, size_t(tables) * 9 * cells * 2)) != hipSuccess) return drop();
+    const size_t entries = size_t(place_base(tables, uint32_t(plans[0].wx * plans[0].wy)));
+    if (hipMalloc((void **)&multi_place, std::max<size_t>(1, entries * 2)) != hipSuccess) return drop();
     HIP_TRY(hipMemcpy(multi_table, mark.data(), nw * 4, hipMemcpyHostToDevice));
     HIP_TRY(plan(multi_place));
     for (int i = 0; i < ncase; ++i) {

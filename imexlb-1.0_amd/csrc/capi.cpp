@@ -552,7 +552,7 @@ static int build_multi(imexlb_ctx *c, const DeviceTables &t)
     }
     int32_t tables = 0;
     for (int32_t &v : mark) v = v ? tables++ : -1;
-    if (hipMalloc((void **)&c->multi_place, std::max<size_t>(1, size_t(tables) * 9 * size_t(m.wx * m.wy) * 2)) != hipSuccess)
+    if (hipMalloc((void **)&c->multi_place, std::max<size_t>(1, size_t(place_base(tables, uint32_t(m.wx * m.wy))) * 2)) != hipSuccess)
         return no_memory();
     HIP_TRY(hipMemcpy(c->multi_table, mark.data(), nw * sizeof(int32_t), hipMemcpyHostToDevice));
     HIP_TRY(plan(c->multi_place));

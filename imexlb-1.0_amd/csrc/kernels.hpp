@@ -128,6 +128,11 @@ struct MultiPlan {
     const uint16_t *place = nullptr;  // the tables
 };
 
+// First entry of a window's table of places (9 directions of `cells` cells).
+// In 64 bits: the tables of a large ensemble or of a long channel two windows
+// high pass 2^32 entries (116,509 of 64 x 64 cells, 466,034 of 32 x 32).
+__host__ __device__ inline int64_t place_base(int32_t table, uint32_t cells) { return int64_t(table) * 9 * cells; }
+
 // One case of a batched ensemble: its parameters and where its populations
 // and node types start in the shared arrays.
 struct BatchCase {

@@ -1339,7 +1339,7 @@ __global__ __launch_bounds__((win_threads<WX, WY>())) void k_multi_plan(const in
                     }
                 }
             }
-            if (place && mark[blockIdx.x] >= 0) place[(uint32_t(mark[blockIdx.x]) * 9u + uint32_t(q)) * N + l] = uint16_t(at);
+            if (place && mark[blockIdx.x] >= 0) place[place_base(mark[blockIdx.x], N) + (uint32_t(q) * N + l)] = uint16_t(at);
         }
         right[0][l] = fluid ? m.halo : 0;
     }
@@ -1431,10 +1431,11 @@ __device__ __forceinline__ void multi_window(const S *__restrict__ src, S *__res
         }
     } else {
         uint32_t at[P][L::Q];
+        const uint16_t *const place = m.place + place_base(table, N);
 #pragma unroll
         for (uint32_t p = 0; p < P; ++p) {
 #pragma unroll
-            for (int q = 0; q < L::Q; ++q) at[p][q] = m.place[(uint32_t(table) * 9u + uint32_t(q)) * N + th + p * T];
+            for (int q = 0; q < L::Q; ++q) at[p][q] = place[uint32_t(q) * N + th + p * T];
             g[p] = g[p] ? geo[c[p]] : 0u;
         }
         if (th < 2) cells[th][9 * N] = U(0);
