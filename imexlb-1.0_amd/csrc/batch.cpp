@@ -838,4 +838,15 @@ int imexlb_batch_info(imexlb_batch *b, int64_t out[4])
     return IMEXLB_OK;
 }
 
+int imexlb_batch_step_form(imexlb_batch *b, int32_t out[4])
+{
+    if (!b || !out) return fail(IMEXLB_E_ARG, "null pointer");
+    const MultiPlan &m = b->cases[0].multi;
+    out[0] = b->multi_on ? m.halo : 1;
+    out[1] = b->multi_on ? m.wx : 0;
+    out[2] = b->multi_on ? m.wy : 0;
+    out[3] = b->multi_on ? int32_t(b->nwindows) : 0;
+    return IMEXLB_OK;
+}
+
 }  // extern "C"

@@ -1352,4 +1352,16 @@ int imexlb_info(imexlb_ctx *c, int64_t out[6])
     return IMEXLB_OK;
 }
 
+int imexlb_step_form(imexlb_ctx *c, int32_t out[4])
+{
+    CHECK_DEV(c);
+    if (!out) return fail(IMEXLB_E_ARG, "null pointer");
+    if (!c->geom_set) return fail(IMEXLB_E_STATE, "SetGeometry not called");
+    out[0] = c->multi_on ? c->multi.halo : c->dbl_on ? 2 : 1;
+    out[1] = c->multi_on ? c->multi.wx : 0;
+    out[2] = c->multi_on ? c->multi.wy : 0;
+    out[3] = int32_t(c->Px);
+    return IMEXLB_OK;
+}
+
 }  // extern "C"

@@ -57,6 +57,7 @@ SIGNATURES = {
     "imexlb_profile": (C.c_int, [_P, C.c_int]),
     "imexlb_profile_read": (C.c_int, [_P, _I64P, _DP]),
     "imexlb_info": (C.c_int, [_P, _I64P]),
+    "imexlb_step_form": (C.c_int, [_P, _I32P]),
     "imexlb_batch_create": (C.c_int, [C.POINTER(_P), C.c_int, _I32P, _DP, C.c_int, C.c_int]),
     "imexlb_batch_create_shapes": (C.c_int, [C.POINTER(_P), C.c_int, _I32P, _DP, _DP, C.c_int, C.c_int]),
     "imexlb_batch_destroy": (C.c_int, [_P]),
@@ -72,6 +73,7 @@ SIGNATURES = {
     "imexlb_batch_monitor": (C.c_int, [_P, _DP]),
     "imexlb_batch_download_fields": (C.c_int, [_P, C.c_int, _DP, _DP]),
     "imexlb_batch_info": (C.c_int, [_P, _I64P]),
+    "imexlb_batch_step_form": (C.c_int, [_P, _I32P]),
     # warm-start network kernels (include/imexlb_nn.h); float pointers are device addresses
     "imexlb_nn_conv3x3": (C.c_int, [_P, _P, _P, _P, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _P]),
     "imexlb_nn_conv3x3_into": (C.c_int, [_P, _P, _P, _P] + [C.c_int] * 8 + [_P]),

@@ -134,6 +134,13 @@ class Batch:
               "imexlb_batch_download_fields")
         return p, u
 
+    def step_form(self):
+        """How advance() steps the cases: the most steps a launch makes, the
+        window they are made in (None: none), windows per launch."""
+        out = (C.c_int32 * 4)()
+        check(lib().imexlb_batch_step_form(self._h, out), "imexlb_batch_step_form")
+        return {"steps_per_pass": out[0], "window": (out[1], out[2]) if out[1] else None, "windows": out[3]}
+
     def synchronize(self):
         check(lib().imexlb_batch_synchronize(self._h), "imexlb_batch_synchronize")
 

@@ -198,6 +198,13 @@ class Lattice:
         keys = ("nodes", "fluid", "plane_bytes", "device_bytes", "value_bytes", "bc_entries")
         return dict(zip(keys, list(out)))
 
+    def step_form(self):
+        """How advance() steps this lattice: the most steps a pass makes,
+        the window they are made in (None: none), cells of a padded row."""
+        out = (C.c_int32 * 4)()
+        check(lib().imexlb_step_form(self._h, out), "imexlb_step_form")
+        return {"steps_per_pass": out[0], "window": (out[1], out[2]) if out[1] else None, "row_cells": out[3]}
+
 
 def setup(deck: Deck, r_vec, device=0, precision=_lib.F64):
     """DataInput .. InitPDF of main.f90:19-40 for one deck; returns (Lattice, Derived)."""

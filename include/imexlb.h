@@ -208,8 +208,8 @@ int imexlb_synchronize(imexlb_ctx *ctx);
 /* Kernel timing with HIP events on the context stream.  While enabled,
  * every launch is bracketed by events; imexlb_profile_read returns, for
  * kernel class k (0 fused step, 1 boundary fill, 2 other), the launch count
- * and the summed milliseconds since the last reset.  A pass that makes two
- * steps counts as two launches. */
+ * and the summed milliseconds since the last reset.  A pass that makes several
+ * steps counts as so many launches. */
 int imexlb_profile(imexlb_ctx *ctx, int enable);
 int imexlb_profile_read(imexlb_ctx *ctx, int64_t launches[3], double ms[3]);
 
@@ -217,6 +217,13 @@ int imexlb_profile_read(imexlb_ctx *ctx, int64_t launches[3], double ms[3]);
  * array on the device, [3] device bytes allocated, [4] storage bytes per
  * population value, [5] boundary-table entries. */
 int imexlb_info(imexlb_ctx *ctx, int64_t out[6]);
+
+/* How the fused steps of imexlb_advance and of the queued phase calls run on
+ * this lattice, as SetGeometry chose (results do not depend on it): [0] the
+ * most steps one pass over the lattice makes (1; 2; 3 to 9: several per
+ * launch, in windows), [1], [2] a window's cells along x and y (0 without
+ * windows), [3] cells of a padded row. */
+int imexlb_step_form(imexlb_ctx *ctx, int32_t out[4]);
 
 /* ---------------------------------------------------------------------
  * Batched ensemble.  No counterpart in the reference, which runs one
@@ -275,6 +282,10 @@ int imexlb_batch_monitor(imexlb_batch *b, double *um);
 int imexlb_batch_download_fields(imexlb_batch *b, int i, double *p, double *u);
 /* [0] nodes of all cases, [1] cases, [2] tiles, [3] device bytes */
 int imexlb_batch_info(imexlb_batch *b, int64_t out[4]);
+/* [0] to [2] as imexlb_step_form, for every case of the ensemble; [3] windows
+ * per launch.  One case that several steps per launch do not suit keeps the
+ * whole ensemble on single steps. */
+int imexlb_batch_step_form(imexlb_batch *b, int32_t out[4]);
 
 #ifdef __cplusplus
 }
