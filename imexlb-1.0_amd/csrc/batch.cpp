@@ -54,6 +54,8 @@ struct imexlb_batch {
     uint32_t *tile_case = nullptr, *tile_first = nullptr;
     uint32_t ntiles = 0;
     size_t dev_bytes = 0;
+    AllocHook hook;
+    PlanMemory multi_mem;
 
     int block = 256, cpt = 1, persist = 0;
     unsigned persist_grid = 1024;
@@ -273,6 +275,7 @@ namespace {
 
 int balloc(imexlb_batch *b, void **ptr, size_t bytes)
 {
+    if (b->hook.fails()) return fail(IMEXLB_E_OOM, "batch hipMalloc: failure injected by IMEXLB_FAIL_ALLOC");
     hipError_t e = hipMalloc(ptr, bytes);
     if (e != hipSuccess) {
         *ptr = nullptr;
@@ -283,14 +286,6 @@ int balloc(imexlb_batch *b, void **ptr, size_t bytes)
     if (e != hipSuccess) return fail(IMEXLB_E_HIP, "batch hipMemset failed");
     return IMEXLB_OK;
 }
-
-struct DeviceTemp {  // freed on every return
-    void *p = nullptr;
-    ~DeviceTemp()
-    {
-        if (p) (void)hipFree(p);
-    }
-};
 
 #define CHECK_BATCH(b)                                                    \
     do {                                                                  \
@@ -319,18 +314,18 @@ int imexlb_batch::build_multi(const std::vector<int32_t> &fd, const std::vector<
     }
     DeviceTemp from, dbad, dfd, dfs;
     const auto drop = [&] {
-        (void)hipGetLastError();
         for (void *q : {(void *)window_case, (void *)multi_table, (void *)multi_place})
             if (q) (void)hipFree(q);
         window_case = nullptr;
         multi_table = nullptr;
         multi_place = nullptr;
+        multi_mem = PlanMemory{};
         return IMEXLB_OK;
     };
     const size_t nw = wc.size(), nf = std::max<size_t>(fd.size(), 1);
-    if (hipMalloc((void **)&window_case, nw * 4) != hipSuccess || hipMalloc((void **)&multi_table, nw * 4) != hipSuccess ||
-        hipMalloc(&from.p, size_t(slots) * 4) != hipSuccess || hipMalloc(&dbad.p, 4) != hipSuccess ||
-        hipMalloc(&dfd.p, nf * 4) != hipSuccess || hipMalloc(&dfs.p, nf * 4) != hipSuccess)
+    if (!multi_mem.get(hook, (void **)&window_case, nw * 4) || !multi_mem.get(hook, (void **)&multi_table, nw * 4) ||
+        !PlanMemory::temp(hook, &from.p, size_t(slots) * 4) || !PlanMemory::temp(hook, &dbad.p, 4) ||
+        !PlanMemory::temp(hook, &dfd.p, nf * 4) || !PlanMemory::temp(hook, &dfs.p, nf * 4))
         return drop();
     HIP_TRY(hipMemcpy(window_case, wc.data(), nw * 4, hipMemcpyHostToDevice));
     if (!fd.empty()) {
@@ -362,7 +357,7 @@ int imexlb_batch::build_multi(const std::vector<int32_t> &fd, const std::vector<
     int32_t tables = 0;
     for (int32_t &v : mark) v = v ? tables++ : -1;
     const size_t entries = size_t(place_base(tables, uint32_t(plans[0].wx * plans[0].wy)));
-    if (hipMalloc((void **)&multi_place, std::max<size_t>(1, entries * 2)) != hipSuccess) return drop();
+    if (!multi_mem.get(hook, (void **)&multi_place, std::max<size_t>(1, entries * 2))) return drop();
     HIP_TRY(hipMemcpy(multi_table, mark.data(), nw * 4, hipMemcpyHostToDevice));
     HIP_TRY(plan(multi_place));
     for (int i = 0; i < ncase; ++i) {
@@ -402,6 +397,7 @@ int imexlb_batch_create_shapes(imexlb_batch **out, int ncase, const int32_t *nxn
                                                                   }
                                                               });
     if (!b) return fail(IMEXLB_E_OOM, "batch");
+    b->hook.read();
     b->ncase = ncase;
     b->prec = precision;
     b->device = device;
@@ -529,9 +525,10 @@ int imexlb_batch_create_shapes(imexlb_batch **out, int ncase, const int32_t *nxn
         HIP_TRY(hipMemcpy(B->link_back, lbk.data(), lbk.size() * 8, hipMemcpyHostToDevice));
         HIP_TRY(hipMemcpy(B->link_q, lq.data(), lq.size(), hipMemcpyHostToDevice));
     }
+    // (what the ensemble needs first, so that the windows' tables leave room for it)
+    if ((rc = B->build_tiles())) return rc;
     if (multi && (rc = B->build_multi(mfd, mfs, mfirst))) return rc;
     HIP_TRY(hipMemcpy(B->d_cases, B->cases.data(), size_t(ncase) * sizeof(BatchCase), hipMemcpyHostToDevice));
-    if ((rc = B->build_tiles())) return rc;
     *out = b.release();
     return IMEXLB_OK;
 }
@@ -834,7 +831,7 @@ int imexlb_batch_info(imexlb_batch *b, int64_t out[4])
     out[0] = b->node_total;
     out[1] = b->ncase;
     out[2] = int64_t(b->ntiles);
-    out[3] = int64_t(b->dev_bytes);
+    out[3] = int64_t(b->dev_bytes + b->multi_mem.bytes);
     return IMEXLB_OK;
 }
 

@@ -376,7 +376,7 @@ int imexlb_create(imexlb_ctx **out, int dim, int nx, int ny, int nz, int device,
     k.xcd_remap = xv ? uint32_t(std::max(0, std::atoi(xv)))
                      : uint32_t(int64_t(k.ncell) <= c->small_cells);
 
-    if (const char *fv = std::getenv("IMEXLB_FAIL_ALLOC")) c->fail_alloc_at = std::atoll(fv);
+    c->hook.read();
     if (device >= 0) {
         int ndev = 0;
         HIP_TRY(hipGetDeviceCount(&ndev));
@@ -459,28 +459,22 @@ static bool double_suits(const imexlb_ctx *c)
 
 // The two-steps-per-pass plan of the new geometry: the frame's lists, the
 // bulk's marks in the node types, the scratch buffer.  A lattice it does not
-// suit, or without memory for the scratch buffer, keeps single steps.
+// suit, or without memory for it, keeps single steps.
 static int build_double(imexlb_ctx *c)
 {
     c->drop_double();
     if (!c->dbl_enabled || !c->push_on || c->multi_on || !double_suits(c)) return IMEXLB_OK;
     DoublePlan &d = c->dbl;
-    struct Tmp {  // freed on every return
-        void *p = nullptr;
-        ~Tmp()
-        {
-            if (p) (void)hipFree(p);
-        }
-    } zones, counts;
+    DeviceTemp zones, counts;
     const size_t pop = size_t(c->Q) * size_t(c->plane) * c->ssz, n = size_t(c->plane);
-    if (hipMalloc(&d.scratch, pop) != hipSuccess) {
-        (void)hipGetLastError();
-        d.scratch = nullptr;
+    const auto no_memory = [&] {
+        c->drop_double();
         return IMEXLB_OK;
-    }
+    };
+    if (!c->dbl_mem.get(c->hook, &d.scratch, pop) || !PlanMemory::temp(c->hook, &zones.p, 3 * n) ||
+        !PlanMemory::temp(c->hook, &counts.p, 4 * sizeof(uint32_t)))
+        return no_memory();
     HIP_TRY(hipMemset(d.scratch, 0, pop));
-    HIP_TRY(hipMalloc(&zones.p, 3 * n));
-    HIP_TRY(hipMalloc(&counts.p, 4 * sizeof(uint32_t)));
     HIP_TRY(hipMemset(zones.p, 0, 3 * n));
     HIP_TRY(hipMemset(counts.p, 0, 4 * sizeof(uint32_t)));
     uint8_t *const z = static_cast<uint8_t *>(zones.p);
@@ -495,7 +489,8 @@ static int build_double(imexlb_ctx *c)
         HIP_TRY(launch_zone(c->dim, 2, a, c->geo, z + (2 - k) * n, nullptr, cnt + k, nullptr, k, nullptr));
     HIP_TRY(hipMemcpy(d.count, cnt, sizeof(d.count), hipMemcpyDeviceToHost));
     for (int k = 0; k < 2; ++k) {
-        HIP_TRY(hipMalloc((void **)&d.list[k], std::max<size_t>(d.count[k], 1) * sizeof(uint32_t)));
+        if (!c->dbl_mem.get(c->hook, (void **)&d.list[k], std::max<size_t>(d.count[k], 1) * sizeof(uint32_t)))
+            return no_memory();
         HIP_TRY(launch_zone(c->dim, 2, a, c->geo, z + (2 - k) * n, nullptr, cnt + 2 + k, d.list[k], 0, nullptr));
     }
     HIP_TRY(hipDeviceSynchronize());
@@ -516,22 +511,15 @@ static int build_multi(imexlb_ctx *c, const DeviceTables &t)
     std::vector<MultiPlan> plans;
     plan_multi(int(c->ssz), {&c->kp}, plans);
     c->multi = plans[0];
-    struct Tmp {  // freed on every return
-        void *p = nullptr;
-        ~Tmp()
-        {
-            if (p) (void)hipFree(p);
-        }
-    } dfrom, dbad;
+    DeviceTemp dfrom, dbad;
     const MultiPlan &m = c->multi;
     const size_t nw = size_t(m.nx) * size_t(m.ny), nslots = size_t(c->Q) * size_t(c->plane);
     const auto no_memory = [&] {
-        (void)hipGetLastError();
         c->drop_multi();
         return IMEXLB_OK;
     };
-    if (hipMalloc((void **)&c->multi_table, nw * sizeof(int32_t)) != hipSuccess ||
-        hipMalloc(&dfrom.p, nslots * sizeof(int32_t)) != hipSuccess || hipMalloc(&dbad.p, 4) != hipSuccess)
+    if (!c->multi_mem.get(c->hook, (void **)&c->multi_table, nw * sizeof(int32_t)) ||
+        !PlanMemory::temp(c->hook, &dfrom.p, nslots * sizeof(int32_t)) || !PlanMemory::temp(c->hook, &dbad.p, 4))
         return no_memory();
     uint32_t bad = 0;
     std::vector<int32_t> mark(nw);
@@ -552,7 +540,8 @@ static int build_multi(imexlb_ctx *c, const DeviceTables &t)
     }
     int32_t tables = 0;
     for (int32_t &v : mark) v = v ? tables++ : -1;
-    if (hipMalloc((void **)&c->multi_place, std::max<size_t>(1, size_t(place_base(tables, uint32_t(m.wx * m.wy))) * 2)) != hipSuccess)
+    if (!c->multi_mem.get(c->hook, (void **)&c->multi_place,
+                          std::max<size_t>(1, size_t(place_base(tables, uint32_t(m.wx * m.wy))) * 2)))
         return no_memory();
     HIP_TRY(hipMemcpy(c->multi_table, mark.data(), nw * sizeof(int32_t), hipMemcpyHostToDevice));
     HIP_TRY(plan(c->multi_place));
@@ -1346,7 +1335,7 @@ int imexlb_info(imexlb_ctx *c, int64_t out[6])
     out[0] = int64_t(c->kp.N);
     out[1] = int64_t(c->g.fluid_id.size());
     out[2] = int64_t(c->plane) * int64_t(c->ssz);
-    out[3] = int64_t(c->dev_bytes);
+    out[3] = int64_t(c->dev_bytes + c->dbl_mem.bytes + c->multi_mem.bytes);
     out[4] = int64_t(c->ssz);
     out[5] = int64_t(c->bc.entries.size());
     return IMEXLB_OK;

@@ -58,6 +58,46 @@ struct FieldCopy {
     double *to;          // the caller's dense interior array
 };
 
+// Test hook: IMEXLB_FAIL_ALLOC=N (read when a lattice or an ensemble is
+// created) makes its N-th device allocation fail.
+struct AllocHook {
+    int64_t calls = 0, fail_at = 0;
+    void read()
+    {
+        if (const char *v = std::getenv("IMEXLB_FAIL_ALLOC")) fail_at = std::atoll(v);
+    }
+    bool fails() { return fail_at > 0 && ++calls == fail_at; }
+};
+
+// Device memory of a plan that its owner does without if there is none: no
+// error is left behind, and what the plan keeps is counted while it does.
+struct PlanMemory {
+    size_t bytes = 0;
+    bool get(AllocHook &hook, void **ptr, size_t n)
+    {
+        if (!temp(hook, ptr, n)) return false;
+        bytes += n;
+        return true;
+    }
+    static bool temp(AllocHook &hook, void **ptr, size_t n)
+    {
+        *ptr = nullptr;
+        if (hook.fails()) return false;
+        if (hipMalloc(ptr, n) == hipSuccess) return true;
+        (void)hipGetLastError();
+        *ptr = nullptr;
+        return false;
+    }
+};
+
+struct DeviceTemp {  // freed on every return
+    void *p = nullptr;
+    ~DeviceTemp()
+    {
+        if (p) (void)hipFree(p);
+    }
+};
+
 // The interior of padded device arrays to dense host arrays, after the work on
 // the stream; false if there is no memory for the buffers (nothing was copied).
 bool download_interior(Staging &s, int device, hipStream_t stream, int dim, const KParams &kp,
@@ -106,9 +146,7 @@ struct imexlb_ctx {
     Staging staging;
     double *mass_partial = nullptr;  // MASS_BLOCKS partial sums, then the total
     size_t dev_bytes = 0;
-    // test hook: IMEXLB_FAIL_ALLOC=N (read at creation) makes this
-    // context's N-th device allocation fail with IMEXLB_E_OOM
-    int64_t alloc_calls = 0, fail_alloc_at = 0;
+    AllocHook hook;
 
     // Forget the geometry after a failed SetGeometry: every call that needs
     // one (InitUP, the phases, Monitor, downloads) then returns
@@ -165,12 +203,14 @@ struct imexlb_ctx {
     // Two steps in one pass over memory, for lattices that do not stay in the
     // caches (built with the geometry; IMEXLB_DOUBLE=0 keeps single steps)
     DoublePlan dbl;
+    PlanMemory dbl_mem;
     bool dbl_enabled = true, dbl_on = false;
     hipGraphExec_t quad_graph[kGraphSizes][2] = {};  // kQuads[j] pairs of double steps, by starting buffer
     static constexpr int kQuads[kGraphSizes] = {16, 4, 1};
     // Several steps in one launch (built with the geometry; IMEXLB_MULTI=0
     // keeps the other forms)
     MultiPlan multi;
+    PlanMemory multi_mem;
     int32_t *multi_table = nullptr;
     uint16_t *multi_place = nullptr;
     bool multi_enabled = true, multi_on = false;
@@ -183,6 +223,7 @@ struct imexlb_ctx {
         multi_table = nullptr;
         multi_place = nullptr;
         multi = MultiPlan{};
+        multi_mem = PlanMemory{};
         multi_on = false;
     }
     void drop_double()
@@ -190,6 +231,7 @@ struct imexlb_ctx {
         for (void *q : {(void *)dbl.list[0], (void *)dbl.list[1], dbl.scratch})
             if (q) (void)hipFree(q);
         dbl = DoublePlan{};
+        dbl_mem = PlanMemory{};
         dbl_on = false;
     }
 
@@ -356,7 +398,7 @@ namespace imexlb {
 
 inline int dev_alloc(imexlb_ctx *c, void **ptr, size_t bytes)
 {
-    if (c->fail_alloc_at > 0 && ++c->alloc_calls == c->fail_alloc_at) {
+    if (c->hook.fails()) {
         *ptr = nullptr;
         return fail(IMEXLB_E_OOM, "hipMalloc(" + std::to_string(bytes) + "): failure injected by IMEXLB_FAIL_ALLOC");
     }
