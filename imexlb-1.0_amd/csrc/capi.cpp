@@ -317,12 +317,30 @@ int imexlb_create(imexlb_ctx **out, int dim, int nx, int ny, int nz, int device,
                      : c->ssz == 2                    ? int64_t(8) << 20
                                                       : int64_t(5) << 19;
     if (std::getenv("IMEXLB_SMALL_CELLS")) c->multi_cells = c->small_cells;
-    const char *dv = std::getenv("IMEXLB_DOUBLE");
-    c->dbl_enabled = !(dv && dv[0] == '0');
     const char *mv = std::getenv("IMEXLB_MULTI");
     c->multi_enabled = !(mv && mv[0] == '0');
-    // rows of whole tiles where two steps are made per pass (k_double2)
-    if (device >= 0 && c->dbl_enabled && dim == 2 && int64_t(nx + 3) * (ny + 3) > c->small_cells) align = 64;
+    c->cells = int64_t(nx + 3) * (ny + 3) * (dim == 3 ? nz + 3 : 1);
+    // Two steps per pass (k_double2) take rows of whole tiles and populations
+    // that 32 bits address.  They pay from the width on where most of a strip
+    // of 256 columns does work and the frame beside it is a small part: us a
+    // step, single and two per pass, of 6 M cells (16 M): FP64 120 wide 180 and
+    // 174 (484 and 489), 190 168 and 147, 500 154 and 115; FP32 300 77 and 81,
+    // 380 77 and 71, 500 75 and 64; FP16, of which it takes those above 8 Mi cells,
+    // (640 110 and 120, 760 108 and 102, 1100 106 and 100, 2000 102 and 87); with
+    // stochastic rounding 640 48.2 and 51.1, 760 47.2 and 47.4, 2000 45.5 and
+    // 41.0; 20 wide 349 and 753, FP16 72 and 380.  IMEXLB_DOUBLE=1, and IMEXLB_SMALL_CELLS
+    // for lattices above it, take them at every width from 16 on.
+    const char *dv = std::getenv("IMEXLB_DOUBLE");
+    const bool everywhere = (dv && dv[0] == '1') || std::getenv("IMEXLB_SMALL_CELLS");
+    const int64_t tiles = (int64_t(nx) + 3 + 63) / 64 * 64;
+    c->dbl_enabled = !(dv && dv[0] == '0') && device >= 0 && dim == 2 && IMEXLB_TILE == 64 && nx >= 16 && ny >= 16 &&
+                     c->cells > c->small_cells &&
+                     (everywhere || nx >= (c->ssz == 8 ? 120 : c->ssz == 4 ? 360 : 720)) &&
+                     size_t(c->Q) * size_t(tiles * (ny + 3) + 128) * c->ssz < (size_t(1) << 32) - (size_t(1) << 16);
+    // Where several steps per launch are tried first, two per pass only serve
+    // the bodies that those do not suit: rows are padded for them if that adds
+    // at most a sixteenth.
+    if (c->dbl_enabled && !(c->multi_enabled && c->cells <= c->multi_cells && (tiles - nx - 3) * 16 > nx + 3)) align = 64;
     if (const char *av = std::getenv("IMEXLB_ROW_ALIGN")) align = std::max<int64_t>(1, std::atoll(av));
     if (align > 4096) return fail(IMEXLB_E_ARG, "IMEXLB_ROW_ALIGN above 4096 cells");
     c->Px = ((int64_t(nx) + 3 + align - 1) / align) * align;
@@ -374,7 +392,7 @@ int imexlb_create(imexlb_ctx **out, int dim, int nx, int ny, int nz, int device,
     // IMEXLB_XCD_REMAP=0/1/R overrides
     const char *xv = std::getenv("IMEXLB_XCD_REMAP");
     k.xcd_remap = xv ? uint32_t(std::max(0, std::atoi(xv)))
-                     : uint32_t(int64_t(k.ncell) <= c->small_cells);
+                     : uint32_t(c->cells <= c->small_cells);
 
     c->hook.read();
     if (device >= 0) {
@@ -450,23 +468,18 @@ int imexlb_set_params(imexlb_ctx *c, double ome, double rho0, double uu)
     return IMEXLB_OK;
 }
 
-static bool double_suits(const imexlb_ctx *c)
-{
-    return c->dim == 2 && IMEXLB_TILE == 64 && c->Px % 64 == 0 && c->kp.nx >= 16 && c->kp.ny >= 16 &&
-           size_t(c->Q) * size_t(c->plane) * c->ssz < (size_t(1) << 32) - (size_t(1) << 16) &&
-           int64_t(c->kp.ncell) > c->small_cells;
-}
-
 // The two-steps-per-pass plan of the new geometry: the frame's lists, the
 // bulk's marks in the node types, the scratch buffer.  A lattice it does not
 // suit, or without memory for it, keeps single steps.
 static int build_double(imexlb_ctx *c)
 {
     c->drop_double();
-    if (!c->dbl_enabled || !c->push_on || c->multi_on || !double_suits(c)) return IMEXLB_OK;
+    const size_t pop = size_t(c->Q) * size_t(c->plane) * c->ssz, n = size_t(c->plane);
+    if (!c->dbl_enabled || !c->push_on || c->multi_on || c->Px % 64 != 0 ||
+        pop >= (size_t(1) << 32) - (size_t(1) << 16))  // (IMEXLB_ROW_ALIGN)
+        return IMEXLB_OK;
     DoublePlan &d = c->dbl;
     DeviceTemp zones, counts;
-    const size_t pop = size_t(c->Q) * size_t(c->plane) * c->ssz, n = size_t(c->plane);
     const auto no_memory = [&] {
         c->drop_double();
         return IMEXLB_OK;
@@ -506,7 +519,7 @@ static int build_multi(imexlb_ctx *c, const DeviceTables &t)
 {
     c->drop_multi();
     if (!c->multi_enabled || !c->push_on || !c->fill32 || c->dim != 2 || IMEXLB_TILE != 64 ||
-        int64_t(c->kp.ncell) > c->multi_cells || !body_copies_zero(t))
+        c->cells > c->multi_cells || !body_copies_zero(t))
         return IMEXLB_OK;
     std::vector<MultiPlan> plans;
     plan_multi(int(c->ssz), {&c->kp}, plans);

@@ -322,14 +322,15 @@ struct imexlb_ctx {
     }
 
     // mode bits of the fused collide step for this lattice (K_SMALL in 2D and
-    // K_CACHED in 3D for lattices of at most small_cells padded cells)
+    // K_CACHED in 3D for lattices of at most small_cells cells)
     int collide_mode() const
     {
         if (!push_on) return K_COLLIDE;
         if (!fill32) return K_COLLIDE | K_PUSH | K_IDX64;
-        if (int64_t(kp.ncell) > small_cells) return K_COLLIDE | K_PUSH;
+        if (cells > small_cells) return K_COLLIDE | K_PUSH;
         return K_COLLIDE | K_PUSH | (dim == 2 ? K_SMALL : K_CACHED);
     }
+    int64_t cells = 0;        // with the ghost layer, without padding of rows
     int64_t small_cells = 0;  // set at creation (IMEXLB_SMALL_CELLS)
     int64_t multi_cells = 0;  // up to it several steps per launch
 
