@@ -490,35 +490,50 @@ __device__ __forceinline__ void st_px(float *p, const Px<K> &v)
     }
 }
 
-// Pooling and upsampling: a wave takes a low-resolution row of one channel
-// of one image, its place found once with scalar divisions (a 64-bit
-// division per value cost more than the memory access), two pixels per
-// thread with 8- and 16-byte accesses (A) where w is even and the buffers
-// are aligned, else one.  Bound by HBM: the three upsamplings of a training
-// step of 8 cases on 128 x 512 took 64 us each, now 18; the gradients with the
-// ReLU and the skip connection joined 19 and 22 us instead of 46 and 104 in
-// two and four launches.
+// Pooling and upsampling: a thread takes one low-resolution pixel of one
+// channel of one image, or two with 8- and 16-byte accesses (A) where w is even
+// and the buffers are aligned; their place by three 32-bit multiplications
+// (64-bit divisions cost more than the memory access).  Bound by HBM: the three
+// upsamplings of a training step of 8 cases on 128 x 512 take 45 us in all; 8 x
+// 64 channels of 64 x 256, gradients with the ReLU 29 us, joined with the skip
+// connection 76.  A wave per row, its place by scalar divisions, was as fast
+// from 128 columns on (78 us for the join, 64 columns 18 against 8) and idle on
+// narrow ones (40 x 256 of 64 x 4: 165 us against 11); it takes the calls whose
+// values 32 bits do not count.
+struct LowRes {
+    int N, C, h, w;
+    uint32_t items;  // threads with work; 0 where they are 2^31 or more
+    FastDiv per_row, rows, chans;
+};
 template <bool A, class F>
-__device__ __forceinline__ void for_rows(int N, int C, int h, int w, F f)
+__device__ __forceinline__ void for_values(const LowRes &g, F f)
 {
     constexpr int V = A ? 2 : 1;
-    const int64_t rows = int64_t(N) * C * h;
+    const auto div = [](uint32_t n, const FastDiv &d) { return (__umulhi(n, d.m) + n) >> d.s; };  // n < 2^31
+    if (g.items) {
+        const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+        if (i >= g.items) return;
+        const uint32_t r = div(i, g.per_row), nc = div(r, g.rows), n = div(nc, g.chans);
+        f(int64_t(n), int(nc - n * uint32_t(g.C)), int(r - nc * uint32_t(g.h)), int(i - r * uint32_t(g.w / V)) * V);
+        return;
+    }
+    const int64_t rows = int64_t(g.N) * g.C * g.h;
     for (int64_t r = int64_t(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x / 64); r < rows;
          r += int64_t(gridDim.x) * 4) {
-        const int64_t nc = r / h, n = nc / C;
-        const int y = int(r - nc * h), c = int(nc - n * C);
-        for (int x = int(threadIdx.x % 64) * V; x < w; x += 64 * V) f(n, c, y, x);
+        const int64_t nc = r / g.h, n = nc / g.C;
+        const int y = int(r - nc * g.h), c = int(nc - n * g.C);
+        for (int x = int(threadIdx.x % 64) * V; x < g.w; x += 64 * V) f(n, c, y, x);
     }
 }
 
 // 2x2 average pool of channels [coff, coff + C) of in [N][Ctot][2h][2w]
 // (in points at channel coff) into out [N][C][h][w]
 template <bool A>
-__global__ __launch_bounds__(256) void k_pool2(const float *__restrict__ in, int Ctot, float *__restrict__ out, int N,
-                                               int C, int h, int w)
+__global__ __launch_bounds__(256) void k_pool2(const float *__restrict__ in, int Ctot, float *__restrict__ out, LowRes lr)
 {
     constexpr int V = A ? 2 : 1;
-    for_rows<A>(N, C, h, w, [&](int64_t n, int c, int y, int x) {
+    const int C = lr.C, h = lr.h, w = lr.w;
+    for_values<A>(lr, [&](int64_t n, int c, int y, int x) {
         const float *p = in + ((n * Ctot + c) * 2 * h + 2 * y) * (2 * int64_t(w)) + 2 * x;
         const Px<2 * V> a = ld_px<A, 2 * V>(p), b = ld_px<A, 2 * V>(p + 2 * int64_t(w));
         Px<V> o;
@@ -534,11 +549,12 @@ __global__ __launch_bounds__(256) void k_pool2(const float *__restrict__ in, int
 template <bool A>
 __global__ __launch_bounds__(256) void k_pool2_bwd(const float *__restrict__ dout, const float *__restrict__ skip,
                                                    int stot, const float *__restrict__ gate, int gtot,
-                                                   float *__restrict__ din, int N, int C, int h, int w)
+                                                   float *__restrict__ din, LowRes lr)
 {
     constexpr int V = A ? 2 : 1;
+    const int C = lr.C, h = lr.h, w = lr.w;
     const int64_t W = 2 * int64_t(w);
-    for_rows<A>(N, C, h, w, [&](int64_t n, int c, int y, int x) {
+    for_values<A>(lr, [&](int64_t n, int c, int y, int x) {
         const Px<V> g = ld_px<A, V>(dout + ((n * C + c) * h + y) * int64_t(w) + x);
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
@@ -560,12 +576,12 @@ __global__ __launch_bounds__(256) void k_pool2_bwd(const float *__restrict__ dou
 // nearest 2x upsample: in [N][C][h][w] -> C channels of out [N][Ctot][2h][2w]
 // (out points at the first)
 template <bool A>
-__global__ __launch_bounds__(256) void k_up2(const float *__restrict__ in, float *__restrict__ out, int N, int C, int h,
-                                             int w, int Ctot)
+__global__ __launch_bounds__(256) void k_up2(const float *__restrict__ in, float *__restrict__ out, int Ctot, LowRes lr)
 {
     constexpr int V = A ? 2 : 1;
+    const int C = lr.C, h = lr.h, w = lr.w;
     const int64_t W = 2 * int64_t(w);
-    for_rows<A>(N, C, h, w, [&](int64_t n, int c, int y, int x) {
+    for_values<A>(lr, [&](int64_t n, int c, int y, int x) {
         const Px<V> v = ld_px<A, V>(in + ((n * C + c) * h + y) * int64_t(w) + x);
         Px<2 * V> o;
 #pragma unroll
@@ -580,10 +596,11 @@ __global__ __launch_bounds__(256) void k_up2(const float *__restrict__ in, float
 template <bool A>
 __global__ __launch_bounds__(256) void k_up2_bwd(const float *__restrict__ dout, int Ctot,
                                                  const float *__restrict__ gate, int gtot, float *__restrict__ din,
-                                                 int N, int C, int h, int w)
+                                                 LowRes lr)
 {
     constexpr int V = A ? 2 : 1;
-    for_rows<A>(N, C, h, w, [&](int64_t n, int c, int y, int x) {
+    const int C = lr.C, h = lr.h, w = lr.w;
+    for_values<A>(lr, [&](int64_t n, int c, int y, int x) {
         const float *p = dout + ((n * Ctot + c) * 2 * h + 2 * y) * (2 * int64_t(w)) + 2 * x;
         const Px<2 * V> a = ld_px<A, 2 * V>(p), b = ld_px<A, 2 * V>(p + 2 * int64_t(w));
         Px<V> o, t;
@@ -1061,17 +1078,28 @@ __global__ void k_up2_bf16(const uint4 *__restrict__ in, uint4 *__restrict__ out
 
 inline unsigned blocks(int64_t n) { return unsigned((n + 255) / 256); }
 
-// blocks of a kernel that walks rows (four per block, at most 2^20 blocks)
-inline dim3 row_blocks(int N, int C, int h)
-{
-    return dim3(unsigned(std::min<int64_t>((int64_t(N) * C * h + 3) / 4, int64_t(1) << 20)));
-}
 // the buffers of a pooling or upsampling call take 8- and 16-byte accesses
 inline bool vec_ok(int w, std::initializer_list<const void *> ptrs)
 {
     uintptr_t bits = 0;
     for (const void *p : ptrs) bits |= reinterpret_cast<uintptr_t>(p);
     return w % 2 == 0 && bits % 16 == 0;
+}
+template <class K, class... Args>
+int launch_low_res(bool wide, K aligned, K plain, int N, int C, int h, int w, void *stream, Args... args)
+{
+    LowRes g{N, C, h, w, 0, {}, {}, {}};
+    const int per_row = wide ? w / 2 : w;
+    const int64_t rows = int64_t(N) * C * h;
+    if (rows <= 0x7fffffff / per_row) {
+        g.items = uint32_t(rows * per_row);
+        g.per_row.init(uint32_t(per_row));
+        g.rows.init(uint32_t(h));
+        g.chans.init(uint32_t(C));
+    }
+    const unsigned nb = g.items ? blocks(g.items) : unsigned(std::min<int64_t>((rows + 3) / 4, int64_t(1) << 20));
+    hipLaunchKernelGGL(wide ? aligned : plain, dim3(nb), dim3(256), 0, (hipStream_t)stream, args..., g);
+    return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
 // the convolution's tile for these sizes and its launch
@@ -1282,8 +1310,7 @@ int imexlb_nn_pool2_from(const float *in, int Ctot, int coff, float *out, int N,
 {
     if (!in || !out || N <= 0 || C <= 0 || h <= 0 || w <= 0 || coff < 0 || coff + C > Ctot) return -1;
     in += int64_t(coff) * 4 * h * w;
-    NN_LAUNCH(vec_ok(w, {in, out}) ? k_pool2<true> : k_pool2<false>, row_blocks(N, C, h), dim3(256), 0,
-              (hipStream_t)stream, in, Ctot, out, N, C, h, w);
+    return launch_low_res(vec_ok(w, {in, out}), k_pool2<true>, k_pool2<false>, N, C, h, w, stream, in, Ctot, out);
 }
 
 int imexlb_nn_pool2(const float *in, float *out, int N, int C, int h, int w, void *stream)
@@ -1300,8 +1327,8 @@ int imexlb_nn_pool2_bwd_join(const float *dout, const float *skip, int stotal, i
     const int64_t hw = int64_t(4) * h * w;
     if (skip) skip += soff * hw;
     if (gate) gate += goff * hw;
-    NN_LAUNCH(vec_ok(w, {dout, skip, gate, din}) ? k_pool2_bwd<true> : k_pool2_bwd<false>, row_blocks(N, C, h),
-              dim3(256), 0, (hipStream_t)stream, dout, skip, stotal, gate, gtotal, din, N, C, h, w);
+    return launch_low_res(vec_ok(w, {dout, skip, gate, din}), k_pool2_bwd<true>, k_pool2_bwd<false>, N, C, h, w, stream,
+                          dout, skip, stotal, gate, gtotal, din);
 }
 
 int imexlb_nn_pool2_bwd(const float *dout, float *din, int N, int C, int h, int w, void *stream)
@@ -1313,8 +1340,7 @@ int imexlb_nn_up2(const float *in, float *out, int N, int C, int h, int w, int C
 {
     if (!in || !out || N <= 0 || C <= 0 || h <= 0 || w <= 0 || coff < 0 || coff + C > Ctot) return -1;
     out += int64_t(coff) * 4 * h * w;
-    NN_LAUNCH(vec_ok(w, {in, out}) ? k_up2<true> : k_up2<false>, row_blocks(N, C, h), dim3(256), 0,
-              (hipStream_t)stream, in, out, N, C, h, w, Ctot);
+    return launch_low_res(vec_ok(w, {in, out}), k_up2<true>, k_up2<false>, N, C, h, w, stream, in, out, Ctot);
 }
 
 int imexlb_nn_up2_bwd_gate(const float *dout, int Ctot, int coff, const float *gate, int gtotal, int goff, float *din,
@@ -1325,8 +1351,8 @@ int imexlb_nn_up2_bwd_gate(const float *dout, int Ctot, int coff, const float *g
         return -1;
     dout += int64_t(coff) * 4 * h * w;
     if (gate) gate += int64_t(goff) * h * w;
-    NN_LAUNCH(vec_ok(w, {dout, gate, din}) ? k_up2_bwd<true> : k_up2_bwd<false>, row_blocks(N, C, h), dim3(256), 0,
-              (hipStream_t)stream, dout, Ctot, gate, gtotal, din, N, C, h, w);
+    return launch_low_res(vec_ok(w, {dout, gate, din}), k_up2_bwd<true>, k_up2_bwd<false>, N, C, h, w, stream, dout, Ctot,
+                          gate, gtotal, din);
 }
 
 int imexlb_nn_up2_bwd(const float *dout, float *din, int N, int C, int h, int w, int Ctot, int coff, void *stream)

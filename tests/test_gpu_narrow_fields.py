@@ -1,0 +1,50 @@
+"""The network's kernels on fields of few columns: the same results, and no
+slower per value than on wide ones."""
+import ctypes as C
+
+import pytest
+
+import test_gpu_nn_kernels as K
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("shape", [(2, 3, 7, 2), (3, 5, 11, 4), (2, 7, 3, 6), (1, 2, 300, 1), (2, 2, 2, 128),
+                                   (5, 3, 2, 130), (1, 1, 70, 3)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_pooling_and_upsampling_of_narrow_fields(shape, shift):
+    K.test_pooling_and_upsampling(shape, shift)
+
+
+def _time(f, repeat=20):
+    import torch
+    for _ in range(3):
+        f()
+    best = 1e9
+    for _ in range(5):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(repeat):
+            f()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) / repeat)
+    return best
+
+
+@pytest.mark.parametrize("call", ["pool2", "pool2_bwd", "up2", "up2_bwd"])
+def test_narrow_fields_take_the_time_of_wide_ones(call):
+    """40 x 256 fields of 64 x 4 and of 4 x 64 pixels, the same values: up to
+    19 times slower where a wave took a row."""
+    import torch
+    from imexlb._lib import lib
+    ms = []
+    for h, w in ((4, 64), (64, 4)):
+        low = torch.zeros((40, 256, h, w), device="cuda")
+        high = torch.zeros((40, 256, 2 * h, 2 * w), device="cuda")
+        a, b = (high, low) if call in ("pool2", "up2_bwd") else (low, high)
+        args = (40, 256, h, w) + ((256, 0) if call.startswith("up2") else ())
+        f = getattr(lib(), "imexlb_nn_" + call)
+        ms.append(_time(lambda: f(C.c_void_p(a.data_ptr()), C.c_void_p(b.data_ptr()), *args, None)))
+    print(f"[narrow] {call}: {ms[0] * 1e3:.1f} us wide, {ms[1] * 1e3:.1f} us narrow", flush=True)
+    assert ms[1] < 3.0 * ms[0], ms
