@@ -1451,11 +1451,19 @@ int imexlb_nn_conv3x3_bf16_join(const uint16_t *low, int CL, const uint16_t *in,
     const bool wide = CI % 32 == 0 && CL % 32 == 0;
 #define CONV_BF16(MT, WY, TC) (wide ? k_conv3_bf16<MT, WY, TC, 32> : k_conv3_bf16<MT, WY, TC, 16>)
 #define CONV_BF16_DEEP(TC) (wide ? k_conv3_bf16_deep<TC, 32> : k_conv3_bf16_deep<TC, 16>)
+    // Rows of at most 16 pixels: three chunks ahead up to a block per CU, and of
+    // many input channels somewhat above (us, ahead and plain, blocks: 32
+    // channels 6.8 and 6.7 at 208, 13.8 and 8.2 at 800; 128 7.2 and 10.2 at 208,
+    // 11.6 and 11.6 at 320, 21.9 and 17.7 at 800; 512 40 and 43 at 640).
     if (W <= 16)
-        return count(8, 16, 32) < 1024 ? run(CONV_BF16_DEEP(16), 8, 16, 32) : run(CONV_BF16(1, 4, 16), 8, 16, 32);
+        return count(8, 16, 32) <= std::max<int64_t>(256, (int64_t(CL) + CI) * 5 / 2) ? run(CONV_BF16_DEEP(16), 8, 16, 32)
+                                                                                 : run(CONV_BF16(1, 4, 16), 8, 16, 32);
     if (COP % 64 == 0 && count(8, 32, 64) >= 512) return run(CONV_BF16(4, 2, 32), 8, 32, 64);
     if (CL + CI <= 32 && count(16, 32, 32) >= 512) return run(k_conv3_bf16<4, 4, 32, 16>, 16, 32, 32);
     if (count(8, 32, 32) >= 512) return run(CONV_BF16(2, 4, 32), 8, 32, 32);
+    // (one or two chunks in more blocks than CUs: 40 x 64 x 24, 32 -> 16 channels
+    // 11.0 and, plain, 7.1 us; 8 x 128 x 48, 64 -> 32 10.1 and 8.8)
+    if (wide && CL + CI <= 64 && count(4, 32, 32) > 256) return run(CONV_BF16(2, 4, 32), 8, 32, 32);
     return run(CONV_BF16_DEEP(32), 4, 32, 32);
 #undef CONV_BF16_DEEP
 #undef CONV_BF16

@@ -48,3 +48,27 @@ def test_narrow_fields_take_the_time_of_wide_ones(call):
         ms.append(_time(lambda: f(C.c_void_p(a.data_ptr()), C.c_void_p(b.data_ptr()), *args, None)))
     print(f"[narrow] {call}: {ms[0] * 1e3:.1f} us wide, {ms[1] * 1e3:.1f} us narrow", flush=True)
     assert ms[1] < 3.0 * ms[0], ms
+
+
+# one block a CU and fewer (three chunks ahead), somewhat more with many input
+# channels, more with few (plain); rows of more than 16 pixels with one chunk
+@pytest.mark.parametrize("shape", [(20, 32, 70, 40, 8), (20, 128, 70, 40, 8), (20, 16, 70, 41, 5), (40, 32, 16, 64, 24),
+                                   (7, 64, 40, 61, 33)])
+def test_bf16_convolution_of_narrow_fields(shape):
+    """Against the exact sums, and every image equal to itself alone, which
+    few blocks compute: the tile does not change the sums."""
+    import torch
+    K.test_bf16_convolution_at_tile_edges(shape)
+    N, ci, co, H, W = shape
+    g = torch.Generator("cuda").manual_seed(17)
+    x = torch.randn(N, H, W, ci, generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn(co, ci, 3, 3, generator=g, device="cuda")
+    cop = 32 * -(-co // 32)
+    wp = torch.empty(ci * 9 * cop, dtype=torch.bfloat16, device="cuda")
+    K._call("pack_weights_bf16", w, wp, ci, co, ci, cop)
+    out = torch.empty(N, co, H, W, device="cuda")
+    K._call("conv3x3_bf16", x, wp, torch.zeros(co, device="cuda"), out, N, ci, co, cop, H, W, 0, 0, 1, 1)
+    one = torch.empty(1, co, H, W, device="cuda")
+    for k in (0, N - 1):
+        K._call("conv3x3_bf16", x[k].contiguous(), wp, torch.zeros(co, device="cuda"), one, 1, ci, co, cop, H, W, 0, 0, 1, 1)
+        assert torch.equal(one[0], out[k]), k
