@@ -99,7 +99,8 @@ struct DeviceTemp {  // freed on every return
 };
 
 // The interior of padded device arrays to dense host arrays, after the work on
-// the stream; false if there is no memory for the buffers (nothing was copied).
+// the stream; false if there is no memory for the buffers, or the fields are
+// small enough for a plain copy (nothing was copied).
 bool download_interior(Staging &s, int device, hipStream_t stream, int dim, const KParams &kp,
                        const std::vector<FieldCopy> &fields, hipError_t &err);
 

@@ -6,7 +6,8 @@
 // caller's fresh pages (8193 x 2049: 81 ms for 403 MB).  Here a kernel writes
 // runs of interior values straight into pinned buffers, and a few threads, each
 // with a buffer of its own, copy them out while the next runs arrive: 11.5 ms
-// (35 GB/s); 513 x 129 x 129 49 to 8.4 ms, 401 x 101 0.52 to 0.10 ms.
+// (35 GB/s); 513 x 129 x 129 49 to 8.4 ms, 401 x 101 0.52 to 0.10 ms.  Small
+// fields keep the single copy.
 #include "context.hpp"
 
 #include <algorithm>
@@ -59,6 +60,11 @@ bool download_interior(Staging &s, int device, hipStream_t stream, int dim, cons
     constexpr int64_t kRun = int64_t(256) << 10, kLeast = int64_t(48) << 10;
     err = hipSuccess;
     const int64_t n = kp.N, total = n * int64_t(fields.size());
+    // Few values: the whole padded arrays through a vector cost less than
+    // launches and events (us, 61 x 61 34 and 45, 17 x 17 x 17 48 and 59, 151 x
+    // 151 62 and 64, 181 x 181 79 and 76), but not copies of up to 16 KiB, which
+    // the runtime makes in 23 us each instead of 11 (41 x 41 68 and 44).
+    if (kp.plane * int64_t(sizeof(double)) > (int64_t(16) << 10) && total < (int64_t(80) << 10)) return false;
     const int64_t cores = std::max(1u, std::thread::hardware_concurrency());
     const int workers = int(std::clamp<int64_t>(total / (2 * kLeast), 1, std::min<int64_t>(Staging::kWorkers, cores)));
     const int64_t run = std::min(kRun, std::max(kLeast, (total + 2 * workers - 1) / (2 * workers)));
