@@ -69,7 +69,10 @@ constexpr int CIB = 8;  // input channels per LDS chunk
 // transposed -- the data gradient of a layer from CO to CI channels -- and,
 // with a gate (gtotal channels per image), the value is kept only where the
 // gate is positive: the ReLU of the layer before.
-template <int MT, int NT, int TC, bool DGRAD>
+// FEW: at most 6 input channels, whose missing pairs are left out (8 x 512 x
+// 512: 1 -> 1 channels 100 to 58 us, 4 -> 1 99 to 73; the test costs the others
+// 3 %, the products being scheduled pair by pair).
+template <int MT, int NT, int TC, bool DGRAD, bool FEW>
 __global__ __launch_bounds__(256) void k_conv3(const float *__restrict__ in, const float *__restrict__ w,
                                                const float *__restrict__ bias, float *__restrict__ out, int ototal,
                                                const float *__restrict__ gate, int gtotal, int CI, int CO, int H, int W,
@@ -174,6 +177,7 @@ __global__ __launch_bounds__(256) void k_conv3(const float *__restrict__ in, con
         fetch(0, a[0], b[0]);
 #pragma unroll
         for (int k2 = 0; k2 < CIB * 9 / 2; ++k2) {
+            if (FEW && k2 % 9 == 0 && k2 * 2 >= CI * 9) break;  // (pairs of channels past the last)
             if (k2 + 1 < CIB * 9 / 2) fetch(k2 + 1, a[(k2 + 1) % 2], b[(k2 + 1) % 2]);
 #pragma unroll
             for (int s = 0; s < NT; ++s)
@@ -1120,10 +1124,14 @@ int launch_conv(const float *in, const float *w, const float *bias, float *out, 
                            gtotal, CI, CO, H, W, relu, uint32_t(tx), uint32_t(ty), uint32_t(tc));
         return hipGetLastError() == hipSuccess ? 0 : -2;
     };
-    if (W <= 16) return run(k_conv3<1, 1, 16, DGRAD>, 8, 16, 32, true);
-    int rc = CO > 32 ? run(k_conv3<2, 2, 32, DGRAD>, 8, 32, 64, false) : 1;
-    if (rc > 0) rc = run(k_conv3<2, 1, 32, DGRAD>, 8, 32, 32, false);
-    return rc <= 0 ? rc : run(k_conv3<1, 1, 32, DGRAD>, 4, 32, 32, true);
+    const auto tile = [&](auto few) {
+        constexpr bool F = decltype(few)::value;
+        if (W <= 16) return run(k_conv3<1, 1, 16, DGRAD, F>, 8, 16, 32, true);
+        int rc = CO > 32 ? run(k_conv3<2, 2, 32, DGRAD, F>, 8, 32, 64, false) : 1;
+        if (rc > 0) rc = run(k_conv3<2, 1, 32, DGRAD, F>, 8, 32, 32, false);
+        return rc <= 0 ? rc : run(k_conv3<1, 1, 32, DGRAD, F>, 4, 32, 32, true);
+    };
+    return CI <= 6 ? tile(std::true_type{}) : tile(std::false_type{});
 }
 
 // weight gradient: the tiles' sums to `work` and from there to dw in tile
