@@ -699,6 +699,13 @@ int imexlb_batch_tune(imexlb_batch *b, int trial_steps, int32_t best[3], double 
                 if (x) (void)hipEventDestroy(x);
         }
     } ev;
+    // the shapes are those of single steps
+    struct Single {
+        imexlb_batch *b;
+        const bool multi;
+        ~Single() { b->multi_on = multi; }
+    } single{b, b->multi_on};
+    b->multi_on = false;
     HIP_TRY(hipEventCreate(&ev.e[0]));
     HIP_TRY(hipEventCreate(&ev.e[1]));
     double bms = 1e300;

@@ -5,7 +5,9 @@
 generates the cases (Nx = 4*U{64..256}, Ny = Nx/4, radius = Ny/10, Re
 log-uniform in [40, 400], inlet velocity 0.05, body at x = 0.2 Nx), tunes the
 step-kernel shape, and reports the aggregate MLUPS of the batch against the
-same cases run one after another as single lattices.
+same cases run one after another as single lattices.  The shape is that of the
+single-step kernel; "form" tells how many steps a launch makes where all the
+cases suit several (IMEXLB_MULTI=0: single steps).
 """
 from __future__ import annotations
 
@@ -198,8 +200,9 @@ def main(argv=None):
     t_batch = time.perf_counter() - t0
     F = b.forces()
     _, diverged = b.monitor()
+    form = b.step_form()
     b.close()
-    out = {"cases": a.cases, "nodes": nodes, "precision": a.precision, "tuned": best,
+    out = {"cases": a.cases, "nodes": nodes, "precision": a.precision, "tuned": best, "form": form,
            "batch_steps": a.steps, "batch_s": round(t_batch, 3),
            "batch_MLUPS": round(nodes * a.steps / t_batch / 1e6, 1),
            "nonfinite_cases": int(diverged.size), "diverged": diverged.tolist(),

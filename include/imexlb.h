@@ -261,12 +261,13 @@ int imexlb_batch_init_fields_f32(imexlb_batch *b, const float *fields, int H, in
 int imexlb_batch_body_mask_f32(imexlb_batch *b, float *out, int H, int W, int64_t stride);
 /* nsteps complete iterations of every case. */
 int imexlb_batch_advance(imexlb_batch *b, int64_t nsteps);
-/* Step-kernel shape: threads per block (64, 128, 256, 512), nodes per
- * thread (1, 2, 4), persistent blocks taking tiles from a queue (1) or one
- * block per tile (0).  Results do not depend on it. */
+/* Shape of the single-step kernel: threads per block (64, 128, 256, 512),
+ * nodes per thread (1, 2, 4), persistent blocks taking tiles from a queue (1)
+ * or one block per tile (0).  Results do not depend on it, nor do the steps
+ * that imexlb_batch_advance makes several per launch. */
 int imexlb_batch_set_config(imexlb_batch *b, int block, int cells_per_thread, int persistent);
-/* Times every shape over trial_steps steps (advancing the ensemble) and
- * keeps the fastest; best = (block, cells_per_thread, persistent). */
+/* Times every shape over trial_steps single steps (advancing the ensemble)
+ * and keeps the fastest; best = (block, cells_per_thread, persistent). */
 int imexlb_batch_tune(imexlb_batch *b, int trial_steps, int32_t best[3], double *best_ms_per_step);
 /* Waits for every step queued on the batch's stream. */
 int imexlb_batch_synchronize(imexlb_batch *b);
