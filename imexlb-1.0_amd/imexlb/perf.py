@@ -6,17 +6,18 @@
 
 For each (workload, form): set up the lattice on device 0, warm up, time
 ``--timed-steps`` steps launch by launch with HIP events (the average
-duration of the fused step kernel), then advance for about ``--seconds`` of
-GPU time the ordinary way (graph replay of step pairs) for MLUPS over the
-wall clock.  One JSON line per case: MLUPS, the kernel's average duration,
-and the algorithmic HBM rate of that kernel,
-2*Q*s bytes per node update (s = bytes per stored population), against the
-MI355X peak of 8000 GB/s.  Lattices that fit in the 256 MB last-level cache
+duration of a step in the fused kernels), then advance for about
+``--seconds`` of GPU time the ordinary way (graph replay) for MLUPS over the
+wall clock.  One JSON line per case: MLUPS, the step's average duration,
+how many steps a pass over the lattice makes, and the algorithmic HBM rate,
+2*Q*s bytes per node and pass (s = bytes per stored population; a pass reads
+and writes every population once, whatever number of steps it makes), against
+the MI355X peak of 8000 GB/s.  Lattices that fit in the 256 MB last-level cache
 (the 400x100 cylinder) are launch-bound, not HBM-bound; their GB/s is
 reported for completeness.
 
 --no-graphs launches every step on its own (IMEXLB_GRAPHS=0) instead of
-replaying captured step pairs: the form used under a profiler's kernel
+replaying captured ones: the form used under a profiler's kernel
 trace, where every launch then appears as its own dispatch.
 """
 from __future__ import annotations
@@ -36,6 +37,12 @@ from .lattice import setup
 HBM_PEAK_GBS = 8000.0
 FORMS = {"f64": (_lib.F64, 8), "f32": (_lib.F32, 4), "f16_f32": (_lib.F16_F32, 2), "bf16_f32": (_lib.BF16_F32, 2),
          "bf16sr_f32": (_lib.BF16SR_F32, 2)}
+
+
+def bytes_per_update(Q, s, steps_per_pass):
+    """Bytes that a node update cannot do without: a pass reads and writes
+    the Q populations of s bytes once."""
+    return 2 * Q * s / steps_per_pass
 
 
 def measure(deck_name, form, seconds=2.0, timed_steps=200, seed=2021):
@@ -64,15 +71,18 @@ def measure(deck_name, form, seconds=2.0, timed_steps=200, seed=2021):
     lat.synchronize()
     wall = time.perf_counter() - t0
     um = lat.monitor()
+    how = lat.step_form()
     lat.close()
     k_ms = ms[0] / max(launches[0], 1)
-    gbps = n * 2 * Q * s / (k_ms * 1e-3) / 1e9
+    per_update = bytes_per_update(Q, s, how["steps_per_pass"])
+    gbps = n * per_update / (k_ms * 1e-3) / 1e9
     return {"workload": deck_name, "form": form, "nodes": n, "steps": steps,
             "MLUPS": round(n * steps / wall / 1e6, 1),
             "ms_per_step": round(wall / steps * 1e3, 5),
             "timed_steps": timed_steps, "fused_kernel_ms": round(k_ms, 5),
             "fill_kernel_ms": round(ms[1] / max(launches[1], 1), 5),
-            "algorithmic_bytes_per_update": 2 * Q * s, "achieved_GBps": round(gbps, 1),
+            "steps_per_pass": how["steps_per_pass"], "window": how["window"],
+            "algorithmic_bytes_per_update": round(per_update, 3), "achieved_GBps": round(gbps, 1),
             "frac_of_peak": round(gbps / HBM_PEAK_GBS, 4), "umax": um}
 
 
