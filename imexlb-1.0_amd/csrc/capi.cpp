@@ -475,7 +475,7 @@ static int build_double(imexlb_ctx *c)
 {
     c->drop_double();
     const size_t pop = size_t(c->Q) * size_t(c->plane) * c->ssz, n = size_t(c->plane);
-    if (!c->dbl_enabled || !c->push_on || c->multi_on || c->Px % 64 != 0 ||
+    if (!c->dbl_enabled || !c->push_on || !c->fill32 || c->multi_on || c->Px % 64 != 0 ||
         pop >= (size_t(1) << 32) - (size_t(1) << 16))  // (IMEXLB_ROW_ALIGN)
         return IMEXLB_OK;
     DoublePlan &d = c->dbl;
@@ -495,20 +495,19 @@ static int build_double(imexlb_ctx *c)
     const StepArgs a = c->args();
     // special nodes, the second step's frame (one node around them), the
     // first step's (one more)
-    HIP_TRY(launch_zone(c->dim, 0, a, c->geo, nullptr, z, nullptr, nullptr, 0, nullptr));
-    HIP_TRY(launch_zone(c->dim, 1, a, c->geo, z, z + n, nullptr, nullptr, 0, nullptr));
-    HIP_TRY(launch_zone(c->dim, 1, a, c->geo, z + n, z + 2 * n, nullptr, nullptr, 0, nullptr));
+    HIP_TRY(launch_zone(0, a, c->geo, nullptr, z, nullptr, nullptr, 0, nullptr));
+    HIP_TRY(launch_zone(1, a, c->geo, z, z + n, nullptr, nullptr, 0, nullptr));
+    HIP_TRY(launch_zone(1, a, c->geo, z + n, z + 2 * n, nullptr, nullptr, 0, nullptr));
     for (int k = 0; k < 2; ++k)
-        HIP_TRY(launch_zone(c->dim, 2, a, c->geo, z + (2 - k) * n, nullptr, cnt + k, nullptr, k, nullptr));
+        HIP_TRY(launch_zone(2, a, c->geo, z + (2 - k) * n, nullptr, cnt + k, nullptr, k, nullptr));
     HIP_TRY(hipMemcpy(d.count, cnt, sizeof(d.count), hipMemcpyDeviceToHost));
     for (int k = 0; k < 2; ++k) {
         if (!c->dbl_mem.get(c->hook, (void **)&d.list[k], std::max<size_t>(d.count[k], 1) * sizeof(uint32_t)))
             return no_memory();
-        HIP_TRY(launch_zone(c->dim, 2, a, c->geo, z + (2 - k) * n, nullptr, cnt + 2 + k, d.list[k], 0, nullptr));
+        HIP_TRY(launch_zone(2, a, c->geo, z + (2 - k) * n, nullptr, cnt + 2 + k, d.list[k], 0, nullptr));
     }
     HIP_TRY(hipDeviceSynchronize());
-    d.idx64 = !c->fill32;
-    plan_double(c->dim, int(c->ssz), c->kp, d);
+    plan_double(int(c->ssz), c->kp, d);
     c->dbl_on = true;
     return IMEXLB_OK;
 }
@@ -1004,7 +1003,7 @@ static int run_double_steps(imexlb_ctx *c, int A, int64_t n, int64_t *done)
             StepArgs a = c->args();
             a.src = c->fb[A ^ int(k & 1)];
             a.dst = c->fb[A ^ 1 ^ int(k & 1)];
-            int rc = c->launch(0, [&] { return launch_double(c->dim, c->prec, a, c->dbl, c->stream); }, 2);
+            int rc = c->launch(0, [&] { return launch_double(c->prec, a, c->dbl, c->stream); }, 2);
             if (rc) return rc;
         }
         return IMEXLB_OK;
@@ -1014,7 +1013,7 @@ static int run_double_steps(imexlb_ctx *c, int A, int64_t n, int64_t *done)
         if (reps <= 0) continue;
         hipGraphExec_t &g = c->quad_graph[j][A];
         int rc = capture_passes(c, 2 * imexlb_ctx::kQuads[j], A, g,
-                                [&](const StepArgs &a) { return launch_double(c->dim, c->prec, a, c->dbl, c->stream); });
+                                [&](const StepArgs &a) { return launch_double(c->prec, a, c->dbl, c->stream); });
         if (rc) return rc;
         for (int64_t k = 0; k < reps; ++k) HIP_TRY(hipGraphLaunch(g, c->stream));
         quads -= reps * imexlb_ctx::kQuads[j];

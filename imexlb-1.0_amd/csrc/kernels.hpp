@@ -161,7 +161,6 @@ struct DoublePlan {
     uint32_t *list[2] = {nullptr, nullptr};
     uint32_t count[2] = {0, 0};
     void *scratch = nullptr;
-    bool idx64 = false;  // the push table's slots are int64
     uint32_t strips = 0, segments = 0;
     int rows = 0;
 };
@@ -176,13 +175,13 @@ hipError_t launch_batch_multi(int prec, const MultiPlan &m, const void *src, voi
                               bool copies, hipStream_t s);
 // copies: also the boundary copies of the last step
 hipError_t launch_multi(int prec, const StepArgs &a, const MultiPlan &m, int steps, bool copies, hipStream_t s);
-void plan_double(int dim, int bytes, const KParams &kp, DoublePlan &d);
-hipError_t launch_double(int dim, int prec, const StepArgs &a, const DoublePlan &d, hipStream_t s);
+void plan_double(int bytes, const KParams &kp, DoublePlan &d);
+hipError_t launch_double(int prec, const StepArgs &a, const DoublePlan &d, hipStream_t s);
 // passes that find the frame: 0 special nodes to out; 1 in grown by a node to
 // out; 2 the nodes marked in `in` appended to list (nullptr: counted), the
 // others marked G_BULK in geo with bulk
-hipError_t launch_zone(int dim, int pass, const StepArgs &a, uint8_t *geo, const uint8_t *in, uint8_t *out,
-                       uint32_t *count, uint32_t *list, int bulk, hipStream_t s);
+hipError_t launch_zone(int pass, const StepArgs &a, uint8_t *geo, const uint8_t *in, uint8_t *out, uint32_t *count,
+                       uint32_t *list, int bulk, hipStream_t s);
 
 // prec: 0 FP64, 1 FP32, 2 FP16 storage + FP32 arithmetic, 3 BF16 storage + FP32 arithmetic
 hipError_t launch_step(int dim, int prec, int mode, const StepArgs &a, hipStream_t s);

@@ -1006,7 +1006,7 @@ constexpr int kStripX = 256;          // columns a block of k_double2 writes
 constexpr int kDouble2 = kStripX + 64;  // its threads: one more wave for the columns beside the strip
 
 // One step of the cells of a list.
-template <int D, class S, class C, int MODE>
+template <class S, class C>
 __global__ __launch_bounds__(256) void k_step_list(const S *__restrict__ src, S *__restrict__ dst,
                                                    const uint8_t *__restrict__ geo, KParams kp, PushTable pt,
                                                    const uint32_t *__restrict__ list, uint32_t n)
@@ -1015,8 +1015,8 @@ __global__ __launch_bounds__(256) void k_step_list(const S *__restrict__ src, S 
     if (i >= n) return;
     int x, y, z;
     uint32_t c;
-    if (!decode_cell<D>(kp, list[i], x, y, z, c)) return;
-    step_node<D, S, C, MODE>(src, dst, nullptr, nullptr, nullptr, nullptr, nullptr, geo, kp, x, y, z, c, pt);
+    if (!decode_cell<2>(kp, list[i], x, y, z, c)) return;
+    step_node<2, S, C, K_COLLIDE | K_PUSH>(src, dst, nullptr, nullptr, nullptr, nullptr, nullptr, geo, kp, x, y, z, c, pt);
 }
 
 // Two steps of the bulk of a D2Q9 lattice.  A block takes a strip of columns
@@ -1159,39 +1159,36 @@ __global__ __launch_bounds__(kDouble2) void k_double2(const S *__restrict__ src,
 // Zones of a lattice, one byte per padded cell.  k_zone_special: interior
 // nodes whose step is more than a pull from fluid neighbours -- solid, next
 // to a solid or ghost cell, or the source of boundary copies.
-template <int D>
 __global__ __launch_bounds__(256) void k_zone_special(const uint8_t *__restrict__ geo, uint8_t *__restrict__ out,
                                                       KParams kp)
 {
     int x, y, z;
     uint32_t c;
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (!decode_cell<D>(kp, i, x, y, z, c)) return;
+    if (!decode_cell<2>(kp, i, x, y, z, c)) return;
     bool plain = !(geo[c] & G_PUSH);
 #pragma unroll
-    for (int q = 0; q < Lat<D>::Q; ++q) plain &= (geo[c - shift32<D>(kp, q)] & G_FLUID) != 0;
+    for (int q = 0; q < Lat<2>::Q; ++q) plain &= (geo[c - shift32<2>(kp, q)] & G_FLUID) != 0;
     out[c] = plain ? 0 : 1;
 }
 
 // out: interior nodes with a marked neighbour (or marked themselves)
-template <int D>
 __global__ __launch_bounds__(256) void k_zone_grow(const uint8_t *__restrict__ in, uint8_t *__restrict__ out,
                                                    KParams kp)
 {
     int x, y, z;
     uint32_t c;
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (!decode_cell<D>(kp, i, x, y, z, c)) return;
+    if (!decode_cell<2>(kp, i, x, y, z, c)) return;
     uint8_t any = 0;
 #pragma unroll
-    for (int q = 0; q < Lat<D>::Q; ++q) any |= in[c - shift32<D>(kp, q)];
+    for (int q = 0; q < Lat<2>::Q; ++q) any |= in[c - shift32<2>(kp, q)];
     out[c] = any;
 }
 
 // The marked cells with work (fluid, or body cells that copy) as a list: a
 // wave appends its 64 cells' in order (list == nullptr: counts only).  With
 // bulk the unmarked interior cells get G_BULK.
-template <int D>
 __global__ __launch_bounds__(256) void k_zone_list(const uint8_t *__restrict__ mark, uint8_t *__restrict__ geo,
                                                    KParams kp, int bulk, uint32_t *__restrict__ count,
                                                    uint32_t *__restrict__ list)
@@ -1199,7 +1196,7 @@ __global__ __launch_bounds__(256) void k_zone_list(const uint8_t *__restrict__ m
     int x, y, z;
     uint32_t c;
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    const bool in = decode_cell<D>(kp, i, x, y, z, c);
+    const bool in = decode_cell<2>(kp, i, x, y, z, c);
     const bool take = in && mark[c] && (geo[c] & (G_FLUID | G_PUSH));
     const uint64_t m = __ballot(take);
     uint32_t base = 0;
@@ -1892,46 +1889,23 @@ hipError_t launch_step(int dim, int prec, int mode, const StepArgs &a, hipStream
     return dim == 2 ? step_d<2>(prec, mode, a, s) : step_d<3>(prec, mode, a, s);
 }
 
-template <int D, int MODE>
-static hipError_t list_dm(int prec, const StepArgs &a, const uint32_t *list, uint32_t n, hipStream_t s)
+hipError_t launch_double(int prec, const StepArgs &a, const DoublePlan &d, hipStream_t s)
 {
     return dispatch_prec(prec, [&](auto *sp, auto *cp) {
         using S = std::remove_pointer_t<decltype(sp)>;
         using C = std::remove_pointer_t<decltype(cp)>;
-        hipLaunchKernelGGL((k_step_list<D, S, C, MODE>), dim3(nblocks(n)), dim3(256), 0, s, (const S *)a.src,
-                           (S *)a.dst, a.geo, a.kp, a.push, list, n);
-        return hipGetLastError();
-    });
-}
-
-static hipError_t launch_step_list(int dim, int prec, bool idx64, const StepArgs &a, const uint32_t *list, uint32_t n,
-                                   hipStream_t s)
-{
-    constexpr int M = K_COLLIDE | K_PUSH, M64 = M | K_IDX64;
-    if (n == 0) return hipSuccess;
-    if (dim == 2) return idx64 ? list_dm<2, M64>(prec, a, list, n, s) : list_dm<2, M>(prec, a, list, n, s);
-    return idx64 ? list_dm<3, M64>(prec, a, list, n, s) : list_dm<3, M>(prec, a, list, n, s);
-}
-
-hipError_t launch_double(int dim, int prec, const StepArgs &a, const DoublePlan &d, hipStream_t s)
-{
-    StepArgs first = a, second = a;
-    first.dst = d.scratch;
-    second.src = d.scratch;
-    hipError_t e = launch_step_list(dim, prec, d.idx64, first, d.list[0], d.count[0], s);
-    if (e != hipSuccess) return e;
-    if (dim != 2) return hipErrorInvalidValue;
-    e = dispatch_prec(prec, [&](auto *sp, auto *cp) {
-        using S = std::remove_pointer_t<decltype(sp)>;
-        using C = std::remove_pointer_t<decltype(cp)>;
-        const uint32_t nbulk = d.strips * d.segments, n = d.idx64 ? 0u : d.count[1];
-        hipLaunchKernelGGL((k_double2<S, C>), dim3(nbulk + (n + kDouble2 - 1) / kDouble2), dim3(kDouble2), 0, s,
+        if (d.count[0]) {
+            hipLaunchKernelGGL((k_step_list<S, C>), dim3(nblocks(d.count[0])), dim3(256), 0, s, (const S *)a.src,
+                               (S *)d.scratch, a.geo, a.kp, a.push, d.list[0], d.count[0]);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+        }
+        const uint32_t nbulk = d.strips * d.segments;
+        hipLaunchKernelGGL((k_double2<S, C>), dim3(nbulk + (d.count[1] + kDouble2 - 1) / kDouble2), dim3(kDouble2), 0, s,
                            (const S *)a.src, (S *)a.dst, a.geo, a.kp, d.rows, d.strips, nbulk, a.push,
-                           (const S *)d.scratch, d.list[1], n);
+                           (const S *)d.scratch, d.list[1], d.count[1]);
         return hipGetLastError();
     });
-    if (e != hipSuccess || !d.idx64) return e;
-    return launch_step_list(dim, prec, d.idx64, second, d.list[1], d.count[1], s);
 }
 
 template <int BYTES, class F>
@@ -2049,21 +2023,17 @@ hipError_t launch_batch_multi(int prec, const MultiPlan &m, const void *src, voi
     });
 }
 
-hipError_t launch_zone(int dim, int pass, const StepArgs &a, uint8_t *geo, const uint8_t *in, uint8_t *out,
-                       uint32_t *count, uint32_t *list, int bulk, hipStream_t s)
+hipError_t launch_zone(int pass, const StepArgs &a, uint8_t *geo, const uint8_t *in, uint8_t *out, uint32_t *count,
+                       uint32_t *list, int bulk, hipStream_t s)
 {
     const dim3 grid(nblocks(a.kp.ncell)), block(256);
-    const auto go = [&](auto dtag) {
-        constexpr int D = decltype(dtag)::value;
-        if (pass == 0)
-            hipLaunchKernelGGL((k_zone_special<D>), grid, block, 0, s, geo, out, a.kp);
-        else if (pass == 1)
-            hipLaunchKernelGGL((k_zone_grow<D>), grid, block, 0, s, in, out, a.kp);
-        else
-            hipLaunchKernelGGL((k_zone_list<D>), grid, block, 0, s, in, geo, a.kp, bulk, count, list);
-        return hipGetLastError();
-    };
-    return dim == 2 ? go(std::integral_constant<int, 2>{}) : go(std::integral_constant<int, 3>{});
+    if (pass == 0)
+        hipLaunchKernelGGL(k_zone_special, grid, block, 0, s, geo, out, a.kp);
+    else if (pass == 1)
+        hipLaunchKernelGGL(k_zone_grow, grid, block, 0, s, in, out, a.kp);
+    else
+        hipLaunchKernelGGL(k_zone_list, grid, block, 0, s, in, geo, a.kp, bulk, count, list);
+    return hipGetLastError();
 }
 
 // The bulk of k_double2 in strips of columns and segments of rows: as many
@@ -2072,9 +2042,8 @@ hipError_t launch_zone(int dim, int pass, const StepArgs &a, uint8_t *geo, const
 // per step: FP64 0.243 ms with 768 blocks, 0.245 with 1024, 0.266 with 1536;
 // FP16 0.098 with 1024, 0.082 with 1280, 0.100 with 1536).  A segment costs
 // two more rows, so it has at least 8.
-void plan_double(int dim, int bytes, const KParams &kp, DoublePlan &d)
+void plan_double(int bytes, const KParams &kp, DoublePlan &d)
 {
-    (void)dim;
     const uint32_t fit = bytes == 2 ? 1280 : 768, rows = uint32_t(kp.ny - 3);  // rows 2 .. ny-2
     d.strips = uint32_t((kp.nx + kStripX - 1) / kStripX);                       // columns -1 .. nx-2
     const uint32_t seg = std::max(1u, fit / d.strips);

@@ -116,3 +116,18 @@ def test_single_steps_batch_shapes(single_steps, block, cpt, persist, r_vec):
 
 def test_single_steps_ensemble96(single_steps, r_vec):
     C.test_ensemble96_matches_oracle(r_vec)
+
+
+def test_int64_slot_tables_keep_single_steps(monkeypatch, r_vec):
+    """(Only lattices whose populations 32 bits do not address have them.)"""
+    monkeypatch.setenv("IMEXLB_SLOTS64", "1")
+    for small in (None, "0"):
+        if small is not None:
+            monkeypatch.setenv("IMEXLB_SMALL_CELLS", small)
+        lat, o, _ = P._run_pair("tiny2d", r_vec, 0)
+        assert lat.step_form()["steps_per_pass"] == 1
+        lat.advance(41)
+        o.run(0, 40, 0)
+        P.assert_state_equal(lat, o)
+        lat.close()
+        o.close()
