@@ -1454,7 +1454,7 @@ int imexlb_nn_conv3x3_bf16_join(const uint16_t *low, int CL, const uint16_t *in,
     // (bound by memory) 16 rows of 16-channel chunks, else 8 rows (40 x 128 x
     // 512, 32 -> 32 channels 93 against 100 us, 96 -> 32 245 against 229 us).
     // Below that the chain of chunks is the time: three chunks ahead (a batch
-    // of one on 128 x 512: 118 us for the whole network, 137 with the plain
+    // of one on 128 x 512: 116 us for the whole network, 137 with the plain
     // 4-row tile for the layers of one and two chunks, 223 for all).
     const bool wide = CI % 32 == 0 && CL % 32 == 0;
 #define CONV_BF16(MT, WY, TC) (wide ? k_conv3_bf16<MT, WY, TC, 32> : k_conv3_bf16<MT, WY, TC, 16>)

@@ -228,9 +228,10 @@ int imexlb_step_form(imexlb_ctx *ctx, int32_t out[4]);
 /* ---------------------------------------------------------------------
  * Batched ensemble.  No counterpart in the reference, which runs one
  * lattice per process: ncase independent D2Q9 lattices, each with its own
- * size and parameters, advanced together by one boundary-fill and one step
- * launch per time step (pairs of steps replayed as a HIP graph).  Every case
- * follows the single-lattice semantics above exactly.
+ * size and parameters, advanced together, several steps per launch where every
+ * case suits that, else by one step launch per time step (pairs of steps
+ * replayed as a HIP graph).  Every case follows the single-lattice semantics
+ * above exactly.
  * --------------------------------------------------------------------- */
 typedef struct imexlb_batch imexlb_batch;
 
