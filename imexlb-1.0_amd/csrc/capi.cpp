@@ -558,6 +558,16 @@ static int build_multi(imexlb_ctx *c, const DeviceTables &t)
     HIP_TRY(hipMemcpy(c->multi_table, mark.data(), nw * sizeof(int32_t), hipMemcpyHostToDevice));
     HIP_TRY(plan(c->multi_place));
     HIP_TRY(hipDeviceSynchronize());
+    // A launch of three steps takes as long as three or more single ones where
+    // loading and storing the windows is most of it (single steps' time = 1: FP16
+    // 1.0 M nodes 0.87, 1.5 M 1.08, 5 M 1.06 to 1.9; FP64 1.06 M 0.75, 1.4 M 1.05
+    // to 1.54; FP32 0.6 to 1.0 at every size), and so do short runs of 16-bit
+    // lattices most of whose windows read tables, while their single steps
+    // stay in the caches (5 steps of 43 x 111109 nodes 1.28, 91 x 53761 1.40).
+    if (c->ssz != 4 && c->cells > (int64_t(5) << 18)) c->multi.least = 5;
+    if (c->ssz == 2 && c->cells > (int64_t(4) << 20) && c->cells <= c->small_cells &&
+        5 * int64_t(tables) >= 3 * int64_t(nw))
+        c->multi.from = 3 * m.halo + 1;
     c->multi.table = c->multi_table;
     c->multi.place = c->multi_place;
     c->multi_on = true;
@@ -1021,21 +1031,17 @@ static int run_double_steps(imexlb_ctx *c, int A, int64_t n, int64_t *done)
     return IMEXLB_OK;
 }
 
-// The part of n fused steps from fb[A] that runs several steps per launch,
-// leaving at least one single step.  Every launch makes an odd number of
-// steps, so that the buffers end up as after as many single steps; only the
-// last leaves the boundary copies that single steps read.
+// The part of n fused steps from fb[A] that runs several steps per launch;
+// only the last launch leaves the boundary copies that single steps read.
 static int run_multi_steps(imexlb_ctx *c, int A, int64_t n, int64_t *done)
 {
     *done = 0;
-    if (!c->multi_on || n < 4) return IMEXLB_OK;
+    if (!c->multi_on) return IMEXLB_OK;
     const int K = c->multi.halo;
-    int64_t full = (n - 1) / K;
-    int rest = int((n - 1) % K);
-    if (!(rest & 1)) --rest;
-    if (rest < 3) rest = 0;
-    *done = K * full + rest;
-    if (rest == 0) --full;  // the last launch, with copies
+    const MultiRun run = multi_run(c->multi, n);
+    int64_t full = run.full;
+    *done = run.done;
+    if (run.done == 0) return IMEXLB_OK;
     if (c->graphs && !c->prof) {
         for (int j = 0; j < imexlb_ctx::kGraphSizes; ++j)
             for (; full >= imexlb_ctx::kMulti[j]; full -= imexlb_ctx::kMulti[j]) {
@@ -1048,7 +1054,7 @@ static int run_multi_steps(imexlb_ctx *c, int A, int64_t n, int64_t *done)
             }
     }
     for (; full >= 0; --full, A = 1 - A) {
-        const int steps = full > 0 || rest == 0 ? K : rest;
+        const int steps = full > 0 ? K : run.last;
         StepArgs a = c->args();
         a.src = c->fb[A];
         a.dst = c->fb[1 - A];
@@ -1083,6 +1089,13 @@ static int run_fused_steps(imexlb_ctx *c, int A, int64_t n)
         --n;
     }
     int64_t pairs = n / 2;
+    // the two steps after several per launch as they are: replaying a graph of
+    // two costs more (9.9 and 8.0 us a step of five, 401 x 101 nodes)
+    for (; pairs == 1 && done > 0; --pairs)
+        for (int k = 0; k < 2; ++k, A = 1 - A) {
+            int rc = c->run_step(c->collide_mode(), c->fb[A], c->fb[1 - A], nullptr);
+            if (rc) return rc;
+        }
     for (int j = 0; j < imexlb_ctx::kGraphSizes && pairs > 0; ++j) {
         const int64_t reps = pairs / imexlb_ctx::kGraphPairs[j];
         if (reps <= 0) continue;

@@ -438,6 +438,31 @@ int build_device_tables(const imexlb_ctx *c, DeviceTables &t);
 // itself) and stay the 0 they start with.
 bool body_copies_zero(const DeviceTables &t);
 
+// A run of several steps per launch.
+struct MultiRun {
+    int64_t full = 0;  // launches of m.halo steps before the last one
+    int last = 0;      // steps of the last launch, which leaves the boundary copies (0: no launch at all)
+    int64_t done = 0;  // steps in all
+};
+// n steps as launches of an odd number of steps each, the last one of m.least
+// or more, with at least one single step left: the buffers end up as after as
+// many single steps.
+inline MultiRun multi_run(const MultiPlan &m, int64_t n)
+{
+    MultiRun r;
+    if (n < m.from) return r;
+    r.full = (n - 1) / m.halo;
+    r.last = int((n - 1) % m.halo);
+    if (!(r.last & 1)) --r.last;
+    if (r.last < m.least) r.last = 0;
+    r.done = r.full * m.halo + r.last;
+    if (r.last == 0 && r.full > 0) {
+        r.last = m.halo;
+        --r.full;
+    }
+    return r;
+}
+
 // The boundary fill's slot tables fit int32 entries when every slot and its
 // previous-step encoding (-slot-2) do.
 inline bool fill_fits_32(int64_t nslots) { return nslots < (int64_t(1) << 31) - 2; }

@@ -124,6 +124,7 @@ struct PushTable {
 // at most (odd), and where each cell of a window pulls from.
 struct MultiPlan {
     int nx = 0, ny = 0, wx = 0, wy = 0, halo = 0;
+    int least = 3, from = 4;  // fewest steps of a launch and of a run that are worth it (multi_run)
     const int32_t *table = nullptr;   // a window's table of places, -1: plain
     const uint16_t *place = nullptr;  // the tables
 };

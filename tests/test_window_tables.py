@@ -30,6 +30,26 @@ def test_tables_do_not_overlap(tool, cells):
         assert [int(v) for v in line.split()] == [t * 9 * cells, (t + 1) * 9 * cells - 1], t
 
 
+def test_runs_of_several_steps_per_launch(tmp_path):
+    """Launches of odd numbers of steps, the last of enough, a single step left;
+    no steps at all where the run is too short."""
+    exe = str(tmp_path / "multi_run_check")
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-isystem", "/opt/rocm/include",
+                    "-I", os.path.join(ROOT, "imexlb-1.0_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "sanitize", "multi_run_check.cpp"), "-o", exe,
+                    "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib"], check=True)
+    out = subprocess.run([exe], capture_output=True, text=True, check=True).stdout.splitlines()
+    assert len(out) == 4 * 2 * 2 * 400
+    for line in out:
+        halo, least, first, n, full, last, done = map(int, line.split())
+        assert done == full * halo + last
+        if done == 0:
+            assert last == full == 0 and (n < first or n - 1 < max(least, 3) or (n - 1) < halo), line
+            continue
+        assert n >= first and done <= n - 1 and last % 2 == 1 and (last >= least or last == halo), line
+        assert n - 1 - done < max(least, 3) + 1, line  # nothing left that a launch would have taken
+
+
 def test_kernels_index_through_the_table_base():
     """Both kernels and both allocations take the table's place from there."""
     src = os.path.join(ROOT, "imexlb-1.0_amd", "csrc")
