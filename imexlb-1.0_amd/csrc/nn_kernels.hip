@@ -776,20 +776,45 @@ __device__ __forceinline__ void conv_store(const f32x16 (&acc)[MT], uint4 *sh, c
     }
     __syncthreads();
     uint16_t *const o = static_cast<uint16_t *>(out);
-    for (int e = tid; e < kOut; e += 256) {
-        const int b = e / (TR * TC * 4), p = e / 4 % (TR * TC), g = e % 4;
-        const int y = y0 + p / TC, x = x0 + p % TC, co = cob + 32 * b + 8 * g;
-        if (y >= H || x >= W || co >= CO) continue;
-        const uint4 v = sh[b * (TR * TC * 4) + 4 * p + turn<4>(g, p)];
-        uint16_t *const d = o + ((int64_t(n) * H + y) * W + x) * ostride + ooff + co;
-        if (vec) {
-            *reinterpret_cast<uint4 *>(d) = v;
-        } else {
-            const uint32_t w4[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-                if (co + k < CO) d[k] = uint16_t(w4[k / 2] >> (16 * (k % 2)));
+    if (vec) {
+        for (int e = tid; e < kOut; e += 256) {
+            const int b = e / (TR * TC * 4), p = e / 4 % (TR * TC), g = e % 4;
+            const int y = y0 + p / TC, x = x0 + p % TC, co = cob + 32 * b + 8 * g;
+            if (y >= H || x >= W || co >= CO) continue;
+            *reinterpret_cast<uint4 *>(o + ((int64_t(n) * H + y) * W + x) * ostride + ooff + co) =
+                sh[b * (TR * TC * 4) + 4 * p + turn<4>(g, p)];
         }
+    } else {
+        // Where 16 bytes do not fit: one channel per access, or two where CO and
+        // the output's place are even, consecutive channels in consecutive
+        // lanes.  A lane keeps its channel and its column modulo 8 or 16, so that
+        // the addresses only step.  (8 channels per lane, each stored alone: 4 x 79
+        // x 507, 16 -> 229 channels 91 us, now 37.5; 15 x 97 x 254, 16 -> 58 57 and
+        // 22.6.)
+        const auto narrow = [&](auto access) {
+            using A = decltype(access);
+            constexpr int K = sizeof(A) / 2, L = 32 / K, P = 256 / L;  // lanes per pixel, pixels at a time
+            const int c = tid % L * K, px = tid / L;
+#pragma unroll
+            for (int b = 0; b < WC; ++b) {
+                const int co = cob + 32 * b + c;
+                if (co >= CO) break;
+                const A *const v =
+                    reinterpret_cast<const A *>(sh + (b * (TR * TC * 4) + 4 * px + turn<4>(c / 8, px))) + c % 8 / K;
+                uint16_t *d = o + ((int64_t(n) * H + y0) * W + x0 + px) * ostride + ooff + co;
+                const int rows = min(TR, H - y0);
+                for (int r = 0; r < rows; ++r, d += int64_t(W) * ostride)
+#pragma unroll
+                    for (int i = 0; i < TC / P; ++i)
+                        if (x0 + px + P * i < W)
+                            *reinterpret_cast<A *>(d + int64_t(P * i) * ostride) = v[(r * TC + P * i) * (32 / K)];
+            }
+        };
+        const bool two = CO % 2 == 0 && ostride % 2 == 0 && ooff % 2 == 0 && reinterpret_cast<uintptr_t>(out) % 4 == 0;
+        if (two)
+            narrow(uint32_t{});
+        else
+            narrow(uint16_t{});
     }
     if (!pool) return;
     for (int e = tid; e < kOut / 4; e += 256) {
@@ -1469,9 +1494,12 @@ int imexlb_nn_conv3x3_bf16_join(const uint16_t *low, int CL, const uint16_t *in,
     if (COP % 64 == 0 && count(8, 32, 64) >= 512) return run(CONV_BF16(4, 2, 32), 8, 32, 64);
     if (CL + CI <= 32 && count(16, 32, 32) >= 512) return run(k_conv3_bf16<4, 4, 32, 16>, 16, 32, 32);
     if (count(8, 32, 32) >= 512) return run(CONV_BF16(2, 4, 32), 8, 32, 32);
-    // (one or two chunks in more blocks than CUs: 40 x 64 x 24, 32 -> 16 channels
-    // 11.0 and, plain, 7.1 us; 8 x 128 x 48, 64 -> 32 10.1 and 8.8)
-    if (wide && CL + CI <= 64 && count(4, 32, 32) > 256) return run(CONV_BF16(2, 4, 32), 8, 32, 32);
+    // (more blocks than CUs, of one or two chunks, or of up to eight where 8 rows
+    // cover no more than 4: 40 x 64 x 24, 32 -> 16 channels 11.0 and, plain, 7.1
+    // us; 8 x 128 x 48, 64 -> 32 10.1 and 8.8; 32 x 5 x 41, 96 -> 210 20.2 and 11.6)
+    if (wide && count(4, 32, 32) > 256 &&
+        (CL + CI <= 64 || (CL + CI <= 256 && 2 * count(8, 32, 32) <= count(4, 32, 32))))
+        return run(CONV_BF16(2, 4, 32), 8, 32, 32);
     return run(CONV_BF16_DEEP(32), 4, 32, 32);
 #undef CONV_BF16_DEEP
 #undef CONV_BF16

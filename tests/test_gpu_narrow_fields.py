@@ -72,3 +72,29 @@ def test_bf16_convolution_of_narrow_fields(shape):
     for k in (0, N - 1):
         K._call("conv3x3_bf16", x[k].contiguous(), wp, torch.zeros(co, device="cuda"), one, 1, ci, co, cop, H, W, 0, 0, 1, 1)
         assert torch.equal(one[0], out[k]), k
+
+
+# output channels and place in a wider buffer: 16-byte, 4-byte and 2-byte
+# accesses; tiles of 16 and 32 columns, one and two blocks of channels, the
+# look-ahead form
+@pytest.mark.parametrize("co,extra,off", [(8, 0, 0), (64, 8, 8), (64, 2, 2), (30, 0, 0), (58, 4, 2), (10, 1, 0), (6, 2, 1),
+                                          (33, 0, 0), (31, 1, 1), (229, 0, 0), (12, 3, 3)])
+@pytest.mark.parametrize("shape", [(3, 32, 9, 13), (2, 16, 18, 70), (24, 32, 61, 97), (20, 16, 40, 8)])
+def test_bf16_output_of_any_channel_count(shape, co, extra, off):
+    """The bf16 output is the FP32 output rounded, in its channels only."""
+    import torch
+    N, ci, H, W = shape
+    g = torch.Generator("cuda").manual_seed(19)
+    x = torch.randn(N, H, W, ci, generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn(co, ci, 3, 3, generator=g, device="cuda")
+    b = torch.randn(co, generator=g, device="cuda")
+    cop = 32 * -(-co // 32)
+    wp = torch.empty(ci * 9 * cop, dtype=torch.bfloat16, device="cuda")
+    K._call("pack_weights_bf16", w, wp, ci, co, ci, cop)
+    f32 = torch.empty(N, co, H, W, device="cuda")
+    out = torch.full((N, H, W, co + extra), 7.0, dtype=torch.bfloat16, device="cuda")
+    K._call("conv3x3_bf16", x, wp, b, f32, N, ci, co, cop, H, W, 0, 0, 1, 1)
+    K._call("conv3x3_bf16", x, wp, b, out, N, ci, co, cop, H, W, co + extra, off, 1, 0)
+    assert torch.equal(out[..., off:off + co], f32.permute(0, 2, 3, 1).to(torch.bfloat16))
+    rest = torch.cat([out[..., :off], out[..., off + co:]], 3)
+    assert bool((rest == 7.0).all())
